@@ -512,6 +512,16 @@ extern "C" int igap_gpu_create(const igap_mesh_desc *mesh, const igap_phys_desc 
     M.X = c->d_X;
     gauss4(M.gq, M.gw);
     M.separable = (flags & IGAP_GENERAL_GEOMETRY) ? 0 : separable_patch(c);
+    if (M.separable) {
+        const int64_t nt = (int64_t)TAB_STRIDE * (c->nelem[0] + c->nelem[1] + c->nelem[2]);
+        TRY(dalloc(&c->d_tab, nt));
+        TRY(dalloc(&c->d_tabf, nt));
+        for (int d = 0, first = 0; d < 3; first += c->nelem[d++]) {
+            M.tab[d] = c->d_tab + (int64_t)TAB_STRIDE * first;
+            M.tabf[d] = c->d_tabf + (int64_t)TAB_STRIDE * first;
+        }
+        HIPTRY(launch_sep_tables(M, c->d_tab, c->d_tabf, c->stream));
+    }
 
     // CSR pattern: rows 3*cp + i, row length 3 * prod_d stencil_d
     std::vector<int64_t> rowptr(c->ndof + 1);
@@ -561,7 +571,7 @@ extern "C" int igap_gpu_destroy(igap_gpu_ctx *c)
     if (c->stream) note(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     for (int d = 0; d < 3; d++)
         if (c->d_knot[d]) note(hipFree(c->d_knot[d]), "hipFree");
-    void *bufs[] = {c->d_w, c->d_X, c->d_Uh, c->d_R, c->d_Re, c->d_Ke[0], c->d_Ke[1], c->d_rowptr, c->d_col, c->d_pcol, c->d_val64,
+    void *bufs[] = {c->d_w, c->d_X, c->d_tab, c->d_tabf, c->d_Uh, c->d_R, c->d_Re, c->d_Ke[0], c->d_Ke[1], c->d_rowptr, c->d_col, c->d_pcol, c->d_val64,
                     c->d_val32, c->d_mask, c->d_g, c->d_F, c->d_Hd, c->d_H};
     for (void *b : bufs)
         if (b) note(hipFree(b), "hipFree");

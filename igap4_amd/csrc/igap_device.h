@@ -31,7 +31,14 @@ struct MeshK {
     double par_periodic[9];
     double gq[4], gw[4];   // Gauss-Legendre nodes/weights on [0,1]
     int separable;    // x_d depends on xi_d alone and the weights are equal (k_tangent_sep applies)
+    // separable patches: the 1-D tables of each direction's elements (k_sep_tables),
+    // TAB_STRIDE values per element: [Gauss point][order][function], then the four
+    // point weights; tabf the same in FP32
+    const double *tab[3];
+    const float *tabf[3];
 };
+
+constexpr int TAB_STRIDE = 40;
 
 struct PhysK {
     double c2, c3, c4, e0, e345, le;
@@ -217,29 +224,17 @@ constexpr double IS2 = 0.70710678118654752440;
 constexpr double IS3 = 0.57735026918962576451;
 constexpr double IS6 = 0.40824829046386301637;
 
-__device__ __forceinline__ void phys_state(const double *u, const PhysK &P, State &st)
+// S and N (as in State) at the deformation gradient F
+__device__ __forceinline__ void phys_strain(const double *F, const PhysK &P, double *S, double *N)
 {
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int I = 0; I < 3; I++) {
-            st.F[3 * k + I] = (k == I ? 1.0 : 0.0) + u[10 * k + 1 + I];
-#pragma unroll
-            for (int K = 0; K < 3; K++) st.H[9 * k + 3 * I + K] = u[10 * k + sidx(I, K)];
-        }
-    double E[9], EK[9];
+    double E[9];
 #pragma unroll
     for (int I = 0; I < 3; I++)
 #pragma unroll
         for (int J = 0; J < 3; J++) {
-            double s = st.F[I] * st.F[J] + st.F[3 + I] * st.F[3 + J] + st.F[6 + I] * st.F[6 + J];
+            double s = F[I] * F[J] + F[3 + I] * F[3 + J] + F[6 + I] * F[6 + J];
             E[3 * I + J] = 0.5 * (s - (I == J ? 1.0 : 0.0));
         }
-#pragma unroll
-    for (int I = 0; I < 3; I++)
-#pragma unroll
-        for (int K = 0; K < 3; K++)
-            EK[3 * I + K] = st.F[I] * st.H[3 * I + K] + st.F[3 + I] * st.H[9 + 3 * I + K] + st.F[6 + I] * st.H[18 + 3 * I + K];
     const double v24[3] = {IS3, IS3, IS3};
     const double v25[3] = {IS2, -IS2, 0.0};
     const double v26[3] = {IS6, IS6, -2 * IS6};
@@ -254,15 +249,34 @@ __device__ __forceinline__ void phys_state(const double *u, const PhysK &P, Stat
     double P2626 = 6 * P.c3 * e26 + 2 * P.c2 + 4 * P.c4 * rho2 + 8 * P.c4 * e26 * e26;
 #pragma unroll
     for (int I = 0; I < 3; I++) {
-        st.S[4 * I] = 2 * P.e0 * e24 * v24[I] + P25 * v25[I] + P26 * v26[I];
+        S[4 * I] = 2 * P.e0 * e24 * v24[I] + P25 * v25[I] + P26 * v26[I];
 #pragma unroll
         for (int J = 0; J < 3; J++)
-            st.N[3 * I + J] = 2 * P.e0 * v24[I] * v24[J] + P2525 * v25[I] * v25[J]
+            N[3 * I + J] = 2 * P.e0 * v24[I] * v24[J] + P2525 * v25[I] * v25[J]
                             + P2526 * (v25[I] * v26[J] + v26[I] * v25[J]) + P2626 * v26[I] * v26[J];
     }
-    st.S[1] = st.S[3] = P.e345 * E[1];
-    st.S[2] = st.S[6] = P.e345 * E[2];
-    st.S[5] = st.S[7] = P.e345 * E[5];
+    S[1] = S[3] = P.e345 * E[1];
+    S[2] = S[6] = P.e345 * E[2];
+    S[5] = S[7] = P.e345 * E[5];
+}
+
+__device__ __forceinline__ void phys_state(const double *u, const PhysK &P, State &st)
+{
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int I = 0; I < 3; I++) {
+            st.F[3 * k + I] = (k == I ? 1.0 : 0.0) + u[10 * k + 1 + I];
+#pragma unroll
+            for (int K = 0; K < 3; K++) st.H[9 * k + 3 * I + K] = u[10 * k + sidx(I, K)];
+        }
+    phys_strain(st.F, P, st.S, st.N);
+    double EK[9];
+#pragma unroll
+    for (int I = 0; I < 3; I++)
+#pragma unroll
+        for (int K = 0; K < 3; K++)
+            EK[3 * I + K] = st.F[I] * st.H[3 * I + K] + st.F[3 + I] * st.H[9 + 3 * I + K] + st.F[6 + I] * st.H[18 + 3 * I + K];
     double le2 = P.le * P.le;
 #pragma unroll
     for (int K = 0; K < 3; K++) {
@@ -408,23 +422,16 @@ __device__ __forceinline__ void phys_density_transient(const double *J, const Ph
 // ---------------------------------------------------------------- tangent entries
 // The state as stored in LDS: F[0..8], H[9..35], S[36..44], G[45..53], N[54..62]
 constexpr int ST_F = 0, ST_H = 9, ST_S = 36, ST_G = 45, ST_N = 54, STW = 63;
-// Compact layout (48 values): F[9], the symmetric H_k,IK (= u_k,IK), S and N
-// once per index pair (I <= K, in the slot order of sidx), G[9]
-constexpr int STC_H = 9, STC_S = 27, STC_G = 33, STC_N = 42, STWC = 48;
-template <bool CMP>
-__device__ __forceinline__ int st_h(int k, int I, int K) { return CMP ? STC_H + 6 * k + sidx(I, K) - 4 : ST_H + 9 * k + 3 * I + K; }
-template <bool CMP>
-__device__ __forceinline__ int st_s(int I, int J) { return CMP ? STC_S + sidx(I, J) - 4 : ST_S + 3 * I + J; }
-template <bool CMP>
-__device__ __forceinline__ int st_g(int I, int K) { return CMP ? STC_G + 3 * I + K : ST_G + 3 * I + K; }
-template <bool CMP>
-__device__ __forceinline__ int st_n(int I, int J) { return CMP ? STC_N + sidx(I, J) - 4 : ST_N + 3 * I + J; }
+__device__ __forceinline__ int st_h(int k, int I, int K) { return ST_H + 9 * k + 3 * I + K; }
+__device__ __forceinline__ int st_s(int I, int J) { return ST_S + 3 * I + J; }
+__device__ __forceinline__ int st_g(int I, int K) { return ST_G + 3 * I + K; }
+__device__ __forceinline__ int st_n(int I, int J) { return ST_N + 3 * I + J; }
 
 // One row of the (k,l) block of C at one state, accumulated as row[b - A0] +=
 // s * C[(k,a),(l,b)] for the slots b = A0..9.  The row slot a (1..9) is the
 // lane's; all column slots are unrolled at compile time.  Value slots (a or
-// b = 0) carry no stored-energy term.  CMP: the state in the compact layout.
-template <int A0, bool CMP = false>
+// b = 0) carry no stored-energy term.
+template <int A0>
 __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, int a, int l, double s, double *row)
 {
     const double *F = st + ST_F;
@@ -435,17 +442,17 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
         const int L = a - 1;
         const double Fk0 = F[3 * k], Fk1 = F[3 * k + 1], Fk2 = F[3 * k + 2];
         const double FkL = F[3 * k + L], FlL = F[3 * l + L];
-        const double hk0 = st[st_h<CMP>(k, L, 0)], hk1 = st[st_h<CMP>(k, L, 1)], hk2 = st[st_h<CMP>(k, L, 2)];
+        const double hk0 = st[st_h(k, L, 0)], hk1 = st[st_h(k, L, 1)], hk2 = st[st_h(k, L, 2)];
         const double fdot = Fk0 * Fl0 + Fk1 * Fl1 + Fk2 * Fl2;
         const bool dia = (k == l);
 #pragma unroll
         for (int M = 0; M < 3; M++) {
             const double FkM = (M == 0) ? Fk0 : (M == 1 ? Fk1 : Fk2);
-            double v = st[st_n<CMP>(L, M)] * FkL * Fl[M];
+            double v = st[st_n(L, M)] * FkL * Fl[M];
             v += 0.5 * P.e345 * ((M == L) ? (fdot - FkL * FlL) : FkM * FlL);
-            const double hh = hk0 * st[st_h<CMP>(l, M, 0)] + hk1 * st[st_h<CMP>(l, M, 1)] + hk2 * st[st_h<CMP>(l, M, 2)];
+            const double hh = hk0 * st[st_h(l, M, 0)] + hk1 * st[st_h(l, M, 1)] + hk2 * st[st_h(l, M, 2)];
             v += g2 * ((M == L) ? 2.0 / 3.0 : -1.0 / 3.0) * hh;
-            if (dia) v += st[st_s<CMP>(L, M)];
+            if (dia) v += st[st_s(L, M)];
             row[1 + M - A0] += s * v;
         }
         const double hk[3] = {hk0, hk1, hk2};
@@ -456,8 +463,8 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
             double v = g2 * ((L == I) ? 2.0 / 3.0 : -1.0 / 3.0) * hk[K] * Fl[I];
             if (I != K) v += g2 * ((L == K) ? 2.0 / 3.0 : -1.0 / 3.0) * hk[I] * Fl[K];
             if (dia) {
-                if (L == I) v += st[st_g<CMP>(I, K)];
-                if (I != K && L == K) v += st[st_g<CMP>(K, I)];
+                if (L == I) v += st[st_g(I, K)];
+                if (I != K && L == K) v += st[st_g(K, I)];
             }
             row[4 + pp - A0] += s * v;
         }
@@ -469,11 +476,11 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
         // first-gradient columns: C[(k,IK),(l,M)] = C[(l,M),(k,IK)]
 #pragma unroll
         for (int M = 0; M < 3; M++) {
-            double v = g2 * ((M == I) ? 2.0 / 3.0 : -1.0 / 3.0) * st[st_h<CMP>(l, M, K)] * FkI;
-            if (off) v += g2 * ((M == K) ? 2.0 / 3.0 : -1.0 / 3.0) * st[st_h<CMP>(l, M, I)] * FkK;
+            double v = g2 * ((M == I) ? 2.0 / 3.0 : -1.0 / 3.0) * st[st_h(l, M, K)] * FkI;
+            if (off) v += g2 * ((M == K) ? 2.0 / 3.0 : -1.0 / 3.0) * st[st_h(l, M, I)] * FkK;
             if (dia) {
-                if (M == I) v += st[st_g<CMP>(I, K)];
-                if (off && M == K) v += st[st_g<CMP>(K, I)];
+                if (M == I) v += st[st_g(I, K)];
+                if (off && M == K) v += st[st_g(K, I)];
             }
             row[1 + M - A0] += s * v;
         }
@@ -492,7 +499,7 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
     }
 }
 
-// c_row for the separable kernel (slots 1..9, row[b - 1] = C[(k,a),(l,b)]):
+// c_row for the general geometry's static tangent (slots 1..9, row[b - 1] = C[(k,a),(l,b)]):
 // the same entries with the lane's runtime slot indices turned into one-hot
 // vectors and the 2/3 / -1/3 coefficients into per-lane selects, so that
 // every column is straight-line arithmetic at compile-time register
@@ -500,7 +507,6 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
 // from the 3x3 tensor
 //   T[J'][K''] = F_lJ' (d(K'',K) F_kI c(I,J') + [I != K] d(K'',I) F_kK c(K,J')),
 //   C[(k,IK),(l,JK2)] = g2 (T[J][K2] + [J != K2] T[K2][J]),  c(x,y) = d(x,y) - 1/3.
-template <bool CMP>
 __device__ __forceinline__ void c_row_onehot(const double *st, const PhysK &P, int k, int a, int l, double *row)
 {
     const double g2 = 2 * P.le * P.le;
@@ -516,16 +522,16 @@ __device__ __forceinline__ void c_row_onehot(const double *st, const PhysK &P, i
 #pragma unroll
         for (int m = 0; m < 3; m++) { eL[m] = (m == L) ? 1.0 : 0.0; cL[m] = (m == L) ? C1 : C0; }
         const double FkL = F[3 * k + L], FlL = F[3 * l + L];
-        const double hk[3] = {st[st_h<CMP>(k, L, 0)], st[st_h<CMP>(k, L, 1)], st[st_h<CMP>(k, L, 2)]};
+        const double hk[3] = {st[st_h(k, L, 0)], st[st_h(k, L, 1)], st[st_h(k, L, 2)]};
         const double fdot = Fk[0] * Fl[0] + Fk[1] * Fl[1] + Fk[2] * Fl[2];
         const double e1 = 0.5 * P.e345 * (fdot - FkL * FlL), e2 = 0.5 * P.e345 * FlL;
 #pragma unroll
         for (int M = 0; M < 3; M++) {
-            double v = st[st_n<CMP>(L, M)] * FkL * Fl[M];
+            double v = st[st_n(L, M)] * FkL * Fl[M];
             v += eL[M] * e1 + (1.0 - eL[M]) * (e2 * Fk[M]);
-            const double hh = hk[0] * st[st_h<CMP>(l, M, 0)] + hk[1] * st[st_h<CMP>(l, M, 1)] + hk[2] * st[st_h<CMP>(l, M, 2)];
+            const double hh = hk[0] * st[st_h(l, M, 0)] + hk[1] * st[st_h(l, M, 1)] + hk[2] * st[st_h(l, M, 2)];
             v += g2 * cL[M] * hh;
-            v += dd * st[st_s<CMP>(L, M)];
+            v += dd * st[st_s(L, M)];
             row[M] = v;
         }
 #pragma unroll
@@ -533,10 +539,10 @@ __device__ __forceinline__ void c_row_onehot(const double *st, const PhysK &P, i
             constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
             const int I = PI[pp], K = PK[pp];
             double v = g2 * cL[I] * hk[K] * Fl[I];
-            double gv = eL[I] * st[st_g<CMP>(I, K)];
+            double gv = eL[I] * st[st_g(I, K)];
             if (I != K) {
                 v += g2 * cL[K] * hk[I] * Fl[K];
-                gv += eL[K] * st[st_g<CMP>(K, I)];
+                gv += eL[K] * st[st_g(K, I)];
             }
             row[3 + pp] = v + dd * gv;
         }
@@ -554,11 +560,11 @@ __device__ __forceinline__ void c_row_onehot(const double *st, const PhysK &P, i
             cK[m] = (m == K) ? C1 : C0;
         }
         const double FkI = F[3 * k + I], FkK = F[3 * k + K];
-        const double GIK = st[st_g<CMP>(I, K)], GKI = st[st_g<CMP>(K, I)];
+        const double GIK = st[st_g(I, K)], GKI = st[st_g(K, I)];
 #pragma unroll
         for (int M = 0; M < 3; M++) {
-            double v = g2 * cI[M] * st[st_h<CMP>(l, M, K)] * FkI;
-            v += nIK * (g2 * cK[M] * st[st_h<CMP>(l, M, I)] * FkK);
+            double v = g2 * cI[M] * st[st_h(l, M, K)] * FkI;
+            v += nIK * (g2 * cK[M] * st[st_h(l, M, I)] * FkK);
             v += dd * (eI[M] * GIK + nIK * eK[M] * GKI);
             row[M] = v;
         }
@@ -688,40 +694,27 @@ __device__ __forceinline__ void c_row_mom(const double *ms, const PhysK &P, int 
     }
 }
 
-// Compact moment state (87 values; the separable transient tangent keeps one
-// per Gauss point of the element): F^ (9 + 9), H^ once per symmetric index
-// pair (18 + 18, H_k,IK = u_k,IK), Sb and the three N blocks once per
-// symmetric pair (6 each), Gb (9).  Pair slots follow sidx.
-constexpr int MC_F1 = 0, MC_F2 = 9, MC_H1 = 18, MC_H2 = 36, MC_S = 54, MC_G = 60, MC_N11 = 69, MC_N12 = 75, MC_N22 = 81, MWC = 87;
-
-// c_row_mom (slots 1..9, row[b - 1] = C[(k,a),(l,b)]) from the compact moment
-// state, stored in TS, with c_row_onehot's straight-line columns: the lane's
+// c_row_mom (slots 1..9, row[b - 1] = C[(k,a),(l,b)]) from the moment
+// state, with c_row_onehot's straight-line columns: the lane's
 // slot indices as one-hot vectors, the products of two moment-weighted fields as
 // dot2 pairs, the second-gradient block of a second-gradient row from the
 // 3x3 tensor T[J][K2] = e_K[K2] c(I,J) d1[J] + e_I[K2] c(K,J) d2[J] with
 // d1[J] = (F_kI . F_lJ), d2[J] = [I != K] (F_kK . F_lJ).
-template <typename TS, bool CMP = true>
-__device__ __forceinline__ void c_row_momc_onehot(const TS *ms, const PhysK &P, int k, int a, int l, double *row)
+__device__ __forceinline__ void c_row_mom_onehot(const double *ms, const PhysK &P, int k, int a, int l, double *row)
 {
-    // CMP: the compact layout (MC_*); otherwise the full one (M*) of k_tangent_elem
-    constexpr int OF1 = CMP ? MC_F1 : MF1, OF2 = CMP ? MC_F2 : MF2, OH1 = CMP ? MC_H1 : MH1, OH2 = CMP ? MC_H2 : MH2;
-    constexpr int OS = CMP ? MC_S : MS, OG = CMP ? MC_G : MG;
-    constexpr int ON11 = CMP ? MC_N11 : MN11, ON12 = CMP ? MC_N12 : MN12, ON22 = CMP ? MC_N22 : MN22;
-    auto F1 = [&](int i) { return (double)ms[OF1 + i]; };
-    auto F2 = [&](int i) { return (double)ms[OF2 + i]; };
-    auto hidx = [&](int kk, int I, int K) { return CMP ? 6 * kk + sidx(I, K) - 4 : 9 * kk + 3 * I + K; };
-    auto H1 = [&](int kk, int I, int K) { return (double)ms[OH1 + hidx(kk, I, K)]; };
-    auto H2 = [&](int kk, int I, int K) { return (double)ms[OH2 + hidx(kk, I, K)]; };
-    auto sym = [&](int base, int I, int K) { return (double)ms[base + (CMP ? sidx(I, K) - 4 : 3 * I + K)]; };
+    const double *F1 = ms + MF1, *F2 = ms + MF2;
+    auto H1 = [&](int kk, int I, int K) { return ms[MH1 + 9 * kk + 3 * I + K]; };
+    auto H2 = [&](int kk, int I, int K) { return ms[MH2 + 9 * kk + 3 * I + K]; };
+    auto sym = [&](int base, int I, int K) { return ms[base + 3 * I + K]; };
     const double g2 = 2 * P.le * P.le;
     const double dd = (k == l) ? 1.0 : 0.0;
     double Fl1[3], Fl2[3], Fk1[3], Fk2[3];
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-        Fl1[m] = F1(3 * l + m);
-        Fl2[m] = F2(3 * l + m);
-        Fk1[m] = F1(3 * k + m);
-        Fk2[m] = F2(3 * k + m);
+        Fl1[m] = F1[3 * l + m];
+        Fl2[m] = F2[3 * l + m];
+        Fk1[m] = F1[3 * k + m];
+        Fk2[m] = F2[3 * k + m];
     }
     constexpr double C1 = 2.0 / 3.0, C0 = -1.0 / 3.0;
     if (a <= 3) {
@@ -729,7 +722,7 @@ __device__ __forceinline__ void c_row_momc_onehot(const TS *ms, const PhysK &P, 
         double eL[3], cL[3];
 #pragma unroll
         for (int m = 0; m < 3; m++) { eL[m] = (m == L) ? 1.0 : 0.0; cL[m] = (m == L) ? C1 : C0; }
-        const double FkL1 = F1(3 * k + L), FkL2 = F2(3 * k + L), FlL1 = F1(3 * l + L), FlL2 = F2(3 * l + L);
+        const double FkL1 = F1[3 * k + L], FkL2 = F2[3 * k + L], FlL1 = F1[3 * l + L], FlL2 = F2[3 * l + L];
         double hk1[3], hk2[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) { hk1[c] = H1(k, L, c); hk2[c] = H2(k, L, c); }
@@ -737,15 +730,15 @@ __device__ __forceinline__ void c_row_momc_onehot(const TS *ms, const PhysK &P, 
         const double eLL = full - dot2(FkL1, FkL2, FlL1, FlL2);
 #pragma unroll
         for (int M = 0; M < 3; M++) {
-            double v = sym(ON11, L, M) * FkL1 * Fl1[M] + sym(ON12, L, M) * (FkL1 * Fl2[M] + FkL2 * Fl1[M])
-                     + sym(ON22, L, M) * FkL2 * Fl2[M];
+            double v = sym(MN11, L, M) * FkL1 * Fl1[M] + sym(MN12, L, M) * (FkL1 * Fl2[M] + FkL2 * Fl1[M])
+                     + sym(MN22, L, M) * FkL2 * Fl2[M];
             const double e = eL[M] * eLL + (1.0 - eL[M]) * dot2(Fk1[M], Fk2[M], FlL1, FlL2);
             v += 0.5 * P.e345 * e;
             double hh = 0.0;
 #pragma unroll
             for (int c = 0; c < 3; c++) hh += dot2(hk1[c], hk2[c], H1(l, M, c), H2(l, M, c));
             v += g2 * cL[M] * hh;
-            v += dd * sym(OS, L, M);
+            v += dd * sym(MS, L, M);
             row[M] = v;
         }
 #pragma unroll
@@ -753,10 +746,10 @@ __device__ __forceinline__ void c_row_momc_onehot(const TS *ms, const PhysK &P, 
             constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
             const int I = PI[pp], K = PK[pp];
             double v = g2 * cL[I] * dot2(hk1[K], hk2[K], Fl1[I], Fl2[I]);
-            double gv = eL[I] * (double)ms[OG + 3 * I + K];
+            double gv = eL[I] * ms[MG + 3 * I + K];
             if (I != K) {
                 v += g2 * cL[K] * dot2(hk1[I], hk2[I], Fl1[K], Fl2[K]);
-                gv += eL[K] * (double)ms[OG + 3 * K + I];
+                gv += eL[K] * ms[MG + 3 * K + I];
             }
             row[3 + pp] = v + dd * gv;
         }
@@ -773,8 +766,8 @@ __device__ __forceinline__ void c_row_momc_onehot(const TS *ms, const PhysK &P, 
             cI[m] = (m == I) ? C1 : C0;
             cK[m] = (m == K) ? C1 : C0;
         }
-        const double FkI1 = F1(3 * k + I), FkI2 = F2(3 * k + I), FkK1 = F1(3 * k + K), FkK2 = F2(3 * k + K);
-        const double GIK = (double)ms[OG + 3 * I + K], GKI = (double)ms[OG + 3 * K + I];
+        const double FkI1 = F1[3 * k + I], FkI2 = F2[3 * k + I], FkK1 = F1[3 * k + K], FkK2 = F2[3 * k + K];
+        const double GIK = ms[MG + 3 * I + K], GKI = ms[MG + 3 * K + I];
 #pragma unroll
         for (int M = 0; M < 3; M++) {
             double v = g2 * cI[M] * dot2(H1(l, M, K), H2(l, M, K), FkI1, FkI2);

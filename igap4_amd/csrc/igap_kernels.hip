@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include "igap_device.h"
+#include "igap_sep_pipeline.h"
 
 namespace igap {
 
@@ -925,7 +926,7 @@ __global__ __launch_bounds__(256, 2) void k_tangent_elem(MeshK M, PhysK P, const
                 const int q = q0 + ql;
                 const double wgt = sGeo[q * GEOK];
                 double row[NA];
-                c_row_onehot<false>(sSt + q * STW, P, kBlkI[p], ar + A0, kBlkJ[p], row);
+                c_row_onehot(sSt + q * STW, P, kBlkI[p], ar + A0, kBlkJ[p], row);
                 T *D = sD[ql] + p * NN + ar * RS;
 #pragma unroll
                 for (int bb = 0; bb < NA; bb++) D[bb] = (T)(wgt * row[bb]);
@@ -961,7 +962,7 @@ __global__ __launch_bounds__(256, 2) void k_tangent_elem(MeshK M, PhysK P, const
                 for (int bb = 1; bb < NA; bb++) row[bb] = 0.0;
                 if (k == l) row[0] = P.cii / (2. * P.dt) + P.rho / (P.dt * P.dt);
             } else {
-                c_row_momc_onehot<double, false>(sSt + ql * MW, P, k, ar, l, row + 1);
+                c_row_mom_onehot(sSt + ql * MW, P, k, ar, l, row + 1);
             }
             T *D = sD[ql] + p * NN + ar * RS;
 #pragma unroll
@@ -1088,26 +1089,76 @@ __global__ __launch_bounds__(256, 2) void k_tangent_elem(MeshK M, PhysK P, const
 //   K^ij[b][c] = sum_q sum_{a,a'} R_q[a][b] D_q[(i,a),(j,a')] R_q[a'][c],
 // then factors direction by direction (sum factorisation), with s = (dx, dy)
 // the x-y part of a jet slot:
-//   F_q[a][(s',cz)]   = sum_dz' D_q[a][(s',dz')] Pz[qz][dz'][cz]         per point, a lane per row a
-//   E1[(s,bz),(s',cz)] = sum_qz sum_dz Pz[qz][dz][bz] F_q[(s,dz)][(s',cz)]  per (qx, qy) pencil
+//   E1[(s,bz),(s',cz)] = sum_qz sum_{dz,dz'} Pz[qz][dz][bz] D_q[(s,dz)][(s',dz')] Pz[qz][dz'][cz]  per (qx, qy) pencil
 //   E2[(dx,by,bz),(dx',cy,cz)] += sum_{dy,dy'} Py[qy][dy][by] Py[qy][dy'][cy] E1[((dx,dy),bz),((dx',dy'),cz)]
 //   K[(bx,by,bz),(cx,cy,cz)]   += sum_{dx,dx'} Px[qx][dx][bx] Px[qx][dx'][cx] E2   after the fourth qy
 // ~0.7 MFLOP per element on the vector ALUs instead of the 27x27 product per
 // point and jet slot.  The displacement jets come from the same tables by sum
-// factorisation (no quotient or chain rule left to apply), the pointwise
-// tangent rows D_q = w_q C_q are those of k_tangent_elem, and the element
-// matrix is written in its layout (row 3b+i, column 3c+j).
+// factorisation (no quotient or chain rule left to apply); the element matrix
+// is written in k_tangent_elem's layout (row 3b+i, column 3c+j).
 // ============================================================================
-// Per-element set-up on a separable patch (256 threads, no barrier): the 27
-// control displacements -> sU[27][3]; per direction d and 1-D Gauss point q
-// the 1-D rational basis rho_i = N_i / S (S = sum_i N_i) and its derivatives
-// made physical with g = dx_d/dxi_d and g' = d2x_d/dxi_d^2 from the element's
-// three control coordinates along d (x_d depends on the index along d alone):
-//   sPd[d][q][0][i] = rho_i,  [1][i] = rho_i' / g,  [2][i] = (rho_i'' - (g'/g) rho_i') / g^2
-// (the same in the precision T -> sP when given), and g -> sG[d][q].
-template <typename T, int NH = 1>
+// The 1-D tables of a separable patch, one block per element of a direction
+// (blockIdx.y = direction), lane q < 4 its 1-D Gauss point: the rational basis
+// rho_i = N_i / S (S = sum_i N_i) and its derivatives made physical with
+// g = dx_d/dxi_d and g' = d2x_d/dxi_d^2 from the element's three control
+// coordinates along d (x_d depends on the index along d alone):
+//   [q][0][i] = rho_i,  [q][1][i] = rho_i' / g,  [q][2][i] = (rho_i'' - (g'/g) rho_i') / g^2,
+// then the point weight gw_q dX g.  Built once per context, as the knots and
+// control points are: evaluating them in every element's workgroup is a chain of
+// dependent loads and divisions (k_residual_sep at 128x32x32 0.99 -> 0.84 ms).
+__global__ __launch_bounds__(64) void k_sep_tables(MeshK M, double *__restrict__ tab, float *__restrict__ tabf)
+{
+    const int d = blockIdx.y, e = blockIdx.x, q = threadIdx.x;
+    if (e >= M.nelem[d] || q >= 4) return;
+    const int first = (d > 0 ? M.nelem[0] : 0) + (d > 1 ? M.nelem[1] : 0);
+    const double *kV = M.knot[d] + e;
+    const double c = M.gq[q];
+    const double x = (-c + 1.0) * kV[2] + c * kV[3];
+    double t[9];
+    bspline1d(kV, x, t, t + 3, t + 6);
+    // the rational basis of equal weights is N_b / W with W = S_x S_y S_z,
+    // S = sum_i N_i (1 up to the MTOL guard of the B-spline formulas):
+    // a product of the 1-D quotients rho_i = N_i / S, whose derivatives
+    // follow from the 1-D quotient rule
+    const double S0 = t[0] + t[1] + t[2], S1 = t[3] + t[4] + t[5], S2 = t[6] + t[7] + t[8];
+    const double iS = 1.0 / S0;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        t[b] *= iS;
+        t[3 + b] = (t[3 + b] - t[b] * S1) * iS;
+        t[6 + b] = (t[6 + b] - 2.0 * t[3 + b] * S1 - t[b] * S2) * iS;
+    }
+    double xc[3];
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        const int64_t id = d == 0 ? (int64_t)M.na[1] * M.na[2] * (e + b) : d == 1 ? (int64_t)M.na[2] * (e + b) : e + b;
+        xc[b] = M.X[3 * id + d];
+    }
+    const double g = t[3] * xc[0] + t[4] * xc[1] + t[5] * xc[2];
+    const double gp = t[6] * xc[0] + t[7] * xc[1] + t[8] * xc[2];
+    const double ig = 1.0 / g, r = gp * ig;
+    double *o = tab + (int64_t)(first + e) * TAB_STRIDE;
+    float *of = tabf + (int64_t)(first + e) * TAB_STRIDE;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        const double v[3] = {t[b], t[3 + b] * ig, (t[6 + b] - r * t[3 + b]) * (ig * ig)};
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            o[9 * q + 3 * a + b] = v[a];
+            of[9 * q + 3 * a + b] = (float)v[a];
+        }
+    }
+    const double w = M.gw[q] * (kV[3] - kV[2]) * g;
+    o[36 + q] = w;
+    of[36 + q] = (float)w;
+}
+
+// Per-element set-up on a separable patch (at least 256 threads, no barrier):
+// the 27 control displacements -> sU[27][3], the tables of the element's three
+// 1-D elements -> sPd[d][q][order][i] and their point weights -> sW[d][q].
+template <int NH = 1>
 __device__ __forceinline__ void sep_element(const MeshK &M, const double *__restrict__ Uh, const int *ed, double *sU,
-                                            double (*sPd)[4][3][3], T (*sP)[4][3][3], double (*sG)[4], int64_t ndof = 0,
+                                            double (*sPd)[4][3][3], double (*sW)[4], int64_t ndof = 0,
                                             double *sUd = nullptr, double *sV = nullptr, double cv1 = 0.0, double cv2 = 0.0)
 {
     const int tid = threadIdx.x;
@@ -1131,102 +1182,58 @@ __device__ __forceinline__ void sep_element(const MeshK &M, const double *__rest
                 if (sV) sV[3 * tid + k] = cv1 * (u0 - u2) + cv2 * (u0 + u2 - 2 * u1);
             }
         }
-    } else if (tid >= 64 && tid < 64 + 12) {
-        const int d = (tid - 64) >> 2, q = (tid - 64) & 3;
-        const double *kV = M.knot[d] + ed[d];
-        const double c = M.gq[q];
-        const double x = (-c + 1.0) * kV[2] + c * kV[3];
-        double t[9];
-        bspline1d(kV, x, t, t + 3, t + 6);
-        // the rational basis of equal weights is N_b / W with W = S_x S_y S_z,
-        // S = sum_i N_i (1 up to the MTOL guard of the B-spline formulas):
-        // a product of the 1-D quotients rho_i = N_i / S, whose derivatives
-        // follow from the 1-D quotient rule
-        const double S0 = t[0] + t[1] + t[2], S1 = t[3] + t[4] + t[5], S2 = t[6] + t[7] + t[8];
-        const double iS = 1.0 / S0;
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            t[b] *= iS;
-            t[3 + b] = (t[3 + b] - t[b] * S1) * iS;
-            t[6 + b] = (t[6 + b] - 2.0 * t[3 + b] * S1 - t[b] * S2) * iS;
-        }
-        double xc[3];
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            const int ax = ed[0] + (d == 0 ? b : 0), ay = ed[1] + (d == 1 ? b : 0), az = ed[2] + (d == 2 ? b : 0);
-            xc[b] = M.X[3 * (((int64_t)M.na[1] * M.na[2]) * ax + (int64_t)M.na[2] * ay + az) + d];
-        }
-        const double g = t[3] * xc[0] + t[4] * xc[1] + t[5] * xc[2];
-        const double gp = t[6] * xc[0] + t[7] * xc[1] + t[8] * xc[2];
-        const double ig = 1.0 / g, r = gp * ig;
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            const double p1 = t[3 + b] * ig, p2 = (t[6 + b] - r * t[3 + b]) * (ig * ig);
-            sPd[d][q][0][b] = t[b];
-            sPd[d][q][1][b] = p1;
-            sPd[d][q][2][b] = p2;
-            if (sP) {
-                sP[d][q][0][b] = (T)t[b];
-                sP[d][q][1][b] = (T)p1;
-                sP[d][q][2][b] = (T)p2;
-            }
-        }
-        sG[d][q] = g;
+    } else if (tid >= 64 && tid < 64 + 3 * TAB_STRIDE) {
+        const int d = (tid - 64) / TAB_STRIDE, i = (tid - 64) - TAB_STRIDE * d;
+        const double v = M.tab[d][(int64_t)ed[d] * TAB_STRIDE + i];
+        if (i < 36) (&sPd[d][0][0][0])[i] = v;
+        else sW[d][i - 36] = v;
     }
 }
 
 // Physical displacement jets at the 64 Gauss points of a separable element by
 // sum factorisation over the physical tables (z, y, then x; sWork holds 1188
-// doubles), after sep_element and a barrier.  Thread 4q + 1 + k returns in J
-// the jet of component k at point q (par_periodic's macro-field added unless
-// macro is false), thread 4q zeros.
+// doubles), after sep_element and a barrier; at least 192 threads, all of which
+// call it.  Lane q of wave k < 3 returns in J the jet of component k at point q
+// (par_periodic's macro-field added unless macro is false).  The passes are
+// short and serial, so each takes as many threads as it has independent groups
+// of outputs (108, 144 and 192).
 __device__ __forceinline__ void sep_fields(const MeshK &M, const int *ed, const double *sU, const double (*sPd)[4][3][3],
                                            double *sWork, double *J, bool macro = true)
 {
     const int tid = threadIdx.x;
     double *sA = sWork, *sB = sA + 3 * 108;
     // z: sA[k][bx*3+by][qz][dz] = sum_bz U_k(b) Pz[qz][dz][bz]
-    if (tid < 27) {
-        const int k = tid / 9, bxy = tid - 9 * k;
+    if (tid < 108) {
+        const int qz = tid & 3, g = tid >> 2, k = g / 9, bxy = g - 9 * k;
         const double c0 = sU[3 * (3 * bxy) + k], c1 = sU[3 * (3 * bxy + 1) + k], c2 = sU[3 * (3 * bxy + 2) + k];
-        double *o = sA + 108 * k + 12 * bxy;
+        double *o = sA + 108 * k + 12 * bxy + 3 * qz;
 #pragma unroll
-        for (int qz = 0; qz < 4; qz++)
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) {
-                const double *tz = &sPd[2][qz][dz][0];
-                o[3 * qz + dz] = c0 * tz[0] + c1 * tz[1] + c2 * tz[2];
-            }
+        for (int dz = 0; dz < 3; dz++) {
+            const double *tz = &sPd[2][qz][dz][0];
+            o[dz] = c0 * tz[0] + c1 * tz[1] + c2 * tz[2];
+        }
     }
     __syncthreads();
     // y: sB[k][bx][qy][qz][s6] = sum_by sA[k][bx*3+by][qz][dz(s6)] Py[qy][dy(s6)][by],
     //    s6 = (dy, dz) in the order (0,0) (1,0) (0,1) (2,0) (1,1) (0,2)
-    if (tid < 36) {
-        const int k = tid / 12, r = tid - 12 * k, bx = r >> 2, qz = r & 3;
+    if (tid < 144) {
+        const int qz = tid & 3, qy = (tid >> 2) & 3, g = tid >> 4, k = g / 3, bx = g - 3 * k;
         const double *a = sA + 108 * k + 36 * bx + 3 * qz;   // a[12 by + dz]
-        double av[3][3];
+        double *o = sB + 288 * k + 96 * bx + 24 * qy + 6 * qz;
 #pragma unroll
-        for (int by = 0; by < 3; by++)
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) av[by][dz] = a[12 * by + dz];
-        double *o = sB + 288 * k + 96 * bx + 6 * qz;
-#pragma unroll
-        for (int qy = 0; qy < 4; qy++)
-#pragma unroll
-            for (int s6 = 0; s6 < 6; s6++) {
-                const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
-                const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
-                const double *ty = &sPd[1][qy][dy][0];
-                o[24 * qy + s6] = av[0][dz] * ty[0] + av[1][dz] * ty[1] + av[2][dz] * ty[2];
-            }
+        for (int s6 = 0; s6 < 6; s6++) {
+            const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
+            const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
+            const double *ty = &sPd[1][qy][dy][0];
+            o[s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
+        }
     }
     __syncthreads();
     // x
-    const int q = tid >> 2, part = tid & 3;
-    const int qd[3] = {q >> 4, (q >> 2) & 3, q & 3};
-    if (part > 0) {
-        const int k = part - 1;
-        sf_jet(sB + 288 * k + (4 * qd[1] + qd[2]) * 6, &sPd[0][qd[0]][0][0], J);
+    if (tid < 192) {
+        const int q = tid & 63, k = tid >> 6;
+        const int qd[3] = {q >> 4, (q >> 2) & 3, q & 3};
+        sf_jet(sB + 288 * k + (q & 15) * 6, &sPd[0][qd[0]][0][0], J);
         double xq[3];
 #pragma unroll
         for (int d = 0; d < 3; d++) {
@@ -1235,392 +1242,209 @@ __device__ __forceinline__ void sep_fields(const MeshK &M, const int *ed, const 
             xq[d] = (-c + 1.0) * kV[2] + c * kV[3];
         }
         if (macro) add_periodic1(M, xq, k, J);
-    } else {
-#pragma unroll
-        for (int a = 0; a < 10; a++) J[a] = 0.0;
     }
 }
 
 // Gauss weight x span lengths x det G at point q of a separable element
-__device__ __forceinline__ double sep_weight(const MeshK &M, const int *ed, int q, const double (*sG)[4])
+__device__ __forceinline__ double sep_weight(int q, const double (*sW)[4]) { return sW[0][q >> 4] * sW[1][(q >> 2) & 3] * sW[2][q & 3]; }
+
+// Strain-measure states of the 64 points for StaticIn, from the jets of
+// sep_fields (lane q of wave k < 3 holds component k; 256 threads take part):
+// F and H as they come; then wave K < 3 takes column K of the strain gradients
+// and wave 3 the strains.  Ends with a block barrier.
+__device__ __forceinline__ void sep_states(const PhysK &P, const double *J, const double (*sW)[4], double *sSt)
 {
-    const int qd[3] = {q >> 4, (q >> 2) & 3, q & 3};
-    double dX[3];
+    constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+    const int tid = threadIdx.x, q = tid & 63, part = tid >> 6;
+    double *sp = sSt + q * SST_W;
+    if (tid < 192) {
 #pragma unroll
-    for (int d = 0; d < 3; d++) dX[d] = M.knot[d][ed[d] + 3] - M.knot[d][ed[d] + 2];
-    return M.gw[qd[0]] * M.gw[qd[1]] * M.gw[qd[2]] * dX[0] * dX[1] * dX[2] * (sG[0][qd[0]] * sG[1][qd[1]] * sG[2][qd[2]]);
-}
-
-// Row stride of the pencil's F buffer (18 columns): 19, so that the lanes of a
-// row store, each writing its own row, spread over the LDS banks
-constexpr int SEP_FS = 19;
-// Block stride of the F buffer (9 rows per block): 178, 18 modulo the 32 LDS
-// bank pairs, so that the z pass's lanes (18 columns of each of four blocks)
-// and the rows' stores put at most two (z pass) or two to three (stores)
-// lanes on a bank pair; 171 = 9 x 19 gives three
-constexpr int SEP_FB = 178;
-// E1 of the pencil in LDS as [block p][bz][cz][s][s'] (s, s' the x-y parts):
-// a y-pass thread's 36 values (its bz, cz) contiguous, read two at a time.
-// Strides (even: 16-byte aligned pairs): SEP_EC per (bz, cz), SEP_EB per block.
-constexpr int SEP_EC = 38;
-constexpr int SEP_EB = 342;
-
-// jet slot a = 1..9 of the pointwise rows -> order in z, x-y part s = (dx, dy)
-constexpr int SEP_DZ[10] = {0, 0, 0, 1, 0, 0, 1, 0, 1, 2};
-constexpr int SEP_XY[10] = {0, 1, 2, 0, 3, 4, 1, 5, 2, 0};
-
-// z pass of one E1 column (block p, column (s', cz)), task zt < 108 of the
-// pencil: E1[p][(s,bz)][(s',cz)] = sum_qz sum_{a: s(a) = s} Pz[qz][dz(a)][bz]
-// F_qz[p][a][(s',cz)].  HALVES: only the x-y parts s of half h ({0, 1, 3}:
-// five jet slots; {2, 4, 5}: four; h uniform over the wave); otherwise all
-// six.  Every entry takes its terms in the same order either way.
-template <typename T, bool HALVES>
-__device__ __forceinline__ void sep_zcol(const T *sF, const T (*sP)[4][3][3], T *sE, int zt, int h)
-{
-    constexpr int NA = 9;
-    constexpr int ZH[6] = {0, 0, 1, 0, 1, 1};              // half of s
-    constexpr int ZS[6] = {0, 1, 0, 2, 1, 2};              // place of s in its half
-    constexpr int ZI[2][3] = {{0, 1, 3}, {2, 4, 5}};       // s at each place
-    constexpr int NS = HALVES ? 3 : 6;
-    const int zp = zt / 18, zr = zt - 18 * zp;
-    T e1[3 * NS];   // [s][bz]
+        for (int i = 0; i < 3; i++) sp[10 * part + i] = J[1 + i] + (part == i ? 1.0 : 0.0);
 #pragma unroll
-    for (int i = 0; i < 3 * NS; i++) e1[i] = (T)0;
+        for (int t = 0; t < 6; t++) sp[10 * part + 4 + t] = J[4 + t];
+    }
+    __syncthreads();
+    if (tid < 256) {
+        double F[9];
 #pragma unroll
-    for (int qz = 0; qz < 4; qz++) {
-        const T *Fp = sF + (qz * 6 + zp) * SEP_FB + zr;
-        const T *pz = &sP[2][qz][0][0];
-        if (!HALVES) {
+        for (int i = 0; i < 9; i++) F[i] = sp[10 * (i / 3) + i % 3];
+        const double w = sep_weight(q, sW);
+        if (part < 3) {
+            // G_IK = 2 le^2 (E_II,K - their mean), column K = part
+            const int h[3] = {part, part == 0 ? 1 : part + 2, part == 0 ? 2 : part + 3};   // slot of (I, K)
+            double EK[3];
 #pragma unroll
-            for (int bb = 0; bb < NA; bb++) {
-                const int a = bb + 1;
-                const T fv = Fp[SEP_FS * bb];
+            for (int I = 0; I < 3; I++) EK[I] = F[I] * sp[4 + h[I]] + F[3 + I] * sp[14 + h[I]] + F[6 + I] * sp[24 + h[I]];
+            const double tr = (EK[0] + EK[1] + EK[2]) / 3.0, g = w * 2 * P.le * P.le;
 #pragma unroll
-                for (int bz = 0; bz < 3; bz++) e1[3 * SEP_XY[a] + bz] += pz[3 * SEP_DZ[a] + bz] * fv;
-            }
-        } else if (h == 0) {
-#pragma unroll
-            for (int bb = 0; bb < NA; bb++) {
-                const int a = bb + 1;
-                if (ZH[SEP_XY[a]] != 0) continue;
-                const T fv = Fp[SEP_FS * bb];
-#pragma unroll
-                for (int bz = 0; bz < 3; bz++) e1[3 * ZS[SEP_XY[a]] + bz] += pz[3 * SEP_DZ[a] + bz] * fv;
-            }
+            for (int I = 0; I < 3; I++) sp[SST_G + 3 * I + part] = g * (EK[I] - tr);
         } else {
+            double S[9], N[9];
+            phys_strain(F, P, S, N);
 #pragma unroll
-            for (int bb = 0; bb < NA; bb++) {
-                const int a = bb + 1;
-                if (ZH[SEP_XY[a]] != 1) continue;
-                const T fv = Fp[SEP_FS * bb];
+            for (int I = 0; I < 3; I++)
 #pragma unroll
-                for (int bz = 0; bz < 3; bz++) e1[3 * ZS[SEP_XY[a]] + bz] += pz[3 * SEP_DZ[a] + bz] * fv;
-            }
+                for (int K = I; K < 3; K++) {
+                    sp[SST_S + SY[I][K]] = w * S[3 * I + K];
+                    sp[SST_N + SY[I][K]] = w * N[3 * I + K];
+                }
+            sp[SST_WGT] = w;
         }
     }
-    const int sp = zr / 3, cz = zr - 3 * sp;   // column (s', cz)
-    T *o = sE + zp * SEP_EB + cz * SEP_EC + sp;
-#pragma unroll
-    for (int i = 0; i < 3 * NS; i++) o[(i % 3) * 3 * SEP_EC + 6 * (HALVES ? ZI[h][i / 3] : i / 3)] = e1[i];
+    __syncthreads();
 }
 
-// The pencil loop of the separable tangents, after stage A and a barrier
-// (256 threads).  rows(q, p, ar, row) gives row[b - 1] = C_q[(k, ar + 1),
-// (l, b)], b = 1..9, of block p = (k, l) at Gauss point q (unweighted; row
-// arrives zeroed); sWgt holds the point weights, sF and sE the F and E1
-// buffers.  The z pass runs on 108 threads (block p, column (s', cz) of E1;
-// FP64: 216, a column per half of the x-y parts), the y/x pass on 162
-// (block p, bz, cz, by: E2[dx][dx'][cy], K[bx][cx][cy]), all
-// numbered from the rotated thread index rt so that the workgroups sharing a
-// CU put them on different SIMDs.  The y pass of pencil c runs beside the
-// pointwise stage of pencil c + 1 (F and E1 have buffers of their own), so a
-// pencil takes two barriers.  Returns in K the 27 entries [bx][cx][cy] of
-// thread rt < 162.
-template <typename T, class Rows>
-__device__ __forceinline__ void sep_pencils(int rt, const T (*sP)[4][3][3], const double *sWgt, T *sF, T *sE, Rows rows, T *K)
-{
-    constexpr int NA = 9;    // jet slots 1..9 (no value slot in the pointwise rows)
-    constexpr int FR = 18;   // (s', cz) columns of F and E1
-    const int yp = rt / 27, yu = rt - 27 * yp;
-    const int ybz = yu / 9, ycz = (yu / 3) % 3, yby = yu % 3;
-    constexpr int XYX[6] = {0, 1, 0, 2, 1, 0}, XYY[6] = {0, 0, 1, 0, 1, 2};
-    T E2[27];   // [dx][dx'][cy]
-#pragma unroll
-    for (int i = 0; i < 27; i++) { E2[i] = (T)0; K[i] = (T)0; }
-
-    for (int chunk = 0; chunk <= 16; chunk++) {
-        if (chunk > 0 && rt < 162) {
-            // ---- y pass of the previous pencil, x pass after a qx's fourth qy
-            const int pc = chunk - 1, qx = pc >> 2, qy = pc & 3;
-            typedef T pair_t __attribute__((ext_vector_type(2)));
-            const pair_t *E = reinterpret_cast<const pair_t *>(sE + yp * SEP_EB + (3 * ybz + ycz) * SEP_EC);   // [s1][s2]
-            T pyb[3], pyc[9];
-#pragma unroll
-            for (int d = 0; d < 3; d++) pyb[d] = sP[1][qy][d][yby];
-#pragma unroll
-            for (int i = 0; i < 9; i++) pyc[i] = sP[1][qy][i / 3][i % 3];   // [dy'][cy]
-#pragma unroll
-            for (int s1 = 0; s1 < 6; s1++) {
-                T ev[6];
-#pragma unroll
-                for (int v = 0; v < 3; v++) {
-                    const pair_t x = E[3 * s1 + v];
-                    ev[2 * v] = x[0];
-                    ev[2 * v + 1] = x[1];
-                }
-#pragma unroll
-                for (int s2 = 0; s2 < 6; s2++) {
-                    const T t1 = pyb[XYY[s1]] * ev[s2];
-#pragma unroll
-                    for (int cy = 0; cy < 3; cy++) E2[(3 * XYX[s1] + XYX[s2]) * 3 + cy] += t1 * pyc[3 * XYY[s2] + cy];
-                }
-            }
-            if (qy == 3) {
-                T px[9], G[27];   // px[dx][b]; G[dx][cx][cy]
-#pragma unroll
-                for (int i = 0; i < 9; i++) px[i] = sP[0][qx][i / 3][i % 3];
-#pragma unroll
-                for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-                    for (int cx = 0; cx < 3; cx++)
-#pragma unroll
-                        for (int cy = 0; cy < 3; cy++)
-                            G[(3 * dx + cx) * 3 + cy] = px[cx] * E2[(3 * dx) * 3 + cy] + px[3 + cx] * E2[(3 * dx + 1) * 3 + cy]
-                                                      + px[6 + cx] * E2[(3 * dx + 2) * 3 + cy];
-#pragma unroll
-                for (int bx = 0; bx < 3; bx++)
-#pragma unroll
-                    for (int cx = 0; cx < 3; cx++)
-#pragma unroll
-                        for (int cy = 0; cy < 3; cy++)
-                            K[(3 * bx + cx) * 3 + cy] += px[bx] * G[cx * 3 + cy] + px[3 + bx] * G[(3 + cx) * 3 + cy]
-                                                       + px[6 + bx] * G[(6 + cx) * 3 + cy];
-#pragma unroll
-                for (int i = 0; i < 27; i++) E2[i] = (T)0;
-            }
-        }
-        if (chunk == 16) break;
-        // ---- rows of D_q and their z contraction F_q: the pencil's 216 rows
-        //      sorted by kind, so that a wave mostly takes one branch of the
-        //      row function -- tasks 0..71 the first-gradient rows (point
-        //      t / 18, block (t % 18) / 3, row t % 3 + 1), 72..215 the
-        //      second-gradient rows (point u / 36, block (u % 36) / 6, row
-        //      u % 6 + 4, u = t - 72); the mixed wave (tasks 64..127) is the
-        //      one without y-pass work (rt 192..255)
-        {
-            const int t = (rt + 128) & 255;
-            if (t < 216) {
-                int qz, p, ar;
-                if (t < 72) {
-                    qz = t / 18;
-                    const int r = t - 18 * qz;
-                    p = r / 3;
-                    ar = r - 3 * p;
-                } else {
-                    const int u = t - 72;
-                    qz = u / 36;
-                    const int r = u - 36 * qz;
-                    p = r / 6;
-                    ar = 3 + r - 6 * p;
-                }
-                const int q = 4 * chunk + qz;
-                double row[NA];
-#pragma unroll
-                for (int bb = 0; bb < NA; bb++) row[bb] = 0.0;
-                rows(q, p, ar, row);
-                const double wgt = sWgt[q];
-                const T *pz = &sP[2][qz][0][0];
-                T f[FR];
-#pragma unroll
-                for (int i = 0; i < FR; i++) f[i] = (T)0;
-#pragma unroll
-                for (int bb = 0; bb < NA; bb++) {
-                    const int a = bb + 1;
-                    const T v = (T)(wgt * row[bb]);
-#pragma unroll
-                    for (int cz = 0; cz < 3; cz++) f[3 * SEP_XY[a] + cz] += v * pz[3 * SEP_DZ[a] + cz];
-                }
-                T *o = sF + (qz * 6 + p) * SEP_FB + ar * SEP_FS;
-#pragma unroll
-                for (int i = 0; i < FR; i++) o[i] = f[i];
-            }
-        }
-        __syncthreads();
-        // ---- z pass over the pencil's four points -> E1[p][(s,bz)][(s',cz)].
-        //      FP64: on all four waves, each half of rt taking one half of
-        //      the x-y parts s (a wave runs one branch); FP32, capped at 168
-        //      VGPRs for three workgroups per CU, keeps whole columns on 108
-        //      threads (the halves spill there)
-        if constexpr (sizeof(T) == 8) {
-            if ((rt & 127) < 108) sep_zcol<T, true>(sF, sP, sE, rt & 127, rt >> 7);
-        } else if (rt < 108) {
-            sep_zcol<T, false>(sF, sP, sE, rt, 0);
-        }
-        __syncthreads();
-    }
-
-}
-
-// Write-out of the separable tangents: thread rt < 162 holds the entries
-// K[bx][cx][cy] of block (i, j) = (kBlkI[yp], kBlkJ[yp]) for its (by, bz, cz);
-// sWork (at least 972 bytes) is free.
+// Write-out of the separable tangents: a y lane of the pipeline holds the
+// entries K[(3 bx + cx) * 3 + by] of block p = (i, j) for its cy and bc = 3 bz + cz.  DIRECT: sRow and sMsk hold the row starts and Dirichlet flags
+// of the element's 81 rows.
 template <typename T, bool DIRECT>
-__device__ __forceinline__ void sep_write(const MeshK &M, const Scatter &S, T *__restrict__ Ke, int e, int ex, int ey, int ez, int rt,
-                                          const T *K, char *sWork)
+__device__ __forceinline__ void sep_write(const MeshK &M, T *__restrict__ Ke, int e, int ex, int ey, int ez, int p, int bc, int cy, const T *K,
+                                          const int64_t *sRow, const int32_t *sMsk)
 {
-    const int tid = threadIdx.x;
-    const int yp = rt / 27, yu = rt - 27 * yp;
-    const int ybz = yu / 9, ycz = (yu / 3) % 3, yby = yu % 3;
+    // (the lane's place is hidden from the loop around the call: its addresses,
+    // hoisted out of it, would fill the registers)
+    asm volatile("" : "+v"(p), "+v"(bc));
+    const int bz = bc / 3, cz = bc % 3;
+    const int i = blk_k(p), j = blk_l(p);
     if constexpr (DIRECT) {
         // ---- add (row 3b+i, column 3c+j) and the mirrored entry into the CSR
         //      values, Dirichlet rows and columns left at zero; the elements
-        //      of one colour share no row.  Row starts and masks of the
-        //      element's 81 rows staged in LDS (the F buffer is free after
-        //      the last pencil), then per bx all loads of the nine entries
-        //      (and mirrors) before their stores (one round trip for all 27
-        //      measured slower: the scattered read-modify-write of the CSR
-        //      values, not its latency, is the cost).
-        int64_t *sRow = reinterpret_cast<int64_t *>(sWork);
-        int32_t *sMsk = reinterpret_cast<int32_t *>(sWork + 81 * sizeof(int64_t));
-        if (tid < 81) {
-            const int b = tid / 3, i = tid - 3 * (tid / 3);
-            const int64_t cp = ((int64_t)M.nb[1] * M.nb[2]) * (ex + b / 9) + (int64_t)M.nb[2] * (ey + (b / 3) % 3) + (ez + b % 3);
-            sRow[tid] = S.rowptr[3 * cp + i];
-            sMsk[tid] = S.mask[3 * cp + i];
-        }
-        __syncthreads();
-        if (rt < 162) {
-            const int i = kBlkI[yp], j = kBlkJ[yp];
+        //      of one colour share no row.  Per bx all loads of the nine
+        //      entries (and mirrors) before their stores (one round trip for
+        //      all 27 measured slower: the scattered read-modify-write of the
+        //      CSR values, not its latency, is the cost).
 #pragma unroll
-            for (int bx = 0; bx < 3; bx++) {
-                const int b = 9 * bx + 3 * yby + ybz, Bx = ex + bx, By = ey + yby, Bz = ez + ybz;
-                T vp[9], vq[9];
-                int64_t pp[9], pq[9];
-                bool ok[9];
+        for (int bx = 0; bx < 3; bx++) {
+            T vp[9], vq[9];
+            int64_t pp[9], pq[9];
+            bool ok[9];
 #pragma unroll
-                for (int t = 0; t < 9; t++) {
-                    const int cx = t / 3, cy = t % 3, c = 9 * cx + 3 * cy + ycz;
-                    const int Cx = ex + cx, Cy = ey + cy, Cz = ez + ycz;
-                    ok[t] = sMsk[3 * b + i] == 0 && sMsk[3 * c + j] == 0;
-                    pp[t] = stencil_pos(M, sRow[3 * b + i], Bx, By, Bz, Cx, Cy, Cz, j);
-                    pq[t] = stencil_pos(M, sRow[3 * c + j], Cx, Cy, Cz, Bx, By, Bz, i);
-                    vp[t] = vq[t] = (T)0;
-                    if (ok[t]) {
-                        vp[t] = Ke[pp[t]];
-                        if (i != j) vq[t] = Ke[pq[t]];
-                    }
+            for (int t = 0; t < 9; t++) {
+                const int cx = t / 3, by = t % 3, b = 9 * bx + 3 * by + bz, c = 9 * cx + 3 * cy + cz;
+                ok[t] = sMsk[3 * b + i] == 0 && sMsk[3 * c + j] == 0;
+                pp[t] = stencil_pos(M, sRow[3 * b + i], ex + bx, ey + by, ez + bz, ex + cx, ey + cy, ez + cz, j);
+                pq[t] = stencil_pos(M, sRow[3 * c + j], ex + cx, ey + cy, ez + cz, ex + bx, ey + by, ez + bz, i);
+                vp[t] = vq[t] = (T)0;
+                if (ok[t]) {
+                    vp[t] = Ke[pp[t]];
+                    if (i != j) vq[t] = Ke[pq[t]];
                 }
+            }
 #pragma unroll
-                for (int t = 0; t < 9; t++) {
-                    const T v = K[(3 * bx + t / 3) * 3 + t % 3];
-                    if (ok[t]) {
-                        Ke[pp[t]] = vp[t] + v;
-                        if (i != j) Ke[pq[t]] = vq[t] + v;
-                    }
+            for (int t = 0; t < 9; t++) {
+                const T v = K[9 * bx + t];
+                if (ok[t]) {
+                    Ke[pp[t]] = vp[t] + v;
+                    if (i != j) Ke[pq[t]] = vq[t] + v;
                 }
             }
         }
         return;
     }
     // ---- K_e: row 3b+i, column 3c+j, and the mirrored block (3c+j, 3b+i)
-    if (rt < 162) {
-        const int i = kBlkI[yp], j = kBlkJ[yp];
-        T *out = Ke + (int64_t)e * 6561;
+    T *out = Ke + (int64_t)e * 6561;
 #pragma unroll
-        for (int bx = 0; bx < 3; bx++)
+    for (int bx = 0; bx < 3; bx++)
 #pragma unroll
-            for (int cx = 0; cx < 3; cx++)
+        for (int cx = 0; cx < 3; cx++)
 #pragma unroll
-                for (int cy = 0; cy < 3; cy++) {
-                    const int b = 9 * bx + 3 * yby + ybz, c = 9 * cx + 3 * cy + ycz;
-                    const T v = K[(3 * bx + cx) * 3 + cy];
-                    out[(3 * b + i) * 81 + 3 * c + j] = v;
-                    if (i != j) out[(3 * c + j) * 81 + 3 * b + i] = v;
-                }
+            for (int by = 0; by < 3; by++) {
+                const int b = 9 * bx + 3 * by + bz, c = 9 * cx + 3 * cy + cz;
+                const T v = K[(3 * bx + cx) * 3 + by];
+                out[(3 * b + i) * 81 + 3 * c + j] = v;
+                if (i != j) out[(3 * c + j) * 81 + 3 * b + i] = v;
+            }
+}
+
+// element indices of workgroup g: element g, or (DIRECT) element g of the colour S.c
+template <bool DIRECT>
+__device__ __forceinline__ void sep_index(const MeshK &M, const Scatter &S, int g, int *ed)
+{
+    if (DIRECT) {
+        ed[0] = S.c[0] + 3 * (g / (S.nc[1] * S.nc[2]));
+        ed[1] = S.c[1] + 3 * ((g / S.nc[2]) % S.nc[1]);
+        ed[2] = S.c[2] + 3 * (g % S.nc[2]);
+    } else {
+        ed[0] = g / (M.nelem[1] * M.nelem[2]);
+        ed[1] = (g / M.nelem[2]) % M.nelem[1];
+        ed[2] = g % M.nelem[2];
     }
 }
 
-template <typename T, bool DIRECT>
-__global__ __launch_bounds__(256, (sizeof(T) == 8) ? 2 : 3) void k_tangent_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
-                                                        T *__restrict__ Ke, int nel, Scatter S)
+// row starts and Dirichlet flags of the element's 81 rows -> LDS (direct scatter)
+__device__ __forceinline__ void sep_rows(const MeshK &M, const Scatter &S, const int *ed, int64_t *sRow, int32_t *sMsk)
 {
-    constexpr int WORK_A = 3 * (108 + 288) * (int)sizeof(double);   // field passes of the 3 displacement components
-    constexpr int WORK_F = 4 * 6 * SEP_FB * (int)sizeof(T);        // F of the pencil's four points (9 rows x 18 columns)
-    __shared__ double sPd[3][4][3][3];          // 1-D tables of physical derivatives [d][q_d][order][i]
-    __shared__ T sP[3][4][3][3];                // the same in the contraction's precision
-    __shared__ double sG[3][4];                 // dx_d / dxi_d at the 1-D Gauss points
-    __shared__ double sU[27 * 3];
-    __shared__ double sWgt[64];
-    // strain-measure states, compact layout, at a stride of 50 doubles: a wave's
-    // rows cover the pencil's four points, and 48 would put points two apart
-    // on the same LDS banks
-    constexpr int SSTR = 50;
-    __shared__ double sSt[64 * SSTR];
-    __shared__ __attribute__((aligned(16))) T sE[6 * SEP_EB];   // E1 of the current pencil
-    __shared__ __attribute__((aligned(16))) char sWork[WORK_A > WORK_F ? WORK_A : WORK_F];
-    T *sF = reinterpret_cast<T *>(sWork);
-
     const int tid = threadIdx.x;
-    const int e = blockIdx.x;
-    int ex, ey, ez;
-    if (DIRECT) {   // element e of the colour S.c
-        const int k = e % S.nc[2], j = (e / S.nc[2]) % S.nc[1], i = e / (S.nc[1] * S.nc[2]);
-        ex = S.c[0] + 3 * i;
-        ey = S.c[1] + 3 * j;
-        ez = S.c[2] + 3 * k;
-    } else {
-        const int nz = M.nelem[2], ny = M.nelem[1];
-        ex = e / (ny * nz);
-        ey = (e / nz) % ny;
-        ez = e % nz;
+    if (tid < 81) {
+        const int b = tid / 3, i = tid - 3 * b;
+        const int64_t cp = ((int64_t)M.nb[1] * M.nb[2]) * (ed[0] + b / 9) + (int64_t)M.nb[2] * (ed[1] + (b / 3) % 3) + (ed[2] + b % 3);
+        sRow[tid] = S.rowptr[3 * cp + i];
+        sMsk[tid] = S.mask[3 * cp + i];
     }
-    const int ed[3] = {ex, ey, ez};
+}
 
-    sep_element<T>(M, Uh, ed, sU, sPd, sP, sG);
+// shape of the separable tangents' pipeline (pencils per chunk, D waves, E1
+// buffers, D prefetch, deep loads) and the waves per SIMD it is compiled for
+template <typename T, int NH> struct SepPipe;
+template <> struct SepPipe<double, 1> { typedef PipeShape<2, 1, 2, true, true> S; static constexpr int OCC = 2; };
+template <> struct SepPipe<float, 1> { typedef PipeShape<2, 1, 1, false, false> S; static constexpr int OCC = 4; };
+template <> struct SepPipe<double, 3> { typedef PipeShape<2, 1, 1, false, true> S; static constexpr int OCC = 2; };
+template <> struct SepPipe<float, 3> { typedef PipeShape<2, 1, 1, false, false> S; static constexpr int OCC = 4; };
+template <typename T, int NH> using SepShape = typename SepPipe<T, NH>::S;
+
+// Static tangent of a separable patch: a workgroup per element -- tables and
+// displacements, jets and strain-measure states of the 64 points (one pass of
+// all waves each), then the pipeline of igap_sep_pipeline.h.
+// Bound by the vector ALUs' issue: 25.6k FP64 wave instructions per element and
+// CU, 82% of the cycles of an interval.  The stages on waves of their own, D, z
+// and y/x side by side, replace a loop over pencils in which every wave ran all
+// stages with a barrier after each and the matrix cores idle, the z stage as four
+// lanes' partial sums: at 128x32x32 12.9 -> 9.1 ms in FP64 and 8.1 -> 5.3 ms in
+// FP32, at 16x4x4 (FP64) 42 -> 28 us.  FP64 holds two E1 buffers and one
+// workgroup per CU (160 KB of LDS); twelve waves at 168 registers (two sets of y
+// waves) took 9.65 ms, six waves of one pencil and two workgroups per CU 12.5.
+// FP32 fits two workgroups of 79 KB with one E1 buffer.
+template <typename T, bool DIRECT>
+__global__ __launch_bounds__((SepShape<T, 1>::THREADS), (SepPipe<T, 1>::OCC)) void k_tangent_sep(
+    MeshK M, PhysK P, const double *__restrict__ Uh, T *__restrict__ Ke, Scatter S, const T *__restrict__ tabx,
+    const T *__restrict__ taby, const T *__restrict__ tabz)
+{
+    typedef SepShape<T, 1> Sh;
+    __shared__ double sPd[3][4][3][3];          // 1-D tables of physical derivatives [d][q_d][order][i]
+    __shared__ double sW[3][4];                 // 1-D point weights
+    __shared__ double sU[27 * 3];
+    __shared__ __attribute__((aligned(16))) double sSt[64 * SST_W];          // strain-measure states (StaticIn)
+    __shared__ T sX[36];                        // x table in the contraction's precision
+    __shared__ int64_t sRow[DIRECT ? 81 : 1];
+    __shared__ int32_t sMsk[DIRECT ? 81 : 1];
+    __shared__ __attribute__((aligned(16))) T sD[Sh::D_SIZE];
+    __shared__ __attribute__((aligned(16))) T sE[Sh::E_SIZE];   // first the field passes' buffers (1188 doubles)
+    static_assert(Sh::E_SIZE * sizeof(T) >= 3 * (108 + 288) * sizeof(double), "field buffers in sE");
+
+    const int tid = threadIdx.x, e = blockIdx.x;
+    int ed[3];
+    sep_index<DIRECT>(M, S, e, ed);
+    if (DIRECT) sep_rows(M, S, ed, sRow, sMsk);
+    if (tid >= 256 && tid < 256 + 36) sX[tid - 256] = tabx[ed[0] * TAB_STRIDE + tid - 256];
+    sep_element(M, Uh, ed, sU, sPd, sW);
     __syncthreads();
-    // ---- stage A: displacement jets, strain-measure states, point weights
+    // ---- displacement jets and strain-measure states of the first element
     {
         double J[10];
-        sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sWork), J);
-        const int q = tid >> 2, part = tid & 3, lq = (tid & 63) & ~3;
-        double u[30];
-#pragma unroll
-        for (int k = 0; k < 3; k++)
-#pragma unroll
-            for (int a = 0; a < 10; a++) u[10 * k + a] = __shfl(J[a], lq + 1 + k, 64);
-        if (part == 0) {
-            State st;
-            phys_state(u, P, st);
-            double *sp = sSt + q * SSTR;
-            constexpr int PR[6] = {0, 1, 2, 4, 5, 8};   // index pairs I <= J in slot order
-#pragma unroll
-            for (int i = 0; i < 9; i++) { sp[i] = st.F[i]; sp[STC_G + i] = st.G[i]; }
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-#pragma unroll
-                for (int t = 0; t < 6; t++) sp[STC_H + 6 * k + t] = u[10 * k + 4 + t];
-#pragma unroll
-            for (int t = 0; t < 6; t++) { sp[STC_S + t] = st.S[PR[t]]; sp[STC_N + t] = st.N[PR[t]]; }
-            sWgt[q] = sep_weight(M, ed, q, sG);
-        }
+        sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sE), J);
+        sep_states(P, J, sW, sSt);
     }
-    __syncthreads();
-
-    const int rt = (tid + 64 * ((e ^ (e >> 3)) & 3)) & 255;
-    T K[27];
-    // the branch-light rows (FP32: capped at 168 VGPRs for three workgroups
-    // per CU, 5 of them spilled -- faster than the select form of c_row)
-    auto rows = [&](int q, int p, int ar, double *row) {
-        c_row_onehot<true>(sSt + q * SSTR, P, kBlkI[p], ar + 1, kBlkJ[p], row);
+    const StaticIn in{sSt, P.e345, P.le};
+    auto out = [&](int p, int bc, int cy, const T *K) {
+        sep_write<T, DIRECT>(M, Ke, e, ed[0], ed[1], ed[2], p, bc, cy, K, sRow, sMsk);
     };
-    sep_pencils<T>(rt, sP, sWgt, sF, sE, rows, K);
-    sep_write<T, DIRECT>(M, S, Ke, e, ex, ey, ez, rt, K, sWork);
+    sep_pipeline<T, Sh>(sX, taby + ed[1] * TAB_STRIDE, tabz + ed[2] * TAB_STRIDE, sD, sE, in, out);
 }
 
 // Transient tangent on a separable patch (k_tangent_sep_t, gradelasttime):
 // the rule-weighted pointwise rows of k_tangent_elem<..., 3> (c_row_mom: the
-// eight rule-node states us_j = Um + s_j Ud collapsed into moments) in the
-// pencil loop of k_tangent_sep, plus the inertia term.  The inertia block
+// eight rule-node states us_j = Um + s_j Ud collapsed into moments) in
+// the pipeline of k_tangent_sep, plus the inertia term.  The inertia block
 // D[(k,0),(k,0)] = w_q (cii / (2 dt) + rho / dt^2) pairs only basis values,
 // and w_q and the basis value are products over the directions, so its part
 // of K^kk is mc Mx[bx][cx] My[by][cy] Mz[bz][cz] with the 1-D matrices
@@ -1628,70 +1452,62 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 2 : 3) void k_tangent_sep(M
 // Um and Ud (two field passes), then the moment states of all 64 points,
 // compact and in the contraction's precision (one lane per rule node, sums
 // over 8-lane groups), so that the FP32 kernel keeps two workgroups per CU
-// (FP64: 95 KB of LDS, one).
+// (76 KB of LDS; FP64, 149 KB: one).  Bound by vector issue like the static one,
+// and by stage A.  Two pencils per interval and one D wave: 13.5 ms in FP32 at
+// 128x32x32 (14.2 ms as a loop of all waves over the pencils; one pencil and two D
+// waves 18.8, its registers limiting both to two workgroups), 2.06 ms in FP64 at
+// 64x16x16 (one pencil 2.4).
 template <typename T, bool DIRECT>
-__global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t(MeshK M, PhysK P, const double *__restrict__ Uh,
-                                                                               int64_t ndof, T *__restrict__ Ke, int nel, Scatter S)
+__global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) void k_tangent_sep_t(
+    MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof, T *__restrict__ Ke, Scatter S, const T *__restrict__ tabx,
+    const T *__restrict__ taby, const T *__restrict__ tabz)
 {
-    constexpr int WORK_A = 3 * (108 + 288) * (int)sizeof(double);   // field passes of 3 components
-    constexpr int WORK_F = 4 * 6 * SEP_FB * (int)sizeof(T);        // F of the pencil's four points
-    constexpr int WORK_J = 64 * 54 * (int)sizeof(T);               // jets of Um and Ud, slots 1..9
-    constexpr int WORK = WORK_A > WORK_F ? (WORK_A > WORK_J ? WORK_A : WORK_J) : (WORK_F > WORK_J ? WORK_F : WORK_J);
+    typedef SepShape<T, 3> Sh;
     __shared__ double sPd[3][4][3][3];
-    __shared__ T sP[3][4][3][3];
-    __shared__ double sG[3][4];
+    __shared__ double sW[3][4];
     __shared__ double sU[27 * 3], sUd[27 * 3];
     __shared__ double sWgt[64];
     __shared__ double sMass[3][3][3];          // 1-D mass matrices M_d[b][c]
-    __shared__ T sMom[64 * MWC];               // compact moment states
-    __shared__ __attribute__((aligned(16))) T sE[6 * SEP_EB];
-    __shared__ __attribute__((aligned(16))) char sWork[WORK];
-    T *sF = reinterpret_cast<T *>(sWork);
-    T *sJet = reinterpret_cast<T *>(sWork);     // [q][h][k][a - 1], stage A only
+    __shared__ __attribute__((aligned(16))) T sMom[64 * MS_W];   // compact moment states (first the field passes' buffers)
+    __shared__ T sX[36];
+    __shared__ int64_t sRow[DIRECT ? 81 : 1];
+    __shared__ int32_t sMsk[DIRECT ? 81 : 1];
+    __shared__ __attribute__((aligned(16))) T sD[Sh::D_SIZE];
+    __shared__ __attribute__((aligned(16))) T sE[Sh::E_SIZE];
+    static_assert(64 * MS_W * sizeof(T) >= 3 * (108 + 288) * sizeof(double) && Sh::D_SIZE >= 64 * 54, "stage A's buffers");
+    T *sJet = sD;                               // [q][h][k][a - 1], stage A only
 
-    const int tid = threadIdx.x;
-    const int e = blockIdx.x;
-    int ex, ey, ez;
-    if (DIRECT) {
-        const int k = e % S.nc[2], j = (e / S.nc[2]) % S.nc[1], i = e / (S.nc[1] * S.nc[2]);
-        ex = S.c[0] + 3 * i;
-        ey = S.c[1] + 3 * j;
-        ez = S.c[2] + 3 * k;
-    } else {
-        const int nz = M.nelem[2], ny = M.nelem[1];
-        ex = e / (ny * nz);
-        ey = (e / nz) % ny;
-        ez = e % nz;
-    }
-    const int ed[3] = {ex, ey, ez};
+    const int tid = threadIdx.x, e = blockIdx.x;
+    int ed[3];
+    sep_index<DIRECT>(M, S, e, ed);
+    if (DIRECT) sep_rows(M, S, ed, sRow, sMsk);
 
-    sep_element<T, 3>(M, Uh, ed, sU, sPd, sP, sG, ndof, sUd);
+    if (tid >= 256 && tid < 256 + 36) sX[tid - 256] = tabx[ed[0] * TAB_STRIDE + tid - 256];
+    sep_element<3>(M, Uh, ed, sU, sPd, sW, ndof, sUd);
     __syncthreads();
     // ---- stage A: jets of Um and Ud, point weights, 1-D mass matrices
     {
         double J1[10], J2[10];
-        sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sWork), J1, true);
+        sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sMom), J1, true);
         __syncthreads();
-        sep_fields(M, ed, sUd, sPd, reinterpret_cast<double *>(sWork), J2, false);
+        sep_fields(M, ed, sUd, sPd, reinterpret_cast<double *>(sMom), J2, false);
         __syncthreads();
-        const int q = tid >> 2, part = tid & 3;
-        if (part > 0) {
-            const int k = part - 1;
+        const int q = tid & 63, k = tid >> 6;
+        if (k < 3) {
             T *jq = sJet + q * 54;
 #pragma unroll
             for (int a = 1; a < 10; a++) {
                 jq[9 * k + a - 1] = (T)J1[a];
                 jq[27 + 9 * k + a - 1] = (T)J2[a];
             }
-        } else {
-            sWgt[q] = sep_weight(M, ed, q, sG);
+        } else if (k == 3) {
+            sWgt[q] = sep_weight(q, sW);
         }
         if (tid < 27) {
             const int d = tid / 9, b = (tid / 3) % 3, c = tid % 3;
-            const double dX = M.knot[d][ed[d] + 3] - M.knot[d][ed[d] + 2];
             double m = 0.0;
 #pragma unroll
-            for (int qq = 0; qq < 4; qq++) m += M.gw[qq] * dX * sG[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
+            for (int qq = 0; qq < 4; qq++) m += sW[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
             sMass[d][b][c] = m;
         }
     }
@@ -1699,7 +1515,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t
     // ---- moment states: lane 8g + j takes rule node j of point g (32 points
     //      per round, two rounds); node sums over the 8-lane group one entry
     //      at a time; F^ and H^ from the jets, 3-4 entries per lane
-    {
+    if (tid < 256) {
         Mom mu = {0.0, 0.0, 0.0, 0.0, 1.0, 1.0, 1.0};
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -1713,7 +1529,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t
         for (int round = 0; round < 2; round++) {
             const int q = (tid >> 3) + 32 * round;
             const T *jq = sJet + q * 54;
-            T *ms = sMom + q * MWC;
+            T *ms = sMom + q * MS_W;
             {
                 double us[30];
 #pragma unroll
@@ -1737,10 +1553,10 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t
                         n2 += __shfl_xor(n2, o, 64);
                     }
                     if (j == 0) {
-                        ms[MC_S + t] = (T)sv;
-                        ms[MC_N11 + t] = (T)(n0 / mu.m0);
-                        ms[MC_N12 + t] = (T)((n1 - mu.lf * n0) * c12);
-                        ms[MC_N22 + t] = (T)(((mu.lf * n0 - n1) * mu.lf + (n2 - mu.lf * n1)) * c22);
+                        ms[MS_S + t] = (T)sv;
+                        ms[MS_N11 + t] = (T)(n0 / mu.m0);
+                        ms[MS_N12 + t] = (T)((n1 - mu.lf * n0) * c12);
+                        ms[MS_N22 + t] = (T)(((mu.lf * n0 - n1) * mu.lf + (n2 - mu.lf * n1)) * c22);
                     }
                 }
 #pragma unroll
@@ -1748,7 +1564,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t
                     double gv = w0 * st.G[i];
 #pragma unroll
                     for (int o = 1; o < 8; o <<= 1) gv += __shfl_xor(gv, o, 64);
-                    if (j == 0) ms[MC_G + i] = (T)gv;
+                    if (j == 0) ms[MS_G + i] = (T)gv;
                 }
             }
             // F^ (r < 9: F_kL, k = r / 3, L = r % 3) and H^ (r >= 9: H_k,IK in
@@ -1767,37 +1583,34 @@ __global__ __launch_bounds__(256, (sizeof(T) == 8) ? 1 : 2) void k_tangent_sep_t
                 const double xd = (double)jq[27 + src];
                 const double x1 = mu.a11 * (x0 + mu.lf * xd), x2 = mu.a22 * xd;
                 if (r < 9) {
-                    ms[MC_F1 + r] = (T)x1;
-                    ms[MC_F2 + r] = (T)x2;
+                    ms[18 * (r / 3) + r % 3] = (T)x1;
+                    ms[18 * (r / 3) + 3 + r % 3] = (T)x2;
                 } else {
-                    ms[MC_H1 + r - 9] = (T)x1;
-                    ms[MC_H2 + r - 9] = (T)x2;
+                    ms[18 * ((r - 9) / 6) + 6 + (r - 9) % 6] = (T)x1;
+                    ms[18 * ((r - 9) / 6) + 12 + (r - 9) % 6] = (T)x2;
                 }
             }
         }
     }
     __syncthreads();
 
-    const int rt = (tid + 64 * ((e ^ (e >> 3)) & 3)) & 255;
-    T K[27];
-    auto rows = [&](int q, int p, int ar, double *row) { c_row_momc_onehot<T>(sMom + q * MWC, P, kBlkI[p], ar + 1, kBlkJ[p], row); };
-    sep_pencils<T>(rt, sP, sWgt, sF, sE, rows, K);
-    // inertia on the diagonal blocks
-    if (rt < 162) {
-        const int yp = rt / 27, yu = rt - 27 * yp;
-        const int ybz = yu / 9, ycz = (yu / 3) % 3, yby = yu % 3;
-        if (kBlkI[yp] == kBlkJ[yp]) {
+    const MomentIn<T> in{sMom, sWgt, P.e345, P.le};
+    auto out = [&](int p, int bc, int cy, T *K) {
+        // inertia on the diagonal blocks
+        const int bz = bc / 3, cz = bc % 3;
+        if (blk_k(p) == blk_l(p)) {
             const double mc = P.cii / (2. * P.dt) + P.rho / (P.dt * P.dt);
 #pragma unroll
             for (int bx = 0; bx < 3; bx++)
 #pragma unroll
                 for (int cx = 0; cx < 3; cx++)
 #pragma unroll
-                    for (int cy = 0; cy < 3; cy++)
-                        K[(3 * bx + cx) * 3 + cy] += (T)(mc * sMass[0][bx][cx] * sMass[1][yby][cy] * sMass[2][ybz][ycz]);
+                    for (int by = 0; by < 3; by++)
+                        K[(3 * bx + cx) * 3 + by] += (T)(mc * sMass[0][bx][cx] * sMass[1][by][cy] * sMass[2][bz][cz]);
         }
-    }
-    sep_write<T, DIRECT>(M, S, Ke, e, ex, ey, ez, rt, K, sWork);
+        sep_write<T, DIRECT>(M, Ke, e, ed[0], ed[1], ed[2], p, bc, cy, K, sRow, sMsk);
+    };
+    sep_pipeline<T, Sh>(sX, taby + ed[1] * TAB_STRIDE, tabz + ed[2] * TAB_STRIDE, sD, sE, in, out);
 }
 
 // Transposed sum factorisation of the weighted pointwise residual jets
@@ -1875,7 +1688,7 @@ __global__ __launch_bounds__(256, 6) void k_residual_sep(MeshK M, PhysK P, const
                                                          double *__restrict__ Re, int nel)
 {
     __shared__ double sPd[3][4][3][3];
-    __shared__ double sG[3][4];
+    __shared__ double sW[3][4];
     __shared__ double sU[27 * 3];
     __shared__ double sWork[3 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
     __shared__ double sJet[64 * 30];            // u-jets [q][k][a], then the weighted r_q
@@ -1884,15 +1697,15 @@ __global__ __launch_bounds__(256, 6) void k_residual_sep(MeshK M, PhysK P, const
     const int nz = M.nelem[2], ny = M.nelem[1];
     const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
 
-    sep_element<double>(M, Uh, ed, sU, sPd, nullptr, sG);
+    sep_element(M, Uh, ed, sU, sPd, sW);
     __syncthreads();
     {
         double J[10];
         sep_fields(M, ed, sU, sPd, sWork, J);
-        const int q = tid >> 2, part = tid & 3;
-        if (part > 0) {
+        const int q = tid & 63, k = tid >> 6;
+        if (k < 3) {
 #pragma unroll
-            for (int a = 0; a < 10; a++) sJet[q * 30 + 10 * (part - 1) + a] = J[a];
+            for (int a = 0; a < 10; a++) sJet[q * 30 + 10 * k + a] = J[a];
         }
     }
     __syncthreads();
@@ -1904,7 +1717,7 @@ __global__ __launch_bounds__(256, 6) void k_residual_sep(MeshK M, PhysK P, const
 #pragma unroll
         for (int a = 0; a < 30; a++) u[a] = sJet[q * 30 + a];
         phys_residual_static(P, u, r);
-        const double w = sep_weight(M, ed, q, sG);
+        const double w = sep_weight(q, sW);
 #pragma unroll
         for (int a = 0; a < 30; a++) sJet[q * 30 + a] = w * r[a];
     }
@@ -1924,7 +1737,7 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
                                                            double *__restrict__ Re, int nel)
 {
     __shared__ double sPd[3][4][3][3];
-    __shared__ double sG[3][4];
+    __shared__ double sW[3][4];
     __shared__ double sU[27 * 3], sUd[27 * 3], sV[27 * 3];
     __shared__ double sMass[3][3][3];
     __shared__ double sWork[3 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
@@ -1934,27 +1747,26 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
     const int nz = M.nelem[2], ny = M.nelem[1];
     const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
 
-    sep_element<double, 3>(M, Uh, ed, sU, sPd, nullptr, sG, ndof, sUd, sV, P.cii / (2. * P.dt), P.rho / (P.dt * P.dt));
+    sep_element<3>(M, Uh, ed, sU, sPd, sW, ndof, sUd, sV, P.cii / (2. * P.dt), P.rho / (P.dt * P.dt));
     __syncthreads();
     {
         double J1[10], J2[10];
         sep_fields(M, ed, sU, sPd, sWork, J1, true);
         __syncthreads();
         sep_fields(M, ed, sUd, sPd, sWork, J2, false);
-        const int q = tid >> 2, part = tid & 3;
-        if (part > 0) {
+        const int q = tid & 63, k = tid >> 6;
+        if (k < 3) {
 #pragma unroll
             for (int a = 0; a < 10; a++) {
-                sJet[q * 60 + 10 * (part - 1) + a] = J1[a];
-                sJet[q * 60 + 30 + 10 * (part - 1) + a] = J2[a];
+                sJet[q * 60 + 10 * k + a] = J1[a];
+                sJet[q * 60 + 30 + 10 * k + a] = J2[a];
             }
         }
         if (tid < 27) {
             const int d = tid / 9, b = (tid / 3) % 3, c = tid % 3;
-            const double dX = M.knot[d][ed[d] + 3] - M.knot[d][ed[d] + 2];
             double m = 0.0;
 #pragma unroll
-            for (int qq = 0; qq < 4; qq++) m += M.gw[qq] * dX * sG[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
+            for (int qq = 0; qq < 4; qq++) m += sW[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
             sMass[d][b][c] = m;
         }
     }
@@ -1978,7 +1790,7 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
                 for (int a = 0; a < 30; a++) r[a] = 0.0;
                 phys_residual_acc(st, P.cr[j], r);
             }
-            const double w = (j == 0) ? sep_weight(M, ed, q, sG) : 0.0;
+            const double w = (j == 0) ? sep_weight(q, sW) : 0.0;
 #pragma unroll
             for (int a = 0; a < 30; a++) {
                 if (a % 10 == 0) continue;   // value slots: the inertia, added below
@@ -2001,7 +1813,7 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
 #pragma unroll
         for (int cx = 0; cx < 3; cx++)
 #pragma unroll
-            for (int cy = 0; cy < 3; cy++) {
+            for (int cy = 0, ys = 0; cy < 3; cy++) {
                 const double mxy = sMass[0][bx][cx] * sMass[1][by][cy];
 #pragma unroll
                 for (int cz = 0; cz < 3; cz++) in += mxy * sMass[2][bz][cz] * sV[3 * (9 * cx + 3 * cy + cz) + k];
@@ -2449,13 +2261,13 @@ hipError_t launch_tangent_elem(const MeshK &M, const PhysK &P, const double *Uh,
     dim3 grid(nel), block(256);
     const Scatter S{};
     if (P.torder == 0 && M.separable) {
-        if (prec == 0) hipLaunchKernelGGL((k_tangent_sep<double, false>), grid, block, 0, s, M, P, Uh, ndof, (double *)Ke, nel, S);
-        else hipLaunchKernelGGL((k_tangent_sep<float, false>), grid, block, 0, s, M, P, Uh, ndof, (float *)Ke, nel, S);
+        if (prec == 0) hipLaunchKernelGGL((k_tangent_sep<double, false>), grid, dim3(SepShape<double, 1>::THREADS), 0, s, M, P, Uh, (double *)Ke, S, M.tab[0], M.tab[1], M.tab[2]);
+        else hipLaunchKernelGGL((k_tangent_sep<float, false>), grid, dim3(SepShape<float, 1>::THREADS), 0, s, M, P, Uh, (float *)Ke, S, M.tabf[0], M.tabf[1], M.tabf[2]);
         return hipGetLastError();
     }
     if (P.torder == 2 && M.separable) {
-        if (prec == 0) hipLaunchKernelGGL((k_tangent_sep_t<double, false>), grid, block, 0, s, M, P, Uh, ndof, (double *)Ke, nel, S);
-        else hipLaunchKernelGGL((k_tangent_sep_t<float, false>), grid, block, 0, s, M, P, Uh, ndof, (float *)Ke, nel, S);
+        if (prec == 0) hipLaunchKernelGGL((k_tangent_sep_t<double, false>), grid, dim3(SepShape<double, 3>::THREADS), 0, s, M, P, Uh, ndof, (double *)Ke, S, M.tab[0], M.tab[1], M.tab[2]);
+        else hipLaunchKernelGGL((k_tangent_sep_t<float, false>), grid, dim3(SepShape<float, 3>::THREADS), 0, s, M, P, Uh, ndof, (float *)Ke, S, M.tabf[0], M.tabf[1], M.tabf[2]);
         return hipGetLastError();
     }
     if (prec == 0) {
@@ -2481,7 +2293,7 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
     if (prec == 0) hipLaunchKernelGGL(k_fill<double>, dim3((unsigned)fb), dim3(256), 0, s, (double *)vals, 0.0, nnz);
     else hipLaunchKernelGGL(k_fill<float>, dim3((unsigned)fb), dim3(256), 0, s, (float *)vals, 0.0f, nnz);
     for (int cx = 0; cx < 3; cx++)
-        for (int cy = 0; cy < 3; cy++)
+        for (int cy = 0, ys = 0; cy < 3; cy++)
             for (int cz = 0; cz < 3; cz++) {
                 Scatter S;
                 S.rowptr = rowptr;
@@ -2492,11 +2304,11 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
                 if (n <= 0) continue;
                 dim3 grid((unsigned)n), block(256);
                 if (P.torder == 0 && M.separable) {
-                    if (prec == 0) hipLaunchKernelGGL((k_tangent_sep<double, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);
-                    else hipLaunchKernelGGL((k_tangent_sep<float, true>), grid, block, 0, s, M, P, Uh, ndof, (float *)vals, (int)n, S);
+                    if (prec == 0) hipLaunchKernelGGL((k_tangent_sep<double, true>), grid, dim3(SepShape<double, 1>::THREADS), 0, s, M, P, Uh, (double *)vals, S, M.tab[0], M.tab[1], M.tab[2]);
+                    else hipLaunchKernelGGL((k_tangent_sep<float, true>), grid, dim3(SepShape<float, 1>::THREADS), 0, s, M, P, Uh, (float *)vals, S, M.tabf[0], M.tabf[1], M.tabf[2]);
                 } else if (P.torder == 2 && M.separable) {
-                    if (prec == 0) hipLaunchKernelGGL((k_tangent_sep_t<double, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);
-                    else hipLaunchKernelGGL((k_tangent_sep_t<float, true>), grid, block, 0, s, M, P, Uh, ndof, (float *)vals, (int)n, S);
+                    if (prec == 0) hipLaunchKernelGGL((k_tangent_sep_t<double, true>), grid, dim3(SepShape<double, 3>::THREADS), 0, s, M, P, Uh, ndof, (double *)vals, S, M.tab[0], M.tab[1], M.tab[2]);
+                    else hipLaunchKernelGGL((k_tangent_sep_t<float, true>), grid, dim3(SepShape<float, 3>::THREADS), 0, s, M, P, Uh, ndof, (float *)vals, S, M.tabf[0], M.tabf[1], M.tabf[2]);
                 } else if (prec == 0) {
                     if (P.torder == 0) hipLaunchKernelGGL((k_tangent_elem<double, 1, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);
                     else hipLaunchKernelGGL((k_tangent_elem<double, 3, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);
@@ -2526,6 +2338,13 @@ hipError_t launch_csr_cols(const MeshK &M, const int64_t *rowptr, int32_t *col, 
 {
     dim3 grid((unsigned)ncp), block(128);
     hipLaunchKernelGGL(k_csr_cols, grid, block, 0, s, M, rowptr, col);
+    return hipGetLastError();
+}
+
+hipError_t launch_sep_tables(const MeshK &M, double *tab, float *tabf, hipStream_t s)
+{
+    const int m = std::max(M.nelem[0], std::max(M.nelem[1], M.nelem[2]));
+    hipLaunchKernelGGL(k_sep_tables, dim3((unsigned)m, 3), dim3(64), 0, s, M, tab, tabf);
     return hipGetLastError();
 }
 

@@ -20,6 +20,8 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
 hipError_t launch_tangent_gather(const MeshK &M, const void *Ke, int prec, const int64_t *rowptr, const int32_t *mask, void *vals,
                                  int64_t ncp, hipStream_t s);
 hipError_t launch_csr_cols(const MeshK &M, const int64_t *rowptr, int32_t *col, int64_t ncp, hipStream_t s);
+// the 1-D tables of a separable patch (MeshK::tab, tabf: TAB_STRIDE values per element of each direction)
+hipError_t launch_sep_tables(const MeshK &M, double *tab, float *tabf, hipStream_t s);
 hipError_t launch_fill_f64(double *p, double v, int64_t n, hipStream_t s);
 hipError_t launch_copy_f64(double *dst, const double *src, int64_t n, hipStream_t s);
 hipError_t launch_selftest_mfma(double *o64, float *o32, hipStream_t s);
