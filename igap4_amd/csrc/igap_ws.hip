@@ -19,6 +19,12 @@
 // accumulated in one FP32 tile.  Lane l supplies A[l&15][4(l>>4)+j] and
 // B[4(l>>4)+j][l&15] (j = 0..3); result register r of lane l holds
 // D[4(l>>4)+r][l&15] (pinned by igap_ws_selftest_mfma_bf16).
+//
+// The net is a chain of small kernels (a layer of the 66x18x18 grid is 50 ns of
+// matrix-core time), so what bounds a training pair is the number of launches and the
+// load latency inside each: nine dependent launches (pack, four layers, four
+// backward steps that do the input and the weight gradient side by side) and
+// one reduction, every load of a tile issued before its first product.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -44,146 +50,263 @@ __device__ __forceinline__ float4_t mma(short4_t a, short4_t b, float4_t c)
     return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-enum { FWD_RELU = 0, FWD_LAST = 1, BWD_MASK = 2 };
+typedef int int4_t __attribute__((ext_vector_type(4)));
+
+enum { FWD_RELU = 0, FWD_LAST = 1, BWD_MASK = 2, FWD_LOSS = 3 };
+
+// One tap's offset along each axis (the dilation, clamped to the grid's size
+// there: a tap that far off is outside either way, and the products of the
+// offsets then stay within 32 bits).
+struct Shape {
+    int nx, ny, nz, dx, dy, dz;
+};
+
+// Where the tiles of a lane's voxel lie: the voxel's first channel of the
+// lane, and which neighbours along each axis are inside the grid (sgn +1: the
+// taps read v + off, -1: v - off).
+struct Taps {
+    int base;
+    bool in[3][3];   // [axis][tap]
+    __device__ __forceinline__ Taps(const Shape &g, int v, int V, int kg, int sgn)
+    {
+        const bool vin = v < V;
+        if (!vin) v = V - 1;
+        base = v * 16 + 4 * kg;
+        const int x = v / (g.ny * g.nz), y = (v / g.nz) % g.ny, z = v % g.nz;
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const int s = sgn * (t - 1), xx = x + s * g.dx, yy = y + s * g.dy, zz = z + s * g.dz;
+            in[0][t] = vin && xx >= 0 && xx < g.nx;
+            in[1][t] = yy >= 0 && yy < g.ny;
+            in[2][t] = zz >= 0 && zz < g.nz;
+        }
+    }
+    __device__ __forceinline__ bool ok(int t) const { return in[0][t / 9] && in[1][(t / 3) % 3] && in[2][t % 3]; }
+    // the lane's four channels of tap t, from an address inside the array whatever the tap
+    __device__ __forceinline__ short4_t load(const Shape &g, const uint16_t *__restrict__ a, int t, int sgn) const
+    {
+        const int off = sgn * ((t / 9 - 1) * g.dx * (g.ny * g.nz) + ((t / 3) % 3 - 1) * g.dy * g.nz + (t % 3 - 1) * g.dz) * 16;
+        return *reinterpret_cast<const short4_t *>(a + (base + (ok(t) ? off : 0)));
+    }
+};
 
 // One wave per tile of 16 consecutive voxels, all 16 output channels.
 //   FWD_RELU  aout = bf16(relu(sum + bias))
 //   FWD_LAST  yout[v][c] = sum + bias  (c < cout, FP32)
+//   FWD_LOSS  e = sum + bias - target[v][c]: aout = bf16(2 e / (V cout)) (0 for
+//             c >= cout), lpart[tile] = sum of e^2
 //   BWD_MASK  aout = bf16(sum * (mask > 0))   (input gradient through ReLU)
 // sgn = +1 gathers in[v + off_t] (forward), -1 gathers in[v - off_t]
 // (gradient with respect to the layer input).
+// The 54 loads of a tile (27 activation tiles, 27 weight tiles, all in L2) are
+// in flight together; issued tap by tap the kernel waited for each pair:
+// 13.5 us a layer at 66x18x18, now 6.2 us.
 template <int MODE>
-__global__ __launch_bounds__(256) void k_conv(int nx, int ny, int nz, int dil, int sgn, const uint16_t *__restrict__ ain,
-                                              const uint16_t *__restrict__ Wk, const float *__restrict__ bias,
-                                              const uint16_t *__restrict__ mask, uint16_t *__restrict__ aout,
-                                              float *__restrict__ yout, int cout)
+__device__ __forceinline__ void conv_tile(const Shape &g, int tile, int lane, int sgn, const uint16_t *__restrict__ ain,
+                                          const uint16_t *__restrict__ Wk, const float *__restrict__ bias,
+                                          const uint16_t *__restrict__ mask, const float *__restrict__ tg,
+                                          uint16_t *__restrict__ aout, float *__restrict__ yout, float *__restrict__ lpart, int cout)
 {
-    const int V = nx * ny * nz;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int v0 = (blockIdx.x * 4 + wv) * 16;
+    const int V = g.nx * g.ny * g.nz, v0 = tile * 16;
     if (v0 >= V) return;
     const int i = lane & 15, kg = lane >> 4;
-    const int v = v0 + i;
-    const bool vin = v < V;
-    int x = 0, y = 0, z = 0;
-    if (vin) {
-        x = v / (ny * nz);
-        y = (v / nz) % ny;
-        z = v % nz;
-    }
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const Taps tp(g, v0 + i, V, kg, sgn);
+    short4_t a[27], b[27];
+#pragma unroll
     for (int t = 0; t < 27; t++) {
-        const int xx = x + sgn * dil * (t / 9 - 1), yy = y + sgn * dil * ((t / 3) % 3 - 1), zz = z + sgn * dil * (t % 3 - 1);
-        short4_t a = {0, 0, 0, 0};
-        if (vin && xx >= 0 && xx < nx && yy >= 0 && yy < ny && zz >= 0 && zz < nz)
-            a = *reinterpret_cast<const short4_t *>(ain + (size_t)((xx * ny + yy) * nz + zz) * 16 + 4 * kg);
-        const short4_t b = *reinterpret_cast<const short4_t *>(Wk + (t * 16 + i) * 16 + 4 * kg);
-        acc = mma(a, b, acc);
+        a[t] = tp.load(g, ain, t, sgn);
+        b[t] = *reinterpret_cast<const short4_t *>(Wk + (t * 16 + i) * 16 + 4 * kg);
     }
+    const float bi = MODE == BWD_MASK ? 0.f : bias[i];
+    float tv[4];
+    uint16_t mv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int vo = v0 + 4 * kg + r;
+        tv[r] = (MODE == FWD_LOSS && vo < V && i < cout) ? tg[(size_t)vo * cout + i] : 0.f;
+        mv[r] = (MODE == BWD_MASK && vo < V) ? mask[(size_t)vo * 16 + i] : (uint16_t)0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 27; t++) acc = mma(tp.ok(t) ? a[t] : (short4_t){0, 0, 0, 0}, b[t], acc);
+    float e2 = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int vo = v0 + 4 * kg + r;
         if (vo >= V) continue;
         float val = acc[r];
         if (MODE == FWD_RELU) {
-            val += bias[i];
+            val += bi;
             aout[(size_t)vo * 16 + i] = f2bf(val > 0.f ? val : 0.f);
         } else if (MODE == FWD_LAST) {
-            if (i < cout) yout[(size_t)vo * cout + i] = val + bias[i];
+            if (i < cout) yout[(size_t)vo * cout + i] = val + bi;
+        } else if (MODE == FWD_LOSS) {
+            const float e = i < cout ? (val + bi) - tv[r] : 0.f;
+            e2 += e * e;
+            aout[(size_t)vo * 16 + i] = f2bf(i < cout ? 2.f * e / ((float)V * (float)cout) : 0.f);
         } else {
-            aout[(size_t)vo * 16 + i] = f2bf(bf2f(mask[(size_t)vo * 16 + i]) > 0.f ? val : 0.f);
+            aout[(size_t)vo * 16 + i] = f2bf(bf2f(mv[r]) > 0.f ? val : 0.f);
         }
+    }
+    if (MODE == FWD_LOSS) {
+        for (int o = 32; o > 0; o >>= 1) e2 += __shfl_xor(e2, o, 64);
+        if (lane == 0) lpart[tile] = e2;
     }
 }
 
-// Weight-gradient partials of one tap over one voxel chunk:
+template <int MODE>
+__global__ __launch_bounds__(256) void k_conv(Shape g, const uint16_t *__restrict__ ain, const uint16_t *__restrict__ Wk,
+                                              const float *__restrict__ bias, const float *__restrict__ tg,
+                                              uint16_t *__restrict__ aout, float *__restrict__ yout, float *__restrict__ lpart, int cout)
+{
+    conv_tile<MODE>(g, blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63, 1, ain, Wk, bias, nullptr, tg, aout, yout, lpart, cout);
+}
+
+// A 16x16 tile of 16-bit values across the lanes of a wave: X[l&15][4(l>>4)+j]
+// in, X[4(l>>4)+j][l&15] out.  The lane's eight bytes are row l&15 of a 16x32
+// byte matrix; two exact integer products select the low and the high bytes of
+// every column (sel: k == 2n and k == 2n + 1), and the result registers hold them
+// transposed.  No LDS, any bit pattern.
+struct Transposer {
+    long lo, hi;
+    __device__ __forceinline__ explicit Transposer(int lane)
+    {
+        const int k = 2 * (lane & 15) - 8 * (lane >> 4);   // place of column n's low byte in the lane's B[8 kg + j][n]
+        lo = (k >= 0 && k < 8) ? (long)(1ull << (8 * k)) : 0;
+        hi = (k >= 0 && k < 8) ? (long)(1ull << (8 * k + 8)) : 0;
+    }
+    __device__ __forceinline__ short4_t operator()(short4_t x) const
+    {
+        const int4_t zero = {0, 0, 0, 0};
+        const long b = __builtin_bit_cast(long, x);
+        const int4_t l = __builtin_amdgcn_mfma_i32_16x16x32_i8(b, lo, zero, 0, 0, 0);
+        const int4_t h = __builtin_amdgcn_mfma_i32_16x16x32_i8(b, hi, zero, 0, 0, 0);
+        uint32_t p[4];   // low byte, high byte, 0, 0
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[r] = __builtin_amdgcn_perm((uint32_t)h[r], (uint32_t)l[r], 0x0c0c0400u);
+        const uint64_t w = (uint64_t)(p[0] | (p[1] << 16)) | ((uint64_t)(p[2] | (p[3] << 16)) << 32);
+        return __builtin_bit_cast(short4_t, w);
+    }
+};
+
+// Backward step of one layer.  Blocks 0 .. ncb - 1 (CONV): the input gradient,
+// as k_conv.  The others: the gradients of the weights and the bias, as partials
+// of one chunk of 4 tw tiles of 16 voxels and the nine taps of one x offset,
 //   part[t][c][ci][co] = sum_{v in chunk c} a[v + off_t][ci] dz[v][co]
-// M = ci, N = co, K = voxels (16 per product).  One wave per (chunk, tap).
-__global__ __launch_bounds__(64) void k_dw(int nx, int ny, int nz, int dil, const uint16_t *__restrict__ ain,
-                                           const uint16_t *__restrict__ dz, int chunk, int nchunk, float *__restrict__ part)
+//   bpart[c][co]       = sum_{v in chunk c} dz[v][co]           (x offset 0)
+// with M = ci, N = co, K = 16 voxels of a product.  Tiles are read as the
+// convolution reads them (eight bytes a lane) and transposed in registers; the
+// four waves of a block take tw tiles each and add up in LDS.  The gradient of
+// layer l - 1 needs only the input gradient, so both run in one launch.
+// At 66x18x18 one wave per (tap, 512 voxels) gathering two bytes at a time took
+// 42 us a layer for the weights and 16-thread blocks 36 us for the bias;
+// now 11.8 us with the input gradient (13 us before) beside, 8.5 us without.
+template <bool CONV>
+__global__ __launch_bounds__(256) void k_back(Shape g, int ncb, const uint16_t *__restrict__ ain, const uint16_t *__restrict__ dz,
+                                              const uint16_t *__restrict__ WTk, uint16_t *__restrict__ dzprev, int tw, int nchunk,
+                                              float *__restrict__ part, float *__restrict__ bpart)
 {
-    const int V = nx * ny * nz;
-    const int c = blockIdx.x, t = blockIdx.y;
-    const int lane = threadIdx.x, i = lane & 15, kg = lane >> 4;
-    const int vbeg = c * chunk, vend = (vbeg + chunk < V) ? vbeg + chunk : V;
-    const int dx = dil * (t / 9 - 1), dy = dil * ((t / 3) % 3 - 1), dzz = dil * (t % 3 - 1);
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
-    for (int vb = vbeg; vb < vend; vb += 16) {
-        short4_t a, b;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int v = vb + 4 * kg + j;
-            short av = 0, bv = 0;
-            if (v < vend) {
-                const int x = v / (ny * nz), y = (v / nz) % ny, z = v % nz;
-                const int xx = x + dx, yy = y + dy, zz = z + dzz;
-                if (xx >= 0 && xx < nx && yy >= 0 && yy < ny && zz >= 0 && zz < nz)
-                    av = (short)ain[(size_t)((xx * ny + yy) * nz + zz) * 16 + i];
-                bv = (short)dz[(size_t)v * 16 + i];
-            }
-            a[j] = av;
-            b[j] = bv;
-        }
-        acc = mma(a, b, acc);
+    __shared__ float4_t red[3][10][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (CONV && (int)blockIdx.x < ncb) {
+        // the mask of the ReLU that made this layer's input is that input
+        conv_tile<BWD_MASK>(g, blockIdx.x * 4 + wv, lane, -1, dz, WTk, nullptr, ain, nullptr, dzprev, nullptr, nullptr, 16);
+        return;
     }
+    const int V = g.nx * g.ny * g.nz, ntile = (V + 15) / 16;
+    const int bb = blockIdx.x - ncb, c = bb / 3, tx = bb - 3 * c;
+    const int i = lane & 15, kg = lane >> 4;
+    const Transposer tr(lane);
+    const short one = 0x3f80;   // 1 in BF16
+    float4_t acc[10];
 #pragma unroll
-    for (int r = 0; r < 4; r++) part[(((size_t)t * nchunk + c) * 16 + 4 * kg + r) * 16 + i] = acc[r];
-}
-
-// grad W[t][co][ci] = sum over chunks (in order) of part[t][c][ci][co]
-__global__ void k_dw_reduce(int nchunk, const float *__restrict__ part, float *__restrict__ gW)
-{
-    const int id = blockIdx.x * blockDim.x + threadIdx.x;   // t*256 + co*16 + ci
-    if (id >= 27 * 256) return;
-    const int t = id >> 8, co = (id >> 4) & 15, ci = id & 15;
-    float s = 0.f;
-    for (int c = 0; c < nchunk; c++) s += part[(((size_t)t * nchunk + c) * 16 + ci) * 16 + co];
-    gW[id] = s;
-}
-
-// bias-gradient partials: bpart[c][co] = sum_{v in chunk c} dz[v][co]
-__global__ void k_db(int V, const uint16_t *__restrict__ dz, int chunk, float *__restrict__ bpart)
-{
-    const int c = blockIdx.x, co = threadIdx.x;
-    const int vbeg = c * chunk, vend = (vbeg + chunk < V) ? vbeg + chunk : V;
-    float s = 0.f;
-    for (int v = vbeg; v < vend; v++) s += bf2f(dz[(size_t)v * 16 + co]);
-    bpart[c * 16 + co] = s;
-}
-
-__global__ void k_db_reduce(int nchunk, const float *__restrict__ bpart, float *__restrict__ gb)
-{
-    const int co = threadIdx.x;
-    float s = 0.f;
-    for (int c = 0; c < nchunk; c++) s += bpart[c * 16 + co];
-    gb[co] = s;
-}
-
-// mean-square loss over V x cout: dz = bf16(2 (y - target) / (V cout)) on the
-// first cout channels (0 on the rest); lpart[block] = sum of squared errors
-__global__ __launch_bounds__(256) void k_loss(int V, int cout, const float *__restrict__ y, const float *__restrict__ tg,
-                                              uint16_t *__restrict__ dz, float *__restrict__ lpart)
-{
-    __shared__ float red[256];
-    const int id = blockIdx.x * 256 + threadIdx.x;   // v*16 + c
-    float e2 = 0.f;
-    if (id < V * 16) {
-        const int v = id >> 4, c = id & 15;
-        float g = 0.f;
-        if (c < cout) {
-            const float e = y[(size_t)v * cout + c] - tg[(size_t)v * cout + c];
-            e2 = e * e;
-            g = 2.f * e / ((float)V * (float)cout);
+    for (int t = 0; t < 10; t++) acc[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
+    const int beg = (c * 4 + wv) * tw, end = beg + tw < ntile ? beg + tw : ntile;
+    for (int tile = beg; tile < end; tile++) {
+        const int v = tile * 16 + i;
+        const Taps tp(g, v, V, kg, 1);
+        // the nine taps of this x offset: in range along x, and along y and z
+        const bool okx = tx == 0 ? tp.in[0][0] : (tx == 1 ? tp.in[0][1] : tp.in[0][2]);
+        const uint16_t *a0 = ain + tp.base;
+        const int offx = (tx - 1) * g.dx * (g.ny * g.nz);
+        short4_t a[9];
+        short4_t d = *reinterpret_cast<const short4_t *>(dz + tp.base);
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+            const bool ok = okx && tp.in[1][t / 3] && tp.in[2][t % 3];
+            const int off = (offx + (t / 3 - 1) * g.dy * g.nz + (t % 3 - 1) * g.dz) * 16;
+            a[t] = *reinterpret_cast<const short4_t *>(a0 + (ok ? off : 0));
         }
-        dz[id] = f2bf(g);
+        if (v >= V) d = (short4_t){0, 0, 0, 0};
+        const short4_t b = tr(d);
+#pragma unroll
+        for (int t = 0; t < 9; t++) {
+            const bool ok = okx && tp.in[1][t / 3] && tp.in[2][t % 3];
+            acc[t] = mma(tr(ok ? a[t] : (short4_t){0, 0, 0, 0}), b, acc[t]);
+        }
+        if (tx == 1) acc[9] = mma((short4_t){one, one, one, one}, b, acc[9]);
     }
-    red[threadIdx.x] = e2;
+    if (wv > 0) {
+#pragma unroll
+        for (int t = 0; t < 10; t++) red[wv - 1][t][lane] = acc[t];
+    }
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int t = 0; t < 10; t++) acc[t] = ((acc[t] + red[0][t][lane]) + red[1][t][lane]) + red[2][t][lane];
+#pragma unroll
+    for (int t = 0; t < 9; t++) {
+        // lane (co = i): ci = 4 kg + r, stored [ci][co]
+        float *o = part + (((size_t)(9 * tx + t) * nchunk + c) * 16 + 4 * kg) * 16 + i;
+#pragma unroll
+        for (int r = 0; r < 4; r++) o[16 * r] = acc[t][r];
     }
-    if (threadIdx.x == 0) lpart[blockIdx.x] = red[0];
+    if (tx == 1 && kg == 0) bpart[c * 16 + i] = acc[9][0];
+}
+
+// The sums over chunks, every layer in one launch (grid.y = layer): blocks
+// 0..26 one tap of the weights, grad W[t][co][ci] = sum_c part[t][c][ci][co];
+// block 27 the bias, and for layer 0 block 28 the sum of the loss partials (in
+// FP64).  Four groups of 256 threads take a quarter of the chunks each, every
+// quarter in order.  The gradients go to the device copy and, where the caller
+// takes them (hG), straight to pinned host memory.
+__global__ __launch_bounds__(1024) void k_grad_reduce(int nchunk, const float *__restrict__ part, const float *__restrict__ bpart,
+                                                      int ntile, const float *__restrict__ lpart, float *__restrict__ G,
+                                                      float *__restrict__ hG, double *__restrict__ hloss)
+{
+    __shared__ double dred[1024];
+    float *red = reinterpret_cast<float *>(dred);
+    const int l = blockIdx.y, t = blockIdx.x, tid = threadIdx.x;
+    if (t == 28) {
+        if (l > 0) return;
+        double s = 0.0;
+        for (int i = tid; i < ntile; i += 1024) s += lpart[i];
+        dred[tid] = s;
+        __syncthreads();
+        for (int o = 512; o > 0; o >>= 1) {
+            if (tid < o) dred[tid] += dred[tid + o];
+            __syncthreads();
+        }
+        if (tid == 0) *hloss = dred[0];
+        return;
+    }
+    const int n = t < 27 ? 256 : 16, id = tid & 255, grp = tid >> 8;
+    const int per = (nchunk + 3) / 4, c0 = grp * per, c1 = c0 + per < nchunk ? c0 + per : nchunk;
+    const float *p = t < 27 ? part + (((size_t)l * 27 + t) * nchunk) * 256 + id : bpart + (size_t)l * nchunk * 16 + id;
+    float s = 0.f;
+    if (id < n) {
+#pragma unroll 8
+        for (int c = c0; c < c1; c++) s += p[(size_t)c * n];
+    }
+    red[tid] = s;
+    __syncthreads();
+    if (grp > 0 || id >= n) return;
+    s = ((red[id] + red[id + 256]) + red[id + 512]) + red[id + 768];
+    // id = ci*16 + co of a tap, co of the bias
+    const size_t o = (size_t)l * LAYER_P + (t < 27 ? t * 256 + (id & 15) * 16 + (id >> 4) : LAYER_W + id);
+    G[o] = s;
+    if (hG) hG[o] = s;
 }
 
 // FP32 input [V][cin] -> BF16 [V][16], zero padded
@@ -236,6 +359,12 @@ __global__ void k_selftest_bf16(float *out)
 }
 
 // ---------------------------------------------------------------- launchers
+static Shape shape(const Net &n, int layer)
+{
+    const int d = n.dil[layer];
+    return {n.nx, n.ny, n.nz, d < n.nx ? d : n.nx, d < n.ny ? d : n.ny, d < n.nz ? d : n.nz};
+}
+
 hipError_t conv_forward(const Net &n, int layer, const uint16_t *ain, uint16_t *aout, float *yout, hipStream_t s)
 {
     const int V = n.nx * n.ny * n.nz;
@@ -243,37 +372,37 @@ hipError_t conv_forward(const Net &n, int layer, const uint16_t *ain, uint16_t *
     const uint16_t *W = n.Wb + (size_t)layer * LAYER_W;
     const float *bias = n.P + (size_t)layer * LAYER_P + LAYER_W;
     if (layer < NL - 1)
-        hipLaunchKernelGGL(k_conv<FWD_RELU>, g, b, 0, s, n.nx, n.ny, n.nz, n.dil[layer], 1, ain, W, bias, nullptr, aout, nullptr, 16);
+        hipLaunchKernelGGL(k_conv<FWD_RELU>, g, b, 0, s, shape(n, layer), ain, W, bias, nullptr, aout, nullptr, nullptr, 16);
     else
-        hipLaunchKernelGGL(k_conv<FWD_LAST>, g, b, 0, s, n.nx, n.ny, n.nz, n.dil[layer], 1, ain, W, bias, nullptr, nullptr, yout, n.cout);
+        hipLaunchKernelGGL(k_conv<FWD_LAST>, g, b, 0, s, shape(n, layer), ain, W, bias, nullptr, nullptr, yout, nullptr, n.cout);
     return hipGetLastError();
 }
 
-hipError_t conv_input_grad(const Net &n, int layer, const uint16_t *dz, const uint16_t *mask, uint16_t *dzprev, hipStream_t s)
+hipError_t conv_loss(const Net &n, const uint16_t *ain, const float *tg, uint16_t *dz, hipStream_t s)
 {
-    const int V = n.nx * n.ny * n.nz;
-    const dim3 g((unsigned)((V + 63) / 64)), b(256);
-    hipLaunchKernelGGL(k_conv<BWD_MASK>, g, b, 0, s, n.nx, n.ny, n.nz, n.dil[layer], -1, dz, n.WTb + (size_t)layer * LAYER_W,
-                       nullptr, mask, dzprev, nullptr, 16);
+    const int V = n.nx * n.ny * n.nz, l = NL - 1;
+    hipLaunchKernelGGL(k_conv<FWD_LOSS>, dim3((unsigned)((V + 63) / 64)), dim3(256), 0, s, shape(n, l), ain,
+                       n.Wb + (size_t)l * LAYER_W, n.P + (size_t)l * LAYER_P + LAYER_W, tg, dz, nullptr, n.lpart, n.cout);
     return hipGetLastError();
 }
 
-hipError_t weight_grad(const Net &n, int layer, const uint16_t *ain, const uint16_t *dz, hipStream_t s)
+hipError_t layer_back(const Net &n, int layer, const uint16_t *ain, const uint16_t *dz, uint16_t *dzprev, hipStream_t s)
 {
-    const int V = n.nx * n.ny * n.nz;
-    hipLaunchKernelGGL(k_dw, dim3((unsigned)n.nchunk, 27), dim3(64), 0, s, n.nx, n.ny, n.nz, n.dil[layer], ain, dz, CHUNK, n.nchunk,
-                       n.part);
-    float *gW = n.G + (size_t)layer * LAYER_P;
-    hipLaunchKernelGGL(k_dw_reduce, dim3(27), dim3(256), 0, s, n.nchunk, n.part, gW);
-    hipLaunchKernelGGL(k_db, dim3((unsigned)n.nchunk), dim3(16), 0, s, V, dz, CHUNK, n.bpart);
-    hipLaunchKernelGGL(k_db_reduce, dim3(1), dim3(16), 0, s, n.nchunk, n.bpart, gW + LAYER_W);
+    const int V = n.nx * n.ny * n.nz, ncb = dzprev ? (V + 63) / 64 : 0, nb = ncb + 3 * n.nchunk;
+    float *part = n.part + (size_t)layer * 27 * n.nchunk * 256, *bpart = n.bpart + (size_t)layer * n.nchunk * 16;
+    if (dzprev)
+        hipLaunchKernelGGL(k_back<true>, dim3((unsigned)nb), dim3(256), 0, s, shape(n, layer), ncb, ain, dz,
+                           n.WTb + (size_t)layer * LAYER_W, dzprev, n.tw, n.nchunk, part, bpart);
+    else
+        hipLaunchKernelGGL(k_back<false>, dim3((unsigned)nb), dim3(256), 0, s, shape(n, layer), 0, ain, dz, nullptr, nullptr, n.tw,
+                           n.nchunk, part, bpart);
     return hipGetLastError();
 }
 
-hipError_t loss_grad(const Net &n, const float *y, const float *tg, uint16_t *dz, hipStream_t s)
+hipError_t grad_reduce(const Net &n, float *hG, double *hloss, hipStream_t s)
 {
     const int V = n.nx * n.ny * n.nz;
-    hipLaunchKernelGGL(k_loss, dim3((unsigned)((V * 16 + 255) / 256)), dim3(256), 0, s, V, n.cout, y, tg, dz, n.lpart);
+    hipLaunchKernelGGL(k_grad_reduce, dim3(29, NL), dim3(1024), 0, s, n.nchunk, n.part, n.bpart, (V + 15) / 16, n.lpart, n.G, hG, hloss);
     return hipGetLastError();
 }
 

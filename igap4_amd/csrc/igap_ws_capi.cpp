@@ -31,6 +31,7 @@ static void free_net(Net &n)
     void *bufs[] = {n.P, n.G, n.M, n.S, n.Wb, n.WTb, n.y, n.tg, n.x, n.part, n.bpart, n.lpart};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    if (n.hG) (void)hipHostFree(n.hG);
     for (int l = 0; l < W::NL; l++) {
         if (n.a[l]) (void)hipFree(n.a[l]);
         if (n.dz[l]) (void)hipFree(n.dz[l]);
@@ -59,7 +60,9 @@ extern "C" int igap_ws_create(int device, const int grid[3], int cin, int cout, 
     n.cout = cout;
     for (int l = 0; l < W::NL; l++) n.dil[l] = dil[l];
     const int V = (int)V64;
-    n.nchunk = (V + W::CHUNK - 1) / W::CHUNK;
+    const int ntile = (V + 15) / 16;
+    n.tw = (ntile + 4 * W::MAX_CHUNKS - 1) / (4 * W::MAX_CHUNKS);
+    n.nchunk = (ntile + 4 * n.tw - 1) / (4 * n.tw);
     const size_t np = (size_t)W::NL * W::LAYER_P;
     auto fail_free = [&](int rc) {
         free_net(n);
@@ -87,9 +90,11 @@ extern "C" int igap_ws_create(int device, const int grid[3], int cin, int cout, 
     WSCHK(hipMalloc(&n.y, sizeof(float) * (size_t)V * cout));
     WSCHK(hipMalloc(&n.tg, sizeof(float) * (size_t)V * cout));
     WSCHK(hipMalloc(&n.x, sizeof(float) * (size_t)V * cin));
-    WSCHK(hipMalloc(&n.part, sizeof(float) * 27 * (size_t)n.nchunk * 256));
-    WSCHK(hipMalloc(&n.bpart, sizeof(float) * (size_t)n.nchunk * 16));
-    WSCHK(hipMalloc(&n.lpart, sizeof(float) * (size_t)((V * 16 + 255) / 256)));
+    WSCHK(hipMalloc(&n.part, sizeof(float) * W::NL * 27 * (size_t)n.nchunk * 256));
+    WSCHK(hipMalloc(&n.bpart, sizeof(float) * W::NL * (size_t)n.nchunk * 16));
+    WSCHK(hipMalloc(&n.lpart, sizeof(float) * (size_t)ntile));
+    WSCHK(hipHostMalloc(&n.hG, sizeof(float) * np + sizeof(double), hipHostMallocDefault));
+    n.hloss = reinterpret_cast<double *>(n.hG + np);
     // parameters: He-uniform hidden layers over the real input channels, zero last layer
     std::vector<float> P(np, 0.f);
     uint64_t st = seed;
@@ -151,46 +156,41 @@ extern "C" int igap_ws_set_params(igap_ws_ctx *c, const float *params)
     return IGAP_OK;
 }
 
-static int forward(igap_ws_ctx *c, const float *x)
+// the packed input and layers 0 .. NL - 2
+static int hidden_layers(igap_ws_ctx *c, const float *x)
 {
     Net &n = c->n;
     const size_t V = (size_t)n.nx * n.ny * n.nz;
     HIPCHK(hipMemcpyAsync(n.x, x, sizeof(float) * V * n.cin, hipMemcpyHostToDevice, c->stream));
     HIPCHK(W::pack_input(n, n.x, n.a[0], c->stream));
     for (int l = 0; l < W::NL - 1; l++) HIPCHK(W::conv_forward(n, l, n.a[l], n.a[l + 1], nullptr, c->stream));
-    HIPCHK(W::conv_forward(n, W::NL - 1, n.a[W::NL - 1], nullptr, n.y, c->stream));
     return IGAP_OK;
 }
 
-// loss and parameter gradients into n.G (after forward)
-static int backward(igap_ws_ctx *c, const float *target, double *loss)
+// forward and backward: parameter gradients into n.G (and the pinned copy, if
+// the caller takes them), the sum of squared errors into *n.hloss
+static int loss_gradients(igap_ws_ctx *c, const float *x, const float *target, bool to_host)
 {
     Net &n = c->n;
     const size_t V = (size_t)n.nx * n.ny * n.nz;
     HIPCHK(hipMemcpyAsync(n.tg, target, sizeof(float) * V * n.cout, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(W::loss_grad(n, n.y, n.tg, n.dz[W::NL - 1], c->stream));
-    for (int l = W::NL - 1; l >= 0; l--) {
-        HIPCHK(W::weight_grad(n, l, n.a[l], n.dz[l], c->stream));
-        if (l > 0) HIPCHK(W::conv_input_grad(n, l, n.dz[l], n.a[l], n.dz[l - 1], c->stream));
-    }
-    if (loss) {
-        const int nb = (int)((V * 16 + 255) / 256);
-        std::vector<float> lp(nb);
-        HIPCHK(hipMemcpyAsync(lp.data(), n.lpart, sizeof(float) * nb, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(hipStreamSynchronize(c->stream));
-        double s = 0.0;
-        for (int i = 0; i < nb; i++) s += lp[i];
-        *loss = s / ((double)V * n.cout);
-    }
+    const int rc = hidden_layers(c, x);
+    if (rc) return rc;
+    HIPCHK(W::conv_loss(n, n.a[W::NL - 1], n.tg, n.dz[W::NL - 1], c->stream));
+    for (int l = W::NL - 1; l >= 0; l--) HIPCHK(W::layer_back(n, l, n.a[l], n.dz[l], l > 0 ? n.dz[l - 1] : nullptr, c->stream));
+    HIPCHK(W::grad_reduce(n, to_host ? n.hG : nullptr, n.hloss, c->stream));
     return IGAP_OK;
 }
+
+static double mean_loss(const Net &n) { return *n.hloss / ((double)n.nx * n.ny * n.nz * n.cout); }
 
 extern "C" int igap_ws_forward(igap_ws_ctx *c, const float *x, float *y)
 {
     if (!c || !x || !y) return igap::fail(IGAP_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(c->device));
-    int rc = forward(c, x);
+    int rc = hidden_layers(c, x);
     if (rc) return rc;
+    HIPCHK(W::conv_forward(c->n, W::NL - 1, c->n.a[W::NL - 1], nullptr, c->n.y, c->stream));
     const size_t V = (size_t)c->n.nx * c->n.ny * c->n.nz;
     HIPCHK(hipMemcpyAsync(y, c->n.y, sizeof(float) * V * c->n.cout, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -201,11 +201,11 @@ extern "C" int igap_ws_gradients(igap_ws_ctx *c, const float *x, const float *ta
 {
     if (!c || !x || !target || !grad) return igap::fail(IGAP_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(c->device));
-    int rc = forward(c, x);
-    if (!rc) rc = backward(c, target, loss);
+    const int rc = loss_gradients(c, x, target, true);
     if (rc) return rc;
-    HIPCHK(hipMemcpyAsync(grad, c->n.G, sizeof(float) * W::NL * W::LAYER_P, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(grad, c->n.hG, sizeof(float) * W::NL * W::LAYER_P);
+    if (loss) *loss = mean_loss(c->n);
     return IGAP_OK;
 }
 
@@ -213,8 +213,7 @@ extern "C" int igap_ws_train_step(igap_ws_ctx *c, const float *x, const float *t
 {
     if (!c || !x || !target) return igap::fail(IGAP_ERR_ARG, "null argument");
     HIPCHK(hipSetDevice(c->device));
-    int rc = forward(c, x);
-    if (!rc) rc = backward(c, target, loss);
+    const int rc = loss_gradients(c, x, target, false);
     if (rc) return rc;
     Net &n = c->n;
     n.step++;
@@ -222,6 +221,7 @@ extern "C" int igap_ws_train_step(igap_ws_ctx *c, const float *x, const float *t
     HIPCHK(W::adam(n, lr, c1, c2, c->stream));
     HIPCHK(W::pack_weights(n, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
+    if (loss) *loss = mean_loss(n);
     return IGAP_OK;
 }
 

@@ -11,13 +11,13 @@ constexpr int NL = 4;                  // convolution layers
 constexpr int CH = 16;                 // channels between layers (and padded in/out)
 constexpr int LAYER_W = 27 * CH * CH;  // weights of one layer
 constexpr int LAYER_P = LAYER_W + CH;  // weights + bias
-constexpr int CHUNK = 512;             // voxels per weight-gradient partial
+constexpr int MAX_CHUNKS = 128;        // weight-gradient partials per layer at most
 constexpr float ADAM_B1 = 0.9f, ADAM_B2 = 0.999f, ADAM_EPS = 1e-8f;
 
 struct Net {
     int nx = 0, ny = 0, nz = 0, cin = 0, cout = 0;
     int dil[NL] = {1, 1, 1, 1};
-    int nchunk = 0;
+    int tw = 0, nchunk = 0;             // weight gradients: tiles of 16 voxels per wave, chunks of 4 tw tiles
     int64_t step = 0;                   // Adam step count
     float *P = nullptr, *G = nullptr, *M = nullptr, *S = nullptr;   // FP32 params, grads, moments
     uint16_t *Wb = nullptr, *WTb = nullptr;                          // BF16 weight copies
@@ -25,12 +25,17 @@ struct Net {
     uint16_t *dz[NL] = {};              // gradients w.r.t. each layer's pre-activation output
     float *y = nullptr, *tg = nullptr, *x = nullptr;
     float *part = nullptr, *bpart = nullptr, *lpart = nullptr;
+    float *hG = nullptr;                // pinned host memory: gradients, then the loss sum (8-byte aligned)
+    double *hloss = nullptr;
 };
 
 hipError_t conv_forward(const Net &n, int layer, const uint16_t *ain, uint16_t *aout, float *yout, hipStream_t s);
-hipError_t conv_input_grad(const Net &n, int layer, const uint16_t *dz, const uint16_t *mask, uint16_t *dzprev, hipStream_t s);
-hipError_t weight_grad(const Net &n, int layer, const uint16_t *ain, const uint16_t *dz, hipStream_t s);
-hipError_t loss_grad(const Net &n, const float *y, const float *tg, uint16_t *dz, hipStream_t s);
+// the last layer, its loss partials and the gradient of its output in one launch
+hipError_t conv_loss(const Net &n, const uint16_t *ain, const float *tg, uint16_t *dz, hipStream_t s);
+// weight and bias partials of a layer and, with dzprev, its input gradient
+hipError_t layer_back(const Net &n, int layer, const uint16_t *ain, const uint16_t *dz, uint16_t *dzprev, hipStream_t s);
+// G of every layer and the sum of squared errors; hG (pinned) may be null
+hipError_t grad_reduce(const Net &n, float *hG, double *hloss, hipStream_t s);
 hipError_t pack_input(const Net &n, const float *x, uint16_t *a, hipStream_t s);
 hipError_t pack_weights(const Net &n, hipStream_t s);
 hipError_t adam(const Net &n, float lr, float c1, float c2, hipStream_t s);

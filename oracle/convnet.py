@@ -46,6 +46,8 @@ def shift(a, dx, dy, dz):
     """s[x,y,z] = a[x+dx, y+dy, z+dz] with zeros outside the grid."""
     nx, ny, nz = a.shape[:3]
     s = np.zeros_like(a)
+    if abs(dx) >= nx or abs(dy) >= ny or abs(dz) >= nz:
+        return s
     xs = slice(max(0, -dx), min(nx, nx - dx))
     ys = slice(max(0, -dy), min(ny, ny - dy))
     zs = slice(max(0, -dz), min(nz, nz - dz))

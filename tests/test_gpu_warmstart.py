@@ -171,3 +171,41 @@ def test_residual_training_lowers_the_candidate_residual(ws):
         print(arm, s[arm])
         assert s[arm]["all_converged"]
         assert s[arm]["final_rel_diff_vs_plain"] < 1e-8
+
+
+# grids below one 16-point tile, of a ragged last tile, with axes of one point
+# and dilations beyond the grid, and of enough points (over 8192) for a wave of
+# the weight gradients to take several tiles
+@pytest.mark.parametrize("grid,cin,cout,dil", [
+    ((3, 2, 2), 9, 3, (1, 2, 4, 1)),
+    ((1, 1, 17), 1, 1, (1, 40, 2, 1)),
+    ((5, 7, 3), 16, 16, (2, 1, 9, 3)),
+    ((16, 8, 4), 9, 3, (1, 1, 1, 1)),
+    ((33, 18, 15), 9, 3, (1, 2, 4, 1)),
+])
+def test_gradients_at_the_edges_of_tiles(ws, grid, cin, cout, dil):
+    """Loss and gradients against the oracle.  An FP32 sum of 432 products is off by
+    about 6e-7, so about 3e-4 of the activations round to the other BF16 neighbour
+    (2^-8) than the oracle's: 7e-5 a layer, a few layers deep; a tap or a point
+    that is missing is 1e-2 and more."""
+    rng = np.random.default_rng(7)
+    p = np.zeros(cn.NL * cn.LAYER_P, dtype=np.float32)
+    for l in range(cn.NL):
+        o = l * cn.LAYER_P
+        ci, co = (cin if l == 0 else cn.CH), (cout if l == cn.NL - 1 else cn.CH)
+        W = np.zeros((27, cn.CH, cn.CH))
+        W[:, :co, :ci] = rng.uniform(-1, 1, (27, co, ci)) * np.sqrt(6.0 / (27 * ci))
+        p[o:o + cn.LAYER_W] = W.reshape(-1)
+        p[o + cn.LAYER_W:o + cn.LAYER_W + co] = rng.standard_normal(co) * 0.05
+    V = int(np.prod(grid))
+    x = rng.standard_normal((V, cin)).astype(np.float32)
+    t = rng.standard_normal((V, cout)).astype(np.float32)
+    with ws.WarmStartNet(grid, cin, cout, dil) as net:
+        net.set_params(p)
+        loss, g = net.gradients(x, t)
+    loss_ref, g_ref = cn.gradients(p, x, t, grid, cin, cout, dil, emulate=True)
+    assert abs(loss - loss_ref) < 1e-3 * loss_ref
+    for l in range(cn.NL):
+        o = l * cn.LAYER_P
+        for sl in (slice(o, o + cn.LAYER_W), slice(o + cn.LAYER_W, o + cn.LAYER_P)):
+            assert np.linalg.norm(g[sl] - g_ref[sl]) <= 1e-3 * np.linalg.norm(g_ref[sl])
