@@ -57,8 +57,19 @@ enum { FWD_RELU = 0, FWD_LAST = 1, BWD_MASK = 2, FWD_LOSS = 3 };
 // One tap's offset along each axis (the dilation, clamped to the grid's size
 // there: a tap that far off is outside either way, and the products of the
 // offsets then stay within 32 bits).
+// myz, mz: reciprocals 2^64 / d of ny nz and nz, rounded up (0 for d = 1): the
+// upper half of v m is v / d for every v d < 2^64.  (The 32-bit divisions of a
+// run-time divisor were much of a weight-gradient wave's instructions: k_back 18.1 -> 16.7 us.)
 struct Shape {
     int nx, ny, nz, dx, dy, dz;
+    uint64_t myz, mz;
+    __device__ __forceinline__ void point(int v, int &x, int &y, int &z) const
+    {
+        const int r = mz ? (int)__umul64hi((uint64_t)(uint32_t)v, mz) : v;
+        x = myz ? (int)__umul64hi((uint64_t)(uint32_t)v, myz) : v;
+        y = r - x * ny;
+        z = v - r * nz;
+    }
 };
 
 // Where the tiles of a lane's voxel lie: the voxel's first channel of the
@@ -72,7 +83,8 @@ struct Taps {
         const bool vin = v < V;
         if (!vin) v = V - 1;
         base = v * 16 + 4 * kg;
-        const int x = v / (g.ny * g.nz), y = (v / g.nz) % g.ny, z = v % g.nz;
+        int x, y, z;
+        g.point(v, x, y, z);
 #pragma unroll
         for (int t = 0; t < 3; t++) {
             const int s = sgn * (t - 1), xx = x + s * g.dx, yy = y + s * g.dy, zz = z + s * g.dz;
@@ -191,120 +203,128 @@ struct Transposer {
 };
 
 // Backward step of one layer.  Blocks 0 .. ncb - 1 (CONV): the input gradient,
-// as k_conv.  The others: the gradients of the weights and the bias, as partials
-// of one chunk of 4 tw tiles of 16 voxels and the nine taps of one x offset,
+// as k_conv.  The others: the gradients of the weights and the bias, one wave per
+// chunk of CHUNK voxels and tap (t = 27: the bias),
 //   part[t][c][ci][co] = sum_{v in chunk c} a[v + off_t][ci] dz[v][co]
-//   bpart[c][co]       = sum_{v in chunk c} dz[v][co]           (x offset 0)
-// with M = ci, N = co, K = 16 voxels of a product.  Tiles are read as the
-// convolution reads them (eight bytes a lane) and transposed in registers; the
-// four waves of a block take tw tiles each and add up in LDS.  The gradient of
-// layer l - 1 needs only the input gradient, so both run in one launch.
-// At 66x18x18 one wave per (tap, 512 voxels) gathering two bytes at a time took
-// 42 us a layer for the weights and 16-thread blocks 36 us for the bias;
-// now 11.8 us with the input gradient (13 us before) beside, 8.5 us without.
+//   bpart[c][co]       = sum_{v in chunk c} dz[v][co]
+// with M = ci, N = co, K = 16 voxels of a product, the chunk's tiles in order.
+// Tiles are read as the convolution reads them (eight bytes a lane, eight tiles
+// in flight) and transposed in registers.  The gradient of layer l - 1 needs
+// only the input gradient, so both run in one launch.
+// At 66x18x18 gathering two bytes a lane and tile at a time took 42 us a
+// layer for the weights and a loop over single voxels 36 us for the bias;
+// now 14.1 us with the input gradient (13 us before) beside, 11.6 us without.
 template <bool CONV>
 __global__ __launch_bounds__(256) void k_back(Shape g, int ncb, const uint16_t *__restrict__ ain, const uint16_t *__restrict__ dz,
-                                              const uint16_t *__restrict__ WTk, uint16_t *__restrict__ dzprev, int tw, int nchunk,
+                                              const uint16_t *__restrict__ WTk, uint16_t *__restrict__ dzprev, int nchunk,
                                               float *__restrict__ part, float *__restrict__ bpart)
 {
-    __shared__ float4_t red[3][10][64];
+    __shared__ uint4 sdz[CHUNK * 32 / 16];   // one wave's: the bias sums of a chunk
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (CONV && (int)blockIdx.x < ncb) {
         // the mask of the ReLU that made this layer's input is that input
         conv_tile<BWD_MASK>(g, blockIdx.x * 4 + wv, lane, -1, dz, WTk, nullptr, ain, nullptr, dzprev, nullptr, nullptr, 16);
         return;
     }
-    const int V = g.nx * g.ny * g.nz, ntile = (V + 15) / 16;
-    const int bb = blockIdx.x - ncb, c = bb / 3, tx = bb - 3 * c;
+    static_assert(CHUNK % 128 == 0, "eight tiles a round");
+    const int V = g.nx * g.ny * g.nz;
+    const int bb = blockIdx.x - ncb, c = bb / 7, t = __builtin_amdgcn_readfirstlane(4 * (bb - 7 * c) + wv);
     const int i = lane & 15, kg = lane >> 4;
+    const int vbeg = c * CHUNK, vend = vbeg + CHUNK < V ? vbeg + CHUNK : V;
+    if (t == 27) {
+        // the whole chunk in flight at once; the sum itself is a chain of CHUNK additions per channel
+        constexpr int NL16 = CHUNK * 32 / (64 * 16);
+        uint4 d[NL16];
+#pragma unroll
+        for (int j = 0; j < NL16; j++) {
+            const int at = (j * 64 + lane) / 2, v = vbeg + at < V ? vbeg + at : V - 1;   // half a voxel a lane
+            d[j] = *reinterpret_cast<const uint4 *>(dz + (size_t)v * 16 + 8 * (lane & 1));
+        }
+#pragma unroll
+        for (int j = 0; j < NL16; j++) sdz[j * 64 + lane] = d[j];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const uint16_t *q = reinterpret_cast<const uint16_t *>(sdz) + i;
+        const int n = vend - vbeg;
+        float s = 0.f;
+        int v = 0;
+        for (; v + 32 <= n; v += 32) {
+            uint16_t e[32];
+#pragma unroll
+            for (int j = 0; j < 32; j++) e[j] = q[16 * (v + j)];
+#pragma unroll
+            for (int j = 0; j < 32; j++) s += bf2f(e[j]);
+        }
+        for (; v < n; v++) s += bf2f(q[16 * v]);
+        if (kg == 0) bpart[c * 16 + i] = s;
+        return;
+    }
     const Transposer tr(lane);
-    const short one = 0x3f80;   // 1 in BF16
-    float4_t acc[10];
+    const int tx = t / 9 - 1, ty = (t / 3) % 3 - 1, tz = t % 3 - 1;
+    const int sx = tx * g.dx, sy = ty * g.dy, sz = tz * g.dz, off = (sx * (g.ny * g.nz) + sy * g.nz + sz) * 16;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    for (int vb = vbeg; vb < vend; vb += 128) {
+        short4_t a[8], d[8];
+        bool ok[8], in[8];
 #pragma unroll
-    for (int t = 0; t < 10; t++) acc[t] = (float4_t){0.f, 0.f, 0.f, 0.f};
-    const int beg = (c * 4 + wv) * tw, end = beg + tw < ntile ? beg + tw : ntile;
-    for (int tile = beg; tile < end; tile++) {
-        const int v = tile * 16 + i;
-        const Taps tp(g, v, V, kg, 1);
-        // the nine taps of this x offset: in range along x, and along y and z
-        const bool okx = tx == 0 ? tp.in[0][0] : (tx == 1 ? tp.in[0][1] : tp.in[0][2]);
-        const uint16_t *a0 = ain + tp.base;
-        const int offx = (tx - 1) * g.dx * (g.ny * g.nz);
-        short4_t a[9];
-        short4_t d = *reinterpret_cast<const short4_t *>(dz + tp.base);
-#pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const bool ok = okx && tp.in[1][t / 3] && tp.in[2][t % 3];
-            const int off = (offx + (t / 3 - 1) * g.dy * g.nz + (t % 3 - 1) * g.dz) * 16;
-            a[t] = *reinterpret_cast<const short4_t *>(a0 + (ok ? off : 0));
+        for (int j = 0; j < 8; j++) {
+            int v = vb + 16 * j + i;
+            in[j] = v < vend;
+            if (!in[j]) v = V - 1;
+            int x, y, z;
+            g.point(v, x, y, z);
+            x += sx;
+            y += sy;
+            z += sz;
+            ok[j] = in[j] && x >= 0 && x < g.nx && y >= 0 && y < g.ny && z >= 0 && z < g.nz;
+            const int base = v * 16 + 4 * kg;
+            a[j] = *reinterpret_cast<const short4_t *>(ain + (base + (ok[j] ? off : 0)));
+            d[j] = *reinterpret_cast<const short4_t *>(dz + base);
         }
-        if (v >= V) d = (short4_t){0, 0, 0, 0};
-        const short4_t b = tr(d);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < 9; t++) {
-            const bool ok = okx && tp.in[1][t / 3] && tp.in[2][t % 3];
-            acc[t] = mma(tr(ok ? a[t] : (short4_t){0, 0, 0, 0}), b, acc[t]);
+        for (int j = 0; j < 8; j++) {
+            const short4_t zero = {0, 0, 0, 0};
+            if (vb + 16 * j < vend) acc = mma(tr(ok[j] ? a[j] : zero), tr(in[j] ? d[j] : zero), acc);
         }
-        if (tx == 1) acc[9] = mma((short4_t){one, one, one, one}, b, acc[9]);
     }
-    if (wv > 0) {
+    // lane (co = i): ci = 4 kg + r, stored [ci][co]
+    float *o = part + (((size_t)t * nchunk + c) * 16 + 4 * kg) * 16 + i;
 #pragma unroll
-        for (int t = 0; t < 10; t++) red[wv - 1][t][lane] = acc[t];
-    }
-    __syncthreads();
-    if (wv > 0) return;
-#pragma unroll
-    for (int t = 0; t < 10; t++) acc[t] = ((acc[t] + red[0][t][lane]) + red[1][t][lane]) + red[2][t][lane];
-#pragma unroll
-    for (int t = 0; t < 9; t++) {
-        // lane (co = i): ci = 4 kg + r, stored [ci][co]
-        float *o = part + (((size_t)(9 * tx + t) * nchunk + c) * 16 + 4 * kg) * 16 + i;
-#pragma unroll
-        for (int r = 0; r < 4; r++) o[16 * r] = acc[t][r];
-    }
-    if (tx == 1 && kg == 0) bpart[c * 16 + i] = acc[9][0];
+    for (int r = 0; r < 4; r++) o[16 * r] = acc[r];
 }
 
-// The sums over chunks, every layer in one launch (grid.y = layer): blocks
-// 0..26 one tap of the weights, grad W[t][co][ci] = sum_c part[t][c][ci][co];
+// The sums over chunks (in order), every layer in one launch (grid.y = layer):
+// blocks 0..26 one tap of the weights, grad W[t][co][ci] = sum_c part[t][c][ci][co];
 // block 27 the bias, and for layer 0 block 28 the sum of the loss partials (in
-// FP64).  Four groups of 256 threads take a quarter of the chunks each, every
-// quarter in order.  The gradients go to the device copy and, where the caller
-// takes them (hG), straight to pinned host memory.
-__global__ __launch_bounds__(1024) void k_grad_reduce(int nchunk, const float *__restrict__ part, const float *__restrict__ bpart,
-                                                      int ntile, const float *__restrict__ lpart, float *__restrict__ G,
-                                                      float *__restrict__ hG, double *__restrict__ hloss)
+// FP64).  The gradients go to the device copy and, where the caller takes them
+// (hG), straight to pinned host memory.
+__global__ __launch_bounds__(256) void k_grad_reduce(int nchunk, const float *__restrict__ part, const float *__restrict__ bpart,
+                                                     int ntile, const float *__restrict__ lpart, float *__restrict__ G,
+                                                     float *__restrict__ hG, double *__restrict__ hloss)
 {
-    __shared__ double dred[1024];
-    float *red = reinterpret_cast<float *>(dred);
+    __shared__ double dred[256];
     const int l = blockIdx.y, t = blockIdx.x, tid = threadIdx.x;
     if (t == 28) {
         if (l > 0) return;
         double s = 0.0;
-        for (int i = tid; i < ntile; i += 1024) s += lpart[i];
+        for (int i = tid; i < ntile; i += 256) s += lpart[i];
         dred[tid] = s;
         __syncthreads();
-        for (int o = 512; o > 0; o >>= 1) {
+        for (int o = 128; o > 0; o >>= 1) {
             if (tid < o) dred[tid] += dred[tid + o];
             __syncthreads();
         }
         if (tid == 0) *hloss = dred[0];
         return;
     }
-    const int n = t < 27 ? 256 : 16, id = tid & 255, grp = tid >> 8;
-    const int per = (nchunk + 3) / 4, c0 = grp * per, c1 = c0 + per < nchunk ? c0 + per : nchunk;
-    const float *p = t < 27 ? part + (((size_t)l * 27 + t) * nchunk) * 256 + id : bpart + (size_t)l * nchunk * 16 + id;
+    const int n = t < 27 ? 256 : 16;
+    if (tid >= n) return;
+    const float *p = t < 27 ? part + (((size_t)l * 27 + t) * nchunk) * 256 + tid : bpart + (size_t)l * nchunk * 16 + tid;
     float s = 0.f;
-    if (id < n) {
-#pragma unroll 8
-        for (int c = c0; c < c1; c++) s += p[(size_t)c * n];
-    }
-    red[tid] = s;
-    __syncthreads();
-    if (grp > 0 || id >= n) return;
-    s = ((red[id] + red[id + 256]) + red[id + 512]) + red[id + 768];
-    // id = ci*16 + co of a tap, co of the bias
-    const size_t o = (size_t)l * LAYER_P + (t < 27 ? t * 256 + (id & 15) * 16 + (id >> 4) : LAYER_W + id);
+#pragma unroll 16
+    for (int c = 0; c < nchunk; c++) s += p[(size_t)c * n];
+    // tid = ci*16 + co of a tap, co of the bias
+    const size_t o = (size_t)l * LAYER_P + (t < 27 ? t * 256 + (tid & 15) * 16 + (tid >> 4) : LAYER_W + tid);
     G[o] = s;
     if (hG) hG[o] = s;
 }
@@ -362,7 +382,8 @@ __global__ void k_selftest_bf16(float *out)
 static Shape shape(const Net &n, int layer)
 {
     const int d = n.dil[layer];
-    return {n.nx, n.ny, n.nz, d < n.nx ? d : n.nx, d < n.ny ? d : n.ny, d < n.nz ? d : n.nz};
+    auto recip = [](uint64_t q) { return q > 1 ? ~0ull / q + 1 : 0ull; };   // ceil(2^64 / q)
+    return {n.nx, n.ny, n.nz, d < n.nx ? d : n.nx, d < n.ny ? d : n.ny, d < n.nz ? d : n.nz, recip((uint64_t)n.ny * n.nz), recip(n.nz)};
 }
 
 hipError_t conv_forward(const Net &n, int layer, const uint16_t *ain, uint16_t *aout, float *yout, hipStream_t s)
@@ -388,13 +409,13 @@ hipError_t conv_loss(const Net &n, const uint16_t *ain, const float *tg, uint16_
 
 hipError_t layer_back(const Net &n, int layer, const uint16_t *ain, const uint16_t *dz, uint16_t *dzprev, hipStream_t s)
 {
-    const int V = n.nx * n.ny * n.nz, ncb = dzprev ? (V + 63) / 64 : 0, nb = ncb + 3 * n.nchunk;
+    const int V = n.nx * n.ny * n.nz, ncb = dzprev ? (V + 63) / 64 : 0, nb = ncb + 7 * n.nchunk;
     float *part = n.part + (size_t)layer * 27 * n.nchunk * 256, *bpart = n.bpart + (size_t)layer * n.nchunk * 16;
     if (dzprev)
         hipLaunchKernelGGL(k_back<true>, dim3((unsigned)nb), dim3(256), 0, s, shape(n, layer), ncb, ain, dz,
-                           n.WTb + (size_t)layer * LAYER_W, dzprev, n.tw, n.nchunk, part, bpart);
+                           n.WTb + (size_t)layer * LAYER_W, dzprev, n.nchunk, part, bpart);
     else
-        hipLaunchKernelGGL(k_back<false>, dim3((unsigned)nb), dim3(256), 0, s, shape(n, layer), 0, ain, dz, nullptr, nullptr, n.tw,
+        hipLaunchKernelGGL(k_back<false>, dim3((unsigned)nb), dim3(256), 0, s, shape(n, layer), 0, ain, dz, nullptr, nullptr,
                            n.nchunk, part, bpart);
     return hipGetLastError();
 }
@@ -402,7 +423,7 @@ hipError_t layer_back(const Net &n, int layer, const uint16_t *ain, const uint16
 hipError_t grad_reduce(const Net &n, float *hG, double *hloss, hipStream_t s)
 {
     const int V = n.nx * n.ny * n.nz;
-    hipLaunchKernelGGL(k_grad_reduce, dim3(29, NL), dim3(1024), 0, s, n.nchunk, n.part, n.bpart, (V + 15) / 16, n.lpart, n.G, hG, hloss);
+    hipLaunchKernelGGL(k_grad_reduce, dim3(29, NL), dim3(256), 0, s, n.nchunk, n.part, n.bpart, (V + 15) / 16, n.lpart, n.G, hG, hloss);
     return hipGetLastError();
 }
 

@@ -61,8 +61,7 @@ extern "C" int igap_ws_create(int device, const int grid[3], int cin, int cout, 
     for (int l = 0; l < W::NL; l++) n.dil[l] = dil[l];
     const int V = (int)V64;
     const int ntile = (V + 15) / 16;
-    n.tw = (ntile + 4 * W::MAX_CHUNKS - 1) / (4 * W::MAX_CHUNKS);
-    n.nchunk = (ntile + 4 * n.tw - 1) / (4 * n.tw);
+    n.nchunk = (V + W::CHUNK - 1) / W::CHUNK;
     const size_t np = (size_t)W::NL * W::LAYER_P;
     auto fail_free = [&](int rc) {
         free_net(n);

@@ -11,13 +11,13 @@ constexpr int NL = 4;                  // convolution layers
 constexpr int CH = 16;                 // channels between layers (and padded in/out)
 constexpr int LAYER_W = 27 * CH * CH;  // weights of one layer
 constexpr int LAYER_P = LAYER_W + CH;  // weights + bias
-constexpr int MAX_CHUNKS = 128;        // weight-gradient partials per layer at most
+constexpr int CHUNK = 512;             // voxels per weight-gradient partial
 constexpr float ADAM_B1 = 0.9f, ADAM_B2 = 0.999f, ADAM_EPS = 1e-8f;
 
 struct Net {
     int nx = 0, ny = 0, nz = 0, cin = 0, cout = 0;
     int dil[NL] = {1, 1, 1, 1};
-    int tw = 0, nchunk = 0;             // weight gradients: tiles of 16 voxels per wave, chunks of 4 tw tiles
+    int nchunk = 0;
     int64_t step = 0;                   // Adam step count
     float *P = nullptr, *G = nullptr, *M = nullptr, *S = nullptr;   // FP32 params, grads, moments
     uint16_t *Wb = nullptr, *WTb = nullptr;                          // BF16 weight copies

@@ -174,8 +174,8 @@ def test_residual_training_lowers_the_candidate_residual(ws):
 
 
 # grids below one 16-point tile, of a ragged last tile, with axes of one point
-# and dilations beyond the grid, and of enough points (over 8192) for a wave of
-# the weight gradients to take several tiles
+# and dilations beyond the grid, of exactly one chunk of the weight gradients
+# and of many with a ragged last one
 @pytest.mark.parametrize("grid,cin,cout,dil", [
     ((3, 2, 2), 9, 3, (1, 2, 4, 1)),
     ((1, 1, 17), 1, 1, (1, 40, 2, 1)),
