@@ -1134,8 +1134,9 @@ __global__ __launch_bounds__(64) void k_sep_tables(MeshK M, double *__restrict__
         const int64_t id = d == 0 ? (int64_t)M.na[1] * M.na[2] * (e + b) : d == 1 ? (int64_t)M.na[2] * (e + b) : e + b;
         xc[b] = M.X[3 * id + d];
     }
-    const double g = t[3] * xc[0] + t[4] * xc[1] + t[5] * xc[2];
-    const double gp = t[6] * xc[0] + t[7] * xc[1] + t[8] * xc[2];
+    // (parametric tables of a patch that is not separable: g = 1, g' = 0)
+    const double g = M.separable ? t[3] * xc[0] + t[4] * xc[1] + t[5] * xc[2] : 1.0;
+    const double gp = M.separable ? t[6] * xc[0] + t[7] * xc[1] + t[8] * xc[2] : 0.0;
     const double ig = 1.0 / g, r = gp * ig;
     double *o = tab + (int64_t)(first + e) * TAB_STRIDE;
     float *of = tabf + (int64_t)(first + e) * TAB_STRIDE;
@@ -1154,9 +1155,9 @@ __global__ __launch_bounds__(64) void k_sep_tables(MeshK M, double *__restrict__
 }
 
 // Per-element set-up on a separable patch (at least 256 threads, no barrier):
-// the 27 control displacements -> sU[27][3], the tables of the element's three
+// the 27 control displacements -> sU[27][STR], the tables of the element's three
 // 1-D elements -> sPd[d][q][order][i] and their point weights -> sW[d][q].
-template <int NH = 1>
+template <int NH = 1, int STR = 3>
 __device__ __forceinline__ void sep_element(const MeshK &M, const double *__restrict__ Uh, const int *ed, double *sU,
                                             double (*sPd)[4][3][3], double (*sW)[4], int64_t ndof = 0,
                                             double *sUd = nullptr, double *sV = nullptr, double cv1 = 0.0, double cv2 = 0.0)
@@ -1168,7 +1169,7 @@ __device__ __forceinline__ void sep_element(const MeshK &M, const double *__rest
                          + (int64_t)M.nb[2] * own1(ed[1] + by, M.nb[1], M.periodic[1]) + own1(ed[2] + bz, M.nb[2], M.periodic[2]);
         if (NH == 1) {
 #pragma unroll
-            for (int k = 0; k < 3; k++) sU[3 * tid + k] = Uh[3 * oc + k];
+            for (int k = 0; k < 3; k++) sU[STR * tid + k] = Uh[3 * oc + k];
         } else {
             // the transient rule's two fields: Um = (U^1 + U^2)/2 -> sU and
             // Ud = (U - U^2)/2 -> sUd (rule node j: Um + s_j Ud); with sV, the
@@ -1435,6 +1436,201 @@ __global__ __launch_bounds__((SepShape<T, 1>::THREADS), (SepPipe<T, 1>::OCC)) vo
         sep_states(P, J, sW, sSt);
     }
     const StaticIn in{sSt, P.e345, P.le};
+    auto out = [&](int p, int bc, int cy, const T *K) {
+        sep_write<T, DIRECT>(M, Ke, e, ed[0], ed[1], ed[2], p, bc, cy, K, sRow, sMsk);
+    };
+    sep_pipeline<T, Sh>(sX, taby + ed[1] * TAB_STRIDE, tabz + ed[2] * TAB_STRIDE, sD, sE, in, out);
+}
+
+// Static tangent of a patch with equal weights and any geometry (k_tangent_gen):
+// the basis is a tensor product in the parametric directions, so the pipeline of
+// k_tangent_sep contracts the parametric tables, and GeneralIn pulls the
+// pointwise tangent back to parametric slots.  Set-up: the jets of the three
+// coordinates and the three displacements by sum factorisation (one wave per
+// field in the last pass), then per point the map's inverse gradient,
+// connection and metric (one wave) and the physical displacement jets (three),
+// then the strain-measure state.
+// Bound by the SIMD that holds the D wave (870 vector instructions an interval
+// beside a z wave's 180; the y/z SIMDs have 620).  64x16x16, FP64: 3.47 ms for
+// k_tangent_elem, whose matrix-core product of 27 x 27 per point and jet slot alone
+// is 55k cycles an element and CU, 2.05 ms here.  A rational basis (unequal
+// weights) needs the value slot too and stays with k_tangent_elem.
+template <typename T> struct GenPipe;
+template <> struct GenPipe<double> { typedef PipeShape<2, 1, 1, false, true> S; };
+template <> struct GenPipe<float> { typedef PipeShape<2, 1, 2, false, true> S; };
+
+// field passes of k_tangent_gen: c[b][f] the six nodal fields (x, u), sWork 6 *
+// (108 + 288) doubles; lane q of wave f < 6 returns the parametric jet of field f at point q
+__device__ __forceinline__ void gen_fields(const double (*c)[6], const double (*sPd)[4][3][3], double *sWork, double *J)
+{
+    const int tid = threadIdx.x;
+    double *sA = sWork, *sB = sA + 6 * 108;
+    if (tid < 216) {
+        const int qz = tid & 3, g = tid >> 2, f = g / 9, bxy = g - 9 * f;
+        const double c0 = c[3 * bxy][f], c1 = c[3 * bxy + 1][f], c2 = c[3 * bxy + 2][f];
+        double *o = sA + 108 * f + 12 * bxy + 3 * qz;
+#pragma unroll
+        for (int dz = 0; dz < 3; dz++) {
+            const double *tz = &sPd[2][qz][dz][0];
+            o[dz] = c0 * tz[0] + c1 * tz[1] + c2 * tz[2];
+        }
+    }
+    __syncthreads();
+    if (tid < 288) {
+        const int qz = tid & 3, qy = (tid >> 2) & 3, g = tid >> 4, f = g / 3, bx = g - 3 * f;
+        const double *a = sA + 108 * f + 36 * bx + 3 * qz;   // a[12 by + dz]
+        double *o = sB + 288 * f + 96 * bx + 24 * qy + 6 * qz;
+#pragma unroll
+        for (int s6 = 0; s6 < 6; s6++) {
+            const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
+            const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
+            const double *ty = &sPd[1][qy][dy][0];
+            o[s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
+        }
+    }
+    __syncthreads();
+    const int q = tid & 63, f = tid >> 6;
+    if (f < 6) sf_jet(sB + 288 * f + (q & 15) * 6, &sPd[0][q >> 4][0][0], J);
+}
+
+// the states of GeneralIn at the 64 points (eight waves; J as gen_fields leaves it); ends with a block barrier
+__device__ __forceinline__ void gen_states(const MeshK &M, const PhysK &P, const int *ed, double *J, const double (*sW)[4], double *sSt)
+{
+    constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+    constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
+    const int tid = threadIdx.x, q = tid & 63, part = tid >> 6;
+    double *sp = sSt + q * GST_W;
+    // the coordinates' jets wait in the places of S, N and G
+    if (part < 3) {
+#pragma unroll
+        for (int a = 0; a < 9; a++) sp[GST_S + 9 * part + a] = J[1 + a];
+    }
+    __syncthreads();
+    if (part >= 3 && part < 7) {
+        double G[9], Gi[9], X2[18];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+#pragma unroll
+            for (int i = 0; i < 3; i++) G[3 * d + i] = sp[GST_S + 9 * d + i];
+#pragma unroll
+            for (int s = 0; s < 6; s++) X2[6 * d + s] = sp[GST_S + 9 * d + 3 + s];
+        }
+        const double det = inv3(G, Gi);
+        if (part < 6) {
+            const int k = part - 3;
+            double xq[3];
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double *kV = M.knot[d] + ed[d];
+                const double c = M.gq[d == 0 ? q >> 4 : d == 1 ? (q >> 2) & 3 : q & 3];
+                xq[d] = (-c + 1.0) * kV[2] + c * kV[3];
+            }
+            phys_jet(J, Gi, X2);
+            add_periodic1(M, xq, k, J);
+#pragma unroll
+            for (int i = 0; i < 3; i++) sp[10 * k + i] = J[1 + i] + (k == i ? 1.0 : 0.0);
+#pragma unroll
+            for (int t = 0; t < 6; t++) sp[10 * k + 4 + t] = J[4 + t];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 9; i++) sp[GST_GI + i] = Gi[i];
+            sp[GST_WGT] = sep_weight(q, sW) * det;
+#pragma unroll
+            for (int n = 0; n < 3; n++)
+#pragma unroll
+                for (int s = 0; s < 6; s++)
+                    sp[GST_GA + 6 * n + s] = Gi[3 * n] * X2[s] + Gi[3 * n + 1] * X2[6 + s] + Gi[3 * n + 2] * X2[12 + s];
+#pragma unroll
+            for (int s = 0; s < 6; s++)
+                sp[GST_M + s] = Gi[3 * PI[s]] * Gi[3 * PK[s]] + Gi[3 * PI[s] + 1] * Gi[3 * PK[s] + 1] + Gi[3 * PI[s] + 2] * Gi[3 * PK[s] + 2];
+        }
+    }
+    __syncthreads();
+    if (part < 4) {
+        double F[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) F[i] = sp[10 * (i / 3) + i % 3];
+        const double w = sp[GST_WGT];
+        if (part < 3) {
+            // row L = part of G_LK = 2 le^2 (E_LL,K - their mean over L), its second index pulled back
+            const int L = part;
+            const double g = w * 2 * P.le * P.le;
+            double GL[3], Gi[9], gh[3];
+#pragma unroll
+            for (int K = 0; K < 3; K++) {
+                double EK[3];
+#pragma unroll
+                for (int I = 0; I < 3; I++)
+                    EK[I] = F[I] * sp[4 + SY[I][K]] + F[3 + I] * sp[14 + SY[I][K]] + F[6 + I] * sp[24 + SY[I][K]];
+                const double tr = (EK[0] + EK[1] + EK[2]) / 3.0;
+                GL[K] = g * ((L == 0 ? EK[0] : L == 1 ? EK[1] : EK[2]) - tr);
+            }
+#pragma unroll
+            for (int i = 0; i < 9; i++) Gi[i] = sp[GST_GI + i];
+            double gl[3];   // Gi_rL
+#pragma unroll
+            for (int r = 0; r < 3; r++) {
+                gh[r] = GL[0] * Gi[3 * r] + GL[1] * Gi[3 * r + 1] + GL[2] * Gi[3 * r + 2];
+                gl[r] = L == 0 ? Gi[3 * r] : L == 1 ? Gi[3 * r + 1] : Gi[3 * r + 2];
+            }
+#pragma unroll
+            for (int s = 0; s < 6; s++) {
+                double x = gl[PI[s]] * gh[PK[s]];
+                if (PI[s] != PK[s]) x += gl[PK[s]] * gh[PI[s]];
+                sp[GST_G + 6 * L + s] = x;
+            }
+        } else {
+            double S[9], N[9];
+            phys_strain(F, P, S, N);
+#pragma unroll
+            for (int I = 0; I < 3; I++)
+#pragma unroll
+                for (int K = I; K < 3; K++) {
+                    sp[GST_S + SY[I][K]] = w * S[3 * I + K];
+                    sp[GST_N + SY[I][K]] = w * N[3 * I + K];
+                }
+        }
+    }
+    __syncthreads();
+}
+
+template <typename T, bool DIRECT>
+__global__ __launch_bounds__((GenPipe<T>::S::THREADS), 2) void k_tangent_gen(
+    MeshK M, PhysK P, const double *__restrict__ Uh, T *__restrict__ Ke, Scatter S, const T *__restrict__ tabx,
+    const T *__restrict__ taby, const T *__restrict__ tabz)
+{
+    typedef typename GenPipe<T>::S Sh;
+    __shared__ double sPd[3][4][3][3];          // 1-D parametric tables [d][q_d][order][i]
+    __shared__ double sW[3][4];                 // 1-D point weights
+    __shared__ double sC[27][6];                // control points, then displacements
+    __shared__ __attribute__((aligned(16))) double sSt[64 * GST_W];
+    __shared__ T sX[36];
+    __shared__ int64_t sRow[DIRECT ? 81 : 1];
+    __shared__ int32_t sMsk[DIRECT ? 81 : 1];
+    __shared__ __attribute__((aligned(16))) T sD[Sh::D_SIZE];
+    __shared__ __attribute__((aligned(16))) T sE[Sh::E_SIZE];   // first the field passes' buffers (2376 doubles)
+    static_assert(Sh::THREADS == 512, "gen_states takes eight waves");
+    static_assert(Sh::E_SIZE * sizeof(T) >= 6 * (108 + 288) * sizeof(double), "field buffers in sE");
+
+    const int tid = threadIdx.x, e = blockIdx.x;
+    int ed[3];
+    sep_index<DIRECT>(M, S, e, ed);
+    if (DIRECT) sep_rows(M, S, ed, sRow, sMsk);
+    if (tid >= 256 && tid < 256 + 36) sX[tid - 256] = tabx[ed[0] * TAB_STRIDE + tid - 256];
+    if (tid >= 320 && tid < 320 + 27) {
+        const int b = tid - 320, ax = ed[0] + b / 9, ay = ed[1] + (b / 3) % 3, az = ed[2] + b % 3;
+        const int64_t id = ((int64_t)M.na[1] * M.na[2]) * ax + (int64_t)M.na[2] * ay + az;
+#pragma unroll
+        for (int d = 0; d < 3; d++) sC[b][d] = M.X[3 * id + d];
+    }
+    sep_element<1, 6>(M, Uh, ed, &sC[0][3], sPd, sW);
+    __syncthreads();
+    {
+        double J[10];
+        gen_fields(sC, sPd, reinterpret_cast<double *>(sE), J);
+        gen_states(M, P, ed, J, sW, sSt);
+    }
+    const GeneralIn in{sSt, P.e345, P.le};
     auto out = [&](int p, int bc, int cy, const T *K) {
         sep_write<T, DIRECT>(M, Ke, e, ed[0], ed[1], ed[2], p, bc, cy, K, sRow, sMsk);
     };
@@ -2270,6 +2466,11 @@ hipError_t launch_tangent_elem(const MeshK &M, const PhysK &P, const double *Uh,
         else hipLaunchKernelGGL((k_tangent_sep_t<float, false>), grid, dim3(SepShape<float, 3>::THREADS), 0, s, M, P, Uh, ndof, (float *)Ke, S, M.tabf[0], M.tabf[1], M.tabf[2]);
         return hipGetLastError();
     }
+    if (P.torder == 0 && M.equalw) {
+        if (prec == 0) hipLaunchKernelGGL((k_tangent_gen<double, false>), grid, dim3(512), 0, s, M, P, Uh, (double *)Ke, S, M.tab[0], M.tab[1], M.tab[2]);
+        else hipLaunchKernelGGL((k_tangent_gen<float, false>), grid, dim3(512), 0, s, M, P, Uh, (float *)Ke, S, M.tabf[0], M.tabf[1], M.tabf[2]);
+        return hipGetLastError();
+    }
     if (prec == 0) {
         if (P.torder == 0) hipLaunchKernelGGL((k_tangent_elem<double, 1, false>), grid, block, 0, s, M, P, Uh, ndof, (double *)Ke, nel, S);
         else hipLaunchKernelGGL((k_tangent_elem<double, 3, false>), grid, block, 0, s, M, P, Uh, ndof, (double *)Ke, nel, S);
@@ -2309,6 +2510,9 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
                 } else if (P.torder == 2 && M.separable) {
                     if (prec == 0) hipLaunchKernelGGL((k_tangent_sep_t<double, true>), grid, dim3(SepShape<double, 3>::THREADS), 0, s, M, P, Uh, ndof, (double *)vals, S, M.tab[0], M.tab[1], M.tab[2]);
                     else hipLaunchKernelGGL((k_tangent_sep_t<float, true>), grid, dim3(SepShape<float, 3>::THREADS), 0, s, M, P, Uh, ndof, (float *)vals, S, M.tabf[0], M.tabf[1], M.tabf[2]);
+                } else if (P.torder == 0 && M.equalw) {
+                    if (prec == 0) hipLaunchKernelGGL((k_tangent_gen<double, true>), grid, dim3(512), 0, s, M, P, Uh, (double *)vals, S, M.tab[0], M.tab[1], M.tab[2]);
+                    else hipLaunchKernelGGL((k_tangent_gen<float, true>), grid, dim3(512), 0, s, M, P, Uh, (float *)vals, S, M.tabf[0], M.tabf[1], M.tabf[2]);
                 } else if (prec == 0) {
                     if (P.torder == 0) hipLaunchKernelGGL((k_tangent_elem<double, 1, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);
                     else hipLaunchKernelGGL((k_tangent_elem<double, 3, true>), grid, block, 0, s, M, P, Uh, ndof, (double *)vals, (int)n, S);

@@ -374,7 +374,189 @@ struct StaticIn {
     }
 };
 
-// The same from the moment state of the transient rule: every product of two
+// D block (k, l) of the stored energy in parametric slots, for a geometry that
+// is no product: the pointwise tangent of the physical jet, pulled back to the
+// parametric jets of the tensor-product basis (rows and columns through
+//   u_,L = sum_i Gi_iL u_i,   u_,IK = sum_ij Gi_iI Gi_jK (u_ij - sum_n Ga^n_ij u_n),
+// Gi the inverse of the map's gradient, Ga its connection).  Nothing is pulled
+// back entry by entry: with E_IK = sum_L F_LI H_LIK the gradient part of the block is a product
+// in each index, so that with
+//   a^k_rI = F_kI Gi_rI,  a'^k_Mr = g sum_I c_MI a^k_rI (c = 1 - 1/3 on, -1/3 off the diagonal),
+//   h^k_Ls = sum_K H_kLK Gi_sK,  m_rs = sum_K Gi_rK Gi_sK,  B_rn = sum_L a'^k_Lr a^l_nL
+// the second-second entry of ((r, s), (n, m)) is B_rn m_sm, symmetrised, the
+// physical-first one of (M, (r, s)) is a'_Mr h_Ms, symmetrised, and only the
+// connection is left to apply: 860 FMAs per block against 1300 for pulling back the
+// physical block.  State layout (16-byte pairs; the stride of 94 puts the eight
+// points of a chunk on different banks): per component k at 10 k F (3), a gap, H
+// (6); times the point weight S at 30, N at 36 (6 each) and at 42 + 6 L
+// G_L(rs) = sum_K G_LK Gi_rL Gi_sK, symmetrised; Gi at 60 (3 r + I), the weight
+// at 69, Ga at 70 + 6 n, m at 88.
+constexpr int GST_S = 30, GST_N = 36, GST_G = 42, GST_GI = 60, GST_WGT = 69, GST_GA = 70, GST_M = 88, GST_W = 94;
+struct GeneralIn {
+    const double *sSt;
+    double e345, le;
+    const double *st;
+    int ok, ol;
+    __device__ __forceinline__ void load(int q, int k, int l, int)
+    {
+        st = sSt + q * GST_W;
+        ok = 10 * k;
+        ol = 10 * l;
+    }
+    __device__ __forceinline__ void get(double *dst, int at, int n) const
+    {
+        typedef double pair_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int i = 0; i < n / 2; i++) {
+            const pair_t x = *reinterpret_cast<const pair_t *>(st + at + 2 * i);
+            dst[2 * i] = x[0];
+            dst[2 * i + 1] = x[1];
+        }
+    }
+    // a[r][I] = F_I Gi_rI and ac[M][r] = g sum_I c_MI a[r][I]
+    static __device__ __forceinline__ void pull(const double *F, const double *Gi, double g, double (*a)[3], double (*ac)[3])
+    {
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+#pragma unroll
+            for (int I = 0; I < 3; I++) a[r][I] = F[I] * Gi[3 * r + I];
+            const double t = (a[r][0] + a[r][1] + a[r][2]) * (1.0 / 3.0);
+#pragma unroll
+            for (int I = 0; I < 3; I++) ac[I][r] = g * (a[r][I] - t);
+        }
+    }
+    // h[L][s] = sum_K H_LK Gi_sK
+    static __device__ __forceinline__ void lower(const double *H, const double *Gi, double (*h)[3])
+    {
+        constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+#pragma unroll
+        for (int L = 0; L < 3; L++)
+#pragma unroll
+            for (int s = 0; s < 3; s++) h[L][s] = H[SY[L][0]] * Gi[3 * s] + H[SY[L][1]] * Gi[3 * s + 1] + H[SY[L][2]] * Gi[3 * s + 2];
+    }
+    template <typename T>
+    __device__ __forceinline__ void rows(int k, int l, int, T *dst) const
+    {
+        constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
+        constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
+        double Gi[10], Ga[18], Fk[4], Fl[4], Hk[6], Hl[6];
+        get(Gi, GST_GI, 10);
+        get(Ga, GST_GA, 18);
+        const double dd = (k == l) ? 1.0 : 0.0, w = Gi[9], eh = w * 0.5 * e345, g = w * 2.0 * le * le;
+        double W[3][3], V[3][6];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+#pragma unroll
+            for (int n = 0; n < 3; n++) W[i][n] = 0.0;
+#pragma unroll
+            for (int c = 0; c < 6; c++) V[i][c] = 0.0;
+        }
+        {
+            // second rows (r, s); their part of the first rows through the connection
+            // (the states are read again below rather than kept: 256 registers hold
+            // Ga, W, V and what a row takes)
+            double B[3][3], hl[3][3], a[3][3], al[3][3], akc[3][3], mt[6];
+            get(Fk, ok, 4);
+            get(Fl, ol, 4);
+            get(Hl, ol + 4, 6);
+            get(mt, GST_M, 6);
+            pull(Fl, Gi, g, al, a);
+            pull(Fk, Gi, g, a, akc);
+            lower(Hl, Gi, hl);
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+#pragma unroll
+                for (int n = 0; n < 3; n++) B[r][n] = akc[0][r] * al[n][0] + akc[1][r] * al[n][1] + akc[2][r] * al[n][2];
+#pragma unroll
+            for (int t = 0; t < 6; t++) {
+                const int r = PI[t], s = PK[t];
+                double f[3], v[9];
+#pragma unroll
+                for (int M = 0; M < 3; M++) {
+                    f[M] = akc[M][r] * hl[M][s] + dd * st[GST_G + 6 * M + t];
+                    if (r != s) f[M] += akc[M][s] * hl[M][r];
+                }
+#pragma unroll
+                for (int c = 0; c < 6; c++) {
+                    const int n = PI[c], m = PK[c];
+                    double x = B[r][n] * mt[SY[s][m]];
+                    if (n != m) x += B[r][m] * mt[SY[s][n]];
+                    if (r != s) x += B[s][n] * mt[SY[r][m]];
+                    if (r != s && n != m) x += B[s][m] * mt[SY[r][n]];
+                    v[3 + c] = x;
+                }
+#pragma unroll
+                for (int n = 0; n < 3; n++) {
+                    double x = f[0] * Gi[3 * n] + f[1] * Gi[3 * n + 1] + f[2] * Gi[3 * n + 2];
+#pragma unroll
+                    for (int c = 0; c < 6; c++) x -= v[3 + c] * Ga[6 * n + c];
+                    v[n] = x;
+                }
+                d_store<T>(dst + PIPE_DR * (3 + t), v);
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+#pragma unroll
+                    for (int n = 0; n < 3; n++) W[i][n] -= Ga[6 * i + t] * v[n];
+#pragma unroll
+                    for (int c = 0; c < 6; c++) V[i][c] -= Ga[6 * i + t] * v[3 + c];
+                }
+            }
+        }
+        // first rows
+        double hk[3][3], al[3][3], alc[3][3], S[6], N[6];
+        get(Fk, ok, 4);
+        get(Fl, ol, 4);
+        get(Hk, ok + 4, 6);
+        get(Hl, ol + 4, 6);
+        pull(Fl, Gi, g, al, alc);
+        lower(Hk, Gi, hk);
+        get(S, GST_S, 6);
+        get(N, GST_N, 6);
+#pragma unroll
+        for (int L = 0; L < 3; L++) {
+            double f[3], x[6];
+#pragma unroll
+            for (int M = 0; M < 3; M++) {
+                const double hh = Hk[SY[L][0]] * Hl[SY[M][0]] + Hk[SY[L][1]] * Hl[SY[M][1]] + Hk[SY[L][2]] * Hl[SY[M][2]];
+                double y = N[SY[L][M]] * (Fk[L] * Fl[M]) + dd * S[SY[L][M]];
+                y += eh * (L == M ? Fk[(L + 1) % 3] * Fl[(L + 1) % 3] + Fk[(L + 2) % 3] * Fl[(L + 2) % 3] : Fk[M] * Fl[L]);
+                y += g * (L == M ? 2.0 / 3.0 : -1.0 / 3.0) * hh;
+                f[M] = y;
+            }
+#pragma unroll
+            for (int c = 0; c < 6; c++) {
+                const int n = PI[c], m = PK[c];
+                x[c] = alc[L][n] * hk[L][m] + dd * st[GST_G + 6 * L + c];
+                if (n != m) x[c] += alc[L][m] * hk[L][n];
+            }
+            double y[3];
+#pragma unroll
+            for (int n = 0; n < 3; n++) {
+                y[n] = f[0] * Gi[3 * n] + f[1] * Gi[3 * n + 1] + f[2] * Gi[3 * n + 2];
+#pragma unroll
+                for (int c = 0; c < 6; c++) y[n] -= x[c] * Ga[6 * n + c];
+            }
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+#pragma unroll
+                for (int n = 0; n < 3; n++) W[i][n] += Gi[3 * i + L] * y[n];
+#pragma unroll
+                for (int c = 0; c < 6; c++) V[i][c] += Gi[3 * i + L] * x[c];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            double v[9];
+#pragma unroll
+            for (int n = 0; n < 3; n++) v[n] = W[i][n];
+#pragma unroll
+            for (int c = 0; c < 6; c++) v[3 + c] = V[i][c];
+            d_store<T>(dst + PIPE_DR * i, v);
+        }
+    }
+};
+
+// The block of StaticIn from the moment state of the transient rule: every product of two
 // state factors is the sum over the two transformed components, every N-weighted
 // one the form X^T N^ Y.  State layout: per component k at 18 k F^ (3 + 3) and H^
 // (6 + 6), then Sb and the three N^ blocks (6 each, symmetric pairs) and Gb (9);
