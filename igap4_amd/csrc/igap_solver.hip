@@ -134,18 +134,70 @@ __global__ void k_point_cols(int64_t ncp, const int64_t *__restrict__ rp, const 
     }
 }
 
+// One Chebyshev step with point-block Jacobi, in the epilogue of the product
+// A v that it needs: r = rin - A v, dn = alpha v + beta Dinv r and the update of
+// x.  v is the step's direction d (or x itself, X_NONE: the first step of a
+// smoothing that starts from x), which other rows still read, so dn is another buffer and
+// the first step's own update of x waits for the second (X_ADD2).  rout and
+// dn may be null (last step), rout may be rin.  As a kernel of its own the step
+// re-read r, d and x and was a launch more per product: a step at 64x16x16
+// (FP64) 12.7 + 3.4 us -> @CHEB64@.
+enum { X_NONE, X_SET, X_ADD2, X_ADD };   // x unchanged; v + dn; x + v + dn; x + dn
+struct Cheb {
+    const double *Dinv, *rin;
+    double *rout, *dn, *x;
+    double alpha, beta;
+    int xmode;
+};
+
+// lane i < 3 of the lanes that sum row block p takes row i; the constructor's
+// loads are issued before the product's
+struct ChebRow {
+    double m0, m1, m2, r0, r1, r2, v, x;
+    __device__ __forceinline__ ChebRow(const Cheb &c, const double *vec, int64_t p, int i, bool ok)
+    {
+        m0 = m1 = m2 = r0 = r1 = r2 = v = x = 0.0;
+        if (ok && i < 3) {
+            const double *m = c.Dinv + 9 * p + 3 * i;
+            m0 = m[0];
+            m1 = m[1];
+            m2 = m[2];
+            r0 = c.rin[3 * p];
+            r1 = c.rin[3 * p + 1];
+            r2 = c.rin[3 * p + 2];
+            v = vec[3 * p + i];
+            if (c.xmode == X_ADD2 || c.xmode == X_ADD) x = c.x[3 * p + i];
+        }
+    }
+    __device__ __forceinline__ void finish(const Cheb &c, int64_t p, int i, double s0, double s1, double s2)
+    {
+        r0 -= s0;
+        r1 -= s1;
+        r2 -= s2;
+        const double z = m0 * r0 + m1 * r1 + m2 * r2;
+        double d = c.beta * z;
+        if (c.alpha != 0.0) d += c.alpha * v;
+        if (c.rout) c.rout[3 * p + i] = i == 0 ? r0 : i == 1 ? r1 : r2;
+        if (c.dn) c.dn[3 * p + i] = d;
+        if (c.xmode == X_SET) c.x[3 * p + i] = v + d;
+        else if (c.xmode == X_ADD2) c.x[3 * p + i] = (x + v) + d;
+        else if (c.xmode == X_ADD) c.x[3 * p + i] = x + d;
+    }
+};
+
 // y = A x on the point-block pattern: one wave per control point, lane k
 // takes neighbour points k and k+64 (one index load, three x loads and the
 // nine values of the block for the three rows)
-// MODE 0: y = A x;  1: y = b - A x;  2: y -= A x
+// MODE 0: y = A x;  1: y = b - A x;  2: the Chebyshev step ch with v = x
 template <typename T, int MODE>
 __global__ __launch_bounds__(256) void k_spmv_pb(int64_t ncp, const int64_t *__restrict__ rp, const int32_t *__restrict__ pcol,
                                                  const T *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
-                                                 double *__restrict__ y)
+                                                 double *__restrict__ y, Cheb ch)
 {
     const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (p >= ncp) return;
+    ChebRow row(ch, x, p, lane, MODE == 2);
     const int64_t b0 = rp[3 * p], b1 = rp[3 * p + 1], b2 = rp[3 * p + 2];
     const int nn = (int)((b1 - b0) / 3);
     const int32_t *pc = pcol + b0 / 9;
@@ -164,19 +216,17 @@ __global__ __launch_bounds__(256) void k_spmv_pb(int64_t ncp, const int64_t *__r
         s1 += __shfl_xor(s1, o, 64);
         s2 += __shfl_xor(s2, o, 64);
     }
-    if (lane == 0) {
+    if (MODE == 2) {
+        if (lane < 3) row.finish(ch, p, lane, s0, s1, s2);
+    } else if (lane == 0) {
         if (MODE == 0) {
             y[3 * p] = s0;
             y[3 * p + 1] = s1;
             y[3 * p + 2] = s2;
-        } else if (MODE == 1) {
+        } else {
             y[3 * p] = b[3 * p] - s0;
             y[3 * p + 1] = b[3 * p + 1] - s1;
             y[3 * p + 2] = b[3 * p + 2] - s2;
-        } else {
-            y[3 * p] -= s0;
-            y[3 * p + 1] -= s1;
-            y[3 * p + 2] -= s2;
         }
     }
 }
@@ -239,16 +289,29 @@ struct PointGrid {
     int nb[3];
     int64_t L12;   // stencil_prefix(nb1, nb1) * stencil_prefix(nb2, nb2)
     int64_t L2;    // stencil_prefix(nb2, nb2)
+    uint64_t m12, m2;   // reciprocals of nb1 nb2 and nb2 (recip64)
 };
+
+// division of a 32-bit number by a run-time divisor d > 1: the upper half of v
+// times 2^64 / d rounded up is v / d (v d < 2^64); d = 1 is the reciprocal 0
+__host__ __forceinline__ uint64_t recip64(uint64_t d) { return d > 1 ? ~0ull / d + 1 : 0; }
+__device__ __forceinline__ uint32_t div32(uint32_t v, uint64_t m) { return m ? (uint32_t)__umul64hi(v, m) : v; }
 
 // sum over the points a' < a of one direction (n points) of their clipped
 // stencil lengths min(a' + 2, n - 1) - max(a' - 2, 0) + 1
-__host__ __device__ __forceinline__ int64_t stencil_prefix(int64_t a, int64_t n)
+__host__ __forceinline__ int64_t stencil_prefix(int64_t a, int64_t n)
 {
     const int64_t m = a < (n - 2 > 0 ? n - 2 : 0) ? a : (n - 2 > 0 ? n - 2 : 0);
     const int64_t smin = m * (m - 1) / 2 + 2 * m + (a - m) * (n - 1);
     const int64_t smax = a >= 3 ? (a - 3) * (a - 2) / 2 : 0;
     return smin - smax + a;
+}
+
+// the same for a < n, n >= 3, in closed form: five a point but for the ends' points
+__device__ __forceinline__ int stencil_before(int a, int n)
+{
+    if (n == 3) return 3 * a;
+    return 5 * a - (a > 1 ? 3 : 2 * a) - (a == n - 1 ? 1 : 0);
 }
 
 // y = A x with the 16-bit blocks (the layout of k_spmv_pb, FP64 sums, the
@@ -259,25 +322,32 @@ __host__ __device__ __forceinline__ int64_t stencil_prefix(int64_t a, int64_t n)
 // per wave, 64 / PPW lanes each: a point's 20-byte blocks are few (at most
 // 125), so a wave per point spends its time waiting on its loads rather
 // than on the blocks; every load of a lane is issued before the sums.
+// The index arithmetic is 32-bit multiplications by reciprocals: 64-bit divisions per
+// point and two 32-bit ones per block took longer than the blocks' bytes
+// (128x32x32, 346 MB: 95 -> @H16@ us).
 template <int MODE, int PPW>
 __global__ __launch_bounds__(256) void k_spmv_h16(int64_t ncp, PointGrid G, const uint32_t *__restrict__ h16, const float *__restrict__ rs,
-                                                  const double *__restrict__ x, const double *__restrict__ b, double *__restrict__ y)
+                                                  const double *__restrict__ x, const double *__restrict__ b, double *__restrict__ y,
+                                                  Cheb ch)
 {
     constexpr int LW = 64 / PPW;   // lanes per control point
     const int lane = threadIdx.x & 63, sl = lane & (LW - 1);
     const int64_t p = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PPW + lane / LW;
     const bool ok = p < ncp;
+    ChebRow row(ch, x, p, sl, MODE == 2 && ok);
     double s0 = 0, s1 = 0, s2 = 0;
     if (ok) {
         const int n1 = G.nb[1], n2 = G.nb[2];
-        const int pz = (int)(p % n2), py = (int)((p / n2) % n1), px = (int)(p / ((int64_t)n1 * n2));
+        const int pq = (int)div32((uint32_t)p, G.m2), px = (int)div32((uint32_t)p, G.m12), py = pq - px * n1, pz = (int)p - pq * n2;
         const int lox = px - 2 > 0 ? px - 2 : 0, loy = py - 2 > 0 ? py - 2 : 0, loz = pz - 2 > 0 ? pz - 2 : 0;
         const int lx = (px + 2 < G.nb[0] - 1 ? px + 2 : G.nb[0] - 1) - lox + 1;
         const int ly = (py + 2 < n1 - 1 ? py + 2 : n1 - 1) - loy + 1;
         const int lz = (pz + 2 < n2 - 1 ? pz + 2 : n2 - 1) - loz + 1;
         const int nn = lx * ly * lz, lyz = ly * lz;
-        const int64_t blk = stencil_prefix(px, G.nb[0]) * G.L12 + lx * (stencil_prefix(py, n1) * G.L2 + ly * stencil_prefix(pz, n2));
+        const int64_t blk = stencil_before(px, G.nb[0]) * G.L12 + lx * (stencil_before(py, n1) * G.L2 + ly * stencil_before(pz, n2));
         const uint32_t *hb = h16 + 5 * blk;
+        // k / lyz and r / lz of k < 125 by multiplication: exact while k d < 2^16
+        const int iyz = (65535 + lyz) / lyz, iz = (65535 + lz) / lz;
         // at most 125 neighbours: a fixed number of rounds
         constexpr int NIT = (125 + LW - 1) / LW;
         uint32_t w[NIT][5];
@@ -286,8 +356,8 @@ __global__ __launch_bounds__(256) void k_spmv_h16(int64_t ncp, PointGrid G, cons
         for (int it = 0; it < NIT; it++) {
             const int k = sl + it * LW;
             if (k < nn) {
-                const int kx = k / lyz, r = k - kx * lyz, ky = r / lz, kz = r - ky * lz;
-                const int64_t q = ((int64_t)(lox + kx) * n1 + (loy + ky)) * n2 + (loz + kz);
+                const int kx = (k * iyz) >> 16, r = k - kx * lyz, ky = (r * iz) >> 16, kz = r - ky * lz;
+                const int64_t q = ((lox + kx) * n1 + (loy + ky)) * n2 + (loz + kz);
 #pragma unroll
                 for (int j = 0; j < 3; j++) xv[it][j] = x[3 * q + j];
 #pragma unroll
@@ -312,7 +382,9 @@ __global__ __launch_bounds__(256) void k_spmv_h16(int64_t ncp, PointGrid G, cons
         s1 += __shfl_xor(s1, o, 64);
         s2 += __shfl_xor(s2, o, 64);
     }
-    if (ok && sl == 0) {
+    if (MODE == 2) {
+        if (ok && sl < 3) row.finish(ch, p, sl, s0 * (double)rs[3 * p], s1 * (double)rs[3 * p + 1], s2 * (double)rs[3 * p + 2]);
+    } else if (ok && sl == 0) {
         s0 *= (double)rs[3 * p];
         s1 *= (double)rs[3 * p + 1];
         s2 *= (double)rs[3 * p + 2];
@@ -320,14 +392,10 @@ __global__ __launch_bounds__(256) void k_spmv_h16(int64_t ncp, PointGrid G, cons
             y[3 * p] = s0;
             y[3 * p + 1] = s1;
             y[3 * p + 2] = s2;
-        } else if (MODE == 1) {
+        } else {
             y[3 * p] = b[3 * p] - s0;
             y[3 * p + 1] = b[3 * p + 1] - s1;
             y[3 * p + 2] = b[3 * p + 2] - s2;
-        } else {
-            y[3 * p] -= s0;
-            y[3 * p + 1] -= s1;
-            y[3 * p + 2] -= s2;
         }
     }
 }
@@ -625,6 +693,12 @@ __global__ __launch_bounds__(64) void k_mcb_ilu(int r0, int npts, const int32_t 
 
 __global__ void k_set_i32(int *p, int v) { *p = v; }
 
+// a 1-D transfer operator in CSR form as a kernel sees it
+struct Op1K {
+    const int *rp, *ci;
+    const double *w;
+};
+
 // One direction of a tensor-product transfer between control-point grids:
 // out(i0,i1,i2)[c] = sum_e w[e] in(i0,i1,i2 with the coordinate along dir
 // replaced by ci[e])[c] over the entries e of row (coordinate along dir) of a
@@ -657,20 +731,85 @@ __global__ void k_apply1d(int dir, int o0, int o1, int o2, int min, const int *_
     }
 }
 
-// x = s D^-1 b, d = x, r = b   (first Chebyshev step from x = 0)
-__global__ void k_cheb_first(int64_t ncp, const double *__restrict__ Dinv, const double *__restrict__ b, double *__restrict__ x,
-                             double *__restrict__ d, double *__restrict__ r, double sc)
+// A transfer over all three directions in one pass, for operators of at most
+// E entries per row (prolongation 2, its transpose 4; a direction that is
+// not coarsened has rp null): out = (op0 x op1 x op2) in with the inner sums in
+// the order of k_apply1d's passes, every load of a thread in flight at once.
+// Three passes were three launches of 4 us at 64x16x16 and on every coarser level.
+// With E = 4 an output takes four lanes, one per entry along z.
+template <int E>
+__global__ __launch_bounds__(256) void k_apply3(Op1K p0, Op1K p1, Op1K p2, int o0, int o1, int o2, int n1, int n2, uint64_t m12, uint64_t m2,
+                                                const double *__restrict__ in, double *__restrict__ out,
+                                                const int32_t *__restrict__ mask, int accumulate)
+{
+    constexpr int LN = E == 4 ? 4 : 1, E2 = E / LN;
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / LN;
+    const int ln = threadIdx.x & (LN - 1);
+    if (t >= 3LL * o0 * o1 * o2) return;   // (whole groups of LN lanes)
+    const uint32_t pt = (uint32_t)((uint64_t)t / 3), c = (uint32_t)(t - 3 * (int64_t)pt);
+    const int pq = (int)div32(pt, m2), px = (int)div32(pt, m12);
+    const int i[3] = {px, pq - px * o1, (int)pt - pq * o2};
+    const Op1K *op[3] = {&p0, &p1, &p2};
+    int j[3][E], m[3];
+    double w[3][E];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        int r0 = 0;
+        m[d] = 1;
+        if (op[d]->rp) {
+            r0 = op[d]->rp[i[d]];
+            m[d] = op[d]->rp[i[d] + 1] - r0;
+        }
+#pragma unroll
+        for (int e = 0; e < (d == 2 ? E2 : E); e++) {
+            const int x = d == 2 ? ln + e : e, q = m[d] > 0 ? r0 + (x < m[d] ? x : 0) : 0;
+            j[d][e] = op[d]->rp ? op[d]->ci[q] : i[d];
+            w[d][e] = op[d]->rp ? op[d]->w[q] : 1.0;
+        }
+    }
+    double v[E2][E][E], a[E2];
+#pragma unroll
+    for (int e2 = 0; e2 < E2; e2++)
+#pragma unroll
+        for (int e1 = 0; e1 < E; e1++)
+#pragma unroll
+            for (int e0 = 0; e0 < E; e0++) v[e2][e1][e0] = in[3 * (((int64_t)j[0][e0] * n1 + j[1][e1]) * n2 + j[2][e2]) + c];
+    const bool last = ln == 0;
+    const double old = last && accumulate ? out[t] : 0.0;
+    const bool zero = last && mask && mask[t];
+#pragma unroll
+    for (int e2 = 0; e2 < E2; e2++) {
+        a[e2] = 0.0;
+#pragma unroll
+        for (int e1 = 0; e1 < E; e1++) {
+            double a1 = 0.0;
+#pragma unroll
+            for (int e0 = 0; e0 < E; e0++)
+                if (e0 < m[0]) a1 += w[0][e0] * v[e2][e1][e0];
+            if (e1 < m[1]) a[e2] += w[1][e1] * a1;
+        }
+    }
+    double acc = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        const double av = LN == 1 ? a[e % E2] : __shfl(a[0], e, LN), wv = LN == 1 ? w[2][e % E2] : __shfl(w[2][0], e, LN);
+        if (e < m[2]) acc += wv * av;
+    }
+    if (!last) return;
+    if (zero) acc = 0.0;
+    out[t] = accumulate ? old + acc : acc;
+}
+
+// d = s D^-1 b   (first Chebyshev step from x = 0, where x = d and r = b)
+__global__ void k_cheb_first(int64_t ncp, const double *__restrict__ Dinv, const double *__restrict__ b, double *__restrict__ d, double sc)
 {
     const int64_t st = (int64_t)gridDim.x * blockDim.x;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < ncp; p += st) {
         const double *m = Dinv + 9 * p;
         const double b0 = b[3 * p], b1 = b[3 * p + 1], b2 = b[3 * p + 2];
-        const double z0 = sc * (m[0] * b0 + m[1] * b1 + m[2] * b2);
-        const double z1 = sc * (m[3] * b0 + m[4] * b1 + m[5] * b2);
-        const double z2 = sc * (m[6] * b0 + m[7] * b1 + m[8] * b2);
-        x[3 * p] = z0; x[3 * p + 1] = z1; x[3 * p + 2] = z2;
-        d[3 * p] = z0; d[3 * p + 1] = z1; d[3 * p + 2] = z2;
-        r[3 * p] = b0; r[3 * p + 1] = b1; r[3 * p + 2] = b2;
+        d[3 * p] = sc * (m[0] * b0 + m[1] * b1 + m[2] * b2);
+        d[3 * p + 1] = sc * (m[3] * b0 + m[4] * b1 + m[5] * b2);
+        d[3 * p + 2] = sc * (m[6] * b0 + m[7] * b1 + m[8] * b2);
     }
 }
 
@@ -715,31 +854,16 @@ __global__ void k_block_diag_inv(int64_t ncp, const int64_t *__restrict__ rp, co
     }
 }
 
-// d = alpha d + beta Dinv r; x += d   (one Chebyshev step, point-block Jacobi)
-__global__ void k_cheb_step(int64_t ncp, const double *__restrict__ Dinv, const double *__restrict__ r, double *__restrict__ d,
-                            double *__restrict__ x, double alpha, double beta, int add)
+// d = Dinv r
+__global__ void k_block_apply(int64_t ncp, const double *__restrict__ Dinv, const double *__restrict__ r, double *__restrict__ d)
 {
     const int64_t st = (int64_t)gridDim.x * blockDim.x;
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < ncp; p += st) {
         const double *m = Dinv + 9 * p;
         const double r0 = r[3 * p], r1 = r[3 * p + 1], r2 = r[3 * p + 2];
-        const double z0 = m[0] * r0 + m[1] * r1 + m[2] * r2;
-        const double z1 = m[3] * r0 + m[4] * r1 + m[5] * r2;
-        const double z2 = m[6] * r0 + m[7] * r1 + m[8] * r2;
-        double d0 = beta * z0, d1 = beta * z1, d2 = beta * z2;
-        if (alpha != 0.0) {   // (d is not read on the first step)
-            d0 += alpha * d[3 * p];
-            d1 += alpha * d[3 * p + 1];
-            d2 += alpha * d[3 * p + 2];
-        }
-        d[3 * p] = d0;
-        d[3 * p + 1] = d1;
-        d[3 * p + 2] = d2;
-        if (add) {
-            x[3 * p] += d0;
-            x[3 * p + 1] += d1;
-            x[3 * p + 2] += d2;
-        }
+        d[3 * p] = m[0] * r0 + m[1] * r1 + m[2] * r2;
+        d[3 * p + 1] = m[3] * r0 + m[4] * r1 + m[5] * r2;
+        d[3 * p + 2] = m[6] * r0 + m[7] * r1 + m[8] * r2;
     }
 }
 
@@ -779,7 +903,20 @@ __global__ __launch_bounds__(256) void k_dot_part(int64_t n, int64_t ld, const d
     const int64_t i1 = i0 + DOT_CHUNK < n ? i0 + DOT_CHUNK : n;
     const double *v = V + (int64_t)k * ld;
     double s = 0;
-    for (int64_t i = i0 + tid; i < i1; i += 256) s += v[i] * w[i];
+    if (i1 - i0 == DOT_CHUNK) {
+        // a whole chunk: its loads in flight together, the sum in the same order
+        double a[DOT_CHUNK / 256], b[DOT_CHUNK / 256];
+#pragma unroll
+        for (int j = 0; j < DOT_CHUNK / 256; j++) {
+            a[j] = v[i0 + tid + 256 * j];
+            b[j] = w[i0 + tid + 256 * j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < DOT_CHUNK / 256; j++) s += a[j] * b[j];
+    } else {
+        for (int64_t i = i0 + tid; i < i1; i += 256) s += v[i] * w[i];
+    }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((tid & 63) == 0) red[tid >> 6] = s;
@@ -1368,7 +1505,8 @@ static int ensure_pcol(igap_gpu_ctx *c)
     return IGAP_OK;
 }
 
-static int spmv(igap_gpu_ctx *c, int p, const double *x, double *y, int mode = 0, const double *b = nullptr)
+// y = A x (mode 0), y = b - A x (1) or a Chebyshev step on d = x (2) with the context's tangent values
+static int spmv(igap_gpu_ctx *c, int p, const double *x, double *y, int mode = 0, const double *b = nullptr, const Cheb &ch = Cheb())
 {
     const int64_t n = c->ndof, ncp = n / 3;
     int rc = ensure_pcol(c);
@@ -1376,7 +1514,7 @@ static int spmv(igap_gpu_ctx *c, int p, const double *x, double *y, int mode = 0
     const dim3 g((unsigned)((ncp + 3) / 4)), bs(256);
     const int64_t *rp = (const int64_t *)c->d_rowptr;
     const int32_t *pc = (const int32_t *)c->d_pcol;
-#define IGAP_SPMV(T, V, M) hipLaunchKernelGGL((k_spmv_pb<T, M>), g, bs, 0, c->stream, ncp, rp, pc, (const T *)V, x, b, y)
+#define IGAP_SPMV(T, V, M) hipLaunchKernelGGL((k_spmv_pb<T, M>), g, bs, 0, c->stream, ncp, rp, pc, (const T *)V, x, b, y, ch)
     if (p == IGAP_F64) {
         if (mode == 0) IGAP_SPMV(double, c->d_val64, 0);
         else if (mode == 1) IGAP_SPMV(double, c->d_val64, 1);
@@ -1441,7 +1579,7 @@ constexpr int MG_POWER_ITS = 20;        // power iterations of the first set-up 
 constexpr int MG_POWER_ITS_WARM = 8;    // of later ones, from the previous set-up's vector
 
 struct Op1 {   // 1-D operator in CSR form on the device
-    int rows = 0, cols = 0;
+    int rows = 0, cols = 0, width = 0;   // width: the most entries of a row
     int *rp = nullptr, *ci = nullptr;
     double *w = nullptr;
 };
@@ -1451,7 +1589,7 @@ struct MGLevel {
     Solver *s = nullptr;         // level 0: the caller's solver (not owned)
     int halve[3] = {0, 0, 0};    // directions halved towards level l+1
     Op1 P[3], R[3], T[3];        // to level l+1: prolongation, P^T, interpolation
-    double *r = nullptr, *t = nullptr, *b = nullptr, *x = nullptr;
+    double *r = nullptr, *t = nullptr, *t2 = nullptr, *b = nullptr, *x = nullptr;
     double *Dinv = nullptr;      // 3x3 diagonal-block inverses (smoother)
     double lmax = 1.0;           // lambda_max(D^-1 A) estimate
     double *pv = nullptr;        // the power iteration's last vector, the next set-up's start
@@ -1487,7 +1625,7 @@ void mg_destroy(MGHier *g)
             op1_free(L.R[d]);
             op1_free(L.T[d]);
         }
-        double *v[] = {L.r, L.t, L.b, L.x, L.pv, L.Dinv, L.dense};
+        double *v[] = {L.r, L.t, L.t2, L.b, L.x, L.pv, L.Dinv, L.dense};
         for (double *q : v)
             if (q) (void)hipFree(q);
         if (L.h16) (void)hipFree(L.h16);
@@ -1568,6 +1706,7 @@ static int op1_upload(const std::vector<double> &M, int rows, int cols, Op1 &o)
                 w.push_back(M[(size_t)r * cols + j]);
             }
         rp[r + 1] = (int)ci.size();
+        o.width = std::max(o.width, rp[r + 1] - rp[r]);
     }
     o.rows = rows;
     o.cols = cols;
@@ -1690,6 +1829,31 @@ static int mg_transfer(igap_gpu_ctx *c, MGHier *g, int l, int which, const doubl
     for (int d = 0; d < 3; d++)
         if (F.halve[d]) dl[nd++] = d;
     if (nd == 0) return fail(IGAP_ERR_STATE, "multigrid: level without coarsening");
+    if (which != 2) {
+        // P and its transpose have few entries a row (2 and 4 in the interior): one
+        // pass.  (T interpolates with full rows: one direction at a time.)
+        Op1K k[3] = {};
+        int od[3], width = 0;
+        for (int d = 0; d < 3; d++) {
+            const Op1 &o = which == 0 ? F.P[d] : F.R[d];
+            od[d] = F.halve[d] ? o.rows : dims[d];
+            if (!F.halve[d]) continue;
+            k[d] = Op1K{o.rp, o.ci, o.w};
+            width = std::max(width, o.width);
+        }
+        if (width <= 4) {
+            const int64_t n = 3LL * od[0] * od[1] * od[2];
+            const uint64_t m12 = recip64((uint64_t)od[1] * od[2]), m2 = recip64(od[2]);
+            if (width <= 2)
+                hipLaunchKernelGGL(k_apply3<2>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, k[0], k[1], k[2], od[0], od[1],
+                                   od[2], dims[1], dims[2], m12, m2, in, out, mask, accumulate);
+            else
+                hipLaunchKernelGGL(k_apply3<4>, dim3((unsigned)((4 * n + 255) / 256)), dim3(256), 0, c->stream, k[0], k[1], k[2], od[0],
+                                   od[1], od[2], dims[1], dims[2], m12, m2, in, out, mask, accumulate);
+            HIPCHK(hipGetLastError());
+            return IGAP_OK;
+        }
+    }
     const double *src = in;
     for (int q = 0; q < nd; q++) {
         const int d = dl[q];
@@ -1806,7 +1970,7 @@ static int mg_build_levels(igap_gpu_ctx *c, Solver *s, MGHier *g, int maxlev)
     for (int l = 0; l < g->nlev; l++) {
         MGLevel &L = g->lev[l];
         const size_t b = sizeof(double) * (size_t)L.c->ndof;
-        double **v[] = {&L.r, &L.t, &L.b, &L.x, &L.pv};
+        double **v[] = {&L.r, &L.t, &L.t2, &L.b, &L.x, &L.pv};
         for (double **q : v) DALLOC(q, b);
         DALLOC(&L.Dinv, sizeof(double) * 3 * (size_t)L.c->ndof);
     }
@@ -1821,10 +1985,11 @@ static int mg_build_levels(igap_gpu_ctx *c, Solver *s, MGHier *g, int maxlev)
 }
 
 // A x on multigrid level l in the preconditioner's precision (MODE of k_spmv_pb)
-static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, double *y, int mode = 0, const double *b = nullptr)
+static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, double *y, int mode = 0, const double *b = nullptr,
+                    const Cheb &ch = Cheb())
 {
     MGLevel &L = g->lev[l];
-    if (p != PC_F16 || !L.h16) return spmv(L.c, p == PC_F16 ? IGAP_F32 : p, x, y, mode, b);
+    if (p != PC_F16 || !L.h16) return spmv(L.c, p == PC_F16 ? IGAP_F32 : p, x, y, mode, b, ch);
     const int64_t ncp = L.c->ndof / 3;
     const dim3 gr((unsigned)((ncp + 4 * H16_PPW - 1) / (4 * H16_PPW))), bs(256);
     const uint32_t *hv = (const uint32_t *)L.h16;
@@ -1835,9 +2000,11 @@ static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, d
     for (int d = 0; d < 3; d++) G.nb[d] = M.nb[d];
     G.L2 = stencil_prefix(M.nb[2], M.nb[2]);
     G.L12 = stencil_prefix(M.nb[1], M.nb[1]) * G.L2;
-    if (mode == 0) hipLaunchKernelGGL((k_spmv_h16<0, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y);
-    else if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y);
-    else hipLaunchKernelGGL((k_spmv_h16<2, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y);
+    G.m2 = recip64(M.nb[2]);
+    G.m12 = recip64((uint64_t)M.nb[1] * M.nb[2]);
+    if (mode == 0) hipLaunchKernelGGL((k_spmv_h16<0, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
+    else if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
+    else hipLaunchKernelGGL((k_spmv_h16<2, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
     HIPCHK(hipGetLastError());
     return IGAP_OK;
 }
@@ -1849,26 +2016,32 @@ static int mg_cheb(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *b, do
     MGLevel &L = g->lev[l];
     igap_gpu_ctx *cl = L.c;
     const int64_t n = cl->ndof, ncp = n / 3;
-    const dim3 gn = grid1(n), gp = grid1(ncp), bs(256);
+    const dim3 gp = grid1(ncp), bs(256);
     // lower end 0.02 lambda_max, measured on 64x16x16 and 160x40x40 load steps:
     // 0.1 is 5-7% slower, 0.005 needs more Krylov iterations on the small patch
     const double lo = 0.02 * L.lmax, hi = 1.1 * L.lmax;
     const double theta = 0.5 * (hi + lo), delta = 0.5 * (hi - lo), sigma = theta / delta;
+    if (deg < 2) return fail(IGAP_ERR_STATE, "Chebyshev degree %d", deg);
     int rc;
-    (void)gn;
+    Cheb ch{L.Dinv, b, L.r, L.t, x, 0.0, 1.0 / theta, X_NONE};
     if (zero_init) {
-        hipLaunchKernelGGL(k_cheb_first, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, b, x, L.t, L.r, 1.0 / theta);
+        hipLaunchKernelGGL(k_cheb_first, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, b, L.t, 1.0 / theta);
     } else {
-        if ((rc = lvl_spmv(c, g, l, p, x, L.r, 1, b))) return rc;   // r = b - A x
-        hipLaunchKernelGGL(k_cheb_step, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, (const double *)L.r, L.t, x, 0.0, 1.0 / theta,
-                           1);
+        if ((rc = lvl_spmv(c, g, l, p, x, nullptr, 2, nullptr, ch))) return rc;   // r = b - A x, d = Dinv r / theta
+        ch.rin = L.r;
     }
     double rho = 1.0 / sigma;
     for (int k = 1; k < deg; k++) {
-        if ((rc = lvl_spmv(c, g, l, p, L.t, L.r, 2))) return rc;     // r -= A d
         const double rn = 1.0 / (2.0 * sigma - rho);
-        hipLaunchKernelGGL(k_cheb_step, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, (const double *)L.r, L.t, x, rn * rho,
-                           2.0 * rn / delta, 1);
+        const bool last = k == deg - 1;
+        const double *d = k % 2 ? L.t : L.t2;
+        ch.rout = last ? nullptr : L.r;
+        ch.dn = last ? nullptr : (k % 2 ? L.t2 : L.t);
+        ch.alpha = rn * rho;
+        ch.beta = 2.0 * rn / delta;
+        ch.xmode = k > 1 ? X_ADD : zero_init ? X_SET : X_ADD2;
+        if ((rc = lvl_spmv(c, g, l, p, d, nullptr, 2, nullptr, ch))) return rc;   // r -= A d
+        ch.rin = L.r;
         rho = rn;
     }
     HIPCHK(hipGetLastError());
@@ -1905,7 +2078,7 @@ static int mg_smoother_setup(igap_gpu_ctx *c, MGHier *g, int l, int p)
         if ((rc = dots(cl, L.s, L.x, n, 1, L.x, L.s->h))) return rc;
         hipLaunchKernelGGL(k_scale_rsqrt, gn, bs, 0, c->stream, n, (const double *)L.s->h, L.x);
         if ((rc = spmv(cl, p, L.x, L.r))) return rc;
-        hipLaunchKernelGGL(k_cheb_step, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, (const double *)L.r, L.x, L.t, 0.0, 1.0, 0);
+        hipLaunchKernelGGL(k_block_apply, gp, bs, 0, c->stream, ncp, (const double *)L.Dinv, (const double *)L.r, L.x);
     }
     if ((rc = dots(cl, L.s, L.x, n, 1, L.x, L.s->h))) return rc;
     HIPCHK(launch_copy_f64(L.pv, L.x, n, c->stream));
