@@ -134,6 +134,31 @@ __global__ void k_point_cols(int64_t ncp, const int64_t *__restrict__ rp, const 
     }
 }
 
+// the value of the lane N further on in its row of 16 (cyclic)
+template <int N>
+__device__ __forceinline__ double row_ror(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x120 + N, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x120 + N, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// the sum over groups of LW lanes (32 or 64) as the butterfly with distances
+// LW/2 .. 1 gives it: after the step at distance d a value depends on its lane
+// modulo d alone, so rotations of rows of 16 pair the same values as exchanges do,
+// without the LDS round trip of a permutation
+template <int LW>
+__device__ __forceinline__ double group_sum(double s)
+{
+#pragma unroll
+    for (int o = LW / 2; o > 8; o >>= 1) s += __shfl_xor(s, o, 64);
+    s += row_ror<8>(s);
+    s += row_ror<4>(s);
+    s += row_ror<2>(s);
+    s += row_ror<1>(s);
+    return s;
+}
+
 // One Chebyshev step with point-block Jacobi, in the epilogue of the product
 // A v that it needs: r = rin - A v, dn = alpha v + beta Dinv r and the update of
 // x.  v is the step's direction d (or x itself, X_NONE: the first step of a
@@ -141,7 +166,7 @@ __global__ void k_point_cols(int64_t ncp, const int64_t *__restrict__ rp, const 
 // the first step's own update of x waits for the second (X_ADD2).  rout and
 // dn may be null (last step), rout may be rin.  As a kernel of its own the step
 // re-read r, d and x and was a launch more per product: a step at 64x16x16
-// (FP64) 12.7 + 3.4 us -> @CHEB64@.
+// (FP64, finest level) 27.4 + 3.4 us, now 28.8.
 enum { X_NONE, X_SET, X_ADD2, X_ADD };   // x unchanged; v + dn; x + v + dn; x + dn
 struct Cheb {
     const double *Dinv, *rin;
@@ -187,17 +212,15 @@ struct ChebRow {
 
 // y = A x on the point-block pattern: one wave per control point, lane k
 // takes neighbour points k and k+64 (one index load, three x loads and the
-// nine values of the block for the three rows)
-// MODE 0: y = A x;  1: y = b - A x;  2: the Chebyshev step ch with v = x
-template <typename T, int MODE>
+// nine values of the block for the three rows).  Patches with a periodic
+// direction; the others take k_spmv_grid.
+template <typename T>
 __global__ __launch_bounds__(256) void k_spmv_pb(int64_t ncp, const int64_t *__restrict__ rp, const int32_t *__restrict__ pcol,
-                                                 const T *__restrict__ val, const double *__restrict__ x, const double *__restrict__ b,
-                                                 double *__restrict__ y, Cheb ch)
+                                                 const T *__restrict__ val, const double *__restrict__ x, double *__restrict__ y)
 {
     const int64_t p = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (p >= ncp) return;
-    ChebRow row(ch, x, p, lane, MODE == 2);
     const int64_t b0 = rp[3 * p], b1 = rp[3 * p + 1], b2 = rp[3 * p + 2];
     const int nn = (int)((b1 - b0) / 3);
     const int32_t *pc = pcol + b0 / 9;
@@ -216,18 +239,10 @@ __global__ __launch_bounds__(256) void k_spmv_pb(int64_t ncp, const int64_t *__r
         s1 += __shfl_xor(s1, o, 64);
         s2 += __shfl_xor(s2, o, 64);
     }
-    if (MODE == 2) {
-        if (lane < 3) row.finish(ch, p, lane, s0, s1, s2);
-    } else if (lane == 0) {
-        if (MODE == 0) {
-            y[3 * p] = s0;
-            y[3 * p + 1] = s1;
-            y[3 * p + 2] = s2;
-        } else {
-            y[3 * p] = b[3 * p] - s0;
-            y[3 * p + 1] = b[3 * p + 1] - s1;
-            y[3 * p + 2] = b[3 * p + 2] - s2;
-        }
+    if (lane == 0) {
+        y[3 * p] = s0;
+        y[3 * p + 1] = s1;
+        y[3 * p + 2] = s2;
     }
 }
 
@@ -287,9 +302,11 @@ __global__ __launch_bounds__(256) void k_pack_h16(int64_t ncp, const int64_t *__
 // (rowptr[3p] / 9) and its k-th neighbour are arithmetic.
 struct PointGrid {
     int nb[3];
-    int64_t L12;   // stencil_prefix(nb1, nb1) * stencil_prefix(nb2, nb2)
-    int64_t L2;    // stencil_prefix(nb2, nb2)
-    uint64_t m12, m2;   // reciprocals of nb1 nb2 and nb2 (recip64)
+    int nch, per;      // chunks of a line of points along z, points of a chunk
+    int nblk;          // nb0 nb1 nch
+    int64_t L12;       // stencil_prefix(nb1, nb1) * stencil_prefix(nb2, nb2)
+    int64_t L2;        // stencil_prefix(nb2, nb2)
+    uint64_t mch, m1;  // reciprocals of nch and nb1 (recip64)
 };
 
 // division of a 32-bit number by a run-time divisor d > 1: the upper half of v
@@ -314,92 +331,194 @@ __device__ __forceinline__ int stencil_before(int a, int n)
     return 5 * a - (a > 1 ? 3 : 2 * a) - (a == n - 1 ? 1 : 0);
 }
 
-// y = A x with the 16-bit blocks (the layout of k_spmv_pb, FP64 sums, the
-// row scale applied once); MODE as k_spmv_pb.  Multigrid levels have no
-// periodic direction, so the point's first block, its neighbour count and
-// its neighbours come from the point grid G instead of rowptr and the
-// neighbour index (the blocks and x are the only loads).  PPW control points
-// per wave, 64 / PPW lanes each: a point's 20-byte blocks are few (at most
-// 125), so a wave per point spends its time waiting on its loads rather
-// than on the blocks; every load of a lane is issued before the sums.
-// The index arithmetic is 32-bit multiplications by reciprocals: 64-bit divisions per
-// point and two 32-bit ones per block took longer than the blocks' bytes
-// (128x32x32, 346 MB: 95 -> @H16@ us).
-template <int MODE, int PPW>
-__global__ __launch_bounds__(256) void k_spmv_h16(int64_t ncp, PointGrid G, const uint32_t *__restrict__ h16, const float *__restrict__ rs,
-                                                  const double *__restrict__ x, const double *__restrict__ b, double *__restrict__ y,
-                                                  Cheb ch)
+// A workgroup of the grid products: a chunk of at most GRID_TZ points along z of one
+// line (px, py), whose rows need x on the 5 x 5 lines around it: a run of at most
+// GRID_TZ + 4 points of each, read once into LDS.  (Read per row from the caches, the
+// 125 scattered triples are 300 cache-line accesses a point, more than the matrix.)
+// Workgroups of one XCD take consecutive chunks, so that the lines' overlap stays
+// in its L2.
+constexpr int GRID_TZ = 8, GRID_RUN = 3 * (GRID_TZ + 4);
+struct GridChunk {
+    int px, py, lx, ly, lox, loy, z0, npt, sz0;
+    int64_t pre;   // blocks before the points of the line, but for the part that depends on z
+    bool on;
+    __device__ __forceinline__ explicit GridChunk(const PointGrid &G)
+    {
+        const int per8 = (G.nblk + 7) >> 3, b = (blockIdx.x & 7) * per8 + (blockIdx.x >> 3);
+        on = b < G.nblk;
+        if (!on) return;
+        const int line = (int)div32((uint32_t)b, G.mch);
+        px = (int)div32((uint32_t)line, G.m1);
+        py = line - px * G.nb[1];
+        z0 = (b - line * G.nch) * G.per;
+        npt = G.nb[2] - z0 < G.per ? G.nb[2] - z0 : G.per;
+        lox = px - 2 > 0 ? px - 2 : 0;
+        loy = py - 2 > 0 ? py - 2 : 0;
+        lx = (px + 2 < G.nb[0] - 1 ? px + 2 : G.nb[0] - 1) - lox + 1;
+        ly = (py + 2 < G.nb[1] - 1 ? py + 2 : G.nb[1] - 1) - loy + 1;
+        sz0 = z0 - 2 > 0 ? z0 - 2 : 0;
+        pre = stencil_before(px, G.nb[0]) * G.L12 + (int64_t)lx * stencil_before(py, G.nb[1]) * G.L2;
+    }
+    // x of the chunk's neighbourhood -> xs[line][GRID_RUN]; a barrier must follow
+    __device__ __forceinline__ void stage(const PointGrid &G, const double *__restrict__ x, double *xs) const
+    {
+        const int end = z0 + npt + 2 < G.nb[2] ? z0 + npt + 2 : G.nb[2], run = 3 * (end - sz0), n = lx * ly * GRID_RUN;
+        const int iy = (65535 + ly) / ly;
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = threadIdx.x + 256 * j, ln = i / GRID_RUN, o = i - ln * GRID_RUN, kx = (ln * iy) >> 16;
+            const bool in = i < n && o < run;
+            v[j] = x[in ? 3 * (((int64_t)(lox + kx) * G.nb[1] + loy + ln - kx * ly) * G.nb[2] + sz0) + o : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if ((int)threadIdx.x + 256 * j < n) xs[threadIdx.x + 256 * j] = v[j];
+    }
+};
+static_assert(25 * GRID_RUN <= 4 * 256, "four loads a thread");
+
+// one point of a chunk: its number, neighbours and first block
+struct GridPoint {
+    int64_t p, blk;
+    int nn, lz, iz, zo;
+    __device__ __forceinline__ GridPoint(const PointGrid &G, const GridChunk &c, int slot)
+    {
+        const int pz = c.z0 + slot, n2 = G.nb[2], loz = pz - 2 > 0 ? pz - 2 : 0;
+        lz = (pz + 2 < n2 - 1 ? pz + 2 : n2 - 1) - loz + 1;
+        p = ((int64_t)c.px * G.nb[1] + c.py) * n2 + pz;
+        nn = c.lx * c.ly * lz;
+        blk = c.pre + c.lx * c.ly * stencil_before(pz, n2);
+        iz = (65535 + lz) / lz;   // k / lz by multiplication: exact while k lz < 2^16
+        zo = 3 * (loz - c.sz0);
+    }
+    // where block k < nn finds its x in LDS
+    __device__ __forceinline__ int at(int k) const
+    {
+        const int ln = (k * iz) >> 16;
+        return ln * GRID_RUN + zo + 3 * (k - ln * lz);
+    }
+};
+
+// The assembled matrix on a patch without periodic directions: the sums of
+// k_spmv_pb (one wave per point, lane k blocks k and k + 64) with the CSR
+// positions and neighbours from the point grid and x from LDS.
+// MODE 0: y = A x;  1: y = b - A x;  2: the Chebyshev step ch with v = x.
+// Bound by the matrix's bytes in FP64 (128x32x32, 1.25 GB: 218 -> 202 us,
+// 6.2 TB/s; 64x16x16 27.2 -> 25.5 us; FP32 134 -> 113 us).
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void k_spmv_grid(PointGrid G, const T *__restrict__ val, const double *__restrict__ x,
+                                                   const double *__restrict__ b, double *__restrict__ y, Cheb ch)
 {
-    constexpr int LW = 64 / PPW;   // lanes per control point
-    const int lane = threadIdx.x & 63, sl = lane & (LW - 1);
-    const int64_t p = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * PPW + lane / LW;
-    const bool ok = p < ncp;
-    ChebRow row(ch, x, p, sl, MODE == 2 && ok);
-    double s0 = 0, s1 = 0, s2 = 0;
-    if (ok) {
-        const int n1 = G.nb[1], n2 = G.nb[2];
-        const int pq = (int)div32((uint32_t)p, G.m2), px = (int)div32((uint32_t)p, G.m12), py = pq - px * n1, pz = (int)p - pq * n2;
-        const int lox = px - 2 > 0 ? px - 2 : 0, loy = py - 2 > 0 ? py - 2 : 0, loz = pz - 2 > 0 ? pz - 2 : 0;
-        const int lx = (px + 2 < G.nb[0] - 1 ? px + 2 : G.nb[0] - 1) - lox + 1;
-        const int ly = (py + 2 < n1 - 1 ? py + 2 : n1 - 1) - loy + 1;
-        const int lz = (pz + 2 < n2 - 1 ? pz + 2 : n2 - 1) - loz + 1;
-        const int nn = lx * ly * lz, lyz = ly * lz;
-        const int64_t blk = stencil_before(px, G.nb[0]) * G.L12 + lx * (stencil_before(py, n1) * G.L2 + ly * stencil_before(pz, n2));
-        const uint32_t *hb = h16 + 5 * blk;
-        // k / lyz and r / lz of k < 125 by multiplication: exact while k d < 2^16
-        const int iyz = (65535 + lyz) / lyz, iz = (65535 + lz) / lz;
-        // at most 125 neighbours: a fixed number of rounds
-        constexpr int NIT = (125 + LW - 1) / LW;
-        uint32_t w[NIT][5];
-        double xv[NIT][3];
+    __shared__ double xs[25 * GRID_RUN];
+    constexpr int NR = GRID_TZ / 4;
+    const GridChunk c(G);
+    if (!c.on) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    c.stage(G, x, xs);
+    T a[NR][2][9];
 #pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const int k = sl + it * LW;
-            if (k < nn) {
-                const int kx = (k * iyz) >> 16, r = k - kx * lyz, ky = (r * iz) >> 16, kz = r - ky * lz;
-                const int64_t q = ((lox + kx) * n1 + (loy + ky)) * n2 + (loz + kz);
+    for (int r = 0; r < NR; r++) {
+        const int slot = wv + 4 * r < c.npt ? wv + 4 * r : 0;
+        const GridPoint q(G, c, slot);
 #pragma unroll
-                for (int j = 0; j < 3; j++) xv[it][j] = x[3 * q + j];
+        for (int it = 0; it < 2; it++) {
+            const int k = lane + 64 * it < q.nn ? lane + 64 * it : 0;
+            const T *v = val + 9 * q.blk + 3 * k;
 #pragma unroll
-                for (int j = 0; j < 5; j++) w[it][j] = hb[j * nn + k];
-            } else {
+            for (int i = 0; i < 3; i++)
 #pragma unroll
-                for (int j = 0; j < 3; j++) xv[it][j] = 0.0;
+                for (int j = 0; j < 3; j++) a[r][it][3 * i + j] = v[3 * q.nn * i + j];
+        }
+    }
+    __syncthreads();
 #pragma unroll
-                for (int j = 0; j < 5; j++) w[it][j] = 0u;
+    for (int r = 0; r < NR; r++) {
+        if (wv + 4 * r >= c.npt) break;
+        const GridPoint q(G, c, wv + 4 * r);
+        ChebRow row(ch, x, q.p, lane, MODE == 2);
+        double s0 = 0, s1 = 0, s2 = 0;
+#pragma unroll
+        for (int it = 0; it < 2; it++) {
+            const int k = lane + 64 * it;
+            if (k < q.nn) {
+                const double *xk = xs + q.at(k);
+                const double x0 = xk[0], x1 = xk[1], x2 = xk[2];
+                const T *v = a[r][it];
+                s0 += (double)v[0] * x0 + (double)v[1] * x1 + (double)v[2] * x2;
+                s1 += (double)v[3] * x0 + (double)v[4] * x1 + (double)v[5] * x2;
+                s2 += (double)v[6] * x0 + (double)v[7] * x1 + (double)v[8] * x2;
             }
         }
-#pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            s0 += h_lo(w[it][0]) * xv[it][0] + h_hi(w[it][0]) * xv[it][1] + h_lo(w[it][1]) * xv[it][2];
-            s1 += h_hi(w[it][1]) * xv[it][0] + h_lo(w[it][2]) * xv[it][1] + h_hi(w[it][2]) * xv[it][2];
-            s2 += h_lo(w[it][3]) * xv[it][0] + h_hi(w[it][3]) * xv[it][1] + h_lo(w[it][4]) * xv[it][2];
-        }
-    }
-#pragma unroll
-    for (int o = LW / 2; o > 0; o >>= 1) {
-        s0 += __shfl_xor(s0, o, 64);
-        s1 += __shfl_xor(s1, o, 64);
-        s2 += __shfl_xor(s2, o, 64);
-    }
-    if (MODE == 2) {
-        if (ok && sl < 3) row.finish(ch, p, sl, s0 * (double)rs[3 * p], s1 * (double)rs[3 * p + 1], s2 * (double)rs[3 * p + 2]);
-    } else if (ok && sl == 0) {
-        s0 *= (double)rs[3 * p];
-        s1 *= (double)rs[3 * p + 1];
-        s2 *= (double)rs[3 * p + 2];
-        if (MODE == 0) {
-            y[3 * p] = s0;
-            y[3 * p + 1] = s1;
-            y[3 * p + 2] = s2;
-        } else {
-            y[3 * p] = b[3 * p] - s0;
-            y[3 * p + 1] = b[3 * p + 1] - s1;
-            y[3 * p + 2] = b[3 * p + 2] - s2;
+        s0 = group_sum<64>(s0);
+        s1 = group_sum<64>(s1);
+        s2 = group_sum<64>(s2);
+        if (MODE == 2) {
+            if (lane < 3) row.finish(ch, q.p, lane, s0, s1, s2);
+        } else if (lane == 0) {
+            y[3 * q.p] = MODE == 0 ? s0 : b[3 * q.p] - s0;
+            y[3 * q.p + 1] = MODE == 0 ? s1 : b[3 * q.p + 1] - s1;
+            y[3 * q.p + 2] = MODE == 0 ? s2 : b[3 * q.p + 2] - s2;
         }
     }
 }
-constexpr int H16_PPW = 2;   // control points per wave of k_spmv_h16
+
+// The same with the 16-bit blocks (FP64 sums, the row scale applied once):
+// two points per wave, 32 lanes each, since a point's 20-byte blocks are few;
+// every load of a lane is issued before the sums.  128x32x32 (346 MB): 95 us with
+// x read per block from the caches and 64-bit index divisions, 81 us here
+// (4.3 TB/s; the conversions and FP64 products of 32 lanes a point are what
+// is left), 87 us with the Chebyshev step in it.
+template <int MODE>
+__global__ __launch_bounds__(256) void k_spmv_h16(PointGrid G, const uint32_t *__restrict__ h16, const float *__restrict__ rs,
+                                                  const double *__restrict__ x, const double *__restrict__ b, double *__restrict__ y,
+                                                  Cheb ch)
+{
+    __shared__ double xs[25 * GRID_RUN];
+    constexpr int LW = 32, NIT = (125 + LW - 1) / LW;   // lanes per point, rounds
+    static_assert(GRID_TZ * LW == 256, "a chunk a workgroup");
+    const GridChunk c(G);
+    if (!c.on) return;
+    const int sl = threadIdx.x & (LW - 1), slot = threadIdx.x / LW;
+    const bool ok = slot < c.npt;
+    const GridPoint q(G, c, ok ? slot : 0);
+    c.stage(G, x, xs);
+    uint32_t w[NIT][5];
+    const uint32_t *hb = h16 + 5 * q.blk;
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+        const int k = sl + it * LW < q.nn ? sl + it * LW : 0;
+#pragma unroll
+        for (int j = 0; j < 5; j++) w[it][j] = hb[j * q.nn + k];
+    }
+    ChebRow row(ch, x, q.p, sl, MODE == 2 && ok);
+    __syncthreads();
+    double s0 = 0, s1 = 0, s2 = 0;
+#pragma unroll
+    for (int it = 0; it < NIT; it++) {
+        const int k = sl + it * LW;
+        if (k < q.nn) {
+            const double *xk = xs + q.at(k);
+            const double x0 = xk[0], x1 = xk[1], x2 = xk[2];
+            s0 += h_lo(w[it][0]) * x0 + h_hi(w[it][0]) * x1 + h_lo(w[it][1]) * x2;
+            s1 += h_hi(w[it][1]) * x0 + h_lo(w[it][2]) * x1 + h_hi(w[it][2]) * x2;
+            s2 += h_lo(w[it][3]) * x0 + h_hi(w[it][3]) * x1 + h_lo(w[it][4]) * x2;
+        }
+    }
+    s0 = group_sum<LW>(s0);
+    s1 = group_sum<LW>(s1);
+    s2 = group_sum<LW>(s2);
+    if (!ok || sl > 2) return;
+    s0 *= (double)rs[3 * q.p];
+    s1 *= (double)rs[3 * q.p + 1];
+    s2 *= (double)rs[3 * q.p + 2];
+    if (MODE == 2) {
+        row.finish(ch, q.p, sl, s0, s1, s2);
+    } else {
+        const double t = sl == 0 ? s0 : sl == 1 ? s1 : s2;
+        y[3 * q.p + sl] = MODE == 0 ? t : b[3 * q.p + sl] - t;
+    }
+}
 
 // y[i] = x[idx[i]]  (values or vectors into the coloured order)
 // (grid-stride: launched with grid1)
@@ -1505,16 +1624,43 @@ static int ensure_pcol(igap_gpu_ctx *c)
     return IGAP_OK;
 }
 
-// y = A x (mode 0), y = b - A x (1) or a Chebyshev step on d = x (2) with the context's tangent values
+static PointGrid point_grid(const MeshK &M)
+{
+    PointGrid G;
+    for (int d = 0; d < 3; d++) G.nb[d] = M.nb[d];
+    G.nch = (M.nb[2] + GRID_TZ - 1) / GRID_TZ;
+    G.per = (M.nb[2] + G.nch - 1) / G.nch;
+    G.nblk = M.nb[0] * M.nb[1] * G.nch;
+    G.L2 = stencil_prefix(M.nb[2], M.nb[2]);
+    G.L12 = stencil_prefix(M.nb[1], M.nb[1]) * G.L2;
+    G.mch = recip64(G.nch);
+    G.m1 = recip64(M.nb[1]);
+    return G;
+}
+
+// y = A x (mode 0), and on a patch without periodic directions y = b - A x (1)
+// or a Chebyshev step on d = x (2), with the context's tangent values
 static int spmv(igap_gpu_ctx *c, int p, const double *x, double *y, int mode = 0, const double *b = nullptr, const Cheb &ch = Cheb())
 {
     const int64_t n = c->ndof, ncp = n / 3;
-    int rc = ensure_pcol(c);
-    if (rc) return rc;
-    const dim3 g((unsigned)((ncp + 3) / 4)), bs(256);
-    const int64_t *rp = (const int64_t *)c->d_rowptr;
-    const int32_t *pc = (const int32_t *)c->d_pcol;
-#define IGAP_SPMV(T, V, M) hipLaunchKernelGGL((k_spmv_pb<T, M>), g, bs, 0, c->stream, ncp, rp, pc, (const T *)V, x, b, y, ch)
+    const dim3 bs(256);
+    if (c->M.periodic[0] || c->M.periodic[1] || c->M.periodic[2]) {
+        if (mode != 0) return fail(IGAP_ERR_STATE, "product of mode %d on a periodic patch", mode);
+        int rc = ensure_pcol(c);
+        if (rc) return rc;
+        const dim3 g((unsigned)((ncp + 3) / 4));
+        if (p == IGAP_F64)
+            hipLaunchKernelGGL(k_spmv_pb<double>, g, bs, 0, c->stream, ncp, (const int64_t *)c->d_rowptr, (const int32_t *)c->d_pcol,
+                               (const double *)c->d_val64, x, y);
+        else
+            hipLaunchKernelGGL(k_spmv_pb<float>, g, bs, 0, c->stream, ncp, (const int64_t *)c->d_rowptr, (const int32_t *)c->d_pcol,
+                               (const float *)c->d_val32, x, y);
+        HIPCHK(hipGetLastError());
+        return IGAP_OK;
+    }
+    const PointGrid G = point_grid(c->M);
+    const dim3 g((unsigned)((G.nblk + 7) / 8 * 8));
+#define IGAP_SPMV(T, V, M) hipLaunchKernelGGL((k_spmv_grid<T, M>), g, bs, 0, c->stream, G, (const T *)V, x, b, y, ch)
     if (p == IGAP_F64) {
         if (mode == 0) IGAP_SPMV(double, c->d_val64, 0);
         else if (mode == 1) IGAP_SPMV(double, c->d_val64, 1);
@@ -1984,27 +2130,21 @@ static int mg_build_levels(igap_gpu_ctx *c, Solver *s, MGHier *g, int maxlev)
     return IGAP_OK;
 }
 
-// A x on multigrid level l in the preconditioner's precision (MODE of k_spmv_pb)
+// A x on multigrid level l in the preconditioner's precision (MODE of k_spmv_grid)
 static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, double *y, int mode = 0, const double *b = nullptr,
                     const Cheb &ch = Cheb())
 {
     MGLevel &L = g->lev[l];
     if (p != PC_F16 || !L.h16) return spmv(L.c, p == PC_F16 ? IGAP_F32 : p, x, y, mode, b, ch);
-    const int64_t ncp = L.c->ndof / 3;
-    const dim3 gr((unsigned)((ncp + 4 * H16_PPW - 1) / (4 * H16_PPW))), bs(256);
     const uint32_t *hv = (const uint32_t *)L.h16;
     const float *rs = (const float *)L.rs;
     const MeshK &M = L.c->M;
     if (M.periodic[0] || M.periodic[1] || M.periodic[2]) return fail(IGAP_ERR_STATE, "16-bit multigrid level on a periodic patch");
-    PointGrid G;
-    for (int d = 0; d < 3; d++) G.nb[d] = M.nb[d];
-    G.L2 = stencil_prefix(M.nb[2], M.nb[2]);
-    G.L12 = stencil_prefix(M.nb[1], M.nb[1]) * G.L2;
-    G.m2 = recip64(M.nb[2]);
-    G.m12 = recip64((uint64_t)M.nb[1] * M.nb[2]);
-    if (mode == 0) hipLaunchKernelGGL((k_spmv_h16<0, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
-    else if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
-    else hipLaunchKernelGGL((k_spmv_h16<2, H16_PPW>), gr, bs, 0, c->stream, ncp, G, hv, rs, x, b, y, ch);
+    const PointGrid G = point_grid(M);
+    const dim3 gr((unsigned)((G.nblk + 7) / 8 * 8)), bs(256);
+    if (mode == 0) hipLaunchKernelGGL((k_spmv_h16<0>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
+    else if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
+    else hipLaunchKernelGGL((k_spmv_h16<2>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
     HIPCHK(hipGetLastError());
     return IGAP_OK;
 }
@@ -2141,7 +2281,6 @@ static int mg_setup(igap_gpu_ctx *c, Solver *s, int pm)
             if (pm == PC_F16) {
                 igap_gpu_ctx *cl = L.c;
                 const int64_t ncp = cl->ndof / 3;
-                if ((rc = ensure_pcol(cl))) return rc;
                 if (!L.h16) {
                     DALLOC(&L.h16, sizeof(uint32_t) * 5 * (size_t)(cl->nnz / 9));
                     DALLOC(&L.rs, sizeof(float) * (size_t)cl->ndof);
