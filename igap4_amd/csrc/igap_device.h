@@ -58,6 +58,39 @@ __device__ __forceinline__ int sidx(int I, int K)
 
 __host__ __device__ __forceinline__ int own1(int a, int n, int periodic) { return periodic ? (a >= n ? a - n : a) : a; }
 
+// ---------------------------------------------------------------- lanes
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+// Sums over aligned groups of 4, 8 and 16 lanes, in every lane, as the butterfly
+// with distances 1, 2, 4, 8 gives them: once the groups of 2^n lanes hold their
+// sum, a mirror image pairs the same two groups as the exchange does.  Lane
+// moves of the vector ALU in place of permutations through LDS, whose pipe the
+// eight-node sums of the transient kernels filled.
+__device__ __forceinline__ double sum4(double v)
+{
+    v += dpp<0xB1>(v);    // quad_perm 1, 0, 3, 2
+    v += dpp<0x4E>(v);    // quad_perm 2, 3, 0, 1
+    return v;
+}
+__device__ __forceinline__ double sum8(double v)
+{
+    v = sum4(v);
+    v += dpp<0x141>(v);   // mirror in eight lanes
+    return v;
+}
+__device__ __forceinline__ double sum16(double v)
+{
+    v = sum8(v);
+    v += dpp<0x140>(v);   // mirror in sixteen lanes
+    return v;
+}
+
 // ---------------------------------------------------------------- basis
 // value/first/second derivative of the three quadratic B-splines of the span
 // [kV[2], kV[3]] of the five-knot window kV at x

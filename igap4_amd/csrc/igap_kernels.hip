@@ -276,8 +276,7 @@ __global__ __launch_bounds__(256, (NH == 1 ? 4 : 2)) void k_residual_elem(MeshK 
         }
 #pragma unroll
         for (int a = 0; a < 30; a++) {
-            r[a] += __shfl_xor(r[a], 1, 64);
-            r[a] += __shfl_xor(r[a], 2, 64);
+            r[a] = sum4(r[a]);
         }
         if (part == 0) {
 #pragma unroll
@@ -832,9 +831,10 @@ __global__ __launch_bounds__(256, 2) void k_tangent_elem(MeshK M, PhysK P, const
 #pragma unroll
                 for (int a = 0; a < 10; a++) W[a] = wb * N[a];
 #pragma unroll
-                for (int o = 1; o < 32; o <<= 1)
-#pragma unroll
-                    for (int a = 0; a < 10; a++) W[a] += __shfl_xor(W[a], o, 64);
+                for (int a = 0; a < 10; a++) {
+                    W[a] = sum16(W[a]);
+                    W[a] += __shfl_xor(W[a], 16, 64);
+                }
                 if (b < 27) {
                     nurbs_param(N, wb, W, R);
                     phys_jet(R, g + 1, g + 10);
@@ -863,14 +863,11 @@ __global__ __launch_bounds__(256, 2) void k_tangent_elem(MeshK M, PhysK P, const
                 for (int i = 0; i < 9; i++) {
                     double sv = w0 * st.S[i], gv = w0 * st.G[i];
                     double n0 = w0 * st.N[i], n1 = w1 * st.N[i], n2 = w2 * st.N[i];
-#pragma unroll
-                    for (int o = 1; o < 8; o <<= 1) {
-                        sv += __shfl_xor(sv, o, 64);
-                        gv += __shfl_xor(gv, o, 64);
-                        n0 += __shfl_xor(n0, o, 64);
-                        n1 += __shfl_xor(n1, o, 64);
-                        n2 += __shfl_xor(n2, o, 64);
-                    }
+                    sv = sum8(sv);
+                    gv = sum8(gv);
+                    n0 = sum8(n0);
+                    n1 = sum8(n1);
+                    n2 = sum8(n2);
                     if (j == 0) {
                         ms[MS + i] = sv;
                         ms[MG + i] = gv;
@@ -1741,13 +1738,10 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
 #pragma unroll
                 for (int t = 0; t < 6; t++) {
                     double sv = w0 * st.S[PR[t]], n0 = w0 * st.N[PR[t]], n1 = w1 * st.N[PR[t]], n2 = w2 * st.N[PR[t]];
-#pragma unroll
-                    for (int o = 1; o < 8; o <<= 1) {
-                        sv += __shfl_xor(sv, o, 64);
-                        n0 += __shfl_xor(n0, o, 64);
-                        n1 += __shfl_xor(n1, o, 64);
-                        n2 += __shfl_xor(n2, o, 64);
-                    }
+                    sv = sum8(sv);
+                    n0 = sum8(n0);
+                    n1 = sum8(n1);
+                    n2 = sum8(n2);
                     if (j == 0) {
                         ms[MS_S + t] = (T)sv;
                         ms[MS_N11 + t] = (T)(n0 / mu.m0);
@@ -1757,9 +1751,7 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
                 }
 #pragma unroll
                 for (int i = 0; i < 9; i++) {
-                    double gv = w0 * st.G[i];
-#pragma unroll
-                    for (int o = 1; o < 8; o <<= 1) gv += __shfl_xor(gv, o, 64);
+                    const double gv = sum8(w0 * st.G[i]);
                     if (j == 0) ms[MS_G + i] = (T)gv;
                 }
             }
@@ -1990,10 +1982,7 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
 #pragma unroll
             for (int a = 0; a < 30; a++) {
                 if (a % 10 == 0) continue;   // value slots: the inertia, added below
-                double v = r[a];
-#pragma unroll
-                for (int o = 1; o < 8; o <<= 1) v += __shfl_xor(v, o, 64);
-                r[a] = v;
+                r[a] = sum8(r[a]);
             }
             if (j == 0) {
 #pragma unroll

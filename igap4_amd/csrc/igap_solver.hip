@@ -134,15 +134,6 @@ __global__ void k_point_cols(int64_t ncp, const int64_t *__restrict__ rp, const 
     }
 }
 
-// the value of the lane N further on in its row of 16 (cyclic)
-template <int N>
-__device__ __forceinline__ double row_ror(double v)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x120 + N, 0xf, 0xf, true);
-    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x120 + N, 0xf, 0xf, true);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 // the sum over groups of LW lanes (32 or 64) as the butterfly with distances
 // LW/2 .. 1 gives it: after the step at distance d a value depends on its lane
 // modulo d alone, so rotations of rows of 16 pair the same values as exchanges do,
@@ -152,10 +143,10 @@ __device__ __forceinline__ double group_sum(double s)
 {
 #pragma unroll
     for (int o = LW / 2; o > 8; o >>= 1) s += __shfl_xor(s, o, 64);
-    s += row_ror<8>(s);
-    s += row_ror<4>(s);
-    s += row_ror<2>(s);
-    s += row_ror<1>(s);
+    s += dpp<0x120 + 8>(s);
+    s += dpp<0x120 + 4>(s);
+    s += dpp<0x120 + 2>(s);
+    s += dpp<0x120 + 1>(s);
     return s;
 }
 
