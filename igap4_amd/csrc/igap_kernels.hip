@@ -1174,8 +1174,8 @@ __device__ __forceinline__ void sep_element(const MeshK &M, const double *__rest
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 const double u0 = Uh[3 * oc + k], u1 = Uh[ndof + 3 * oc + k], u2 = Uh[2 * ndof + 3 * oc + k];
-                sU[3 * tid + k] = 0.5 * (u1 + u2);
-                sUd[3 * tid + k] = 0.5 * (u0 - u2);
+                sU[STR * tid + k] = 0.5 * (u1 + u2);
+                sUd[STR * tid + k] = 0.5 * (u0 - u2);
                 // the inertia combination of the residual's value slot
                 if (sV) sV[3 * tid + k] = cv1 * (u0 - u2) + cv2 * (u0 + u2 - 2 * u1);
             }
@@ -1188,15 +1188,29 @@ __device__ __forceinline__ void sep_element(const MeshK &M, const double *__rest
     }
 }
 
+// the periodic macro-field at point q added to the jet of component k
+__device__ __forceinline__ void sep_macro(const MeshK &M, const int *ed, int q, int k, double *J)
+{
+    const int qd[3] = {q >> 4, (q >> 2) & 3, q & 3};
+    double xq[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double *kV = M.knot[d] + ed[d];
+        const double c = M.gq[qd[d]];
+        xq[d] = (-c + 1.0) * kV[2] + c * kV[3];
+    }
+    add_periodic1(M, xq, k, J);
+}
+
 // Physical displacement jets at the 64 Gauss points of a separable element by
 // sum factorisation over the physical tables (z, y, then x; sWork holds 1188
 // doubles), after sep_element and a barrier; at least 192 threads, all of which
 // call it.  Lane q of wave k < 3 returns in J the jet of component k at point q
-// (par_periodic's macro-field added unless macro is false).  The passes are
+// (par_periodic's macro-field added).  The passes are
 // short and serial, so each takes as many threads as it has independent groups
 // of outputs (108, 144 and 192).
 __device__ __forceinline__ void sep_fields(const MeshK &M, const int *ed, const double *sU, const double (*sPd)[4][3][3],
-                                           double *sWork, double *J, bool macro = true)
+                                           double *sWork, double *J)
 {
     const int tid = threadIdx.x;
     double *sA = sWork, *sB = sA + 3 * 108;
@@ -1230,19 +1244,47 @@ __device__ __forceinline__ void sep_fields(const MeshK &M, const int *ed, const 
     // x
     if (tid < 192) {
         const int q = tid & 63, k = tid >> 6;
-        const int qd[3] = {q >> 4, (q >> 2) & 3, q & 3};
-        sf_jet(sB + 288 * k + (q & 15) * 6, &sPd[0][qd[0]][0][0], J);
-        double xq[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const double *kV = M.knot[d] + ed[d];
-            const double c = M.gq[qd[d]];
-            xq[d] = (-c + 1.0) * kV[2] + c * kV[3];
-        }
-        if (macro) add_periodic1(M, xq, k, J);
+        sf_jet(sB + 288 * k + (q & 15) * 6, &sPd[0][q >> 4][0][0], J);
+        sep_macro(M, ed, q, k, J);
     }
 }
 
+// Field passes of six nodal fields c[b][f] at once (two of sep_fields' sets, or
+// coordinates and displacements), sWork 6 * (108 + 288) doubles: the z and y
+// passes; six_jet then is the x pass of one field at one point.  One pass of
+// six has half the barriers of two passes of three.
+__device__ __forceinline__ void six_fields(const double (*c)[6], const double (*sPd)[4][3][3], double *sWork)
+{
+    double *sA = sWork, *sB = sA + 6 * 108;
+    for (int i = threadIdx.x; i < 216; i += blockDim.x) {
+        const int qz = i & 3, g = i >> 2, f = g / 9, bxy = g - 9 * f;
+        const double c0 = c[3 * bxy][f], c1 = c[3 * bxy + 1][f], c2 = c[3 * bxy + 2][f];
+        double *o = sA + 108 * f + 12 * bxy + 3 * qz;
+#pragma unroll
+        for (int dz = 0; dz < 3; dz++) {
+            const double *tz = &sPd[2][qz][dz][0];
+            o[dz] = c0 * tz[0] + c1 * tz[1] + c2 * tz[2];
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 288; i += blockDim.x) {
+        const int qz = i & 3, qy = (i >> 2) & 3, g = i >> 4, f = g / 3, bx = g - 3 * f;
+        const double *a = sA + 108 * f + 36 * bx + 3 * qz;   // a[12 by + dz]
+        double *o = sB + 288 * f + 96 * bx + 24 * qy + 6 * qz;
+#pragma unroll
+        for (int s6 = 0; s6 < 6; s6++) {
+            const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
+            const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
+            const double *ty = &sPd[1][qy][dy][0];
+            o[s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
+        }
+    }
+    __syncthreads();
+}
+__device__ __forceinline__ void six_jet(const double *sWork, const double (*sPd)[4][3][3], int f, int q, double *J)
+{
+    sf_jet(sWork + 6 * 108 + 288 * f + (q & 15) * 6, &sPd[0][q >> 4][0][0], J);
+}
 // Gauss weight x span lengths x det G at point q of a separable element
 __device__ __forceinline__ double sep_weight(int q, const double (*sW)[4]) { return sW[0][q >> 4] * sW[1][(q >> 2) & 3] * sW[2][q & 3]; }
 
@@ -1456,41 +1498,7 @@ template <typename T> struct GenPipe;
 template <> struct GenPipe<double> { typedef PipeShape<2, 1, 1, false, true> S; };
 template <> struct GenPipe<float> { typedef PipeShape<2, 1, 2, false, true> S; };
 
-// field passes of k_tangent_gen: c[b][f] the six nodal fields (x, u), sWork 6 *
-// (108 + 288) doubles; lane q of wave f < 6 returns the parametric jet of field f at point q
-__device__ __forceinline__ void gen_fields(const double (*c)[6], const double (*sPd)[4][3][3], double *sWork, double *J)
-{
-    const int tid = threadIdx.x;
-    double *sA = sWork, *sB = sA + 6 * 108;
-    if (tid < 216) {
-        const int qz = tid & 3, g = tid >> 2, f = g / 9, bxy = g - 9 * f;
-        const double c0 = c[3 * bxy][f], c1 = c[3 * bxy + 1][f], c2 = c[3 * bxy + 2][f];
-        double *o = sA + 108 * f + 12 * bxy + 3 * qz;
-#pragma unroll
-        for (int dz = 0; dz < 3; dz++) {
-            const double *tz = &sPd[2][qz][dz][0];
-            o[dz] = c0 * tz[0] + c1 * tz[1] + c2 * tz[2];
-        }
-    }
-    __syncthreads();
-    if (tid < 288) {
-        const int qz = tid & 3, qy = (tid >> 2) & 3, g = tid >> 4, f = g / 3, bx = g - 3 * f;
-        const double *a = sA + 108 * f + 36 * bx + 3 * qz;   // a[12 by + dz]
-        double *o = sB + 288 * f + 96 * bx + 24 * qy + 6 * qz;
-#pragma unroll
-        for (int s6 = 0; s6 < 6; s6++) {
-            const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
-            const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
-            const double *ty = &sPd[1][qy][dy][0];
-            o[s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
-        }
-    }
-    __syncthreads();
-    const int q = tid & 63, f = tid >> 6;
-    if (f < 6) sf_jet(sB + 288 * f + (q & 15) * 6, &sPd[0][q >> 4][0][0], J);
-}
-
-// the states of GeneralIn at the 64 points (eight waves; J as gen_fields leaves it); ends with a block barrier
+// the states of GeneralIn at the 64 points (eight waves; lane q of wave f < 6 holds field f's parametric jet at point q in J); ends with a block barrier
 __device__ __forceinline__ void gen_states(const MeshK &M, const PhysK &P, const int *ed, double *J, const double (*sW)[4], double *sSt)
 {
     constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
@@ -1515,15 +1523,8 @@ __device__ __forceinline__ void gen_states(const MeshK &M, const PhysK &P, const
         const double det = inv3(G, Gi);
         if (part < 6) {
             const int k = part - 3;
-            double xq[3];
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const double *kV = M.knot[d] + ed[d];
-                const double c = M.gq[d == 0 ? q >> 4 : d == 1 ? (q >> 2) & 3 : q & 3];
-                xq[d] = (-c + 1.0) * kV[2] + c * kV[3];
-            }
             phys_jet(J, Gi, X2);
-            add_periodic1(M, xq, k, J);
+            sep_macro(M, ed, q, k, J);
 #pragma unroll
             for (int i = 0; i < 3; i++) sp[10 * k + i] = J[1 + i] + (k == i ? 1.0 : 0.0);
 #pragma unroll
@@ -1624,7 +1625,8 @@ __global__ __launch_bounds__((GenPipe<T>::S::THREADS), 2) void k_tangent_gen(
     __syncthreads();
     {
         double J[10];
-        gen_fields(sC, sPd, reinterpret_cast<double *>(sE), J);
+        six_fields(sC, sPd, reinterpret_cast<double *>(sE));
+        if (tid < 384) six_jet(reinterpret_cast<double *>(sE), sPd, tid >> 6, tid & 63, J);
         gen_states(M, P, ed, J, sW, sSt);
     }
     const GeneralIn in{sSt, P.e345, P.le};
@@ -1646,10 +1648,11 @@ __global__ __launch_bounds__((GenPipe<T>::S::THREADS), 2) void k_tangent_gen(
 // compact and in the contraction's precision (one lane per rule node, sums
 // over 8-lane groups), so that the FP32 kernel keeps two workgroups per CU
 // (76 KB of LDS; FP64, 149 KB: one).  Bound by vector issue like the static one,
-// and by stage A.  Two pencils per interval and one D wave: 13.5 ms in FP32 at
-// 128x32x32 (14.2 ms as a loop of all waves over the pencils; one pencil and two D
-// waves 18.8, its registers limiting both to two workgroups), 2.06 ms in FP64 at
-// 64x16x16 (one pencil 2.4).
+// and by stage A (all six fields in one pass, a lane per rule node and point, sums by
+// lane moves; as two passes, two rounds of half the waves and LDS permutations it took
+// 13.5 ms at 128x32x32 in FP32, 10.9 now; FP64 at 24^3 1.78 -> 1.48 ms).  Two
+// pencils per interval and one D wave: one pencil and two D waves took 18.8 ms,
+// their registers limiting both to two workgroups.
 template <typename T, bool DIRECT>
 __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) void k_tangent_sep_t(
     MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof, T *__restrict__ Ke, Scatter S, const T *__restrict__ tabx,
@@ -1658,7 +1661,7 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
     typedef SepShape<T, 3> Sh;
     __shared__ double sPd[3][4][3][3];
     __shared__ double sW[3][4];
-    __shared__ double sU[27 * 3], sUd[27 * 3];
+    __shared__ double sC[27][6];                // nodal Um, Ud
     __shared__ double sWgt[64];
     __shared__ double sMass[3][3][3];          // 1-D mass matrices M_d[b][c]
     __shared__ __attribute__((aligned(16))) T sMom[64 * MS_W];   // compact moment states (first the field passes' buffers)
@@ -1667,7 +1670,8 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
     __shared__ int32_t sMsk[DIRECT ? 81 : 1];
     __shared__ __attribute__((aligned(16))) T sD[Sh::D_SIZE];
     __shared__ __attribute__((aligned(16))) T sE[Sh::E_SIZE];
-    static_assert(64 * MS_W * sizeof(T) >= 3 * (108 + 288) * sizeof(double) && Sh::D_SIZE >= 64 * 54, "stage A's buffers");
+    static_assert(64 * MS_W * sizeof(T) >= 6 * (108 + 288) * sizeof(double) && Sh::D_SIZE >= 64 * 54, "stage A's buffers");
+    static_assert(Sh::THREADS == 512, "a lane per rule node and point");
     T *sJet = sD;                               // [q][h][k][a - 1], stage A only
 
     const int tid = threadIdx.x, e = blockIdx.x;
@@ -1676,28 +1680,23 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
     if (DIRECT) sep_rows(M, S, ed, sRow, sMsk);
 
     if (tid >= 256 && tid < 256 + 36) sX[tid - 256] = tabx[ed[0] * TAB_STRIDE + tid - 256];
-    sep_element<3>(M, Uh, ed, sU, sPd, sW, ndof, sUd);
+    sep_element<3, 6>(M, Uh, ed, &sC[0][0], sPd, sW, ndof, &sC[0][3]);
     __syncthreads();
     // ---- stage A: jets of Um and Ud, point weights, 1-D mass matrices
     {
-        double J1[10], J2[10];
-        sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sMom), J1, true);
-        __syncthreads();
-        sep_fields(M, ed, sUd, sPd, reinterpret_cast<double *>(sMom), J2, false);
-        __syncthreads();
-        const int q = tid & 63, k = tid >> 6;
-        if (k < 3) {
-            T *jq = sJet + q * 54;
+        double *work = reinterpret_cast<double *>(sMom);
+        six_fields(sC, sPd, work);
+        const int q = tid & 63, f = tid >> 6;   // field f < 3: Um, f < 6: Ud
+        if (f < 6) {
+            double J[10];
+            six_jet(work, sPd, f, q, J);
+            if (f < 3) sep_macro(M, ed, q, f, J);
 #pragma unroll
-            for (int a = 1; a < 10; a++) {
-                jq[9 * k + a - 1] = (T)J1[a];
-                jq[27 + 9 * k + a - 1] = (T)J2[a];
-            }
-        } else if (k == 3) {
+            for (int a = 1; a < 10; a++) sJet[q * 54 + 9 * f + a - 1] = (T)J[a];
+        } else if (f == 6) {
             sWgt[q] = sep_weight(q, sW);
-        }
-        if (tid < 27) {
-            const int d = tid / 9, b = (tid / 3) % 3, c = tid % 3;
+        } else if (q < 27) {
+            const int d = q / 9, b = (q / 3) % 3, c = q % 3;
             double m = 0.0;
 #pragma unroll
             for (int qq = 0; qq < 4; qq++) m += sW[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
@@ -1705,10 +1704,10 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
         }
     }
     __syncthreads();
-    // ---- moment states: lane 8g + j takes rule node j of point g (32 points
-    //      per round, two rounds); node sums over the 8-lane group one entry
-    //      at a time; F^ and H^ from the jets, 3-4 entries per lane
-    if (tid < 256) {
+    // ---- moment states: lane 8g + j takes rule node j of point g; node sums
+    //      over the 8-lane group one entry at a time; F^ and H^ from the jets,
+    //      3-4 entries per lane
+    {
         Mom mu = {0.0, 0.0, 0.0, 0.0, 1.0, 1.0, 1.0};
 #pragma unroll
         for (int j = 0; j < 8; j++) {
@@ -1719,64 +1718,62 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
         mu.factor();
         const double c12 = 1.0 / (mu.a11 * mu.a22), c22 = 1.0 / mu.d2;
         const int j = tid & 7;
-        for (int round = 0; round < 2; round++) {
-            const int q = (tid >> 3) + 32 * round;
-            const T *jq = sJet + q * 54;
-            T *ms = sMom + q * MS_W;
-            {
-                double us[30];
+        const int q = tid >> 3;
+        const T *jq = sJet + q * 54;
+        T *ms = sMom + q * MS_W;
+        {
+            double us[30];
 #pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    us[10 * k] = 0.0;
+            for (int k = 0; k < 3; k++) {
+                us[10 * k] = 0.0;
 #pragma unroll
-                    for (int a = 1; a < 10; a++) us[10 * k + a] = (double)jq[9 * k + a - 1] + P.s[j] * (double)jq[27 + 9 * k + a - 1];
-                }
-                State st;
-                phys_state(us, P, st);
-                const double w0 = P.ct[j], w1 = w0 * P.s[j], w2 = w1 * P.s[j];
-                constexpr int PR[6] = {0, 1, 2, 4, 5, 8};   // index pairs I <= J in slot order
+                for (int a = 1; a < 10; a++) us[10 * k + a] = (double)jq[9 * k + a - 1] + P.s[j] * (double)jq[27 + 9 * k + a - 1];
+            }
+            State st;
+            phys_state(us, P, st);
+            const double w0 = P.ct[j], w1 = w0 * P.s[j], w2 = w1 * P.s[j];
+            constexpr int PR[6] = {0, 1, 2, 4, 5, 8};   // index pairs I <= J in slot order
 #pragma unroll
-                for (int t = 0; t < 6; t++) {
-                    double sv = w0 * st.S[PR[t]], n0 = w0 * st.N[PR[t]], n1 = w1 * st.N[PR[t]], n2 = w2 * st.N[PR[t]];
-                    sv = sum8(sv);
-                    n0 = sum8(n0);
-                    n1 = sum8(n1);
-                    n2 = sum8(n2);
-                    if (j == 0) {
-                        ms[MS_S + t] = (T)sv;
-                        ms[MS_N11 + t] = (T)(n0 / mu.m0);
-                        ms[MS_N12 + t] = (T)((n1 - mu.lf * n0) * c12);
-                        ms[MS_N22 + t] = (T)(((mu.lf * n0 - n1) * mu.lf + (n2 - mu.lf * n1)) * c22);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 9; i++) {
-                    const double gv = sum8(w0 * st.G[i]);
-                    if (j == 0) ms[MS_G + i] = (T)gv;
+            for (int t = 0; t < 6; t++) {
+                double sv = w0 * st.S[PR[t]], n0 = w0 * st.N[PR[t]], n1 = w1 * st.N[PR[t]], n2 = w2 * st.N[PR[t]];
+                sv = sum8(sv);
+                n0 = sum8(n0);
+                n1 = sum8(n1);
+                n2 = sum8(n2);
+                if (j == 0) {
+                    ms[MS_S + t] = (T)sv;
+                    ms[MS_N11 + t] = (T)(n0 / mu.m0);
+                    ms[MS_N12 + t] = (T)((n1 - mu.lf * n0) * c12);
+                    ms[MS_N22 + t] = (T)(((mu.lf * n0 - n1) * mu.lf + (n2 - mu.lf * n1)) * c22);
                 }
             }
-            // F^ (r < 9: F_kL, k = r / 3, L = r % 3) and H^ (r >= 9: H_k,IK in
-            // slot 4 + t of component k = (r - 9) / 6): X^_1 = a11 (X0 + lf Xd),
-            // X^_2 = a22 Xd
-            for (int r = j; r < 27; r += 8) {
-                int src;
-                double x0;
-                if (r < 9) {
-                    src = 9 * (r / 3) + (r % 3);
-                    x0 = (double)jq[src] + ((r / 3) == (r % 3) ? 1.0 : 0.0);
-                } else {
-                    src = 9 * ((r - 9) / 6) + 3 + (r - 9) % 6;
-                    x0 = (double)jq[src];
-                }
-                const double xd = (double)jq[27 + src];
-                const double x1 = mu.a11 * (x0 + mu.lf * xd), x2 = mu.a22 * xd;
-                if (r < 9) {
-                    ms[18 * (r / 3) + r % 3] = (T)x1;
-                    ms[18 * (r / 3) + 3 + r % 3] = (T)x2;
-                } else {
-                    ms[18 * ((r - 9) / 6) + 6 + (r - 9) % 6] = (T)x1;
-                    ms[18 * ((r - 9) / 6) + 12 + (r - 9) % 6] = (T)x2;
-                }
+#pragma unroll
+            for (int i = 0; i < 9; i++) {
+                const double gv = sum8(w0 * st.G[i]);
+                if (j == 0) ms[MS_G + i] = (T)gv;
+            }
+        }
+        // F^ (r < 9: F_kL, k = r / 3, L = r % 3) and H^ (r >= 9: H_k,IK in
+        // slot 4 + t of component k = (r - 9) / 6): X^_1 = a11 (X0 + lf Xd),
+        // X^_2 = a22 Xd
+        for (int r = j; r < 27; r += 8) {
+            int src;
+            double x0;
+            if (r < 9) {
+                src = 9 * (r / 3) + (r % 3);
+                x0 = (double)jq[src] + ((r / 3) == (r % 3) ? 1.0 : 0.0);
+            } else {
+                src = 9 * ((r - 9) / 6) + 3 + (r - 9) % 6;
+                x0 = (double)jq[src];
+            }
+            const double xd = (double)jq[27 + src];
+            const double x1 = mu.a11 * (x0 + mu.lf * xd), x2 = mu.a22 * xd;
+            if (r < 9) {
+                ms[18 * (r / 3) + r % 3] = (T)x1;
+                ms[18 * (r / 3) + 3 + r % 3] = (T)x2;
+            } else {
+                ms[18 * ((r - 9) / 6) + 6 + (r - 9) % 6] = (T)x1;
+                ms[18 * ((r - 9) / 6) + 12 + (r - 9) % 6] = (T)x2;
             }
         }
     }
@@ -1926,24 +1923,25 @@ __global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, con
 {
     __shared__ double sPd[3][4][3][3];
     __shared__ double sW[3][4];
-    __shared__ double sU[27 * 3], sUd[27 * 3], sV[27 * 3];
+    __shared__ double sC[27][6], sV[27 * 3];   // nodal Um, Ud; inertia combination
     __shared__ double sMass[3][3][3];
-    __shared__ double sWork[3 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
+    __shared__ double sWork[6 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
     __shared__ double sJet[64 * 60];            // jets [q][h][k][a] of Um and Ud, then the weighted r_q [q][k][a]
     const int tid = threadIdx.x;
     const int e = blockIdx.x;
     const int nz = M.nelem[2], ny = M.nelem[1];
     const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
 
-    sep_element<3>(M, Uh, ed, sU, sPd, sW, ndof, sUd, sV, P.cii / (2. * P.dt), P.rho / (P.dt * P.dt));
+    sep_element<3, 6>(M, Uh, ed, &sC[0][0], sPd, sW, ndof, &sC[0][3], sV, P.cii / (2. * P.dt), P.rho / (P.dt * P.dt));
     __syncthreads();
     {
-        double J1[10], J2[10];
-        sep_fields(M, ed, sU, sPd, sWork, J1, true);
-        __syncthreads();
-        sep_fields(M, ed, sUd, sPd, sWork, J2, false);
+        six_fields(sC, sPd, sWork);
         const int q = tid & 63, k = tid >> 6;
         if (k < 3) {
+            double J1[10], J2[10];
+            six_jet(sWork, sPd, k, q, J1);
+            six_jet(sWork, sPd, 3 + k, q, J2);
+            sep_macro(M, ed, q, k, J1);
 #pragma unroll
             for (int a = 0; a < 10; a++) {
                 sJet[q * 60 + 10 * k + a] = J1[a];
