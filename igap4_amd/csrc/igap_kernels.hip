@@ -1865,50 +1865,121 @@ __device__ __forceinline__ double sep_project(const double (*sPd)[4][3][3], cons
 // with R_q the tensor product of the physical tables, as the transposed sum
 // factorisation x -> y -> z; no quotient or chain rule to undo.
 // ============================================================================
-// Six workgroups per CU (26 KB of LDS each, 80 VGPRs; the one-wave pointwise
-// stage spills 32 of them): 7.6 ms at 256x64x64 against 8.3 at five and 9.9
-// at four, where nothing spills -- the barriers of the field and projection
-// passes are what the extra workgroups hide.
-__global__ __launch_bounds__(256, 6) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
-                                                         double *__restrict__ Re, int nel)
+// A wave per element: every pass fits 64 lanes component by component (36, 48 and 64
+// of them for z, y, x; 48, 36 and 27 back), the jets of a lane's point stay in
+// its registers, and nothing waits at a block barrier.  10 KB of LDS an element,
+// so 16 elements are in flight per CU.  @RESNOTE@
+__device__ __forceinline__ void wave_sync()
 {
-    __shared__ double sPd[3][4][3][3];
-    __shared__ double sW[3][4];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__global__ __launch_bounds__(64, 4) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
+                                                        double *__restrict__ Re, int nel)
+{
+    __shared__ double sT[3][TAB_STRIDE];   // the element's 1-D tables [q][order][function], then their point weights
     __shared__ double sU[27 * 3];
-    __shared__ double sWork[3 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
-    __shared__ double sJet[64 * 30];            // u-jets [q][k][a], then the weighted r_q
-    const int tid = threadIdx.x;
-    const int e = blockIdx.x;
+    __shared__ double sA[108], sB[288];    // field passes, then the transposed ones
+    __shared__ double sR[10 * 64];         // weighted residual jets of one component [a][q]
+    const int lane = threadIdx.x, e = blockIdx.x;
     const int nz = M.nelem[2], ny = M.nelem[1];
     const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
-
-    sep_element(M, Uh, ed, sU, sPd, sW);
-    __syncthreads();
-    {
-        double J[10];
-        sep_fields(M, ed, sU, sPd, sWork, J);
-        const int q = tid & 63, k = tid >> 6;
-        if (k < 3) {
 #pragma unroll
-            for (int a = 0; a < 10; a++) sJet[q * 30 + 10 * k + a] = J[a];
+    for (int d = 0; d < 3; d++)
+        if (lane < TAB_STRIDE) sT[d][lane] = M.tab[d][(int64_t)ed[d] * TAB_STRIDE + lane];
+    if (lane < 27) {
+        const int bx = lane / 9, by = (lane / 3) % 3, bz = lane % 3;
+        const int64_t oc = ((int64_t)M.nb[1] * M.nb[2]) * own1(ed[0] + bx, M.nb[0], M.periodic[0])
+                         + (int64_t)M.nb[2] * own1(ed[1] + by, M.nb[1], M.periodic[1]) + own1(ed[2] + bz, M.nb[2], M.periodic[2]);
+#pragma unroll
+        for (int k = 0; k < 3; k++) sU[3 * lane + k] = Uh[3 * oc + k];
+    }
+    wave_sync();
+    const int qz = lane & 3, qy = (lane >> 2) & 3, qx = lane >> 4;
+    double u[30];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        // z: sA[bx*3+by][qz][dz]
+        if (lane < 36) {
+            const double *c = sU + 9 * (lane >> 2) + k;
+#pragma unroll
+            for (int dz = 0; dz < 3; dz++) {
+                const double *tz = &sT[2][9 * qz + 3 * dz];
+                sA[3 * lane + dz] = c[0] * tz[0] + c[3] * tz[1] + c[6] * tz[2];
+            }
         }
-    }
-    __syncthreads();
-    // ---- pointwise residual jets, weighted: one wave, lane = Gauss point
-    //      (the wave taking it rotates with the element)
-    if ((tid >> 6) == (e & 3)) {
-        const int q = tid & 63;
-        double u[30], r[30];
+        wave_sync();
+        // y: sB[bx][qy][qz][s6], s6 = (dy, dz) in the order (0,0) (1,0) (0,1) (2,0) (1,1) (0,2); bx = qx here
+        if (lane < 48) {
+            const double *a = sA + 36 * qx + 3 * qz;   // a[12 by + dz]
 #pragma unroll
-        for (int a = 0; a < 30; a++) u[a] = sJet[q * 30 + a];
-        phys_residual_static(P, u, r);
-        const double w = sep_weight(q, sW);
-#pragma unroll
-        for (int a = 0; a < 30; a++) sJet[q * 30 + a] = w * r[a];
+            for (int s6 = 0; s6 < 6; s6++) {
+                const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
+                const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
+                const double *ty = &sT[1][9 * qy + 3 * dy];
+                sB[6 * lane + s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
+            }
+        }
+        wave_sync();
+        sf_jet(sB + (lane & 15) * 6, &sT[0][9 * qx], u + 10 * k);
+        sep_macro(M, ed, lane, k, u + 10 * k);
     }
-    __syncthreads();
-    const double v = sep_project<30>(sPd, sJet, sWork);
-    if (tid < 81) Re[(int64_t)e * 81 + tid] = v;
+    double r[30];
+    phys_residual_static(P, u, r);
+    const double w = sT[0][36 + qx] * sT[1][36 + qy] * sT[2][36 + qz];
+    double out[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+#pragma unroll
+        for (int a = 0; a < 10; a++) sR[64 * a + lane] = w * r[10 * k + a];
+        wave_sync();
+        // x^T: C1[bx][qy][qz][s6] = sum_qx sum_{a: S6(a) = s6} r[a] Px[qx][DX(a)][bx]
+        if (lane < 48) {
+            double c[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const double *rq = sR + 16 * x + (lane & 15), *tx = &sT[0][9 * x + qx];   // bx = qx; tx[3 dx]
+                c[0] += rq[0] * tx[0] + rq[64] * tx[3] + rq[4 * 64] * tx[6];
+                c[1] += rq[2 * 64] * tx[0] + rq[5 * 64] * tx[3];
+                c[2] += rq[3 * 64] * tx[0] + rq[6 * 64] * tx[3];
+                c[3] += rq[7 * 64] * tx[0];
+                c[4] += rq[8 * 64] * tx[0];
+                c[5] += rq[9 * 64] * tx[0];
+            }
+#pragma unroll
+            for (int s6 = 0; s6 < 6; s6++) sB[6 * lane + s6] = c[s6];
+        }
+        wave_sync();
+        // y^T: C2[bx][by][qz][dz] = sum_qy sum_{s6: dz(s6) = dz} C1[..][s6] Py[qy][dy(s6)][by]
+        if (lane < 36) {
+            const int by = (lane >> 2) % 3, bx = lane / 12;
+            double c[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int y = 0; y < 4; y++) {
+                const double *c1 = sB + ((bx * 4 + y) * 4 + qz) * 6, *ty = &sT[1][9 * y + by];   // ty[3 dy]
+                c[0] += c1[0] * ty[0] + c1[1] * ty[3] + c1[3] * ty[6];
+                c[1] += c1[2] * ty[0] + c1[4] * ty[3];
+                c[2] += c1[5] * ty[0];
+            }
+#pragma unroll
+            for (int dz = 0; dz < 3; dz++) sA[3 * lane + dz] = c[dz];
+        }
+        wave_sync();
+        // z^T: R_e[3 b + k] = sum_qz sum_dz C2[bx][by][qz][dz] Pz[qz][dz][bz]
+        double acc = 0.0;
+        if (lane < 27) {
+            const double *c2 = sA + (lane / 3) * 12;
+#pragma unroll
+            for (int z = 0; z < 4; z++)
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++) acc += c2[3 * z + dz] * sT[2][9 * z + 3 * dz + lane % 3];
+        }
+        out[k] = acc;
+    }
+    if (lane < 27) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) Re[(int64_t)e * 81 + 3 * lane + k] = out[k];
+    }
 }
 
 // Transient residual on a separable patch (k_residual_sep_t, gradelasttime):
@@ -2423,7 +2494,7 @@ hipError_t launch_density(const MeshK &M, const PhysK &P, const double *Uh, int6
 hipError_t launch_residual_elem(const MeshK &M, const PhysK &P, const double *Uh, int64_t ndof, double *Re, int nel, hipStream_t s)
 {
     dim3 grid(nel), block(256);
-    if (P.torder == 0 && M.separable) hipLaunchKernelGGL(k_residual_sep, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
+    if (P.torder == 0 && M.separable) hipLaunchKernelGGL(k_residual_sep, grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
     else if (P.torder == 2 && M.separable) hipLaunchKernelGGL(k_residual_sep_t, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
     else if (P.torder == 0) hipLaunchKernelGGL(k_residual_elem<1>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
     else hipLaunchKernelGGL(k_residual_elem<3>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
