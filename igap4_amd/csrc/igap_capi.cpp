@@ -720,19 +720,39 @@ static int t_end(igap_gpu_ctx *c, int slot, int which)
 }
 
 // ---------------------------------------------------------------- callbacks
+// The iterate of an assembly call, kept as U_hist[0] (src/assmcore_iga.c:68, 557).  The
+// static kernels read the caller's U, and the gather that ends the call copies
+// it (*copy) on the way, one launch less; the transient ones read all levels from
+// d_Uh, so there the copy comes first.
+static int take_iterate(igap_gpu_ctx *c, const double *U, const double **src, double **copy)
+{
+    *src = c->d_Uh;
+    *copy = nullptr;
+    if (!U || U == c->d_Uh) return IGAP_OK;
+    if (c->P.torder == 0) {
+        *src = U;
+        *copy = c->d_Uh;
+        return IGAP_OK;
+    }
+    HIPCHK(launch_copy_f64(c->d_Uh, U, c->ndof, c->stream));
+    return IGAP_OK;
+}
+
 extern "C" int igap_gpu_residual(igap_gpu_ctx *c, const double *U, double *R)
 {
     if (!c) return fail(IGAP_ERR_ARG, "null context");
     HIPCHK(hipSetDevice(c->device));
     if (!R) R = c->d_R;
     if (c->timing) HIPCHK(hipEventRecord(c->ev[2], c->stream));
-    if (U && U != c->d_Uh) HIPCHK(launch_copy_f64(c->d_Uh, U, c->ndof, c->stream));   // U_hist[0] = U (:68)
-    int rc = t_begin(c, 0);
+    const double *U0;
+    double *keep;
+    int rc = take_iterate(c, U, &U0, &keep);
+    if (!rc) rc = t_begin(c, 0);
     if (rc) return rc;
-    HIPCHK(launch_residual_elem(c->M, c->P, c->d_Uh, c->ndof, c->d_Re, (int)c->nel, c->stream));
+    HIPCHK(launch_residual_elem(c->M, c->P, U0, c->ndof, c->d_Re, (int)c->nel, c->stream));
     rc = t_end(c, 0, 0);
     if (rc) return rc;
-    HIPCHK(launch_residual_gather(c->M, c->d_Re, c->d_Uh, c->d_F, c->d_mask, c->d_g, R, c->ncp, c->stream));
+    HIPCHK(launch_residual_gather(c->M, c->d_Re, U0, keep, c->d_F, c->d_mask, c->d_g, R, c->ncp, c->stream));
     if (c->timing) {
         HIPCHK(hipEventRecord(c->ev[3], c->stream));
         HIPCHK(hipEventSynchronize(c->ev[3]));
@@ -755,9 +775,12 @@ extern "C" int igap_gpu_residual_noalloc(igap_gpu_ctx *c, const double *U, doubl
     double *scr = scratch_device_ptr(c->device);
     if (!scr) return fail(IGAP_ERR_STATE, "no device array on device %d (contexts set it up)", c->device);
     if (!R) R = c->d_R;
-    if (U && U != c->d_Uh) HIPCHK(launch_copy_f64(c->d_Uh, U, c->ndof, c->stream));   // U_hist[0] = U (:68)
-    HIPCHK(launch_residual_elem(c->M, c->P, c->d_Uh, c->ndof, scr, (int)c->nel, c->stream));
-    HIPCHK(launch_residual_gather(c->M, scr, c->d_Uh, c->d_F, c->d_mask, c->d_g, R, c->ncp, c->stream));
+    const double *U0;
+    double *keep;
+    const int rc = take_iterate(c, U, &U0, &keep);
+    if (rc) return rc;
+    HIPCHK(launch_residual_elem(c->M, c->P, U0, c->ndof, scr, (int)c->nel, c->stream));
+    HIPCHK(launch_residual_gather(c->M, scr, U0, keep, c->d_F, c->d_mask, c->d_g, R, c->ncp, c->stream));
     return IGAP_OK;
 }
 
@@ -810,15 +833,17 @@ extern "C" int igap_gpu_tangent(igap_gpu_ctx *c, const double *U, void *vals, in
         if (e != hipSuccess) return fail(IGAP_ERR_NOMEM, "element tangent buffer (%zu bytes): %s", es * 6561 * (size_t)c->nel, hipGetErrorString(e));
     }
     if (c->timing) HIPCHK(hipEventRecord(c->ev[2], c->stream));
-    if (U && U != c->d_Uh) HIPCHK(launch_copy_f64(c->d_Uh, U, c->ndof, c->stream));   // U_hist[0] = U (:557)
-    int rc = t_begin(c, 0);
+    const double *U0;
+    double *keep;
+    int rc = take_iterate(c, U, &U0, &keep);
+    if (!rc) rc = t_begin(c, 0);
     if (rc) return rc;
-    HIPCHK(launch_tangent_elem(c->M, c->P, c->d_Uh, c->ndof, c->d_Ke[prec], prec, (int)c->nel, c->stream));
+    HIPCHK(launch_tangent_elem(c->M, c->P, U0, c->ndof, c->d_Ke[prec], prec, (int)c->nel, c->stream));
     rc = t_end(c, 0, 1);
     if (rc) return rc;
     rc = t_begin(c, 0);
     if (rc) return rc;
-    HIPCHK(launch_tangent_gather(c->M, c->d_Ke[prec], prec, c->d_rowptr, c->d_mask, vals, c->ncp, c->stream));
+    HIPCHK(launch_tangent_gather(c->M, c->d_Ke[prec], prec, c->d_rowptr, c->d_mask, vals, c->ncp, U0, keep, c->stream));
     rc = t_end(c, 0, 2);
     if (rc) return rc;
     if (c->timing) {

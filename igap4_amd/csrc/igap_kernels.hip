@@ -404,57 +404,62 @@ __global__ __launch_bounds__(256) void k_density_reduce(int nel, int nd, const d
     if (threadIdx.x == 0) H[i] = red[0];
 }
 
-// contributing (element, local index) pairs of owned control point a along one
-// direction, sorted by element (the reference accumulates in element order)
-__device__ __forceinline__ int elem_pairs(int a, int nelem, int nb, int periodic, int *es, int *ls)
-{
-    int cnt = 0;
-    if (!periodic) {
-        for (int l = 2; l >= 0; l--) {
-            int e = a - l;
-            if (e >= 0 && e < nelem) { es[cnt] = e; ls[cnt] = l; cnt++; }
+// The elements of owned control point a along one direction, ascending (the
+// reference accumulates in element order): element e[j] with a its local
+// point l[j], where ok[j].  A periodic direction has at least five elements.
+struct ElemRow {
+    int e[3], l[3];
+    bool ok[3];
+    __device__ __forceinline__ ElemRow(int a, int nelem, int periodic)
+    {
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            // wrapped elements come last: locals 0, 2, 1 at a = 0 and 1, 0, 2 at a = 1
+            const int lp = a == 0 ? (j == 0 ? 0 : 3 - j) : a == 1 ? (j == 2 ? 2 : 1 - j) : 2 - j;
+            l[j] = periodic ? lp : 2 - j;
+            e[j] = a - l[j];
+            if (periodic && e[j] < 0) e[j] += nelem;
+            ok[j] = e[j] >= 0 && e[j] < nelem;
         }
-        return cnt;
     }
-    for (int l = 2; l >= 0; l--) {
-        int e = a - l;
-        if (e < 0) e += nb;
-        es[cnt] = e; ls[cnt] = l; cnt++;
-    }
-    // insertion sort by element
-    for (int i = 1; i < cnt; i++)
-        for (int j = i; j > 0 && es[j] < es[j - 1]; j--) {
-            int te = es[j]; es[j] = es[j - 1]; es[j - 1] = te;
-            int tl = ls[j]; ls[j] = ls[j - 1]; ls[j - 1] = tl;
-        }
-    return cnt;
-}
+};
 
-__global__ __launch_bounds__(256) void k_residual_gather(MeshK M, const double *__restrict__ Re, const double *__restrict__ Uh,
+// One thread per dof, its loads (27 at most) in flight together.  As one thread
+// per control point looping over run-time index lists (in scratch memory) it took 14.6 us at
+// 64x16x16, now 5.3.  Ucopy (may be null): where the iterate U is kept.
+__global__ __launch_bounds__(256) void k_residual_gather(MeshK M, const double *__restrict__ Re, const double *U, double *Ucopy,
                                                          const double *__restrict__ Fneu, const int32_t *__restrict__ mask,
-                                                         const double *__restrict__ g, double *__restrict__ R, int64_t ncp)
+                                                         const double *__restrict__ g, double *R, int64_t ncp)
 {
-    int64_t a = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= ncp) return;
-    int nb1 = M.nb[1], nb2 = M.nb[2];
-    int az = (int)(a % nb2), ay = (int)((a / nb2) % nb1), ax = (int)(a / ((int64_t)nb1 * nb2));
-    int exs[3], lxs[3], eys[3], lys[3], ezs[3], lzs[3];
-    int nx = elem_pairs(ax, M.nelem[0], M.nb[0], M.periodic[0], exs, lxs);
-    int ny = elem_pairs(ay, M.nelem[1], M.nb[1], M.periodic[1], eys, lys);
-    int nz = elem_pairs(az, M.nelem[2], M.nb[2], M.periodic[2], ezs, lzs);
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int x = 0; x < nx; x++)
-        for (int y = 0; y < ny; y++)
-            for (int z = 0; z < nz; z++) {
-                int64_t e = ((int64_t)exs[x] * M.nelem[1] + eys[y]) * M.nelem[2] + ezs[z];
-                int lb = 9 * lxs[x] + 3 * lys[y] + lzs[z];
-                const double *r = Re + e * 81 + 3 * lb;
-                s0 += r[0]; s1 += r[1]; s2 += r[2];
+    const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (d >= 3 * ncp) return;
+    // control-point and dof indices fit in 32 bits (the CSR columns are int32)
+    const int a = (int)((uint32_t)d / 3u), k = (int)d - 3 * a;
+    const int nb1 = M.nb[1], nb2 = M.nb[2], az = a % nb2, axy = a / nb2, ay = axy % nb1, ax = axy / nb1;
+    const ElemRow X(ax, M.nelem[0], M.periodic[0]), Y(ay, M.nelem[1], M.periodic[1]), Z(az, M.nelem[2], M.periodic[2]);
+    const int m = mask[d];
+    const double u = U[d], f = m ? g[d] : Fneu[d];
+    double v[27];
+#pragma unroll
+    for (int x = 0; x < 3; x++)
+#pragma unroll
+        for (int y = 0; y < 3; y++)
+#pragma unroll
+            for (int z = 0; z < 3; z++) {
+                const bool ok = X.ok[x] && Y.ok[y] && Z.ok[z];
+                const int64_t e = ((int64_t)X.e[x] * M.nelem[1] + Y.e[y]) * M.nelem[2] + Z.e[z];
+                v[9 * x + 3 * y + z] = Re[ok ? e * 81 + 27 * X.l[x] + 9 * Y.l[y] + 3 * Z.l[z] + k : 0];
             }
-    int64_t d = 3 * a;
-    R[d + 0] = mask[d + 0] ? Uh[d + 0] - g[d + 0] : s0 + Fneu[d + 0];
-    R[d + 1] = mask[d + 1] ? Uh[d + 1] - g[d + 1] : s1 + Fneu[d + 1];
-    R[d + 2] = mask[d + 2] ? Uh[d + 2] - g[d + 2] : s2 + Fneu[d + 2];
+    double s = 0.0;
+#pragma unroll
+    for (int x = 0; x < 3; x++)
+#pragma unroll
+        for (int y = 0; y < 3; y++)
+#pragma unroll
+            for (int z = 0; z < 3; z++)
+                if (X.ok[x] && Y.ok[y] && Z.ok[z]) s += v[9 * x + 3 * y + z];
+    if (Ucopy) Ucopy[d] = u;
+    R[d] = m ? u - f : s + f;
 }
 
 // ============================================================================
@@ -1868,7 +1873,9 @@ __device__ __forceinline__ double sep_project(const double (*sPd)[4][3][3], cons
 // A wave per element: every pass fits 64 lanes component by component (36, 48 and 64
 // of them for z, y, x; 48, 36 and 27 back), the jets of a lane's point stay in
 // its registers, and nothing waits at a block barrier.  10 KB of LDS an element,
-// so 16 elements are in flight per CU.  @RESNOTE@
+// so 16 elements are in flight per CU.  At 64x16x16 120 -> 83 us (one
+// call), at 16x4x4 9.2 -> 7.9 us, against a workgroup of four waves per element with
+// six in flight per CU and the pointwise stage on one of the waves.
 __device__ __forceinline__ void wave_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -2144,9 +2151,11 @@ __device__ __forceinline__ int elem_pairs2(int a, int b, int nelem, int nb, int 
 // order -- the order k_tangent_gather_rows uses, so the values are the same.
 template <typename TK, typename TV>
 __global__ __launch_bounds__(128) void k_tangent_gather(MeshK M, const TK *__restrict__ Ke, const int64_t *__restrict__ rowptr,
-                                                        const int32_t *__restrict__ mask, TV *__restrict__ vals)
+                                                        const int32_t *__restrict__ mask, TV *__restrict__ vals, const double *U,
+                                                        double *Ucopy)
 {
     const int64_t a = blockIdx.x;
+    if (Ucopy && threadIdx.x < 3) Ucopy[3 * a + threadIdx.x] = U[3 * a + threadIdx.x];   // (where the iterate is kept)
     int nb1 = M.nb[1], nb2 = M.nb[2];
     int az = (int)(a % nb2), ay = (int)((a / nb2) % nb1), ax = (int)(a / ((int64_t)nb1 * nb2));
     int Sx[5], Sy[5], Sz[5];
@@ -2203,12 +2212,14 @@ __global__ __launch_bounds__(128) void k_tangent_gather(MeshK M, const TK *__res
 // write-out does not wait on them.
 template <typename TK, typename TV>
 __global__ __launch_bounds__(256) void k_tangent_gather_rows(MeshK M, const TK *__restrict__ Ke, const int64_t *__restrict__ rowptr,
-                                                             const int32_t *__restrict__ mask, TV *__restrict__ vals)
+                                                             const int32_t *__restrict__ mask, TV *__restrict__ vals, const double *U,
+                                                             double *Ucopy)
 {
     __shared__ double acc[125 * 9];
     // control-point and dof indices fit in 32 bits (the CSR columns are int32)
     const int a = (int)blockIdx.x;
     const int tid = threadIdx.x;
+    if (Ucopy && tid < 3) Ucopy[3 * (int64_t)a + tid] = U[3 * (int64_t)a + tid];   // (where the iterate is kept)
     const int nb1 = M.nb[1], nb2 = M.nb[2];
     const int az = a % nb2, ay = (a / nb2) % nb1, ax = a / (nb1 * nb2);
     int Sx[5], Sy[5], Sz[5];
@@ -2501,11 +2512,11 @@ hipError_t launch_residual_elem(const MeshK &M, const PhysK &P, const double *Uh
     return hipGetLastError();
 }
 
-hipError_t launch_residual_gather(const MeshK &M, const double *Re, const double *Uh, const double *Fneu, const int32_t *mask,
-                                  const double *g, double *R, int64_t ncp, hipStream_t s)
+hipError_t launch_residual_gather(const MeshK &M, const double *Re, const double *U, double *Ucopy, const double *Fneu,
+                                  const int32_t *mask, const double *g, double *R, int64_t ncp, hipStream_t s)
 {
-    dim3 grid((unsigned)((ncp + 255) / 256)), block(256);
-    hipLaunchKernelGGL(k_residual_gather, grid, block, 0, s, M, Re, Uh, Fneu, mask, g, R, ncp);
+    dim3 grid((unsigned)((3 * ncp + 255) / 256)), block(256);
+    hipLaunchKernelGGL(k_residual_gather, grid, block, 0, s, M, Re, U, Ucopy, Fneu, mask, g, R, ncp);
     return hipGetLastError();
 }
 
@@ -2586,13 +2597,13 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
 }
 
 hipError_t launch_tangent_gather(const MeshK &M, const void *Ke, int prec, const int64_t *rowptr, const int32_t *mask, void *vals,
-                                 int64_t ncp, hipStream_t s)
+                                 int64_t ncp, const double *U, double *Ucopy, hipStream_t s)
 {
     dim3 grid((unsigned)ncp), block(256);
     if (prec == 0)
-        hipLaunchKernelGGL((k_tangent_gather_rows<double, double>), grid, block, 0, s, M, (const double *)Ke, rowptr, mask, (double *)vals);
+        hipLaunchKernelGGL((k_tangent_gather_rows<double, double>), grid, block, 0, s, M, (const double *)Ke, rowptr, mask, (double *)vals, U, Ucopy);
     else
-        hipLaunchKernelGGL((k_tangent_gather<float, float>), grid, dim3(128), 0, s, M, (const float *)Ke, rowptr, mask, (float *)vals);
+        hipLaunchKernelGGL((k_tangent_gather<float, float>), grid, dim3(128), 0, s, M, (const float *)Ke, rowptr, mask, (float *)vals, U, Ucopy);
     return hipGetLastError();
 }
 
