@@ -1873,7 +1873,7 @@ __device__ __forceinline__ double sep_project(const double (*sPd)[4][3][3], cons
 // A wave per element: every pass fits 64 lanes component by component (36, 48 and 64
 // of them for z, y, x; 48, 36 and 27 back), the jets of a lane's point stay in
 // its registers, and nothing waits at a block barrier.  10 KB of LDS an element,
-// so 16 elements are in flight per CU.  At 64x16x16 120 -> 83 us (one
+// so at 156 registers (128 spill 38) 12 elements are in flight per CU.  At 64x16x16 120 -> 79 us (one
 // call), at 16x4x4 9.2 -> 7.9 us, against a workgroup of four waves per element with
 // six in flight per CU and the pointwise stage on one of the waves.
 __device__ __forceinline__ void wave_sync()
@@ -1881,7 +1881,7 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
-__global__ __launch_bounds__(64, 4) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
+__global__ __launch_bounds__(64, 3) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
                                                         double *__restrict__ Re, int nel)
 {
     __shared__ double sT[3][TAB_STRIDE];   // the element's 1-D tables [q][order][function], then their point weights
