@@ -222,7 +222,7 @@ def kernel_rooflines(nel, nelem, nnz, avg, avg32, gen, gen32, genr):
         "k_residual_elem<1>": flop(genr, F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
         "k_tangent_gather_rows<double,double>": hbm(avg[2], 8 * (6561 * nelem + nnz),
                                                     "igap::k_tangent_gather_rows<double, double>", 8 * nnz),
-        "k_tangent_gather<float,float>": hbm(avg32[2], 4 * (6561 * nelem + nnz), "igap::k_tangent_gather<float, float>",
+        "k_tangent_gather_rows<float,float>": hbm(avg32[2], 4 * (6561 * nelem + nnz), "igap::k_tangent_gather_rows<float, float>",
                                              4 * nnz),
     }
 

@@ -6,9 +6,8 @@
 //                     Dirichlet rows R_d = U_d - g_d (:258, :273-497)
 //   k_tangent_elem    per-element tangents K_e[81x81] on the matrix cores
 //                     (volume loop of Tangent_iga, :607-764)
-//   k_tangent_gather_rows / k_tangent_gather  deterministic per-nonzero sum of
-//                     K_e into the CSR values with MatZeroRowsColumns(diag=1)
-//                     fused (:763, :844); row-wise for FP64, column-wise FP32
+//   k_tangent_gather_rows  deterministic per-nonzero sum of K_e into the CSR values
+//                     with MatZeroRowsColumns(diag=1) fused (:763, :844)
 //   k_csr_cols        column indices of the CSR pattern
 //
 // Element numbering e = (ex*ny + ey)*nz + ez (the reference's x->y->z loop
@@ -2116,196 +2115,117 @@ __device__ __forceinline__ int stencil1(int a, int n, int periodic, int *S)
     return cnt;
 }
 
-// elements along one direction containing owned points a and b, sorted, with
-// their local indices
-__device__ __forceinline__ int elem_pairs2(int a, int b, int nelem, int nb, int periodic, int *es, int *la, int *lb)
+// acc += v in LDS without a round trip; a wave's additions happen in program order
+__device__ __forceinline__ void lds_add(double *p, double v)
 {
-    int cnt = 0;
-    if (!periodic) {
-        int lo = (a > b ? a : b) - 2, hi = a < b ? a : b;
-        if (lo < 0) lo = 0;
-        if (hi > nelem - 1) hi = nelem - 1;
-        for (int e = lo; e <= hi; e++) { es[cnt] = e; la[cnt] = a - e; lb[cnt] = b - e; cnt++; }
-        return cnt;
-    }
-    for (int l = 2; l >= 0; l--) {
-        int e = a - l;
-        if (e < 0) e += nb;
-        int m = b - e;
-        if (m < 0) m += nb;
-        if (m <= 2) { es[cnt] = e; la[cnt] = l; lb[cnt] = m; cnt++; }
-    }
-    for (int i = 1; i < cnt; i++)
-        for (int j = i; j > 0 && es[j] < es[j - 1]; j--) {
-            int t = es[j]; es[j] = es[j - 1]; es[j - 1] = t;
-            t = la[j]; la[j] = la[j - 1]; la[j - 1] = t;
-            t = lb[j]; lb[j] = lb[j - 1]; lb[j - 1] = t;
-        }
-    return cnt;
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Column-wise variant of the same sums (used for FP32 element matrices, where
-// it is faster): one workgroup per owned control point a, thread t <-> the
-// t-th control point b of the row's column stencil, summing the (at most 27)
-// 3x3 contributions of the elements containing a and b in ascending element
-// order -- the order k_tangent_gather_rows uses, so the values are the same.
-template <typename TK, typename TV>
-__global__ __launch_bounds__(128) void k_tangent_gather(MeshK M, const TK *__restrict__ Ke, const int64_t *__restrict__ rowptr,
-                                                        const int32_t *__restrict__ mask, TV *__restrict__ vals, const double *U,
-                                                        double *Ucopy)
-{
-    const int64_t a = blockIdx.x;
-    if (Ucopy && threadIdx.x < 3) Ucopy[3 * a + threadIdx.x] = U[3 * a + threadIdx.x];   // (where the iterate is kept)
-    int nb1 = M.nb[1], nb2 = M.nb[2];
-    int az = (int)(a % nb2), ay = (int)((a / nb2) % nb1), ax = (int)(a / ((int64_t)nb1 * nb2));
-    int Sx[5], Sy[5], Sz[5];
-    int nsx = stencil1(ax, M.nb[0], M.periodic[0], Sx);
-    int nsy = stencil1(ay, M.nb[1], M.periodic[1], Sy);
-    int nsz = stencil1(az, M.nb[2], M.periodic[2], Sz);
-    int t = threadIdx.x;
-    if (t >= nsx * nsy * nsz) return;
-    int sx = t / (nsy * nsz), sy = (t / nsz) % nsy, sz = t % nsz;
-    int bx = Sx[sx], by = Sy[sy], bz = Sz[sz];
-    int ex[3], lax[3], lbx[3], ey[3], lay[3], lby[3], ez[3], laz[3], lbz[3];
-    int nx = elem_pairs2(ax, bx, M.nelem[0], M.nb[0], M.periodic[0], ex, lax, lbx);
-    int ny = elem_pairs2(ay, by, M.nelem[1], M.nb[1], M.periodic[1], ey, lay, lby);
-    int nz = elem_pairs2(az, bz, M.nelem[2], M.nb[2], M.periodic[2], ez, laz, lbz);
-    double s[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) s[i] = 0.0;
-    for (int x = 0; x < nx; x++)
-        for (int y = 0; y < ny; y++)
-            for (int z = 0; z < nz; z++) {
-                int64_t e = ((int64_t)ex[x] * M.nelem[1] + ey[y]) * M.nelem[2] + ez[z];
-                int la = 9 * lax[x] + 3 * lay[y] + laz[z], lb = 9 * lbx[x] + 3 * lby[y] + lbz[z];
-                const TK *k = Ke + e * 6561 + (3 * la) * 81 + 3 * lb;
-#pragma unroll
-                for (int i = 0; i < 3; i++)
-#pragma unroll
-                    for (int j = 0; j < 3; j++) s[3 * i + j] += (double)k[81 * i + j];
-            }
-    int64_t bcp = ((int64_t)M.nb[1] * M.nb[2]) * bx + (int64_t)M.nb[2] * by + bz;
-#pragma unroll
-    for (int i = 0; i < 3; i++) {
-        int64_t row = 3 * a + i;
-        int64_t pos = rowptr[row] + 3 * t;
-        bool mr = mask[row] != 0;
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            int64_t col = 3 * bcp + j;
-            double v = (mr || mask[col]) ? (row == col ? 1.0 : 0.0) : s[3 * i + j];
-            vals[pos + j] = (TV)v;
-        }
+// the same set in closed form: point k of it and the place of point b in it
+// (wrapped, the points from 0 on come first; a periodic direction has at least five)
+struct Stencil {
+    int lo, f, n5, cnt;
+    __device__ __forceinline__ Stencil(int a, int n, int periodic)
+    {
+        const bool wrap = periodic && (a < 2 || a + 2 > n - 1);
+        const int l = a - 2 > 0 ? a - 2 : 0, h = a + 2 < n - 1 ? a + 2 : n - 1;
+        cnt = periodic ? 5 : h - l + 1;
+        lo = l;
+        f = wrap ? (a + 3 >= n ? a + 3 - n : a + 3) : 0;
+        n5 = wrap ? n - 5 : l;
     }
-}
+    __device__ __forceinline__ int at(int k) const { return k < f ? k : n5 + k; }
+    __device__ __forceinline__ int slot(int b) const { return b < f ? b : b - n5; }
+};
 
-// Deterministic per-nonzero sum of the element tangents into the CSR values,
-// with MatZeroRowsColumns(diag = 1) applied (src/assmcore_iga.c:763,844):
-// one workgroup per owned control point a walks the (at most 27) elements
-// containing a in ascending element order; for each it reads a's three rows
-// of K_e (243 contiguous values, one per thread, all issued before the sums)
-// and adds them into an LDS accumulator indexed by the stencil column point,
-// with a barrier between elements.  Every entry gets its contributions in
-// ascending element order (bitwise repeatable); the loads are whole-row,
-// coalesced segments.  The row starts and the Dirichlet flags of the rows and
-// stencil columns are loaded into LDS before the element rounds, so that the
-// write-out does not wait on them.
+// Sum of the element matrices into the CSR rows of control point a, one wave per
+// row: the row's entries are summed in LDS, element by element in ascending
+// order, by one wave in program order, so nothing waits at a barrier and the sum
+// of every entry has a fixed order.  A row has 81 columns per element: 64 are one
+// load of the wave, the other 17 of the (up to) three elements along z another, 36 loads
+// in flight.  The Dirichlet rows and columns of MatZeroRowsColumns (unit diagonal)
+// go in with the write-out.  Ucopy (may be null): where the iterate U is kept.
+// Bound by the element matrices' bytes: 256x64x64 FP64 14.4 -> 13.2 ms (65 GB, 4.9
+// TB/s), 160x40x40 FP32 3.2 -> 2.0 ms, 16x4x4 (its latency) 17.5 -> 11.4 us, against
+// four waves over the three rows with a barrier per element (FP64) and a thread per
+// pair of points (FP32).
 template <typename TK, typename TV>
-__global__ __launch_bounds__(256) void k_tangent_gather_rows(MeshK M, const TK *__restrict__ Ke, const int64_t *__restrict__ rowptr,
+__global__ __launch_bounds__(192) void k_tangent_gather_rows(MeshK M, const TK *__restrict__ Ke, const int64_t *__restrict__ rowptr,
                                                              const int32_t *__restrict__ mask, TV *__restrict__ vals, const double *U,
                                                              double *Ucopy)
 {
-    __shared__ double acc[125 * 9];
+    __shared__ double sAcc[3][376];
     // control-point and dof indices fit in 32 bits (the CSR columns are int32)
-    const int a = (int)blockIdx.x;
-    const int tid = threadIdx.x;
-    if (Ucopy && tid < 3) Ucopy[3 * (int64_t)a + tid] = U[3 * (int64_t)a + tid];   // (where the iterate is kept)
+    const int a = (int)blockIdx.x, i = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    double *acc = sAcc[i];
+    const int row = 3 * a + i;
+    if (Ucopy && lane == 0) Ucopy[row] = U[row];
     const int nb1 = M.nb[1], nb2 = M.nb[2];
-    const int az = a % nb2, ay = (a / nb2) % nb1, ax = a / (nb1 * nb2);
-    int Sx[5], Sy[5], Sz[5];
-    const int nsx = stencil1(ax, M.nb[0], M.periodic[0], Sx);
-    const int nsy = stencil1(ay, M.nb[1], M.periodic[1], Sy);
-    const int nsz = stencil1(az, M.nb[2], M.periodic[2], Sz);
-    int ex[3], lax[3], ey[3], lay[3], ez[3], laz[3], dummy[3];
-    const int nx = elem_pairs2(ax, ax, M.nelem[0], M.nb[0], M.periodic[0], ex, lax, dummy);
-    const int ny = elem_pairs2(ay, ay, M.nelem[1], M.nb[1], M.periodic[1], ey, lay, dummy);
-    const int nz = elem_pairs2(az, az, M.nelem[2], M.nb[2], M.periodic[2], ez, laz, dummy);
-    const int nst = nsx * nsy * nsz;
-    for (int i = tid; i < nst * 9; i += 256) acc[i] = 0.0;
-    // this thread's value of a's rows: row 3 la + i, column c = 3 lb + j
-    const int i = tid / 81, c = tid - 81 * (tid / 81), lb = c / 3, j = c - 3 * (c / 3);
-    const int lbx = lb / 9, lby = (lb / 3) % 3, lbz = lb % 3;
-    // stencil slot of the thread's column point in element slot (x, y, z)
-    int sxv[3] = {0, 0, 0}, syv[3] = {0, 0, 0}, szv[3] = {0, 0, 0};
+    const int axy = a / nb2, az = a - axy * nb2, ax = axy / nb1, ay = axy - ax * nb1;
+    const Stencil Sx(ax, M.nb[0], M.periodic[0]), Sy(ay, M.nb[1], M.periodic[1]), Sz(az, M.nb[2], M.periodic[2]);
+    const ElemRow X(ax, M.nelem[0], M.periodic[0]), Y(ay, M.nelem[1], M.periodic[1]), Z(az, M.nelem[2], M.periodic[2]);
+    const int nsz = Sz.cnt, nsyz = Sy.cnt * nsz, n = 3 * Sx.cnt * nsyz;
+    // columns c of an element row: c = lane, and 64 + u of element z = h along z
+    const int h = lane / 17, u = lane - 17 * h, c2 = 64 + u, z2 = h < 3 ? h : 0;
+    TK v[27], w[9];
 #pragma unroll
-    for (int x = 0; x < 3; x++) {
-        if (x < nx) {
-            const int bx = own1(ex[x] + lbx, M.nb[0], M.periodic[0]);
-            for (int k = 0; k < nsx; k++) if (Sx[k] == bx) sxv[x] = k;
+    for (int x = 0; x < 3; x++)
+#pragma unroll
+        for (int y = 0; y < 3; y++) {
+            const int64_t exy = ((int64_t)X.e[x] * M.nelem[1] + Y.e[y]) * M.nelem[2];
+            const int lxy = 27 * X.l[x] + 9 * Y.l[y];
+#pragma unroll
+            for (int z = 0; z < 3; z++) {
+                const bool ok = X.ok[x] && Y.ok[y] && Z.ok[z];
+                v[9 * x + 3 * y + z] = Ke[ok ? (exy + Z.e[z]) * 6561 + (lxy + 3 * Z.l[z] + i) * 81 + lane : 0];
+            }
+            const int ez = z2 == 0 ? Z.e[0] : z2 == 1 ? Z.e[1] : Z.e[2], lz = z2 == 0 ? Z.l[0] : z2 == 1 ? Z.l[1] : Z.l[2];
+            const bool okz = z2 == 0 ? Z.ok[0] : z2 == 1 ? Z.ok[1] : Z.ok[2];
+            w[3 * x + y] = Ke[X.ok[x] && Y.ok[y] && okz ? (exy + ez) * 6561 + (lxy + 3 * lz + i) * 81 + c2 : 0];
         }
-        if (x < ny) {
-            const int by = own1(ey[x] + lby, M.nb[1], M.periodic[1]);
-            for (int k = 0; k < nsy; k++) if (Sy[k] == by) syv[x] = k;
-        }
-        if (x < nz) {
-            const int bz = own1(ez[x] + lbz, M.nb[2], M.periodic[2]);
-            for (int k = 0; k < nsz; k++) if (Sz[k] == bz) szv[x] = k;
-        }
+    // the write-out's Dirichlet flags and row start
+    bool dead[6];
+    int col[6];
+    const bool drow = mask[row] != 0;
+    const int64_t start = rowptr[row];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        const int r = lane + 64 * k, t = r / 3, j = r - 3 * t, sx = t / nsyz, q = t - sx * nsyz, sy = q / nsz, sz = q - sy * nsz;
+        col[k] = r < n ? 3 * ((Sx.at(sx) * nb1 + Sy.at(sy)) * nb2 + Sz.at(sz)) + j : 0;
+        dead[k] = drow || mask[col[k]] != 0;
+        if (r < n) acc[r] = 0.0;
     }
-    __shared__ int64_t s_rp[3];
-    __shared__ int32_t s_mrow[3], s_mcol[125 * 3];
-    double v[27];
+    // places of the two columns' points: 3 (slot along x) ns_y ns_z + 3 (slot along y) ns_z + 3 (slot along z) + component
+    int px[3], py[3], pz[3], qx[3], qy[3], qz;
+    {
+        const int lb = lane / 3, j = lane - 3 * lb, lb2 = c2 / 3, j2 = c2 - 3 * lb2;
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            px[e] = 3 * nsyz * Sx.slot(own1(X.e[e] + lb / 9, M.nb[0], M.periodic[0]));
+            py[e] = 3 * nsz * Sy.slot(own1(Y.e[e] + (lb / 3) % 3, M.nb[1], M.periodic[1]));
+            pz[e] = 3 * Sz.slot(own1(Z.e[e] + lb % 3, M.nb[2], M.periodic[2])) + j;
+            qx[e] = 3 * nsyz * Sx.slot(own1(X.e[e] + lb2 / 9, M.nb[0], M.periodic[0]));
+            qy[e] = 3 * nsz * Sy.slot(own1(Y.e[e] + (lb2 / 3) % 3, M.nb[1], M.periodic[1]));
+        }
+        const int ez = z2 == 0 ? Z.e[0] : z2 == 1 ? Z.e[1] : Z.e[2];
+        qz = 3 * Sz.slot(own1(ez + lb2 % 3, M.nb[2], M.periodic[2])) + j2;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
     for (int x = 0; x < 3; x++)
 #pragma unroll
         for (int y = 0; y < 3; y++)
 #pragma unroll
-            for (int z = 0; z < 3; z++) {
-                double t = 0.0;
-                if (tid < 243 && x < nx && y < ny && z < nz) {
-                    const int64_t e = ((int64_t)ex[x] * M.nelem[1] + ey[y]) * M.nelem[2] + ez[z];
-                    const int la = 9 * lax[x] + 3 * lay[y] + laz[z];
-                    t = (double)Ke[e * 6561 + (3 * la + i) * 81 + c];
+            for (int z = 0; z < 3; z++)
+                if (X.ok[x] && Y.ok[y] && Z.ok[z]) {
+                    lds_add(acc + px[x] + py[y] + pz[z], (double)v[9 * x + 3 * y + z]);
+                    if (h == z) lds_add(acc + qx[x] + qy[y] + qz, (double)w[3 * x + y]);
                 }
-                v[9 * x + 3 * y + z] = t;
-            }
-    // the output phase's row starts and Dirichlet flags, loaded now so that
-    // their latency overlaps the element rounds
-    for (int q = tid; q < 3 * nst + 6; q += 256) {
-        if (q < 3 * nst) {
-            const int t = q / 3, jj = q - 3 * t;
-            const int sx = t / (nsy * nsz), sy = (t / nsz) % nsy, sz = t % nsz;
-            const int bcp = (nb1 * nb2) * Sx[sx] + nb2 * Sy[sy] + Sz[sz];
-            s_mcol[q] = mask[3 * bcp + jj];
-        } else if (q < 3 * nst + 3) {
-            s_rp[q - 3 * nst] = rowptr[3 * a + (q - 3 * nst)];
-        } else {
-            s_mrow[q - 3 * nst - 3] = mask[3 * a + (q - 3 * nst - 3)];
-        }
-    }
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-    for (int x = 0; x < 3; x++)
-#pragma unroll
-        for (int y = 0; y < 3; y++)
-#pragma unroll
-            for (int z = 0; z < 3; z++) {
-                if (x < nx && y < ny && z < nz) {
-                    if (tid < 243) {
-                        const int t = (sxv[x] * nsy + syv[y]) * nsz + szv[z];
-                        acc[(3 * t + i) * 3 + j] += v[9 * x + 3 * y + z];
-                    }
-                    __syncthreads();
-                }
-            }
-    // CSR rows 3a+i: positions rowptr + 3t + j, consecutive threads on one row
-    for (int idx = tid; idx < nst * 9; idx += 256) {
-        const int ii = idx / (3 * nst), r = idx - ii * 3 * nst, t = r / 3, jj = r - 3 * t;
-        const int sx = t / (nsy * nsz), sy = (t / nsz) % nsy, sz = t % nsz;
-        const int bcp = (nb1 * nb2) * Sx[sx] + nb2 * Sy[sy] + Sz[sz];
-        const int row = 3 * a + ii, col = 3 * bcp + jj;
-        const double val = (s_mrow[ii] || s_mcol[3 * t + jj]) ? (row == col ? 1.0 : 0.0) : acc[(3 * t + ii) * 3 + jj];
-        vals[s_rp[ii] + r] = (TV)val;
+    for (int k = 0; k < 6; k++) {
+        const int r = lane + 64 * k;
+        if (r < n) vals[start + r] = (TV)(dead[k] ? (row == col[k] ? 1.0 : 0.0) : acc[r]);
     }
 }
 
@@ -2599,11 +2519,11 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
 hipError_t launch_tangent_gather(const MeshK &M, const void *Ke, int prec, const int64_t *rowptr, const int32_t *mask, void *vals,
                                  int64_t ncp, const double *U, double *Ucopy, hipStream_t s)
 {
-    dim3 grid((unsigned)ncp), block(256);
+    dim3 grid((unsigned)ncp), block(192);
     if (prec == 0)
         hipLaunchKernelGGL((k_tangent_gather_rows<double, double>), grid, block, 0, s, M, (const double *)Ke, rowptr, mask, (double *)vals, U, Ucopy);
     else
-        hipLaunchKernelGGL((k_tangent_gather<float, float>), grid, dim3(128), 0, s, M, (const float *)Ke, rowptr, mask, (float *)vals, U, Ucopy);
+        hipLaunchKernelGGL((k_tangent_gather_rows<float, float>), grid, block, 0, s, M, (const float *)Ke, rowptr, mask, (float *)vals, U, Ucopy);
     return hipGetLastError();
 }
 
