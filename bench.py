@@ -216,8 +216,8 @@ def kernel_rooflines(nel, nelem, nnz, avg, avg32, gen, gen32, genr):
     return {
         "k_tangent_sep<double, false>": flop(avg[1], F_K, PEAK_FP64_TFLOPS, "valu", F_SEP),
         "k_tangent_sep<float, false>": flop(avg32[1], F_K, PEAK_FP32_TFLOPS, "valu", F_SEP),
-        "k_tangent_elem<double, 1, false>": flop(gen, F_K, PEAK_FP64_TFLOPS, "mfma"),
-        "k_tangent_elem<float, 1, false>": flop(gen32, F_K, PEAK_FP32_TFLOPS, "mfma"),
+        "k_tangent_gen<double, false>": flop(gen, F_K, PEAK_FP64_TFLOPS, "valu"),
+        "k_tangent_gen<float, false>": flop(gen32, F_K, PEAK_FP32_TFLOPS, "valu"),
         "k_residual_sep": flop(avg[0], F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
         "k_residual_elem<1>": flop(genr, F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
         "k_tangent_gather_rows<double,double>": hbm(avg[2], 8 * (6561 * nelem + nnz),

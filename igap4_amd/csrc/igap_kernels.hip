@@ -1161,7 +1161,7 @@ __global__ __launch_bounds__(64) void k_sep_tables(MeshK M, double *__restrict__
 template <int NH = 1, int STR = 3>
 __device__ __forceinline__ void sep_element(const MeshK &M, const double *__restrict__ Uh, const int *ed, double *sU,
                                             double (*sPd)[4][3][3], double (*sW)[4], int64_t ndof = 0,
-                                            double *sUd = nullptr, double *sV = nullptr, double cv1 = 0.0, double cv2 = 0.0)
+                                            double *sUd = nullptr)
 {
     const int tid = threadIdx.x;
     if (tid < 27) {
@@ -1173,15 +1173,12 @@ __device__ __forceinline__ void sep_element(const MeshK &M, const double *__rest
             for (int k = 0; k < 3; k++) sU[STR * tid + k] = Uh[3 * oc + k];
         } else {
             // the transient rule's two fields: Um = (U^1 + U^2)/2 -> sU and
-            // Ud = (U - U^2)/2 -> sUd (rule node j: Um + s_j Ud); with sV, the
-            // nodal cv1 (U - U^2) + cv2 (U + U^2 - 2 U^1)
+            // Ud = (U - U^2)/2 -> sUd (rule node j: Um + s_j Ud)
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 const double u0 = Uh[3 * oc + k], u1 = Uh[ndof + 3 * oc + k], u2 = Uh[2 * ndof + 3 * oc + k];
                 sU[STR * tid + k] = 0.5 * (u1 + u2);
                 sUd[STR * tid + k] = 0.5 * (u0 - u2);
-                // the inertia combination of the residual's value slot
-                if (sV) sV[3 * tid + k] = cv1 * (u0 - u2) + cv2 * (u0 + u2 - 2 * u1);
             }
         }
     } else if (tid >= 64 && tid < 64 + 3 * TAB_STRIDE) {
@@ -1802,64 +1799,6 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
     sep_pipeline<T, Sh>(sX, taby + ed[1] * TAB_STRIDE, tabz + ed[2] * TAB_STRIDE, sD, sE, in, out);
 }
 
-// Transposed sum factorisation of the weighted pointwise residual jets
-// sR[q * RS + 10 k + a] (after a barrier; sWork holds 1188 doubles): returns
-// R_e[tid] = sum_q sum_a r_q[k][a] R_q[a][b] (tid = 3 b + k < 81), the
-// reference's projection (src/assmcore_iga.c:230-252) as x -> y -> z passes
-// over the physical tables; 0 for tid >= 81.
-template <int RS>
-__device__ __forceinline__ double sep_project(const double (*sPd)[4][3][3], const double *sR, double *sWork)
-{
-    // ---- x^T: C1[k][bx][qy][qz][s6] = sum_qx sum_{a: S6(a) = s6} r[q][k][a] Px[qx][DX(a)][bx]
-    const int tid = threadIdx.x;
-    double *C1 = sWork, *C2 = sWork + 864;
-    for (int i = tid; i < 864; i += 256) {   // s6 slowest: the switch below is mostly wave-uniform
-        const int s6 = i / 144, t = i - 144 * s6, qz = t & 3, qy = (t >> 2) & 3, bx = (t >> 4) % 3, k = t / 48;
-        double acc = 0.0;
-#pragma unroll
-        for (int qx = 0; qx < 4; qx++) {
-            const double *rq = sR + (16 * qx + 4 * qy + qz) * RS + 10 * k;
-            const double *tx = &sPd[0][qx][0][0];   // tx[3 * dx + bx]
-            switch (s6) {
-                case 0: acc += rq[0] * tx[bx] + rq[1] * tx[3 + bx] + rq[4] * tx[6 + bx]; break;
-                case 1: acc += rq[2] * tx[bx] + rq[5] * tx[3 + bx]; break;
-                case 2: acc += rq[3] * tx[bx] + rq[6] * tx[3 + bx]; break;
-                case 3: acc += rq[7] * tx[bx]; break;
-                case 4: acc += rq[8] * tx[bx]; break;
-                default: acc += rq[9] * tx[bx]; break;
-            }
-        }
-        C1[6 * t + s6] = acc;   // [k][bx][qy][qz][s6]
-    }
-    __syncthreads();
-    // ---- y^T: C2[k][bx][by][qz][dz] = sum_qy sum_{s6: dz(s6) = dz} C1[..][s6] Py[qy][dy(s6)][by]
-    for (int i = tid; i < 324; i += 256) {   // dz slowest (mostly wave-uniform branches)
-        const int dz = i / 108, t = i - 108 * dz, qz = t & 3, u = t >> 2, by = u % 3, bx = (u / 3) % 3, k = u / 9;
-        double acc = 0.0;
-#pragma unroll
-        for (int qy = 0; qy < 4; qy++) {
-            const double *c = C1 + (((k * 3 + bx) * 4 + qy) * 4 + qz) * 6;
-            const double *ty = &sPd[1][qy][0][0];   // ty[3 * dy + by]
-            if (dz == 0) acc += c[0] * ty[by] + c[1] * ty[3 + by] + c[3] * ty[6 + by];
-            else if (dz == 1) acc += c[2] * ty[by] + c[4] * ty[3 + by];
-            else acc += c[5] * ty[by];
-        }
-        C2[3 * t + dz] = acc;   // [k][bx][by][qz][dz]
-    }
-    __syncthreads();
-    // ---- z^T: R_e[3 b + k] = sum_qz sum_dz C2[k][bx][by][qz][dz] Pz[qz][dz][bz]
-    double acc = 0.0;
-    if (tid < 81) {
-        const int k = tid % 3, b = tid / 3, bx = b / 9, by = (b / 3) % 3, bz = b % 3;
-        const double *c = C2 + ((k * 3 + bx) * 3 + by) * 12;
-#pragma unroll
-        for (int qz = 0; qz < 4; qz++)
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) acc += c[3 * qz + dz] * sPd[2][qz][dz][bz];
-    }
-    return acc;
-}
-
 // ============================================================================
 // Residual on a separable patch (k_residual_sep, static physics; volume loop
 // of Residual_iga, src/assmcore_iga.c:118-259): the displacement jets of
@@ -1880,205 +1819,222 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
-__global__ __launch_bounds__(64, 3) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
-                                                        double *__restrict__ Re, int nel)
+// Field passes of one nodal component c[STR * b] by a wave: lane q gets its
+// parametric or physical jet (the tables decide) at point q.  sA 108, sB 288 doubles.
+template <int STR>
+__device__ __forceinline__ void wave_field(const double (*sT)[TAB_STRIDE], const double *c, double *sA, double *sB, int lane, double *J)
 {
-    __shared__ double sT[3][TAB_STRIDE];   // the element's 1-D tables [q][order][function], then their point weights
-    __shared__ double sU[27 * 3];
-    __shared__ double sA[108], sB[288];    // field passes, then the transposed ones
-    __shared__ double sR[10 * 64];         // weighted residual jets of one component [a][q]
-    const int lane = threadIdx.x, e = blockIdx.x;
-    const int nz = M.nelem[2], ny = M.nelem[1];
-    const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
+    const int qz = lane & 3, qy = (lane >> 2) & 3, qx = lane >> 4;
+    // z: sA[bx*3+by][qz][dz]
+    if (lane < 36) {
+        const double *cb = c + 3 * STR * (lane >> 2);
+#pragma unroll
+        for (int dz = 0; dz < 3; dz++) {
+            const double *tz = &sT[2][9 * qz + 3 * dz];
+            sA[3 * lane + dz] = cb[0] * tz[0] + cb[STR] * tz[1] + cb[2 * STR] * tz[2];
+        }
+    }
+    wave_sync();
+    // y: sB[bx][qy][qz][s6], s6 = (dy, dz) in the order (0,0) (1,0) (0,1) (2,0) (1,1) (0,2); bx = qx here
+    if (lane < 48) {
+        const double *a = sA + 36 * qx + 3 * qz;   // a[12 by + dz]
+#pragma unroll
+        for (int s6 = 0; s6 < 6; s6++) {
+            const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
+            const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
+            const double *ty = &sT[1][9 * qy + 3 * dy];
+            sB[6 * lane + s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
+        }
+    }
+    wave_sync();
+    sf_jet(sB + (lane & 15) * 6, &sT[0][9 * qx], J);
+}
+
+// Transposed passes by a wave: lane q's weighted residual jet r[10] of one
+// component -> R_e of that component at local point b = lane (0 for lane >= 27).  sR 640 doubles.
+__device__ __forceinline__ double wave_project(const double (*sT)[TAB_STRIDE], const double *r, double w, double *sR, double *sA, double *sB,
+                                               int lane)
+{
+    const int qz = lane & 3, qx = lane >> 4;
+#pragma unroll
+    for (int a = 0; a < 10; a++) sR[64 * a + lane] = w * r[a];
+    wave_sync();
+    // x^T: C1[bx][qy][qz][s6] = sum_qx sum_{a: S6(a) = s6} r[a] Px[qx][DX(a)][bx]
+    if (lane < 48) {
+        double c[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int x = 0; x < 4; x++) {
+            const double *rq = sR + 16 * x + (lane & 15), *tx = &sT[0][9 * x + qx];   // bx = qx; tx[3 dx]
+            c[0] += rq[0] * tx[0] + rq[64] * tx[3] + rq[4 * 64] * tx[6];
+            c[1] += rq[2 * 64] * tx[0] + rq[5 * 64] * tx[3];
+            c[2] += rq[3 * 64] * tx[0] + rq[6 * 64] * tx[3];
+            c[3] += rq[7 * 64] * tx[0];
+            c[4] += rq[8 * 64] * tx[0];
+            c[5] += rq[9 * 64] * tx[0];
+        }
+#pragma unroll
+        for (int s6 = 0; s6 < 6; s6++) sB[6 * lane + s6] = c[s6];
+    }
+    wave_sync();
+    // y^T: C2[bx][by][qz][dz] = sum_qy sum_{s6: dz(s6) = dz} C1[..][s6] Py[qy][dy(s6)][by]
+    if (lane < 36) {
+        const int by = (lane >> 2) % 3, bx = lane / 12;
+        double c[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int y = 0; y < 4; y++) {
+            const double *c1 = sB + ((bx * 4 + y) * 4 + qz) * 6, *ty = &sT[1][9 * y + by];   // ty[3 dy]
+            c[0] += c1[0] * ty[0] + c1[1] * ty[3] + c1[3] * ty[6];
+            c[1] += c1[2] * ty[0] + c1[4] * ty[3];
+            c[2] += c1[5] * ty[0];
+        }
+#pragma unroll
+        for (int dz = 0; dz < 3; dz++) sA[3 * lane + dz] = c[dz];
+    }
+    wave_sync();
+    // z^T: R_e = sum_qz sum_dz C2[bx][by][qz][dz] Pz[qz][dz][bz]
+    double acc = 0.0;
+    if (lane < 27) {
+        const double *c2 = sA + (lane / 3) * 12;
+#pragma unroll
+        for (int z = 0; z < 4; z++)
+#pragma unroll
+            for (int dz = 0; dz < 3; dz++) acc += c2[3 * z + dz] * sT[2][9 * z + 3 * dz + lane % 3];
+    }
+    return acc;
+}
+
+// the element's 1-D tables [q][order][function] with their point weights, by a wave
+__device__ __forceinline__ void wave_tables(const MeshK &M, const int *ed, double (*sT)[TAB_STRIDE], int lane)
+{
 #pragma unroll
     for (int d = 0; d < 3; d++)
         if (lane < TAB_STRIDE) sT[d][lane] = M.tab[d][(int64_t)ed[d] * TAB_STRIDE + lane];
+}
+// owned control point of local point b
+__device__ __forceinline__ int64_t wave_point(const MeshK &M, const int *ed, int b)
+{
+    return ((int64_t)M.nb[1] * M.nb[2]) * own1(ed[0] + b / 9, M.nb[0], M.periodic[0])
+         + (int64_t)M.nb[2] * own1(ed[1] + (b / 3) % 3, M.nb[1], M.periodic[1]) + own1(ed[2] + b % 3, M.nb[2], M.periodic[2]);
+}
+
+__global__ __launch_bounds__(64, 3) void k_residual_sep(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
+                                                        double *__restrict__ Re, int nel)
+{
+    __shared__ double sT[3][TAB_STRIDE], sU[27 * 3], sA[108], sB[288], sR[640];
+    const int lane = threadIdx.x, e = blockIdx.x;
+    const int nz = M.nelem[2], ny = M.nelem[1];
+    const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
+    wave_tables(M, ed, sT, lane);
     if (lane < 27) {
-        const int bx = lane / 9, by = (lane / 3) % 3, bz = lane % 3;
-        const int64_t oc = ((int64_t)M.nb[1] * M.nb[2]) * own1(ed[0] + bx, M.nb[0], M.periodic[0])
-                         + (int64_t)M.nb[2] * own1(ed[1] + by, M.nb[1], M.periodic[1]) + own1(ed[2] + bz, M.nb[2], M.periodic[2]);
+        const int64_t oc = wave_point(M, ed, lane);
 #pragma unroll
         for (int k = 0; k < 3; k++) sU[3 * lane + k] = Uh[3 * oc + k];
     }
     wave_sync();
-    const int qz = lane & 3, qy = (lane >> 2) & 3, qx = lane >> 4;
-    double u[30];
+    double u[30], r[30], out[3];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        // z: sA[bx*3+by][qz][dz]
-        if (lane < 36) {
-            const double *c = sU + 9 * (lane >> 2) + k;
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) {
-                const double *tz = &sT[2][9 * qz + 3 * dz];
-                sA[3 * lane + dz] = c[0] * tz[0] + c[3] * tz[1] + c[6] * tz[2];
-            }
-        }
-        wave_sync();
-        // y: sB[bx][qy][qz][s6], s6 = (dy, dz) in the order (0,0) (1,0) (0,1) (2,0) (1,1) (0,2); bx = qx here
-        if (lane < 48) {
-            const double *a = sA + 36 * qx + 3 * qz;   // a[12 by + dz]
-#pragma unroll
-            for (int s6 = 0; s6 < 6; s6++) {
-                const int dy = (s6 == 1 || s6 == 4) ? 1 : (s6 == 3 ? 2 : 0);
-                const int dz = (s6 == 2 || s6 == 4) ? 1 : (s6 == 5 ? 2 : 0);
-                const double *ty = &sT[1][9 * qy + 3 * dy];
-                sB[6 * lane + s6] = a[dz] * ty[0] + a[12 + dz] * ty[1] + a[24 + dz] * ty[2];
-            }
-        }
-        wave_sync();
-        sf_jet(sB + (lane & 15) * 6, &sT[0][9 * qx], u + 10 * k);
+        wave_field<3>(sT, sU + k, sA, sB, lane, u + 10 * k);
         sep_macro(M, ed, lane, k, u + 10 * k);
     }
-    double r[30];
     phys_residual_static(P, u, r);
-    const double w = sT[0][36 + qx] * sT[1][36 + qy] * sT[2][36 + qz];
-    double out[3];
+    const double w = sT[0][36 + (lane >> 4)] * sT[1][36 + ((lane >> 2) & 3)] * sT[2][36 + (lane & 3)];
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-#pragma unroll
-        for (int a = 0; a < 10; a++) sR[64 * a + lane] = w * r[10 * k + a];
-        wave_sync();
-        // x^T: C1[bx][qy][qz][s6] = sum_qx sum_{a: S6(a) = s6} r[a] Px[qx][DX(a)][bx]
-        if (lane < 48) {
-            double c[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int x = 0; x < 4; x++) {
-                const double *rq = sR + 16 * x + (lane & 15), *tx = &sT[0][9 * x + qx];   // bx = qx; tx[3 dx]
-                c[0] += rq[0] * tx[0] + rq[64] * tx[3] + rq[4 * 64] * tx[6];
-                c[1] += rq[2 * 64] * tx[0] + rq[5 * 64] * tx[3];
-                c[2] += rq[3 * 64] * tx[0] + rq[6 * 64] * tx[3];
-                c[3] += rq[7 * 64] * tx[0];
-                c[4] += rq[8 * 64] * tx[0];
-                c[5] += rq[9 * 64] * tx[0];
-            }
-#pragma unroll
-            for (int s6 = 0; s6 < 6; s6++) sB[6 * lane + s6] = c[s6];
-        }
-        wave_sync();
-        // y^T: C2[bx][by][qz][dz] = sum_qy sum_{s6: dz(s6) = dz} C1[..][s6] Py[qy][dy(s6)][by]
-        if (lane < 36) {
-            const int by = (lane >> 2) % 3, bx = lane / 12;
-            double c[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-            for (int y = 0; y < 4; y++) {
-                const double *c1 = sB + ((bx * 4 + y) * 4 + qz) * 6, *ty = &sT[1][9 * y + by];   // ty[3 dy]
-                c[0] += c1[0] * ty[0] + c1[1] * ty[3] + c1[3] * ty[6];
-                c[1] += c1[2] * ty[0] + c1[4] * ty[3];
-                c[2] += c1[5] * ty[0];
-            }
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) sA[3 * lane + dz] = c[dz];
-        }
-        wave_sync();
-        // z^T: R_e[3 b + k] = sum_qz sum_dz C2[bx][by][qz][dz] Pz[qz][dz][bz]
-        double acc = 0.0;
-        if (lane < 27) {
-            const double *c2 = sA + (lane / 3) * 12;
-#pragma unroll
-            for (int z = 0; z < 4; z++)
-#pragma unroll
-                for (int dz = 0; dz < 3; dz++) acc += c2[3 * z + dz] * sT[2][9 * z + 3 * dz + lane % 3];
-        }
-        out[k] = acc;
-    }
+    for (int k = 0; k < 3; k++) out[k] = wave_project(sT, r + 10 * k, w, sR, sA, sB, lane);
     if (lane < 27) {
 #pragma unroll
         for (int k = 0; k < 3; k++) Re[(int64_t)e * 81 + 3 * lane + k] = out[k];
     }
 }
 
-// Transient residual on a separable patch (k_residual_sep_t, gradelasttime):
-// the jets of Um and Ud, the rule's eight nodes per point (one lane per node
-// at Um + s_j Ud, weighted by cr_j and summed over the 8-lane group), the
-// point weight, and the projection of k_residual_sep.  The value slot's inertia r[10 k] = cii (u - u^2) / (2 dt)
+// Transient residual on a separable patch (k_residual_sep_t, gradelasttime), a
+// wave per element like the static one: the jets of Um and Ud of a lane's point,
+// the rule's eight nodes Um + s_j Ud one after another, weighted by cr_j, all in
+// its registers, then the projection.  The value slot's inertia r[10 k] = cii (u - u^2) / (2 dt)
 // + rho (u + u^2 - 2 u^1) / dt^2 is linear in the nodal values, so its part of
 // R_e is the element mass matrix Mx x My x Mz applied to the nodal
 // combination (k_tangent_sep_t's 1-D mass matrices).
-__global__ __launch_bounds__(256, 2) void k_residual_sep_t(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
-                                                           double *__restrict__ Re, int nel)
+// At 128x32x32 2.70 -> 1.37 ms, against a workgroup of four waves per element with a lane
+// per node and point, the node sums as lane moves and seven block barriers.  Ud's jets
+// wait in LDS: 20 KB an element, eight elements in flight per CU, as many as the registers allow.
+__global__ __launch_bounds__(64, 2) void k_residual_sep_t(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
+                                                          double *__restrict__ Re, int nel)
 {
-    __shared__ double sPd[3][4][3][3];
-    __shared__ double sW[3][4];
-    __shared__ double sC[27][6], sV[27 * 3];   // nodal Um, Ud; inertia combination
-    __shared__ double sMass[3][3][3];
-    __shared__ double sWork[6 * (108 + 288)];   // field passes, then x^T (864) and y^T (324)
-    __shared__ double sJet[64 * 60];            // jets [q][h][k][a] of Um and Ud, then the weighted r_q [q][k][a]
-    const int tid = threadIdx.x;
-    const int e = blockIdx.x;
+    __shared__ double sT[3][TAB_STRIDE], sC[27 * 6], sV[27 * 3], sMass[3][3][3], sA[108], sB[288];
+    __shared__ double sJ[27 * 64];   // the points' jets of Ud [slot][q], then wave_project's buffer
+    const int lane = threadIdx.x, e = blockIdx.x;
     const int nz = M.nelem[2], ny = M.nelem[1];
     const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
-
-    sep_element<3, 6>(M, Uh, ed, &sC[0][0], sPd, sW, ndof, &sC[0][3], sV, P.cii / (2. * P.dt), P.rho / (P.dt * P.dt));
-    __syncthreads();
-    {
-        six_fields(sC, sPd, sWork);
-        const int q = tid & 63, k = tid >> 6;
-        if (k < 3) {
-            double J1[10], J2[10];
-            six_jet(sWork, sPd, k, q, J1);
-            six_jet(sWork, sPd, 3 + k, q, J2);
-            sep_macro(M, ed, q, k, J1);
+    wave_tables(M, ed, sT, lane);
+    if (lane < 27) {
+        const int64_t oc = wave_point(M, ed, lane);
+        const double cv1 = P.cii / (2. * P.dt), cv2 = P.rho / (P.dt * P.dt);
 #pragma unroll
-            for (int a = 0; a < 10; a++) {
-                sJet[q * 60 + 10 * k + a] = J1[a];
-                sJet[q * 60 + 30 + 10 * k + a] = J2[a];
-            }
-        }
-        if (tid < 27) {
-            const int d = tid / 9, b = (tid / 3) % 3, c = tid % 3;
-            double m = 0.0;
-#pragma unroll
-            for (int qq = 0; qq < 4; qq++) m += sW[d][qq] * sPd[d][qq][0][b] * sPd[d][qq][0][c];
-            sMass[d][b][c] = m;
+        for (int k = 0; k < 3; k++) {
+            const double u0 = Uh[3 * oc + k], u1 = Uh[ndof + 3 * oc + k], u2 = Uh[2 * ndof + 3 * oc + k];
+            sC[6 * lane + k] = 0.5 * (u1 + u2);
+            sC[6 * lane + 3 + k] = 0.5 * (u0 - u2);
+            sV[3 * lane + k] = cv1 * (u0 - u2) + cv2 * (u0 + u2 - 2 * u1);
         }
     }
-    __syncthreads();
-    // ---- rule-weighted residual jets of the stored energy, times the weight:
-    //      lane 8g + j takes rule node j of point g + 32 round, the node sums
-    //      over the 8-lane group one entry at a time
+    wave_sync();
+    if (lane < 27) {
+        const int d = lane / 9, b = (lane / 3) % 3, c = lane % 3;
+        double m = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; q++) m += sT[d][36 + q] * sT[d][9 * q + b] * sT[d][9 * q + c];
+        sMass[d][b][c] = m;
+    }
+    double r[30], out[3];
     {
-        const int j = tid & 7;
-        for (int round = 0; round < 2; round++) {
-            const int q = (tid >> 3) + 32 * round;
-            const double *J = sJet + q * 60;
-            double r[30];
-            {
-                double us[30];
+        double J1[30];
 #pragma unroll
-                for (int a = 0; a < 30; a++) us[a] = J[a] + P.s[j] * J[30 + a];
-                State st;
-                phys_state(us, P, st);
+        for (int k = 0; k < 3; k++) {
+            double J2[10];
+            wave_field<6>(sT, sC + 3 + k, sA, sB, lane, J2);
 #pragma unroll
-                for (int a = 0; a < 30; a++) r[a] = 0.0;
-                phys_residual_acc(st, P.cr[j], r);
+            for (int a = 1; a < 10; a++) sJ[64 * (9 * k + a - 1) + lane] = J2[a];
+            wave_field<6>(sT, sC + k, sA, sB, lane, J1 + 10 * k);
+            sep_macro(M, ed, lane, k, J1 + 10 * k);
+        }
+#pragma unroll
+        for (int a = 0; a < 30; a++) r[a] = 0.0;
+#pragma unroll 1
+        for (int j = 0; j < 8; j++) {
+            double us[30];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                us[10 * k] = 0.0;
+#pragma unroll
+                for (int a = 1; a < 10; a++) us[10 * k + a] = J1[10 * k + a] + P.s[j] * sJ[64 * (9 * k + a - 1) + lane];
             }
-            const double w = (j == 0) ? sep_weight(q, sW) : 0.0;
-#pragma unroll
-            for (int a = 0; a < 30; a++) {
-                if (a % 10 == 0) continue;   // value slots: the inertia, added below
-                r[a] = sum8(r[a]);
-            }
-            if (j == 0) {
-#pragma unroll
-                for (int a = 0; a < 30; a++) sJet[q * 60 + a] = (a % 10 == 0) ? 0.0 : w * r[a];
-            }
+            State st;
+            phys_state(us, P, st);
+            phys_residual_acc(st, P.cr[j], r);
         }
     }
-    __syncthreads();
-    double v = sep_project<60>(sPd, sJet, sWork);
-    if (tid < 81) {
-        const int k = tid % 3, b = tid / 3, bx = b / 9, by = (b / 3) % 3, bz = b % 3;
-        double in = 0.0;
+    wave_sync();
+    const double w = sT[0][36 + (lane >> 4)] * sT[1][36 + ((lane >> 2) & 3)] * sT[2][36 + (lane & 3)];
 #pragma unroll
-        for (int cx = 0; cx < 3; cx++)
+    for (int k = 0; k < 3; k++) {
+        r[10 * k] = 0.0;   // value slot: the inertia, added below
+        out[k] = wave_project(sT, r + 10 * k, w, sJ, sA, sB, lane);
+    }
+    if (lane < 27) {
+        const int bx = lane / 9, by = (lane / 3) % 3, bz = lane % 3;
 #pragma unroll
-            for (int cy = 0, ys = 0; cy < 3; cy++) {
-                const double mxy = sMass[0][bx][cx] * sMass[1][by][cy];
+        for (int k = 0; k < 3; k++) {
+            double in = 0.0;
 #pragma unroll
-                for (int cz = 0; cz < 3; cz++) in += mxy * sMass[2][bz][cz] * sV[3 * (9 * cx + 3 * cy + cz) + k];
-            }
-        Re[(int64_t)e * 81 + tid] = v + in;
+            for (int cx = 0; cx < 3; cx++)
+#pragma unroll
+                for (int cy = 0; cy < 3; cy++) {
+                    const double mxy = sMass[0][bx][cx] * sMass[1][by][cy];
+#pragma unroll
+                    for (int cz = 0; cz < 3; cz++) in += mxy * sMass[2][bz][cz] * sV[3 * (9 * cx + 3 * cy + cz) + k];
+                }
+            Re[(int64_t)e * 81 + 3 * lane + k] = out[k] + in;
+        }
     }
 }
 
@@ -2426,7 +2382,7 @@ hipError_t launch_residual_elem(const MeshK &M, const PhysK &P, const double *Uh
 {
     dim3 grid(nel), block(256);
     if (P.torder == 0 && M.separable) hipLaunchKernelGGL(k_residual_sep, grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
-    else if (P.torder == 2 && M.separable) hipLaunchKernelGGL(k_residual_sep_t, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
+    else if (P.torder == 2 && M.separable) hipLaunchKernelGGL(k_residual_sep_t, grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
     else if (P.torder == 0) hipLaunchKernelGGL(k_residual_elem<1>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
     else hipLaunchKernelGGL(k_residual_elem<3>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
     return hipGetLastError();
