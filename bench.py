@@ -219,7 +219,7 @@ def kernel_rooflines(nel, nelem, nnz, avg, avg32, gen, gen32, genr):
         "k_tangent_gen<double, false>": flop(gen, F_K, PEAK_FP64_TFLOPS, "valu"),
         "k_tangent_gen<float, false>": flop(gen32, F_K, PEAK_FP32_TFLOPS, "valu"),
         "k_residual_sep": flop(avg[0], F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
-        "k_residual_elem<1>": flop(genr, F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
+        "k_residual_gen<1, false>": flop(genr, F_R_STATIC, PEAK_FP64_TFLOPS, "valu"),
         "k_tangent_gather_rows<double,double>": hbm(avg[2], 8 * (6561 * nelem + nnz),
                                                     "igap::k_tangent_gather_rows<double, double>", 8 * nnz),
         "k_tangent_gather_rows<float,float>": hbm(avg32[2], 4 * (6561 * nelem + nnz), "igap::k_tangent_gather_rows<float, float>",

@@ -513,7 +513,7 @@ extern "C" int igap_gpu_create(const igap_mesh_desc *mesh, const igap_phys_desc 
     gauss4(M.gq, M.gw);
     M.separable = (flags & IGAP_GENERAL_GEOMETRY) ? 0 : separable_patch(c);
     M.equalw = std::all_of(c->w_h.begin(), c->w_h.end(), [&](double w) { return w == c->w_h[0]; });
-    if (M.equalw) {
+    {
         const int64_t nt = (int64_t)TAB_STRIDE * (c->nelem[0] + c->nelem[1] + c->nelem[2]);
         TRY(dalloc(&c->d_tab, nt));
         TRY(dalloc(&c->d_tabf, nt));

@@ -32,8 +32,8 @@ struct MeshK {
     double gq[4], gw[4];   // Gauss-Legendre nodes/weights on [0,1]
     int separable;    // x_d depends on xi_d alone and the weights are equal (k_tangent_sep applies)
     int equalw;       // the weights are equal: the basis is a tensor product in the parametric directions
-    // equal weights: the 1-D tables of each direction's elements (k_sep_tables;
-    // derivatives physical if separable, else parametric), TAB_STRIDE values per element: [Gauss point][order][function], then the four
+    // the 1-D tables of each direction's elements (k_sep_tables; derivatives
+    // physical if separable, else parametric), TAB_STRIDE values per element: [Gauss point][order][function], then the four
     // point weights; tabf the same in FP32
     const double *tab[3];
     const float *tabf[3];

@@ -1,6 +1,6 @@
 // igap_kernels.hip -- CDNA4 (gfx950) kernels of the IGA residual/tangent assembly.
 //
-//   k_residual_elem   per-element residual vectors R_e[81]
+//   k_residual_gen, k_residual_sep, k_residual_sep_t  per-element residual vectors R_e[81]
 //                     (volume loop of Residual_iga, src/assmcore_iga.c:118-259)
 //   k_residual_gather deterministic per-dof sum of R_e + Neumann load +
 //                     Dirichlet rows R_d = U_d - g_d (:258, :273-497)
@@ -27,17 +27,7 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // ============================================================================
-// residual: one workgroup (4 waves) per element.
-//   A  the Gauss-point fields by sum factorisation (as in the tangent):
-//      geometry, the physical u-jets of every history level -> LDS
-//   P  pointwise residual jets r_q (static: one lane per Gauss point on one
-//      wave; transient: four lanes per point, two rule nodes each)
-//   T  projection R_e[b][k] = sum_q w_q sum_a r_q[k][a] R_a(q, b), written as
-//      w_b sum_q (Q_q^T Phi_q^T w_q r_q[k]) . N_b(q): the transposes of the
-//      chain rule (phys_jet_adj) and of the quotient rule (nurbs_param_adj)
-//      per Gauss point, then the transposed sum factorisation x -> y -> z.
-// ============================================================================
-// Element e's Gauss-point fields for the residual and the density integral
+// Element e's Gauss-point fields for the density integral
 // (256 threads): the control points and 1-D tables to LDS, then by sum
 // factorisation the physical u-jets of every history level
 // (sJet[q][h][k][a], par_periodic added) and the weight, G^-1, d2x/dxi2
@@ -221,134 +211,6 @@ __device__ __forceinline__ void gp_fields(const MeshK &M, const double *__restri
         }
     }
     __syncthreads();
-}
-
-template <int NH>
-__global__ __launch_bounds__(256, (NH == 1 ? 4 : 2)) void k_residual_elem(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
-                                                       double *__restrict__ Re, int nel)
-{
-    constexpr int STR = 4 + 3 * NH;            // X(3) w(1) U(3*NH) per control point
-    constexpr int WA = gp_fields_per_pass<NH>() * (108 + 288);   // stage-A buffers
-    constexpr int GEO_R = 38;                  // wgt, Gi[9], X2[18], W[10]
-    constexpr int WG = 64 * GEO_R;             // the Gauss-point geometry (after stage A)
-    constexpr int WT = 864 + 324;              // x^T and y^T buffers (after the adjoint; rho lives in sJet)
-    constexpr int W1 = WA > WG ? WA : WG;
-    __shared__ double sT[3][4][3][3];
-    __shared__ double sCP[27 * STR];
-    __shared__ double sWork[W1 > WT ? W1 : WT];   // stage A, then sGeo, then x^T / y^T
-    __shared__ double sJet[64 * 30 * NH];      // physical u-jets [q][h][k][a]; then r_q / rho_q [q][k][a]
-    double *sGeo = sWork;
-
-    const int tid = threadIdx.x;
-    const int e = blockIdx.x;
-    // ---- A: fields at the Gauss points
-    gp_fields<NH>(M, Uh, ndof, e, sT, sCP, sWork, sJet, sGeo);
-
-    // ---- P: pointwise residual jets r_q -> sJet[q * 30 * NH + 10 k + a]
-    if (NH == 1) {
-        if ((tid >> 6) == (e & 3)) {                            // one wave, lane = Gauss point
-            const int q = tid & 63;
-            double u[30], r[30];
-#pragma unroll
-            for (int a = 0; a < 30; a++) u[a] = sJet[q * 30 + a];
-            phys_residual_static(P, u, r);
-#pragma unroll
-            for (int a = 0; a < 30; a++) sJet[q * 30 + a] = r[a];
-        }
-    } else {
-        // lanes 4q..4q+3 evaluate two rule nodes each at s_j: m0 + s_j d with
-        // m0 = (u^1 + u^0)/2, d = (u - u^0)/2, then sum over the four lanes
-        const int q = tid >> 2, part = tid & 3;
-        const double *J = sJet + q * 30 * NH;
-        double r[30];
-#pragma unroll
-        for (int a = 0; a < 30; a++) r[a] = 0.0;
-#pragma unroll 1
-        for (int gg = 0; gg < 2; gg++) {
-            const int g = 2 * part + gg;
-            double us[30];
-#pragma unroll
-            for (int a = 0; a < 30; a++) us[a] = 0.5 * (J[30 + a] + J[60 + a]) + P.s[g] * (0.5 * (J[a] - J[60 + a]));
-            State st;
-            phys_state(us, P, st);
-            phys_residual_acc(st, P.cr[g], r);
-        }
-#pragma unroll
-        for (int a = 0; a < 30; a++) {
-            r[a] = sum4(r[a]);
-        }
-        if (part == 0) {
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                r[10 * k] = (P.cii * (J[10 * k] - J[60 + 10 * k])) / (2. * P.dt)
-                          + (P.rho * (J[10 * k] + J[60 + 10 * k] - 2 * J[30 + 10 * k])) / (P.dt * P.dt);
-#pragma unroll
-            for (int a = 0; a < 30; a++) sJet[q * 30 * NH + a] = r[a];
-        }
-    }
-    __syncthreads();
-
-    // ---- T: per (Gauss point, component) adjoint of the basis maps, weighted
-    if ((tid & 3) != 0) {
-        const int q = tid >> 2, k = (tid & 3) - 1;
-        const double *g = sGeo + q * GEO_R;
-        double o[10];
-        double *rq = sJet + q * 30 * NH + 10 * k;
-#pragma unroll
-        for (int a = 0; a < 10; a++) o[a] = g[0] * rq[a];
-        phys_jet_adj(o, g + 1, g + 10);
-        nurbs_param_adj(o, g + 28);
-#pragma unroll
-        for (int a = 0; a < 10; a++) rq[a] = o[a];
-    }
-    __syncthreads();
-    //      x^T: C1[k][bx][qy][qz][s6] = sum_qx sum_{a: S6(a) = s6} rho[q][k][a] tx[qx][DX(a)][bx]
-    double *C1 = sWork, *C2 = sWork + 864;
-    for (int i = tid; i < 864; i += 256) {   // s6 slowest: the switch below is mostly wave-uniform
-        const int s6 = i / 144, t = i - 144 * s6, qz = t & 3, qy = (t >> 2) & 3, bx = (t >> 4) % 3, k = t / 48;
-        double acc = 0.0;
-#pragma unroll
-        for (int qx = 0; qx < 4; qx++) {
-            const double *rq = sJet + (16 * qx + 4 * qy + qz) * 30 * NH + 10 * k;
-            const double *tx = &sT[0][qx][0][0];   // tx[3 * dx + bx]
-            switch (s6) {
-                case 0: acc += rq[0] * tx[bx] + rq[1] * tx[3 + bx] + rq[4] * tx[6 + bx]; break;
-                case 1: acc += rq[2] * tx[bx] + rq[5] * tx[3 + bx]; break;
-                case 2: acc += rq[3] * tx[bx] + rq[6] * tx[3 + bx]; break;
-                case 3: acc += rq[7] * tx[bx]; break;
-                case 4: acc += rq[8] * tx[bx]; break;
-                default: acc += rq[9] * tx[bx]; break;
-            }
-        }
-        C1[6 * t + s6] = acc;   // [k][bx][qy][qz][s6]
-    }
-    __syncthreads();
-    //      y^T: C2[k][bx][by][qz][dz] = sum_qy sum_{s6: dz(s6) = dz} C1[..][s6] ty[qy][dy(s6)][by]
-    for (int i = tid; i < 324; i += 256) {   // dz slowest (mostly wave-uniform branches)
-        const int dz = i / 108, t = i - 108 * dz, qz = t & 3, u = t >> 2, by = u % 3, bx = (u / 3) % 3, k = u / 9;
-        double acc = 0.0;
-#pragma unroll
-        for (int qy = 0; qy < 4; qy++) {
-            const double *c = C1 + (((k * 3 + bx) * 4 + qy) * 4 + qz) * 6;
-            const double *ty = &sT[1][qy][0][0];   // ty[3 * dy + by]
-            if (dz == 0) acc += c[0] * ty[by] + c[1] * ty[3 + by] + c[3] * ty[6 + by];
-            else if (dz == 1) acc += c[2] * ty[by] + c[4] * ty[3 + by];
-            else acc += c[5] * ty[by];
-        }
-        C2[3 * t + dz] = acc;   // [k][bx][by][qz][dz]
-    }
-    __syncthreads();
-    //      z^T: R_e[3 b + k] = w_b sum_qz sum_dz C2[k][bx][by][qz][dz] tz[qz][dz][bz]
-    if (tid < 81) {
-        const int k = tid % 3, b = tid / 3, bx = b / 9, by = (b / 3) % 3, bz = b % 3;
-        const double *c = C2 + ((k * 3 + bx) * 3 + by) * 12;
-        double acc = 0.0;
-#pragma unroll
-        for (int qz = 0; qz < 4; qz++)
-#pragma unroll
-            for (int dz = 0; dz < 3; dz++) acc += c[3 * qz + dz] * sT[2][qz][dz][bz];
-        Re[(int64_t)e * 81 + tid] = sCP[STR * b + 3] * acc;
-    }
 }
 
 // ============================================================================
@@ -2038,6 +1900,131 @@ __global__ __launch_bounds__(64, 2) void k_residual_sep_t(MeshK M, PhysK P, cons
     }
 }
 
+// Residual of any geometry (k_residual_gen), a wave per element: NH = 1 static, 3
+// transient; RAT: unequal weights.  The basis is a tensor product of the
+// parametric tables (k_sep_tables; a common factor of the 1-D functions cancels in the
+// rational basis), so the coordinates' and displacements' parametric jets come
+// from wave_field, with RAT those of w, w X and w U followed by the quotient rule;
+// the chain rule gives the physical jets, and the weighted residual jet goes back
+// through the transposes of both rules (phys_jet_adj, nurbs_param_adj) into
+// wave_project:
+//   R_e[b][k] = w_b sum_q (Q_q^T Phi_q^T w_q r_q[k]) . N_b(q).
+// 64x16x16 distorted beam 282 -> 150 us, 45x23x17 rational 303 -> 265 us (134 registers
+// spilled), whole residual calls at 23x9x14: static 77 -> 39 us (rational 56), transient 155 ->
+// 84 us (89), against a workgroup of four waves per element and eight block barriers.
+template <int NH, bool RAT>
+__global__ __launch_bounds__(64, 2) void k_residual_gen(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,
+                                                        double *__restrict__ Re, int nel)
+{
+    // nodal fields X (3), U (3) or Um, Ud and the inertia combination (9), w
+    constexpr int STR = NH == 1 ? 7 : 13;
+    __shared__ double sT[3][TAB_STRIDE], sC[27 * STR], sA[108], sB[288];
+    __shared__ double sJ[NH == 1 ? 640 : 27 * 64];   // the points' jets of Ud [slot][q], then wave_project's buffer
+    const int lane = threadIdx.x, e = blockIdx.x;
+    const int nz = M.nelem[2], ny = M.nelem[1];
+    const int ed[3] = {e / (ny * nz), (e / nz) % ny, e % nz};
+    wave_tables(M, ed, sT, lane);
+    if (lane < 27) {
+        const int64_t id = ((int64_t)M.na[1] * M.na[2]) * (ed[0] + lane / 9) + (int64_t)M.na[2] * (ed[1] + (lane / 3) % 3) + ed[2] + lane % 3;
+        const int64_t oc = wave_point(M, ed, lane);
+        const double wb = RAT ? M.w[id] : 1.0;
+        double *c = sC + STR * lane;
+        c[STR - 1] = wb;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            c[k] = wb * M.X[3 * id + k];
+            const double u0 = Uh[3 * oc + k];
+            if (NH == 1) {
+                c[3 + k] = wb * u0;
+            } else {
+                const double u1 = Uh[ndof + 3 * oc + k], u2 = Uh[2 * ndof + 3 * oc + k];
+                c[3 + k] = wb * (0.5 * (u1 + u2));
+                c[(NH == 1 ? 0 : 6) + k] = wb * (0.5 * (u0 - u2));
+                c[(NH == 1 ? 0 : 9) + k] = wb * (P.cii * (u0 - u2) / (2. * P.dt) + P.rho * (u0 + u2 - 2 * u1) / (P.dt * P.dt));
+            }
+        }
+    }
+    wave_sync();
+    double W[10], Gi[9], X2[18], r[30], out[3];
+    if (RAT) wave_field<STR>(sT, sC + STR - 1, sA, sB, lane, W);
+    auto field = [&](int f, double *J) {
+        wave_field<STR>(sT, sC + f, sA, sB, lane, J);
+        if (RAT) {
+            double N[10];
+#pragma unroll
+            for (int a = 0; a < 10; a++) N[a] = J[a];
+            nurbs_param(N, 1.0, W, J);
+        }
+    };
+    double w = sT[0][36 + (lane >> 4)] * sT[1][36 + ((lane >> 2) & 3)] * sT[2][36 + (lane & 3)];
+    {
+        double G[9];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            double J[10];
+            field(d, J);
+#pragma unroll
+            for (int i = 0; i < 3; i++) G[3 * d + i] = J[1 + i];
+#pragma unroll
+            for (int t = 0; t < 6; t++) X2[6 * d + t] = J[4 + t];
+        }
+        w *= inv3(G, Gi);
+    }
+    {
+        double u[30], inert[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (NH != 1) {
+                double J[10];
+                field(9 + k, J);
+                inert[k] = J[0];
+                field(6 + k, J);
+                phys_jet(J, Gi, X2);
+#pragma unroll
+                for (int a = 1; a < 10; a++) sJ[64 * (9 * k + a - 1) + lane] = J[a];
+            }
+            field(3 + k, u + 10 * k);
+            phys_jet(u + 10 * k, Gi, X2);
+            sep_macro(M, ed, lane, k, u + 10 * k);
+        }
+        if (NH == 1) {
+            phys_residual_static(P, u, r);
+        } else {
+#pragma unroll
+            for (int a = 0; a < 30; a++) r[a] = 0.0;
+#pragma unroll 1
+            for (int j = 0; j < 8; j++) {
+                double us[30];
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    us[10 * k] = 0.0;
+#pragma unroll
+                    for (int a = 1; a < 10; a++) us[10 * k + a] = u[10 * k + a] + P.s[j] * sJ[64 * (9 * k + a - 1) + lane];
+                }
+                State st;
+                phys_state(us, P, st);
+                phys_residual_acc(st, P.cr[j], r);
+            }
+#pragma unroll
+            for (int k = 0; k < 3; k++) r[10 * k] = inert[k];
+        }
+    }
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        double *o = r + 10 * k;
+#pragma unroll
+        for (int a = 0; a < 10; a++) o[a] *= w;
+        phys_jet_adj(o, Gi, X2);
+        if (RAT) nurbs_param_adj(o, W);
+        out[k] = wave_project(sT, o, 1.0, sJ, sA, sB, lane);
+    }
+    if (lane < 27) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) Re[(int64_t)e * 81 + 3 * lane + k] = RAT ? sC[STR * lane + STR - 1] * out[k] : out[k];
+    }
+}
+
 // the unit diagonal MatZeroRowsColumns(diag = 1) leaves on the Dirichlet rows
 // of a non-periodic patch (their other entries stayed zero)
 template <typename TV>
@@ -2380,11 +2367,13 @@ hipError_t launch_density(const MeshK &M, const PhysK &P, const double *Uh, int6
 
 hipError_t launch_residual_elem(const MeshK &M, const PhysK &P, const double *Uh, int64_t ndof, double *Re, int nel, hipStream_t s)
 {
-    dim3 grid(nel), block(256);
+    dim3 grid(nel);
     if (P.torder == 0 && M.separable) hipLaunchKernelGGL(k_residual_sep, grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
     else if (P.torder == 2 && M.separable) hipLaunchKernelGGL(k_residual_sep_t, grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
-    else if (P.torder == 0) hipLaunchKernelGGL(k_residual_elem<1>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
-    else hipLaunchKernelGGL(k_residual_elem<3>, grid, block, 0, s, M, P, Uh, ndof, Re, nel);
+    else if (P.torder == 0 && M.equalw) hipLaunchKernelGGL((k_residual_gen<1, false>), grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
+    else if (P.torder == 0) hipLaunchKernelGGL((k_residual_gen<1, true>), grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
+    else if (M.equalw) hipLaunchKernelGGL((k_residual_gen<3, false>), grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
+    else hipLaunchKernelGGL((k_residual_gen<3, true>), grid, dim3(64), 0, s, M, P, Uh, ndof, Re, nel);
     return hipGetLastError();
 }
 
