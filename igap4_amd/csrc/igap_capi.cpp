@@ -512,11 +512,11 @@ extern "C" int igap_gpu_create(const igap_mesh_desc *mesh, const igap_phys_desc 
     M.X = c->d_X;
     gauss4(M.gq, M.gw);
     M.separable = (flags & IGAP_GENERAL_GEOMETRY) ? 0 : separable_patch(c);
-    M.equalw = std::all_of(c->w_h.begin(), c->w_h.end(), [&](double w) { return w == c->w_h[0]; });
+    M.equalw = M.separable || std::all_of(c->w_h.begin(), c->w_h.end(), [&](double w) { return w == c->w_h[0]; });
     {
         const int64_t nt = (int64_t)TAB_STRIDE * (c->nelem[0] + c->nelem[1] + c->nelem[2]);
-        TRY(dalloc(&c->d_tab, nt));
-        TRY(dalloc(&c->d_tabf, nt));
+        TRY(dalloc(&c->d_tab, nt + (nt + 1) / 2));   // the FP32 copy behind the FP64 tables
+        c->d_tabf = reinterpret_cast<float *>(c->d_tab + nt);
         for (int d = 0, first = 0; d < 3; first += c->nelem[d++]) {
             M.tab[d] = c->d_tab + (int64_t)TAB_STRIDE * first;
             M.tabf[d] = c->d_tabf + (int64_t)TAB_STRIDE * first;
@@ -572,7 +572,7 @@ extern "C" int igap_gpu_destroy(igap_gpu_ctx *c)
     if (c->stream) note(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
     for (int d = 0; d < 3; d++)
         if (c->d_knot[d]) note(hipFree(c->d_knot[d]), "hipFree");
-    void *bufs[] = {c->d_w, c->d_X, c->d_tab, c->d_tabf, c->d_Uh, c->d_R, c->d_Re, c->d_Ke[0], c->d_Ke[1], c->d_rowptr, c->d_col, c->d_pcol, c->d_val64,
+    void *bufs[] = {c->d_w, c->d_X, c->d_tab, c->d_Uh, c->d_R, c->d_Re, c->d_Ke[0], c->d_Ke[1], c->d_rowptr, c->d_col, c->d_pcol, c->d_val64,
                     c->d_val32, c->d_mask, c->d_g, c->d_F, c->d_Hd, c->d_H};
     for (void *b : bufs)
         if (b) note(hipFree(b), "hipFree");

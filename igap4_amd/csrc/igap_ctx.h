@@ -45,8 +45,8 @@ struct igap_gpu_ctx {
     // device
     double *d_knot[3] = {nullptr, nullptr, nullptr};
     double *d_w = nullptr, *d_X = nullptr;
-    double *d_tab = nullptr;        // separable patches: 1-D tables per direction and element
-    float *d_tabf = nullptr;
+    double *d_tab = nullptr;        // 1-D tables per direction and element
+    float *d_tabf = nullptr;        // their FP32 copy, in the same allocation
     double *d_Uh = nullptr, *d_R = nullptr, *d_Re = nullptr;
     void *d_Ke[2] = {nullptr, nullptr};
     int64_t *d_rowptr = nullptr;

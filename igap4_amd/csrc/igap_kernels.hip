@@ -1481,8 +1481,11 @@ __global__ __launch_bounds__((GenPipe<T>::S::THREADS), 2) void k_tangent_gen(
     if (tid >= 320 && tid < 320 + 27) {
         const int b = tid - 320, ax = ed[0] + b / 9, ay = ed[1] + (b / 3) % 3, az = ed[2] + b % 3;
         const int64_t id = ((int64_t)M.na[1] * M.na[2]) * ax + (int64_t)M.na[2] * ay + az;
+        // (relative to the element's middle point: only derivatives are used, and
+        // their rounding errors then scale with the element's size)
+        const int64_t mid = ((int64_t)M.na[1] * M.na[2]) * (ed[0] + 1) + (int64_t)M.na[2] * (ed[1] + 1) + ed[2] + 1;
 #pragma unroll
-        for (int d = 0; d < 3; d++) sC[b][d] = M.X[3 * id + d];
+        for (int d = 0; d < 3; d++) sC[b][d] = M.X[3 * id + d] - M.X[3 * mid + d];
     }
     sep_element<1, 6>(M, Uh, ed, &sC[0][3], sPd, sW);
     __syncthreads();
@@ -1927,12 +1930,15 @@ __global__ __launch_bounds__(64, 2) void k_residual_gen(MeshK M, PhysK P, const 
     if (lane < 27) {
         const int64_t id = ((int64_t)M.na[1] * M.na[2]) * (ed[0] + lane / 9) + (int64_t)M.na[2] * (ed[1] + (lane / 3) % 3) + ed[2] + lane % 3;
         const int64_t oc = wave_point(M, ed, lane);
+        // coordinates relative to the element's middle point: the jets' derivatives
+        // are the same, and their rounding errors scale with the element's size
+        const int64_t mid = ((int64_t)M.na[1] * M.na[2]) * (ed[0] + 1) + (int64_t)M.na[2] * (ed[1] + 1) + ed[2] + 1;
         const double wb = RAT ? M.w[id] : 1.0;
         double *c = sC + STR * lane;
         c[STR - 1] = wb;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
-            c[k] = wb * M.X[3 * id + k];
+            c[k] = wb * (M.X[3 * id + k] - M.X[3 * mid + k]);
             const double u0 = Uh[3 * oc + k];
             if (NH == 1) {
                 c[3 + k] = wb * u0;
