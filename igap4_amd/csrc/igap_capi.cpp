@@ -723,13 +723,18 @@ static int t_end(igap_gpu_ctx *c, int slot, int which)
 // The iterate of an assembly call, kept as U_hist[0] (src/assmcore_iga.c:68, 557).  The
 // static kernels read the caller's U, and the gather that ends the call copies
 // it (*copy) on the way, one launch less; the transient ones read all levels from
-// d_Uh, so there the copy comes first.
-static int take_iterate(igap_gpu_ctx *c, const double *U, const double **src, double **copy)
+// d_Uh, so there the copy comes first.  So it does where the gather's output
+// (nout bytes) overlaps U: its workgroups would read entries that others have
+// already written.  Only U == out of the residual is safe as it is (`same`): each
+// entry is read and written by one thread.
+static int take_iterate(igap_gpu_ctx *c, const double *U, const void *out, size_t nout, bool same, const double **src, double **copy)
 {
     *src = c->d_Uh;
     *copy = nullptr;
     if (!U || U == c->d_Uh) return IGAP_OK;
-    if (c->P.torder == 0) {
+    const uintptr_t u0 = (uintptr_t)U, o0 = (uintptr_t)out;
+    const bool overlap = u0 < o0 + nout && o0 < u0 + sizeof(double) * (size_t)c->ndof;
+    if (c->P.torder == 0 && (!overlap || (same && u0 == o0))) {
         *src = U;
         *copy = c->d_Uh;
         return IGAP_OK;
@@ -746,7 +751,7 @@ extern "C" int igap_gpu_residual(igap_gpu_ctx *c, const double *U, double *R)
     if (c->timing) HIPCHK(hipEventRecord(c->ev[2], c->stream));
     const double *U0;
     double *keep;
-    int rc = take_iterate(c, U, &U0, &keep);
+    int rc = take_iterate(c, U, R, sizeof(double) * (size_t)c->ndof, true, &U0, &keep);
     if (!rc) rc = t_begin(c, 0);
     if (rc) return rc;
     HIPCHK(launch_residual_elem(c->M, c->P, U0, c->ndof, c->d_Re, (int)c->nel, c->stream));
@@ -777,7 +782,7 @@ extern "C" int igap_gpu_residual_noalloc(igap_gpu_ctx *c, const double *U, doubl
     if (!R) R = c->d_R;
     const double *U0;
     double *keep;
-    const int rc = take_iterate(c, U, &U0, &keep);
+    const int rc = take_iterate(c, U, R, sizeof(double) * (size_t)c->ndof, true, &U0, &keep);
     if (rc) return rc;
     HIPCHK(launch_residual_elem(c->M, c->P, U0, c->ndof, scr, (int)c->nel, c->stream));
     HIPCHK(launch_residual_gather(c->M, scr, U0, keep, c->d_F, c->d_mask, c->d_g, R, c->ncp, c->stream));
@@ -835,7 +840,7 @@ extern "C" int igap_gpu_tangent(igap_gpu_ctx *c, const double *U, void *vals, in
     if (c->timing) HIPCHK(hipEventRecord(c->ev[2], c->stream));
     const double *U0;
     double *keep;
-    int rc = take_iterate(c, U, &U0, &keep);
+    int rc = take_iterate(c, U, vals, (prec == IGAP_F64 ? sizeof(double) : sizeof(float)) * (size_t)c->nnz, false, &U0, &keep);
     if (!rc) rc = t_begin(c, 0);
     if (rc) return rc;
     HIPCHK(launch_tangent_elem(c->M, c->P, U0, c->ndof, c->d_Ke[prec], prec, (int)c->nel, c->stream));
