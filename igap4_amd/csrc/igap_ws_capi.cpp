@@ -62,6 +62,8 @@ extern "C" int igap_ws_create(int device, const int grid[3], int cin, int cout, 
     const int V = (int)V64;
     const int ntile = (V + 15) / 16;
     n.nchunk = (V + W::CHUNK - 1) / W::CHUNK;
+    const size_t layer_part = sizeof(float) * 27 * (size_t)n.nchunk * 256;
+    n.part_layers = W::NL * layer_part <= (size_t)W::PART_ALL_BYTES ? W::NL : 1;
     const size_t np = (size_t)W::NL * W::LAYER_P;
     auto fail_free = [&](int rc) {
         free_net(n);
@@ -89,7 +91,7 @@ extern "C" int igap_ws_create(int device, const int grid[3], int cin, int cout, 
     WSCHK(hipMalloc(&n.y, sizeof(float) * (size_t)V * cout));
     WSCHK(hipMalloc(&n.tg, sizeof(float) * (size_t)V * cout));
     WSCHK(hipMalloc(&n.x, sizeof(float) * (size_t)V * cin));
-    WSCHK(hipMalloc(&n.part, sizeof(float) * W::NL * 27 * (size_t)n.nchunk * 256));
+    WSCHK(hipMalloc(&n.part, n.part_layers * layer_part));
     WSCHK(hipMalloc(&n.bpart, sizeof(float) * W::NL * (size_t)n.nchunk * 16));
     WSCHK(hipMalloc(&n.lpart, sizeof(float) * (size_t)ntile));
     WSCHK(hipHostMalloc(&n.hG, sizeof(float) * np + sizeof(double), hipHostMallocDefault));
@@ -176,8 +178,11 @@ static int loss_gradients(igap_ws_ctx *c, const float *x, const float *target, b
     const int rc = hidden_layers(c, x);
     if (rc) return rc;
     HIPCHK(W::conv_loss(n, n.a[W::NL - 1], n.tg, n.dz[W::NL - 1], c->stream));
-    for (int l = W::NL - 1; l >= 0; l--) HIPCHK(W::layer_back(n, l, n.a[l], n.dz[l], l > 0 ? n.dz[l - 1] : nullptr, c->stream));
-    HIPCHK(W::grad_reduce(n, to_host ? n.hG : nullptr, n.hloss, c->stream));
+    float *hG = to_host ? n.hG : nullptr;
+    for (int l = W::NL - 1; l >= 0; l--) {
+        HIPCHK(W::layer_back(n, l, n.a[l], n.dz[l], l > 0 ? n.dz[l - 1] : nullptr, c->stream));
+        if (n.part_layers == 1 || l == 0) HIPCHK(W::grad_reduce(n, l, hG, n.hloss, c->stream));
+    }
     return IGAP_OK;
 }
 
