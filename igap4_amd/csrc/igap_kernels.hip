@@ -1286,13 +1286,12 @@ __device__ __forceinline__ void sep_rows(const MeshK &M, const Scatter &S, const
     }
 }
 
-// shape of the separable tangents' pipeline (pencils per chunk, D waves, E1
-// buffers, D prefetch, deep loads) and the waves per SIMD it is compiled for
+// shape of the separable tangents' pipeline (E1 buffers, D prefetch, deep loads) and the waves per SIMD it is compiled for
 template <typename T, int NH> struct SepPipe;
-template <> struct SepPipe<double, 1> { typedef PipeShape<2, 1, 2, true, true> S; static constexpr int OCC = 2; };
-template <> struct SepPipe<float, 1> { typedef PipeShape<2, 1, 1, false, false> S; static constexpr int OCC = 4; };
-template <> struct SepPipe<double, 3> { typedef PipeShape<2, 1, 1, false, true> S; static constexpr int OCC = 2; };
-template <> struct SepPipe<float, 3> { typedef PipeShape<2, 1, 1, false, false> S; static constexpr int OCC = 4; };
+template <> struct SepPipe<double, 1> { typedef PipeShape<2, true, true> S; static constexpr int OCC = 2; };
+template <> struct SepPipe<float, 1> { typedef PipeShape<1, false, false> S; static constexpr int OCC = 4; };
+template <> struct SepPipe<double, 3> { typedef PipeShape<1, false, true> S; static constexpr int OCC = 2; };
+template <> struct SepPipe<float, 3> { typedef PipeShape<1, false, false> S; static constexpr int OCC = 4; };
 template <typename T, int NH> using SepShape = typename SepPipe<T, NH>::S;
 
 // Static tangent of a separable patch: a workgroup per element -- tables and
@@ -1358,8 +1357,8 @@ __global__ __launch_bounds__((SepShape<T, 1>::THREADS), (SepPipe<T, 1>::OCC)) vo
 // is 55k cycles an element and CU, 2.05 ms here.  A rational basis (unequal
 // weights) needs the value slot too and stays with k_tangent_elem.
 template <typename T> struct GenPipe;
-template <> struct GenPipe<double> { typedef PipeShape<2, 1, 1, false, true> S; };
-template <> struct GenPipe<float> { typedef PipeShape<2, 1, 2, false, true> S; };
+template <> struct GenPipe<double> { typedef PipeShape<1, false, true> S; };
+template <> struct GenPipe<float> { typedef PipeShape<2, false, true> S; };
 
 // the states of GeneralIn at the 64 points (eight waves; lane q of wave f < 6 holds field f's parametric jet at point q in J); ends with a block barrier
 __device__ __forceinline__ void gen_states(const MeshK &M, const PhysK &P, const int *ed, double *J, const double (*sW)[4], double *sSt)
@@ -2434,7 +2433,7 @@ hipError_t launch_tangent_direct(const MeshK &M, const PhysK &P, const double *U
     if (prec == 0) hipLaunchKernelGGL(k_fill<double>, dim3((unsigned)fb), dim3(256), 0, s, (double *)vals, 0.0, nnz);
     else hipLaunchKernelGGL(k_fill<float>, dim3((unsigned)fb), dim3(256), 0, s, (float *)vals, 0.0f, nnz);
     for (int cx = 0; cx < 3; cx++)
-        for (int cy = 0, ys = 0; cy < 3; cy++)
+        for (int cy = 0; cy < 3; cy++)
             for (int cz = 0; cz < 3; cz++) {
                 Scatter S;
                 S.rowptr = rowptr;

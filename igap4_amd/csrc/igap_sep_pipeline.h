@@ -21,25 +21,23 @@ namespace igap {
 
 // x-y part s of the jet slots, s = (dx, dy) in the order (0,0) (1,0) (0,1) (2,0) (1,1) (0,2)
 constexpr int PIPE_SX[6] = {0, 1, 0, 2, 1, 0}, PIPE_SY[6] = {0, 0, 1, 0, 1, 2};
-// LDS layout.  A D block: nine rows (slots 1..9) of ten columns in the order of
-// PIPE_COL: the two slots of the x-y parts s' = 0, 1, 2 (orders in z ascending),
-// the single ones of s' = 3 and 4, that of s' = 5 and a zero, so that a z lane
-// reads a row's entries as one aligned pair.  E1 as [pencil][block][bz][cz][s][s'],
+// LDS layout.  A D block: nine rows (slots 1..9) of ten columns (AT of d_store): the
+// two slots of the x-y parts s' = 0, 1, 2 (orders in z ascending), the single ones
+// of s' = 3 and 4, that of s' = 5 and a zero, so that a z lane reads a row's entries
+// as one aligned pair.  E1 as [pencil][block][bz][cz][s][s'],
 // the 36 values of a y lane contiguous.
 constexpr int PIPE_DR = 10, PIPE_DB = 90, PIPE_EC = 36, PIPE_EB = 326;
-constexpr int PIPE_COL[9] = {2, 4, 0, 6, 7, 3, 8, 5, 1};   // column of slot a, index a - 1
 
-// The waves of the pipeline: three y waves (wave cy, lanes (block, bz, cz)), ND
-// waves for D (2: first- and second-gradient rows apart) and 2 NP z waves, in
-// this order.  Waves four apart share a SIMD: eight waves (NP = 2, ND = 1) put a
-// z wave (250 instructions per interval in FP64) beside each y wave (260, and
-// every other time 190 more) and beside the D wave (290).
-template <int NP_, int ND_, int NE_, bool PF_, bool DEEP_>
+// The waves of the pipeline: three y waves (wave cy, lanes (block, bz, cz)), one
+// for D and four z waves, in this order.  Waves four apart share a SIMD, so that a z
+// wave (250 instructions per interval in FP64) stands beside each y wave (260, and
+// every other time 190 more) and beside the D wave (290 for StaticIn).
+template <int NE_, bool PF_, bool DEEP_>
 struct PipeShape {
-    static constexpr int NP = NP_, ND = ND_, NE = NE_;
+    static constexpr int NP = 2, NE = NE_;
     static constexpr bool PF = PF_;       // D reads its states an interval ahead
     static constexpr bool DEEP = DEEP_;   // every load of an interval before its first product
-    static constexpr int NZW = 2 * NP, WAVES = 3 + NZW + ND, THREADS = 64 * WAVES, NCH = 16 / NP;
+    static constexpr int NZW = 2 * NP, WAVES = 3 + 1 + NZW, THREADS = 64 * WAVES, NCH = 16 / NP;
     static constexpr int D_SIZE = 2 * NP * 24 * PIPE_DB, E_SIZE = NE * NP * 6 * PIPE_EB;   // entries
     // pencil (qx, qy) = 4 qx + qy of place pen in chunk ch
     static __device__ __forceinline__ int pencil(int ch, int pen) { return ch * NP + pen; }
@@ -209,23 +207,22 @@ __device__ __forceinline__ void pipe_z(const T *__restrict__ tz, const T *sD, T 
     }
 }
 
-// D role, D wave dw: lane (pencil, qz, block) of the chunk.  A chunk's state is
-// read (In::load) before the barrier that ends the interval before (PF, where
-// the registers allow it), and turned into the block's rows (part 2: all,
-// 0: the first-gradient rows, 1: the second-gradient rows) after it.
+// D role: lane (pencil, qz, block) of the chunk.  A chunk's state is read
+// (In::load) before the barrier that ends the interval before (PF, where the
+// registers allow it), and turned into the block's rows after it.
 template <typename T, class S, class In>
-__device__ __forceinline__ void pipe_d(T *sD, int dw, int lane, In in)
+__device__ __forceinline__ void pipe_d(T *sD, int lane, In in)
 {
-    const int p = lane % 6, k = blk_k(p), l = blk_l(p), qz = (lane / 6) & 3, pen = lane / 24, part = S::ND == 1 ? 2 : dw;
+    const int p = lane % 6, k = blk_k(p), l = blk_l(p), qz = (lane / 6) & 3, pen = lane / 24;
     T *Dl = sD + (pen * 24 + qz * 6 + p) * PIPE_DB;
     const bool on = lane < 24 * S::NP;
-    if (S::PF && on) in.load(S::pencil(0, pen) * 4 + qz, k, l, part);
+    if (S::PF && on) in.load(S::pencil(0, pen) * 4 + qz, k, l);
     for (int g = 0; g < S::NCH + 2; g++) {
         if (g < S::NCH && on) {
-            if (!S::PF) in.load(S::pencil(g, pen) * 4 + qz, k, l, part);
+            if (!S::PF) in.load(S::pencil(g, pen) * 4 + qz, k, l);
             __builtin_amdgcn_sched_barrier(0);
-            in.template rows<T>(k, l, part, Dl + (g & 1) * (S::NP * 24 * PIPE_DB));
-            if (S::PF && g + 1 < S::NCH) in.load(S::pencil(g + 1, pen) * 4 + qz, k, l, part);
+            in.template rows<T>(k, l, Dl + (g & 1) * (S::NP * 24 * PIPE_DB));
+            if (S::PF && g + 1 < S::NCH) in.load(S::pencil(g + 1, pen) * 4 + qz, k, l);
         }
         pipe_barrier();
         if (S::NE == 1) pipe_barrier();
@@ -239,8 +236,8 @@ __device__ __forceinline__ void sep_pipeline(const T *sX, const T *__restrict__ 
 {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     if (wave < 3) pipe_y<T, S>(sX, ty, sE, wave, lane, out);
-    else if (wave < 3 + S::ND) pipe_d<T, S>(sD, wave - 3, lane, in);
-    else pipe_z<T, S>(tz, sD, sE, wave - 3 - S::ND, lane);
+    else if (wave < 4) pipe_d<T, S>(sD, lane, in);
+    else pipe_z<T, S>(tz, sD, sE, wave - 4, lane);
 }
 
 // a row of a D block -> LDS: v[a - 1] = D[(k, row), (l, a)], a = 1..9
@@ -288,7 +285,7 @@ struct StaticIn {
     const double *sSt;
     double e345, le;
     double a[10], b[10], S[6], N[6], G[10];
-    __device__ __forceinline__ void load(int q, int k, int l, int)
+    __device__ __forceinline__ void load(int q, int k, int l)
     {
         typedef double pair_t __attribute__((ext_vector_type(2)));
         const double *st = sSt + q * SST_W;
@@ -307,7 +304,7 @@ struct StaticIn {
         get(G, SST_G, 10);
     }
     template <typename T>
-    __device__ __forceinline__ void rows(int k, int l, int part, T *dst) const
+    __device__ __forceinline__ void rows(int k, int l, T *dst) const
     {
         constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
         constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
@@ -320,34 +317,31 @@ struct StaticIn {
 #pragma unroll
             for (int j = 0; j < 3; j++) A[i][j] = Fk[i] * Fl[j];
         // first-gradient rows
-        if (part != 1) {
-            double l1[3], l0[3];   // 2 le^2 (2/3, -1/3) F_l
+        double l1[3], l0[3];   // 2 le^2 (2/3, -1/3) F_l
 #pragma unroll
-            for (int i = 0; i < 3; i++) { l1[i] = g1 * Fl[i]; l0[i] = g0 * Fl[i]; }
+        for (int i = 0; i < 3; i++) { l1[i] = g1 * Fl[i]; l0[i] = g0 * Fl[i]; }
 #pragma unroll
-            for (int L = 0; L < 3; L++) {
-                double v[9];
+        for (int L = 0; L < 3; L++) {
+            double v[9];
 #pragma unroll
-                for (int M = 0; M < 3; M++) {
-                    const double hh = Hk[SY[L][0]] * Hl[SY[M][0]] + Hk[SY[L][1]] * Hl[SY[M][1]] + Hk[SY[L][2]] * Hl[SY[M][2]];
-                    double x = N[SY[L][M]] * A[L][M] + dd * S[SY[L][M]];
-                    x += eh * (L == M ? A[(L + 1) % 3][(L + 1) % 3] + A[(L + 2) % 3][(L + 2) % 3] : A[M][L]);
-                    x += (L == M ? g1 : g0) * hh;
-                    v[M] = x;
-                }
-#pragma unroll
-                for (int s = 0; s < 6; s++) {
-                    const int I = PI[s], K = PK[s];
-                    double x = Hk[SY[L][K]] * (L == I ? l1[I] : l0[I]);
-                    if (I != K) x += Hk[SY[L][I]] * (L == K ? l1[K] : l0[K]);
-                    if (L == I) x += dd * G[3 * I + K];
-                    else if (L == K) x += dd * G[3 * K + I];
-                    v[3 + s] = x;
-                }
-                d_store<T>(dst + PIPE_DR * L, v);
+            for (int M = 0; M < 3; M++) {
+                const double hh = Hk[SY[L][0]] * Hl[SY[M][0]] + Hk[SY[L][1]] * Hl[SY[M][1]] + Hk[SY[L][2]] * Hl[SY[M][2]];
+                double x = N[SY[L][M]] * A[L][M] + dd * S[SY[L][M]];
+                x += eh * (L == M ? A[(L + 1) % 3][(L + 1) % 3] + A[(L + 2) % 3][(L + 2) % 3] : A[M][L]);
+                x += (L == M ? g1 : g0) * hh;
+                v[M] = x;
             }
+#pragma unroll
+            for (int s = 0; s < 6; s++) {
+                const int I = PI[s], K = PK[s];
+                double x = Hk[SY[L][K]] * (L == I ? l1[I] : l0[I]);
+                if (I != K) x += Hk[SY[L][I]] * (L == K ? l1[K] : l0[K]);
+                if (L == I) x += dd * G[3 * I + K];
+                else if (L == K) x += dd * G[3 * K + I];
+                v[3 + s] = x;
+            }
+            d_store<T>(dst + PIPE_DR * L, v);
         }
-        if (part == 0) return;
         // second-gradient rows
         double k1[3], k0[3], B[3][3];   // 2 le^2 (2/3, -1/3) F_k
 #pragma unroll
@@ -397,7 +391,7 @@ struct GeneralIn {
     double e345, le;
     const double *st;
     int ok, ol;
-    __device__ __forceinline__ void load(int q, int k, int l, int)
+    __device__ __forceinline__ void load(int q, int k, int l)
     {
         st = sSt + q * GST_W;
         ok = 10 * k;
@@ -435,7 +429,7 @@ struct GeneralIn {
             for (int s = 0; s < 3; s++) h[L][s] = H[SY[L][0]] * Gi[3 * s] + H[SY[L][1]] * Gi[3 * s + 1] + H[SY[L][2]] * Gi[3 * s + 2];
     }
     template <typename T>
-    __device__ __forceinline__ void rows(int k, int l, int, T *dst) const
+    __device__ __forceinline__ void rows(int k, int l, T *dst) const
     {
         constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
         constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
@@ -569,7 +563,7 @@ struct MomentIn {
     double e345, le;
     const TS *a, *b, *S, *G;   // read entry by entry: in registers they are 70
     double wgt;
-    __device__ __forceinline__ void load(int q, int k, int l, int)
+    __device__ __forceinline__ void load(int q, int k, int l)
     {
         a = sMom + q * MS_W + 18 * k;
         b = sMom + q * MS_W + 18 * l;
@@ -578,7 +572,7 @@ struct MomentIn {
         wgt = sWgt[q];
     }
     template <typename T>
-    __device__ __forceinline__ void rows(int k, int l, int part, T *dst) const
+    __device__ __forceinline__ void rows(int k, int l, T *dst) const
     {
         constexpr int PI[6] = {0, 0, 0, 1, 1, 2}, PK[6] = {0, 1, 2, 1, 2, 2};
         constexpr int SY[3][3] = {{0, 1, 2}, {1, 3, 4}, {2, 4, 5}};
@@ -593,36 +587,33 @@ struct MomentIn {
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = 0; j < 3; j++) A[i][j] = Fk(0, i) * Fl(0, j) + Fk(1, i) * Fl(1, j);
-        if (part != 1) {
-            const double eh = 0.5 * e345 * w;
+        const double eh = 0.5 * e345 * w;
 #pragma unroll
-            for (int L = 0; L < 3; L++) {
-                double v[9];
+        for (int L = 0; L < 3; L++) {
+            double v[9];
 #pragma unroll
-                for (int M = 0; M < 3; M++) {
-                    double hh = 0.0;
+            for (int M = 0; M < 3; M++) {
+                double hh = 0.0;
 #pragma unroll
-                    for (int c = 0; c < 3; c++) hh += Hk(0, SY[L][c]) * Hl(0, SY[M][c]) + Hk(1, SY[L][c]) * Hl(1, SY[M][c]);
-                    double x = (double)S[6 + SY[L][M]] * (Fk(0, L) * Fl(0, M)) + (double)S[12 + SY[L][M]] * (Fk(0, L) * Fl(1, M) + Fk(1, L) * Fl(0, M))
-                             + (double)S[18 + SY[L][M]] * (Fk(1, L) * Fl(1, M));
-                    x = w * x + dd * (double)S[SY[L][M]];
-                    x += eh * (L == M ? A[(L + 1) % 3][(L + 1) % 3] + A[(L + 2) % 3][(L + 2) % 3] : A[M][L]);
-                    x += (L == M ? g1 : g0) * hh;
-                    v[M] = x;
-                }
-#pragma unroll
-                for (int s = 0; s < 6; s++) {
-                    const int I = PI[s], K = PK[s];
-                    double x = (L == I ? g1 : g0) * (Hk(0, SY[L][K]) * Fl(0, I) + Hk(1, SY[L][K]) * Fl(1, I));
-                    if (I != K) x += (L == K ? g1 : g0) * (Hk(0, SY[L][I]) * Fl(0, K) + Hk(1, SY[L][I]) * Fl(1, K));
-                    if (L == I) x += dd * (double)G[3 * I + K];
-                    else if (L == K) x += dd * (double)G[3 * K + I];
-                    v[3 + s] = x;
-                }
-                d_store<T>(dst + PIPE_DR * L, v);
+                for (int c = 0; c < 3; c++) hh += Hk(0, SY[L][c]) * Hl(0, SY[M][c]) + Hk(1, SY[L][c]) * Hl(1, SY[M][c]);
+                double x = (double)S[6 + SY[L][M]] * (Fk(0, L) * Fl(0, M)) + (double)S[12 + SY[L][M]] * (Fk(0, L) * Fl(1, M) + Fk(1, L) * Fl(0, M))
+                         + (double)S[18 + SY[L][M]] * (Fk(1, L) * Fl(1, M));
+                x = w * x + dd * (double)S[SY[L][M]];
+                x += eh * (L == M ? A[(L + 1) % 3][(L + 1) % 3] + A[(L + 2) % 3][(L + 2) % 3] : A[M][L]);
+                x += (L == M ? g1 : g0) * hh;
+                v[M] = x;
             }
+#pragma unroll
+            for (int s = 0; s < 6; s++) {
+                const int I = PI[s], K = PK[s];
+                double x = (L == I ? g1 : g0) * (Hk(0, SY[L][K]) * Fl(0, I) + Hk(1, SY[L][K]) * Fl(1, I));
+                if (I != K) x += (L == K ? g1 : g0) * (Hk(0, SY[L][I]) * Fl(0, K) + Hk(1, SY[L][I]) * Fl(1, K));
+                if (L == I) x += dd * (double)G[3 * I + K];
+                else if (L == K) x += dd * (double)G[3 * K + I];
+                v[3 + s] = x;
+            }
+            d_store<T>(dst + PIPE_DR * L, v);
         }
-        if (part == 0) return;
         double B[3][3];
 #pragma unroll
         for (int i = 0; i < 3; i++)
