@@ -454,7 +454,7 @@ __global__ __launch_bounds__(256) void k_spmv_grid(PointGrid G, const T *__restr
     }
 }
 
-// The same with the 16-bit blocks (FP64 sums, the row scale applied once):
+// The same with the 16-bit blocks, MODE 1 or 2 (FP64 sums, the row scale applied once):
 // two points per wave, 32 lanes each, since a point's 20-byte blocks are few;
 // every load of a lane is issued before the sums.  128x32x32 (346 MB): 95 us with
 // x read per block from the caches and 64-bit index divisions, 81 us here
@@ -468,6 +468,7 @@ __global__ __launch_bounds__(256) void k_spmv_h16(PointGrid G, const uint32_t *_
     __shared__ double xs[25 * GRID_RUN];
     constexpr int LW = 32, NIT = (125 + LW - 1) / LW;   // lanes per point, rounds
     static_assert(GRID_TZ * LW == 256, "a chunk a workgroup");
+    static_assert(MODE == 1 || MODE == 2, "what the cycle takes");
     const GridChunk c(G);
     if (!c.on) return;
     const int sl = threadIdx.x & (LW - 1), slot = threadIdx.x / LW;
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(256) void k_spmv_h16(PointGrid G, const uint32_t *_
         row.finish(ch, q.p, sl, s0, s1, s2);
     } else {
         const double t = sl == 0 ? s0 : sl == 1 ? s1 : s2;
-        y[3 * q.p + sl] = MODE == 0 ? t : b[3 * q.p + sl] - t;
+        y[3 * q.p + sl] = b[3 * q.p + sl] - t;
     }
 }
 
@@ -2121,8 +2122,8 @@ static int mg_build_levels(igap_gpu_ctx *c, Solver *s, MGHier *g, int maxlev)
     return IGAP_OK;
 }
 
-// A x on multigrid level l in the preconditioner's precision (MODE of k_spmv_grid)
-static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, double *y, int mode = 0, const double *b = nullptr,
+// The product on multigrid level l in the preconditioner's precision: MODE 1 or 2 of k_spmv_grid
+static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, double *y, int mode, const double *b,
                     const Cheb &ch = Cheb())
 {
     MGLevel &L = g->lev[l];
@@ -2133,8 +2134,7 @@ static int lvl_spmv(igap_gpu_ctx *c, MGHier *g, int l, int p, const double *x, d
     if (M.periodic[0] || M.periodic[1] || M.periodic[2]) return fail(IGAP_ERR_STATE, "16-bit multigrid level on a periodic patch");
     const PointGrid G = point_grid(M);
     const dim3 gr((unsigned)((G.nblk + 7) / 8 * 8)), bs(256);
-    if (mode == 0) hipLaunchKernelGGL((k_spmv_h16<0>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
-    else if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
+    if (mode == 1) hipLaunchKernelGGL((k_spmv_h16<1>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
     else hipLaunchKernelGGL((k_spmv_h16<2>), gr, bs, 0, c->stream, G, hv, rs, x, b, y, ch);
     HIPCHK(hipGetLastError());
     return IGAP_OK;
