@@ -40,12 +40,12 @@ F_K = 64 * 9 * (2 * 10 * 10 * 27 + 2 * 10 * 27 * 27)
 F_R_STATIC = 64 * (1620 + 1620)
 # floating-point operations the sum-factorised tangent of a separable patch
 # (k_tangent_sep) executes per element in its contraction (the pointwise
-# tangent rows and the field stage come on top, as for F_K):
-#   F_q  54 rows x 64 points x (9 MUL + 27 FMA)
-#   z    108 items x 16 pencils x 108 FMA
-#   y    162 items x 16 pencils x (36 MUL + 108 FMA)
-#   x    162 items x 4 x-slabs x (27 MUL + 135 FMA)
-F_SEP = (54 * 64 * (9 + 2 * 27) + 108 * 16 * 2 * 108 + 162 * 16 * (36 + 2 * 108) + 162 * 4 * (27 + 2 * 135))
+# tangent blocks and the field stage come on top, as for F_K), lanes x
+# pencils (x: slabs) x operations a lane:
+#   z    108 x 16 x 4 x 3 x (3 MUL + 12 FMA)
+#   y    162 x 16 x 6 x (3 MUL + 12 FMA)
+#   x    162 x  4 x 9 x (3 MUL + 15 FMA)
+F_SEP = 108 * 16 * 12 * (3 + 2 * 12) + 162 * 16 * 6 * (3 + 2 * 12) + 162 * 4 * 9 * (3 + 2 * 15)
 
 
 def parse():
