@@ -136,9 +136,9 @@ def pmc_json(nel, fetch_csv, write_csv):
         # copy kernels; other copies of the run are a few bytes)
         copy = [mx for k, (_, mx) in d.items() if "copy" in k.lower() or "elementwise" in k.lower()]
         # the FP64 element tangent of the probe: the sum-factorised kernel on
-        # the (separable) beam, the general-geometry one otherwise
+        # the (separable) beam, that of any geometry with --general-geometry
         tang = [mean for k, (mean, _) in d.items() if "k_tangent_sep<double, false>" in k] or \
-               [mean for k, (mean, _) in d.items() if "k_tangent_elem<double, 1, false>" in k]
+               [mean for k, (mean, _) in d.items() if "k_tangent_gen<double, false>" in k]
         if not copy or not tang:
             raise SystemExit(f"{path}: no copy or tangent dispatch found for {name}")
         factor = max(copy) * 1024.0 / COPY_BYTES
