@@ -6,8 +6,8 @@ quadratic C1 B-spline beam (L = 4:1:1, 1,123,848 control points, 3,371,544
 dofs, 1.21G CSR nonzeros), static gradient elasticity with St Venant-Kirchhoff
 lambda = mu = 1 and strain-gradient length 0.1, clamped at x = 0 with a tip
 displacement on x = L, 4x4x4 Gauss points.  A step is one full residual
-(volume + Neumann + Dirichlet rows) plus one full tangent (element tangents on
-the matrix cores, deterministic CSR gather, MatZeroRowsColumns) in FP64, on a
+(volume + Neumann + Dirichlet rows) plus one full tangent (element tangents by
+sum factorisation, deterministic CSR gather, MatZeroRowsColumns) in FP64, on a
 smooth synthetic displacement resident in HBM.
 
 The second measure is the wall time per Newton load step of the 40-step ramp
@@ -190,9 +190,9 @@ def measured_bytes(nel, kernel):
 
 def kernel_rooflines(nel, nelem, nnz, avg, avg32, gen, gen32, genr):
     """Every assembly kernel against the ceiling that bounds it.  Tangents:
-    the counted F_K per element against the FP64 (FP32) peak -- the
-    sum-factorised kernel also with the operations it executes (F_SEP), the
-    general-geometry kernel on the matrix cores; residual: F_R per element on
+    the counted F_K per element (the block-form contraction's) against the FP64
+    (FP32) peak of the vector ALUs, on which they run -- k_tangent_sep also with
+    the operations its contraction executes (F_SEP); residual: F_R per element on
     the FP64 vector ALUs (counted flops only: basis, geometry and the
     pointwise physics come on top); gathers: the element matrices read once
     and the CSR values written once (8 or 4 bytes each), with the CSR values
@@ -338,7 +338,7 @@ def main():
         step(0)
     A.synchronize()
     t1 = time.perf_counter()
-    # ---- same with the FP32 matrix-core tangent (residual stays FP64)
+    # ---- same with the FP32 tangent (residual stays FP64)
     for _ in range(a.steps):
         step(1)
     A.synchronize()
@@ -407,7 +407,7 @@ def main():
         # achieved = the counted F_K of the element tangent per element (the
         # block-form contraction) / kernel time, against the FP64 peak; the
         # sum-factorised kernel executes F_SEP of them, so frac can pass 1
-        "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+        "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64_TFLOPS, "traffic": traffic,
                      "kernel": "k_tangent_sep<double, false>", "kernel_ms": avg[1],
                      "executed_flop_per_element": F_SEP,
@@ -464,7 +464,7 @@ def newton_load_steps(nel, timed=2, nsteps=40, tip=0.1, ramp_in=2, fp32_maxit=15
                     against linear extrapolation by residual norm; FP64
       fast          the same start, FP64 tangent, multigrid levels in FP32
                     smoothing with 16-bit copies of their matrices
-      fp32_tangent  the same start, Newton on the FP32 matrix-core tangent
+      fp32_tangent  the same start, Newton on the FP32 tangent
                     (the preconditioner as in fast), at most fp32_maxit
                     iterations
 
