@@ -683,7 +683,7 @@ def run_transient(nelem=(128, 32, 32), nsteps=200, ntrain=100, dt=1e-3, epochs=6
             hist = np.concatenate([U[k - 1], U[k - 2]])
             rq = float(np.linalg.norm(A.residual(np.concatenate([cq, hist]))))
             ratios_val.append(float(np.linalg.norm(A.residual(np.concatenate([cl, hist])))) / rq if rq > 0 else 1.0)
-    use_corr = bool(corr_on and ratios_val and np.median(ratios_val) < 1.0)
+    use_corr = bool(tr["correction_enabled"] and ratios_val and np.median(ratios_val) < 1.0)
     say(f"  held-out residual ratio learned/quadratic: "
         f"{np.median(ratios_val) if ratios_val else float('nan'):.3g}; correction {'used' if use_corr else 'off'}")
     t_train = time.perf_counter() - t0
