@@ -533,7 +533,7 @@ __device__ __forceinline__ void c_row(const double *st, const PhysK &P, int k, i
     }
 }
 
-// c_row for the general geometry's static tangent (slots 1..9, row[b - 1] = C[(k,a),(l,b)]):
+// c_row for the static tangent of rational patches, k_tangent_elem (slots 1..9, row[b - 1] = C[(k,a),(l,b)]):
 // the same entries with the lane's runtime slot indices turned into one-hot
 // vectors and the 2/3 / -1/3 coefficients into per-lane selects, so that
 // every column is straight-line arithmetic at compile-time register

@@ -4,8 +4,10 @@
 //                     (volume loop of Residual_iga, src/assmcore_iga.c:118-259)
 //   k_residual_gather deterministic per-dof sum of R_e + Neumann load +
 //                     Dirichlet rows R_d = U_d - g_d (:258, :273-497)
-//   k_tangent_elem    per-element tangents K_e[81x81] on the matrix cores
-//                     (volume loop of Tangent_iga, :607-764)
+//   k_tangent_sep, k_tangent_sep_t, k_tangent_gen, k_tangent_elem
+//                     per-element tangents K_e[81x81] (volume loop of Tangent_iga,
+//                     :607-764): separable patches, static and transient; equal weights
+//                     and any geometry, static; everything else, on the matrix cores
 //   k_tangent_gather_rows  deterministic per-nonzero sum of K_e into the CSR values
 //                     with MatZeroRowsColumns(diag=1) fused (:763, :844)
 //   k_csr_cols        column indices of the CSR pattern
@@ -1286,7 +1288,18 @@ __device__ __forceinline__ void sep_rows(const MeshK &M, const Scatter &S, const
     }
 }
 
-// shape of the separable tangents' pipeline (E1 buffers, D prefetch, deep loads) and the waves per SIMD it is compiled for
+// Shape of the separable tangents' pipeline (E1 buffers, D prefetch, loads of an
+// interval all before its first product) and the waves per SIMD it is compiled for.
+// Measured at 128x32x32 (kernel time; the same order at 64x16x16):
+//   static FP64     two buffers 9.2 ms, one 9.7 (160 KB of LDS leave one workgroup per CU
+//                   either way); without the prefetch 9.4
+//   static FP32     one buffer and two workgroups per CU (79 KB) 5.3 ms, two buffers and
+//                   one workgroup 7.6; with the prefetch 5.8; compiled for one 5.3
+//   transient FP64  one buffer is what fits (149 KB), 13.5 ms; with the prefetch 16.7
+//   transient FP32  one buffer and two workgroups per CU (76 KB) 10.9 ms, two buffers and one
+//                   workgroup 11.5, compiled for one workgroup 12.1; with the prefetch 10.2 (open)
+// The order of the loads makes no difference above 1% anywhere; it is the one that
+// the registers allow.
 template <typename T, int NH> struct SepPipe;
 template <> struct SepPipe<double, 1> { typedef PipeShape<2, true, true> S; static constexpr int OCC = 2; };
 template <> struct SepPipe<float, 1> { typedef PipeShape<1, false, false> S; static constexpr int OCC = 4; };
@@ -1297,8 +1310,10 @@ template <typename T, int NH> using SepShape = typename SepPipe<T, NH>::S;
 // Static tangent of a separable patch: a workgroup per element -- tables and
 // displacements, jets and strain-measure states of the 64 points (one pass of
 // all waves each), then the pipeline of igap_sep_pipeline.h.
-// Bound by the vector ALUs' issue: 25.6k FP64 wave instructions per element and
-// CU, 82% of the cycles of an interval.  The stages on waves of their own, D, z
+// Bound in FP64 by latency with one workgroup per CU: 16.6k vector instructions an
+// element take 41% of the issue slots of the 40.6k cycles its workgroup lives, and a wave
+// waits 44% of them, at the pipeline's barriers and the set-up's; in FP32, two
+// workgroups per CU, by vector issue, 71% of the slots.  The stages on waves of their own, D, z
 // and y/x side by side, replace a loop over pencils in which every wave ran all
 // stages with a barrier after each and the matrix cores idle, the z stage as four
 // lanes' partial sums: at 128x32x32 12.9 -> 9.1 ms in FP64 and 8.1 -> 5.3 ms in
@@ -1330,7 +1345,7 @@ __global__ __launch_bounds__((SepShape<T, 1>::THREADS), (SepPipe<T, 1>::OCC)) vo
     if (tid >= 256 && tid < 256 + 36) sX[tid - 256] = tabx[ed[0] * TAB_STRIDE + tid - 256];
     sep_element(M, Uh, ed, sU, sPd, sW);
     __syncthreads();
-    // ---- displacement jets and strain-measure states of the first element
+    // ---- displacement jets and strain-measure states
     {
         double J[10];
         sep_fields(M, ed, sU, sPd, reinterpret_cast<double *>(sE), J);
@@ -1351,11 +1366,15 @@ __global__ __launch_bounds__((SepShape<T, 1>::THREADS), (SepPipe<T, 1>::OCC)) vo
 // field in the last pass), then per point the map's inverse gradient,
 // connection and metric (one wave) and the physical displacement jets (three),
 // then the strain-measure state.
-// Bound by the SIMD that holds the D wave (870 vector instructions an interval
-// beside a z wave's 180; the y/z SIMDs have 620).  64x16x16, FP64: 3.47 ms for
+// Bound by the D wave: 1005 vector instructions an interval (849 FP64; FP32 1076 and
+// 930) in one stream, for which the other seven waves wait (62% of a wave's life,
+// 32% of the issue slots used), in both precisions.  64x16x16, FP64: 3.47 ms for
 // k_tangent_elem, whose matrix-core product of 27 x 27 per point and jet slot alone
 // is 55k cycles an element and CU, 2.05 ms here.  A rational basis (unequal
 // weights) needs the value slot too and stays with k_tangent_elem.
+// Shape as below (128x32x32, kernel): FP64 fits one E1 buffer (148 KB of LDS); FP32 two,
+// 15.5 ms, one 16.1 (two workgroups do not fit either way).  Loads all before the
+// first product: 16.1 and 15.5 ms, without 16.3 and 15.5.
 template <typename T> struct GenPipe;
 template <> struct GenPipe<double> { typedef PipeShape<1, false, true> S; };
 template <> struct GenPipe<float> { typedef PipeShape<2, false, true> S; };
@@ -1512,8 +1531,10 @@ __global__ __launch_bounds__((GenPipe<T>::S::THREADS), 2) void k_tangent_gen(
 // Um and Ud (two field passes), then the moment states of all 64 points,
 // compact and in the contraction's precision (one lane per rule node, sums
 // over 8-lane groups), so that the FP32 kernel keeps two workgroups per CU
-// (76 KB of LDS; FP64, 149 KB: one).  Bound by vector issue like the static one,
-// and by stage A (all six fields in one pass, a lane per rule node and point, sums by
+// (76 KB of LDS; FP64, 149 KB: one).  Bound by latency: a wave waits 46% of its life in
+// FP64 (44% of the issue slots used) and 64% in FP32 (58% used; 62 registers spilled),
+// for the D wave (534 vector instructions an interval, 363 FP64; FP32 688 and 490) and
+// in stage A (all six fields in one pass, a lane per rule node and point, sums by
 // lane moves; as two passes, two rounds of half the waves and LDS permutations it took
 // 13.5 ms at 128x32x32 in FP32, 10.9 now; FP64 at 24^3 1.78 -> 1.48 ms).  Two
 // pencils per interval and one D wave: one pencil and two D waves took 18.8 ms,
@@ -1675,9 +1696,12 @@ __global__ __launch_bounds__((SepShape<T, 3>::THREADS), (SepPipe<T, 3>::OCC)) vo
 // A wave per element: every pass fits 64 lanes component by component (36, 48 and 64
 // of them for z, y, x; 48, 36 and 27 back), the jets of a lane's point stay in
 // its registers, and nothing waits at a block barrier.  10 KB of LDS an element,
-// so at 156 registers (128 spill 38) 12 elements are in flight per CU.  At 64x16x16 120 -> 79 us (one
-// call), at 16x4x4 9.2 -> 7.9 us, against a workgroup of four waves per element with
-// six in flight per CU and the pointwise stage on one of the waves.
+// so at 156 registers (128 spill 38) 12 elements are in flight per CU, whose LDS
+// instructions (313 a wave) fill the CU's LDS pipe: that is the bound, a wave waits on
+// it 43% of its life.  A whole residual call at 64x16x16, with its gather and back to
+// back, 123 -> 67.6 us (this kernel alone 79 us in a kernel trace, where the write-back of each
+// dispatch counts); at 16x4x4 9.2 -> 7.1 us, against a workgroup of four waves per element
+// with six in flight per CU and the pointwise stage on one of the waves.
 __device__ __forceinline__ void wave_sync()
 {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1911,8 +1935,11 @@ __global__ __launch_bounds__(64, 2) void k_residual_sep_t(MeshK M, PhysK P, cons
 // through the transposes of both rules (phys_jet_adj, nurbs_param_adj) into
 // wave_project:
 //   R_e[b][k] = w_b sum_q (Q_q^T Phi_q^T w_q r_q[k]) . N_b(q).
-// 64x16x16 distorted beam 282 -> 150 us, 45x23x17 rational 303 -> 265 us (134 registers
-// spilled), whole residual calls at 23x9x14: static 77 -> 39 us (rational 56), transient 155 ->
+// Bound by the traffic of its spilled registers (70 static, 134 rational, 118 and 141
+// transient, at 256 registers): at 256x64x64 33 GB in 8.0 ms, 4.2 TB/s, for 0.7 GB of
+// element vectors, and a wave waits 50 to 67% of its life.
+// 64x16x16 distorted beam 282 -> 148 us, 45x23x17 rational 303 -> 248 us, whole
+// residual calls at 23x9x14: static 77 -> 39 us (rational 56), transient 155 ->
 // 84 us (89), against a workgroup of four waves per element and eight block barriers.
 template <int NH, bool RAT>
 __global__ __launch_bounds__(64, 2) void k_residual_gen(MeshK M, PhysK P, const double *__restrict__ Uh, int64_t ndof,

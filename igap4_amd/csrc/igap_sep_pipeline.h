@@ -30,8 +30,9 @@ constexpr int PIPE_DR = 10, PIPE_DB = 90, PIPE_EC = 36, PIPE_EB = 326;
 
 // The waves of the pipeline: three y waves (wave cy, lanes (block, bz, cz)), one
 // for D and four z waves, in this order.  Waves four apart share a SIMD, so that a z
-// wave (250 instructions per interval in FP64) stands beside each y wave (260, and
-// every other time 190 more) and beside the D wave (290 for StaticIn).
+// wave (267 vector instructions per interval in k_tangent_sep<double>) stands beside
+// each y wave (the contraction's 180 FMAs and products, every other time 162 more,
+// and their addresses) and beside the D wave (317; transient 534, any geometry 1005).
 template <int NE_, bool PF_, bool DEEP_>
 struct PipeShape {
     static constexpr int NP = 2, NE = NE_;
@@ -379,7 +380,7 @@ struct StaticIn {
 //   h^k_Ls = sum_K H_kLK Gi_sK,  m_rs = sum_K Gi_rK Gi_sK,  B_rn = sum_L a'^k_Lr a^l_nL
 // the second-second entry of ((r, s), (n, m)) is B_rn m_sm, symmetrised, the
 // physical-first one of (M, (r, s)) is a'_Mr h_Ms, symmetrised, and only the
-// connection is left to apply: 860 FMAs per block against 1300 for pulling back the
+// connection is left to apply: 850 FP64 instructions per block against 1300 for pulling back the
 // physical block.  State layout (16-byte pairs; the stride of 94 puts the eight
 // points of a chunk on different banks): per component k at 10 k F (3), a gap, H
 // (6); times the point weight S at 30, N at 36 (6 each) and at 42 + 6 L

@@ -1,5 +1,5 @@
 """FP32 tangent against FP64 tangent in Newton's method: how far the inexact
-Jacobian of the FP32 matrix-core tangent lets Newton converge at each patch
+Jacobian of the FP32 tangent lets Newton converge at each patch
 size.  The reference's solve is one SNES iteration per sub-iteration
 (src/interface.c:302-328); this driver calls the device Newton one
 iteration at a time the same way and records the history.
@@ -20,7 +20,7 @@ from .warmstart import LearnedGuess
 def study(nel, nsteps=40, tip=0.1, k=4, iters=6):
     """Load step k of the clamped-tip ramp (tip ``tip`` in ``nsteps`` steps)
     from the quadratic extrapolation of the converged steps before it,
-    ``iters`` Newton iterations with the FP64 and with the FP32 matrix-core
+    ``iters`` Newton iterations with the FP64 and with the FP32
     tangent (FP64 residual and update, FP32 multigrid preconditioner, GMRES
     to 1e-8): per iteration the residual over the first residual of the
     reference's iteration and the displacement error against the FP64

@@ -2,7 +2,7 @@
 
   transient  gradelasttime on an L = 4:1:1 beam (default 128x32x32 elements),
              zero displacement and the 8-mode seeded initial velocity, time
-             steps with history shift, FP32 or FP64 matrix-core tangent,
+             steps with history shift, FP32 or FP64 tangent,
              FP64 residual and Krylov
   ramp       static SVK + strain-gradient beam, clamped at x = 0 with a tip
              displacement ramped over load steps (the load-step workloads)

@@ -106,13 +106,14 @@ int igap_mesh_igabeam(const double L[3], const int nelem[3], const int periodic[
  *   IGAP_TANGENT_DIRECT            the element kernel adds its matrix into the
  *       CSR values, one launch per class of the 27-colouring (the elements of
  *       one class share no control point); non-periodic patches only
- * Element kernels of the static physics: on a separable patch -- every
+ * Element kernels: on a separable patch -- every
  * control coordinate x_d depends on the control point's index along d alone
  * and all weights are equal, as on the igabeam patches -- the residual and
  * the element tangents (either way to the CSR values) come from
  * sum-factorised kernels over 1-D tables of physical derivatives; otherwise,
- * and with the flag below, from the general-geometry kernels.  Both give the
- * same values up to rounding.
+ * and with the flag below, from the general-geometry kernels (the static tangent
+ * of equal weights by sum factorisation over parametric tables, other tangents on
+ * the matrix cores).  All give the same values up to rounding.
  *   IGAP_GENERAL_GEOMETRY          the general-geometry kernels on every patch */
 enum { IGAP_TANGENT_ELEMENT_MATRICES = 1, IGAP_TANGENT_DIRECT = 2, IGAP_GENERAL_GEOMETRY = 4 };
 
@@ -190,7 +191,7 @@ double *igap_gpu_rvec(igap_gpu_ctx *ctx);
 /* Tangent_iga: copies U into U_hist level 0 (U may be NULL to use U_hist as
  * it is), zeroes the values, assembles the volume tangent deterministically
  * and applies MatZeroRowsColumns(diag = 1) to the Dirichlet rows.
- * prec = IGAP_F64 writes vals as double, IGAP_F32 as float (FP32 MFMA);
+ * prec = IGAP_F64 writes vals as double, IGAP_F32 as float (contraction in FP32);
  * vals may be NULL for the context's own arrays. */
 int igap_gpu_tangent(igap_gpu_ctx *ctx, const double *U, void *vals, int prec);
 /* MatMult (PETSc's) on the tangent IGAP4 assembles into assm->TT
@@ -239,7 +240,7 @@ typedef struct {
     int    ksp_maxit;     /* Krylov iterations per Newton step                              */
     int    ksp_restart;   /* GMRES restart (reference 10000; bounded to fit HBM)            */
     int    pc;            /* IGAP_PC_ILU0 (the reference's ASM/ILU(0) on one part), ...     */
-    int    tangent_prec;  /* IGAP_F64 or IGAP_F32 (FP32 matrix-core tangent, FP32 ILU)      */
+    int    tangent_prec;  /* IGAP_F64 or IGAP_F32 (FP32 tangent, FP32 ILU)                  */
     int    linesearch;    /* 1: backtracking (SNESLINESEARCHBT, cubic), 0: full steps       */
     int    pc_order;      /* ILU(0) ordering: 0 natural dof order (the reference's), 1     */
                           /* 27 colours of control points (colour 9(i%3)+3(j%3)+k%3, the   */
